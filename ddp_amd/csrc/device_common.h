@@ -316,3 +316,67 @@ __device__ __forceinline__ bool grid_barrier(uint32_t *bar, uint32_t nblocks, ui
     __syncthreads();
     return *s_flag != 0;
 }
+
+// Grid barrier without cache maintenance, for kernels whose workgroups share
+// data only through agent-scope atomics (loads and stores included: ld_gp,
+// ld_u32, st_u64, ...): those go past L1 and are kept coherent between the
+// XCDs' L2s, so a wave's vmcnt(0) is all the release that is needed and a
+// relaxed poll all the acquire.  The fences of grid_barrier (an L2 write-back
+// and invalidate by every workgroup) were most of its cost: 1.9 us with 16
+// workgroups of 64, 4.0 with 64, 14.4 with 256, 28.6 with 512, against 1.4,
+// 1.9, 4.0 and 6.9 us here.  Beyond 64 workgroups the arrivals, which one
+// counter takes at about 11 ns each, are counted in eight groups first (a
+// second dependent round trip, 0.45 us): 2.3 us with 128, 2.6 with 256, 3.0
+// with 512; with 64 and fewer one counter is faster (64: 1.9 against 2.2 us).
+// bar: GRID_SYNC_WORDS zeroed words, a 128-byte line per counter.  Waits are
+// bounded by limit_ticks of the 100 MHz clock; false if one ran out.
+constexpr uint32_t GRID_SYNC_WORDS = 32 * 10;
+
+__device__ __forceinline__ uint32_t add_u32(uint32_t *p, uint32_t v)
+{
+    return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_u64(uint64_t *p, uint64_t v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ bool grid_sync(uint32_t *bar, uint32_t nblocks, uint32_t &gen, uint64_t limit_ticks,
+                                          int32_t *s_flag)
+{
+    block_sync_global();
+    if (threadIdx.x == 0) {
+        constexpr uint32_t kGroups = 8;
+        bool ok = true, last;
+        if (nblocks <= 64) {
+            last = add_u32(bar, 1u) == nblocks - 1;
+        } else {
+            const uint32_t g = blockIdx.x % kGroups, members = (nblocks - g + kGroups - 1) / kGroups;
+            uint32_t *grp = bar + 32 * (2 + g);
+            last = add_u32(grp, 1u) == members - 1;
+            if (last) {
+                st_u32(grp, 0u);
+                wait_vmem();
+                last = add_u32(bar, 1u) == kGroups - 1;
+            }
+        }
+        if (last) {
+            st_u32(bar, 0u);
+            wait_vmem();  // the counters are clear before anyone can arrive again
+            st_u32(bar + 32, gen + 1);
+        } else {
+            const uint64_t t0 = dev_clock_100mhz();
+            while (ld_u32(bar + 32) == gen) {
+                __builtin_amdgcn_s_sleep(1);
+                if (dev_clock_100mhz() - t0 > limit_ticks) {
+                    ok = false;
+                    break;
+                }
+            }
+        }
+        *s_flag = ok ? 1 : 0;
+    }
+    gen += 1;
+    __syncthreads();
+    return *s_flag != 0;
+}

@@ -146,9 +146,10 @@ int ddp_bfs_hops(ddp_ctx *ctx, ddp_graph *g, int32_t t, int32_t reverse,
 /* No reference counterpart.  ddp_bfs_hops for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): it calls no hipMalloc/hipFree.  Its
- * distance array, frontier buffers and control words live in a static device
- * array of 12 bytes per node for at most 2,097,152 nodes (24 MiB, held by
- * every GPU the library runs on until the process ends); a larger graph gets
+ * distance array, queue and control words live in a static device array for
+ * at most 2,097,152 nodes (26 MiB: 12 bytes per node and 2 MiB for the parts of
+ * long rows; held by every GPU the library runs on until the process ends); a
+ * larger graph gets
  * DDP_ERR_CAPACITY.  h_out_dev: N int32 in DEVICE memory the caller owns,
  * written in the caller's node numbering (hops x scale, -1 = not reached).
  * No store_as_h.  All calls on one GPU share that array, so calls that
