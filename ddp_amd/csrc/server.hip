@@ -84,6 +84,7 @@ enum : int {
     CT_HEAD = 0, CT_TAIL = 16, CT_APPLIED = 32, CT_POLL = 48, CT_ERR = 64, CT_STOP = 80, CT_BUSY = 96, CT_WORDS = 112
 };
 constexpr uint32_t kClosed = 0x80000000u;
+constexpr int kLeftWord = 16, kFlagWords = 32;  // pinned flag words: [0] tail, [1] stop, [kLeftWord] left (a line of its own)
 
 struct ServeArgs {
     GraphView g;           // base rows + versioned view fields (ver set per query)
@@ -105,10 +106,12 @@ struct ServeArgs {
     int32_t *rltail;
     int32_t log_cap;
     const Req *ring;       // pinned
+    Req *mirror;           // device copy of the published entries (the poller's)
     Res *res;              // pinned
     const int32_t *arena;  // pinned update payloads
     const uint32_t *tail;  // pinned: requests published
     const uint32_t *stop;  // pinned
+    uint32_t *left;        // pinned: newest launch that has begun to leave
     uint32_t ring_mask;
     uint32_t *ctrl;        // device: claimed count, applied version
     uint64_t *gp;
@@ -129,63 +132,107 @@ __device__ __forceinline__ int32_t sys_ld_i(const int32_t *p)
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// What an update writes is read by slots on other XCDs: everything goes
+// through agent-scope atomics or stores, which a wave's vmcnt(0) publishes, so
+// no L2 write-back is needed before the version is published.  The payload is
+// read over the host link, about 2 us a round trip: a lane asks for all it may
+// need at once.  A row is scanned in groups of 8 loads issued together.
 template <int B, bool BIDI>
 __device__ void apply_update(const ServeArgs &a, const Req &rq, uint32_t *s_err)
 {
     const int32_t V = rq.version;
     const int lane = threadIdx.x;
+    struct Ins {
+        int32_t u, v, w, x, before, after;
+    };
+    auto load_ins = [&](int32_t i) {
+        Ins r{-1, -1, 0, -1, -1, -1};
+        if (i < rq.ins_n) {
+            const int32_t *q = a.arena + rq.ins_off + 4 * i;
+            r.u = sys_ld_i(q);
+            r.v = sys_ld_i(q + 1);
+            r.w = sys_ld_i(q + 2);
+            r.x = sys_ld_i(q + 3);
+            if (i > 0) r.before = sys_ld_i(q - 4);
+            if (i + 1 < rq.ins_n) r.after = sys_ld_i(q + 4);
+        }
+        return r;
+    };
+    Ins in = load_ins(lane);  // under way while the deletes are applied
     // deletes: first instance still live at V-1 (its delete word is INF)
     for (int32_t i = lane; i < rq.del_n; i += B) {
         const int32_t u = sys_ld_i(a.arena + rq.del_off + 2 * i), v = sys_ld_i(a.arena + rq.del_off + 2 * i + 1);
         if (u < 0 || u >= a.N || v < 0 || v >= a.N) continue;
-        bool done = false;
-        for (int32_t j = a.g.off[u]; j < a.g.off[u + 1] && !done; ++j)
-            if (a.g.col[j] == v && atomicCAS(a.dver + j, INT32_MAX, V) == INT32_MAX) {
-                done = true;
-                if constexpr (BIDI)  // the same edge in v's transposed row
-                    for (int32_t r = a.gr.off[v]; r < a.gr.off[v + 1]; ++r)
-                        if (a.reid[r] == j) {
-                            a.rdver[r] = V;
-                            break;
-                        }
-            }
+        constexpr int kG = 8;
+        const int32_t rb = a.g.off[u], re = a.g.off[u + 1];
         uint64_t link = __hip_atomic_load(a.lhead + u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        int32_t hit = -1;
+        for (int32_t j0 = rb; j0 < re && hit < 0; j0 += kG) {
+            int32_t c[kG];
+#pragma unroll
+            for (int k = 0; k < kG; ++k) c[k] = j0 + k < re ? a.g.col[j0 + k] : -1;
+#pragma unroll
+            for (int k = 0; k < kG; ++k)
+                if (hit < 0 && c[k] == v && atomicCAS(a.dver + j0 + k, INT32_MAX, V) == INT32_MAX) hit = j0 + k;
+        }
+        if constexpr (BIDI)  // the same edge in v's transposed row
+            if (hit >= 0)
+                for (int32_t r = a.gr.off[v]; r < a.gr.off[v + 1]; ++r)
+                    if (a.reid[r] == hit) {
+                        st_u32((uint32_t *)a.rdver + r, (uint32_t)V);
+                        break;
+                    }
+        bool done = hit >= 0;
         while (!done && (uint32_t)link < (uint32_t)V) {
             const int32_t x = (int32_t)(link >> 32);
             link = __hip_atomic_load(a.lnext + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (a.lv[x] == v && atomicCAS(a.ldel + x, INT32_MAX, V) == INT32_MAX) done = true;
+            if ((int32_t)ld_u32((const uint32_t *)a.lv + x) == v && atomicCAS(a.ldel + x, INT32_MAX, V) == INT32_MAX) done = true;
         }
     }
     block_sync_global();
-    // inserts: one lane per source (entries arrive sorted by source, entry ids
-    // assigned by the host in arrival order)
+    // inserts (sorted by source, entry ids assigned by the host in arrival
+    // order): every lane fills its own log entry, and the first lane of each
+    // source's group links the group
     for (int32_t i = lane; i < rq.ins_n; i += B) {
-        const int32_t *q = a.arena + rq.ins_off + 4 * i;
-        const int32_t u = sys_ld_i(q);
-        if (i > 0 && sys_ld_i(q - 4) == u) continue;  // not the first of its source's group
-        for (int32_t k = i; k < rq.ins_n; ++k) {
-            const int32_t *e = a.arena + rq.ins_off + 4 * k;
-            if (sys_ld_i(e) != u) break;
-            const int32_t v = sys_ld_i(e + 1), x = sys_ld_i(e + 3);
-            const uint32_t w = (uint32_t)sys_ld_i(e + 2);
-            if (u < 0 || u >= a.N || v < 0 || v >= a.N || x < 0 || x >= a.log_cap) {
-                atomicOr(s_err, (uint32_t)SERR_LOG);
-                continue;
-            }
-            a.lv[x] = v;
-            a.lw[x] = w;
-            a.ldel[x] = INT32_MAX;
-            a.lnext[x] = ~0ull;
+        if (i != lane) in = load_ins(i);
+        const int32_t u = in.u, v = in.v, w = in.w, before = in.before;
+        int32_t x = in.x, after = in.after;
+        auto valid = [&](int32_t vv, int32_t xx) {
+            return u >= 0 && u < a.N && vv >= 0 && vv < a.N && xx >= 0 && xx < a.log_cap;
+        };
+        bool ok = valid(v, x);
+        if (ok) {
+            st_u32((uint32_t *)a.lv + x, (uint32_t)v);
+            st_u32(a.lw + x, (uint32_t)w);
+            st_u32((uint32_t *)a.ldel + x, (uint32_t)INT32_MAX);
             if constexpr (BIDI) {
-                a.lu[x] = u;
-                a.rlnext[x] = ~0ull;
+                st_u32((uint32_t *)a.lu + x, (uint32_t)u);
+                st_u64(a.rlnext + x, ~0ull);
             }
-            const uint64_t link = ((uint64_t)(uint32_t)x << 32) | (uint32_t)V;
-            const int32_t last = a.ltail[u];
-            if (last < 0) a.lhead[u] = link;
-            else a.lnext[last] = link;
-            a.ltail[u] = x;
+        } else {
+            atomicOr(s_err, (uint32_t)SERR_LOG);
         }
+        if (i > 0 && before == u) continue;  // not the first of its source's group
+        bool linked = false;
+        int32_t last = -1;
+        for (int32_t k = i;;) {
+            if (ok) {
+                if (!linked) last = (int32_t)ld_u32((const uint32_t *)a.ltail + u);
+                const uint64_t link = ((uint64_t)(uint32_t)x << 32) | (uint32_t)V;
+                st_u64(a.lnext + x, ~0ull);
+                st_u64(last < 0 ? a.lhead + u : a.lnext + last, link);
+                last = x;
+                linked = true;
+            }
+            if (k + 1 >= rq.ins_n || after != u) break;
+            ++k;
+            const int32_t *e = a.arena + rq.ins_off + 4 * k;
+            const int32_t vk = sys_ld_i(e + 1);
+            x = sys_ld_i(e + 3);
+            after = k + 1 < rq.ins_n ? sys_ld_i(e + 4) : -1;
+            ok = valid(vk, x);  // flagged by its own lane if not
+        }
+        if (linked) st_u32((uint32_t *)a.ltail + u, (uint32_t)last);
     }
     block_sync_global();
     if constexpr (BIDI) {
@@ -202,14 +249,141 @@ __device__ void apply_update(const ServeArgs &a, const Req &rq, uint32_t *s_err)
                 const int32_t x = sys_ld_i(e + 1);
                 if (x < 0 || x >= a.log_cap) continue;
                 const uint64_t link = ((uint64_t)(uint32_t)x << 32) | (uint32_t)V;
-                const int32_t last = a.rltail[v];
-                if (last < 0) a.rlhead[v] = link;
-                else a.rlnext[last] = link;
-                a.rltail[v] = x;
+                const int32_t last = (int32_t)ld_u32((const uint32_t *)a.rltail + v);
+                st_u64(last < 0 ? a.rlhead + v : a.rlnext + last, link);
+                st_u32((uint32_t *)a.rltail + v, (uint32_t)x);
             }
         }
         block_sync_global();
     }
+}
+
+// Claims the next published request for this workgroup (wave 0, every lane
+// active; bounded idle wait); false: the workgroup leaves.
+//
+// Idle slots watch device words only.  One of them at a time holds the poller
+// lease: it reads the host's published count and stop word with relaxed
+// system-scope loads, copies newly published entries (one per lane, six 8-byte
+// loads in flight) into the device mirror of the ring, and only then raises
+// the device's published count.  So a claim costs device round trips (about
+// 0.5 us each) and neither host reads nor system-scope cache invalidations,
+// which it took per claim while entries were read from host memory: a burst of
+// 1,024 requests, every twentieth an update batch, on a 200,000-node map took
+// 62 ms, one claim every 60 us; it takes 13 ms now (5 ms without updates, 3 of
+// them its longest query).
+//
+// A slot counts itself busy once it has claimed, and the launch closes (every
+// slot leaves) only by swapping a busy count of zero for kClosed after an idle
+// time: slots do not leave one by one while others still run, which would
+// strand later requests behind fewer slots until the last running one finished
+// and the host could relaunch.  (A claim that crosses the closing serves its
+// request and leaves then.  Counting before the claim kept the two apart, but
+// every failed attempt of a burst then cost two more atomics on one counter.)
+//
+// The next request is claimed only once the graph version it needs is applied
+// (entries handled by kernels of their own are skipped at once), so no slot
+// holds a claim while it waits: the version may come from an update kernel
+// queued behind this launch, which a stop or an idle close then lets run.  A
+// launch stopped for such an entry (its stop_gen) claims nothing from there
+// on: requests published after it run after its kernels, in the next launch,
+// instead of keeping this one alive while that entry's kernels wait behind it.
+__device__ __forceinline__ bool serve_claim(const ServeArgs &a, uint32_t &ticket)
+{
+    const uint32_t lane = threadIdx.x;
+    constexpr int kWords = sizeof(Req) / 8;
+    static_assert(sizeof(Req) % 8 == 0, "entries are copied as 8-byte words");
+    const uint64_t t0 = dev_clock_100mhz();
+    bool poller = false, have = false;
+    int backoff = 0;  // idle non-pollers back off to ~15 us
+    uint32_t contended = 0;
+    for (;;) {
+        const uint32_t h = __builtin_amdgcn_readfirstlane(ld_u32(a.ctrl + CT_HEAD));
+        const uint32_t tail = __builtin_amdgcn_readfirstlane(ld_u32(a.ctrl + CT_TAIL));
+        const uint32_t bw = __builtin_amdgcn_readfirstlane(ld_u32(a.ctrl + CT_BUSY));
+        const uint32_t applied = __builtin_amdgcn_readfirstlane(ld_u32(a.ctrl + CT_APPLIED));
+        if (bw & kClosed) break;
+        const bool waiting = (int32_t)(tail - h) > 0;
+        if (waiting) {
+            // a stale h reads an entry that its failed claim below ignores
+            const uint32_t *e = (const uint32_t *)(a.mirror + (h & a.ring_mask));
+            const uint32_t type = ld_u32(e + offsetof(Req, type) / 4), ver = ld_u32(e + offsetof(Req, version) / 4),
+                           direct = ld_u32(e + offsetof(Req, direct) / 4),
+                           stop_gen = ld_u32(e + offsetof(Req, stop_gen) / 4);
+            const bool d = __builtin_amdgcn_readfirstlane(direct) != 0;
+            // this launch was stopped for this entry: what follows it starts
+            // after the entry's own kernels, in a later launch
+            if (d && __builtin_amdgcn_readfirstlane(stop_gen) == a.gen) break;
+            const uint32_t v = __builtin_amdgcn_readfirstlane(ver);
+            const uint32_t need = __builtin_amdgcn_readfirstlane(type) == DDP_REQ_UPDATE ? v - 1 : v;
+            if (d || applied >= need) {
+                uint32_t got = 0;
+                if (lane == 0) {
+                    got = atomicCAS(a.ctrl + CT_HEAD, h, h + 1) == h;
+                    if (got) add_u32(a.ctrl + CT_BUSY, 1u);
+                }
+                if (__builtin_amdgcn_readfirstlane(got)) {
+                    ticket = h;
+                    have = true;
+                    break;
+                }
+                // A burst has every idle slot here, and the counter serves one
+                // attempt per 11 ns or so: waits that double with each failure,
+                // spread over the slots, keep it from serving only failures.
+                contended = contended < 7 ? contended + 1 : 7;
+                const uint32_t spread = (blockIdx.x * 2654435761u + h * 40503u) >> 25 & ((1u << contended) - 1);
+                for (uint32_t k = 0; k < spread; ++k) __builtin_amdgcn_s_sleep(1);
+                continue;
+            }
+        }
+        if ((int32_t)(__builtin_amdgcn_readfirstlane(ld_u32(a.ctrl + CT_STOP)) - a.gen) >= 0) break;
+        uint32_t won = 0;
+        if (lane == 0) {
+            if (dev_clock_100mhz() - t0 > a.idle_ticks && bw == 0 && atomicCAS(a.ctrl + CT_BUSY, 0u, kClosed) == 0u)
+                won = 2;
+            else if (!poller) won = atomicCAS(a.ctrl + CT_POLL, 0u, 1u) == 0u;
+        }
+        won = __builtin_amdgcn_readfirstlane(won);
+        if (won == 2) break;
+        poller = poller || won == 1;
+        if (poller) {
+            // the lease holder is the only writer of the tail copy and the mirror
+            const uint32_t from = __builtin_amdgcn_readfirstlane(ld_u32(a.ctrl + CT_TAIL));
+            const uint32_t ht =
+                __builtin_amdgcn_readfirstlane(__hip_atomic_load(a.tail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
+            const uint32_t sg =
+                __builtin_amdgcn_readfirstlane(__hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
+            if ((int32_t)(ht - from) > 0) {
+                // entries were written before the published count; host memory is
+                // not cached here, so the loads only have to come after the count's
+                __atomic_signal_fence(__ATOMIC_ACQUIRE);
+                const uint32_t fresh = ht - from < 64 ? ht - from : 64;
+                if (lane < fresh) {
+                    const uint64_t *src = (const uint64_t *)(a.ring + ((from + lane) & a.ring_mask));
+                    uint64_t *dst = (uint64_t *)(a.mirror + ((from + lane) & a.ring_mask));
+                    uint64_t word[kWords];
+#pragma unroll
+                    for (int k = 0; k < kWords; ++k)
+                        word[k] = __hip_atomic_load(src + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+#pragma unroll
+                    for (int k = 0; k < kWords; ++k) st_u64(dst + k, word[k]);
+                }
+                wait_vmem();
+                if (lane == 0) st_u32(a.ctrl + CT_TAIL, from + fresh);
+                wait_vmem();
+            } else {
+                if ((int32_t)(sg - a.gen) >= 0 && lane == 0) atomicExch(a.ctrl + CT_STOP, sg);
+                __builtin_amdgcn_s_sleep(16);
+            }
+        } else {
+            // waiting for a version, which comes within tens of microseconds: 1.7 us
+            // between looks (0.2 us kept the words they look at so busy that the
+            // update itself took twice as long)
+            backoff = waiting ? 1 : backoff < 8 ? backoff + 1 : 8;
+            for (int k = 0; k < backoff; ++k) __builtin_amdgcn_s_sleep(64);
+        }
+    }
+    if (poller && lane == 0) atomicExch(a.ctrl + CT_POLL, 0u);
+    return have;
 }
 
 template <int B, int HK, int ENG>
@@ -221,6 +395,7 @@ __global__ void __launch_bounds__(B) serve_kernel(ServeArgs a)
     __shared__ uint32_t s_ticket;
     __shared__ int32_t s_have;
     __shared__ uint32_t s_uerr;
+    __shared__ Req s_req;
     const int lane = threadIdx.x;
     const int64_t slot = blockIdx.x;
     const int32_t N = a.N;
@@ -232,115 +407,39 @@ __global__ void __launch_bounds__(B) serve_kernel(ServeArgs a)
     const PilePtrs P{home, home + a.ncap, home + a.ncap + a.fcap, a.ncap, a.fcap, s_heap, a.lring};
     ExpandCounters C;
     uint32_t stale = 0;
+    uint32_t seen = 0;  // newest version whose graph data this workgroup has acquired
+    bool any_seen = false;
     for (;;) {
-        // ---- claim the next published request (bounded idle wait).  Idle
-        // slots watch device words only; one of them at a time holds the
-        // poller lease and copies the host's published count (and the stop
-        // flag) into them with plain relaxed loads of host memory, so idle
-        // slots neither flood the host link nor invalidate caches that the
-        // running searches depend on.
-        //
-        // A slot counts itself busy before it claims, and the launch closes
-        // (every slot leaves) only by swapping a busy count of zero for
-        // kClosed: slots never leave one by one while others still run, which
-        // would strand later requests behind fewer slots until the last
-        // running one finished and the host could relaunch.
-        //
-        // The next request is claimed only once the graph version it needs is
-        // applied (entries handled by kernels of their own are skipped at
-        // once), so no slot holds a claim while it waits: the version may come
-        // from an update kernel queued behind this launch, which a stop or an
-        // idle close then lets run.  A launch stopped for such an entry (its
-        // stop_gen) claims nothing from there on: requests published after it
-        // run after its kernels, in the next launch, instead of keeping this
-        // one alive while that entry's kernels wait behind it.
-        if (lane == 0) {
+        if (threadIdx.x < 64) {
             uint32_t ticket = 0;
-            bool have = false;
-            const uint64_t t0 = dev_clock_100mhz();
-            bool poller = false;
-            int backoff = 0;  // non-pollers back off to ~15 us
-            for (;;) {
-                const uint32_t h = ld_u32(a.ctrl + CT_HEAD);
-                const uint32_t tail = ld_u32(a.ctrl + CT_TAIL);
-                const uint32_t bw = ld_u32(a.ctrl + CT_BUSY);
-                if (bw & kClosed) break;
-                bool ready = false;
-                if ((int32_t)(tail - h) > 0) {
-                    // a stale h reads an entry that its failed claim below ignores
-                    __atomic_thread_fence(__ATOMIC_ACQUIRE);
-                    const Req *hp = a.ring + (h & a.ring_mask);
-                    ready = sys_ld_i(&hp->direct) != 0;
-                    // this launch was stopped for this entry: what follows it
-                    // starts after the entry's own kernels, in a later launch
-                    if (ready && (uint32_t)sys_ld_i(&hp->stop_gen) == a.gen) break;
-                    if (!ready) {
-                        const int32_t ver = sys_ld_i(&hp->version);
-                        const uint32_t need =
-                            sys_ld_i(&hp->type) == DDP_REQ_UPDATE ? (uint32_t)ver - 1 : (uint32_t)ver;
-                        ready = __hip_atomic_load(a.ctrl + CT_APPLIED, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) >=
-                                need;
-                    }
-                }
-                if (ready) {
-                    if (atomicCAS(a.ctrl + CT_BUSY, bw, bw + 1) != bw) continue;
-                    if (atomicCAS(a.ctrl + CT_HEAD, h, h + 1) == h) {
-                        ticket = h;
-                        have = true;
-                        break;
-                    }
-                    atomicSub(a.ctrl + CT_BUSY, 1u);
-                    continue;
-                }
-                if ((int32_t)(ld_u32(a.ctrl + CT_STOP) - a.gen) >= 0) break;
-                if (dev_clock_100mhz() - t0 > a.idle_ticks && bw == 0 && atomicCAS(a.ctrl + CT_BUSY, 0u, kClosed) == 0u)
-                    break;
-                if (!poller) poller = atomicCAS(a.ctrl + CT_POLL, 0u, 1u) == 0u;
-                if (poller) {
-                    // the lease holder is the only writer of the tail copy
-                    const uint32_t ht = __hip_atomic_load(a.tail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                    if ((int32_t)(ht - tail) > 0) st_u32(a.ctrl + CT_TAIL, ht);
-                    const uint32_t sg = __hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                    if ((int32_t)(sg - a.gen) >= 0) atomicExch(a.ctrl + CT_STOP, sg);
-                    __builtin_amdgcn_s_sleep(16);
-                } else {
-                    backoff = backoff < 8 ? backoff + 1 : 8;
-                    for (int k = 0; k < backoff; ++k) __builtin_amdgcn_s_sleep(64);
-                }
+            const bool have = serve_claim(a, ticket);
+            constexpr uint32_t kWords = sizeof(Req) / 4;
+            if (have && threadIdx.x < kWords)
+                ((uint32_t *)&s_req)[threadIdx.x] =
+                    ld_u32((const uint32_t *)(a.mirror + (ticket & a.ring_mask)) + threadIdx.x);
+            if (lane == 0) {
+                s_ticket = ticket;
+                s_have = have ? 1 : 0;
+                s_uerr = 0;
             }
-            if (poller) atomicExch(a.ctrl + CT_POLL, 0u);
-            // the request's fields were written before the published count:
-            // one system-scope acquire per claim orders the reads below
-            if (have) __atomic_thread_fence(__ATOMIC_ACQUIRE);
-            s_ticket = ticket;
-            s_have = have ? 1 : 0;
-            s_uerr = 0;
         }
         __syncthreads();
         const uint32_t ticket = s_ticket;
-        if (!s_have) break;
-        const Req *rp = a.ring + (ticket & a.ring_mask);
-        Req rq;
-        rq.type = sys_ld_i(&rp->type);
-        rq.s = sys_ld_i(&rp->s);
-        rq.t = sys_ld_i(&rp->t);
-        rq.version = sys_ld_i(&rp->version);
-        rq.del_off = sys_ld_i(&rp->del_off);
-        rq.del_n = sys_ld_i(&rp->del_n);
-        rq.ins_off = sys_ld_i(&rp->ins_off);
-        rq.ins_n = sys_ld_i(&rp->ins_n);
-        rq.rins_off = sys_ld_i(&rp->rins_off);
-        rq.relax_min = sys_ld_i(&rp->relax_min);
-        if (sys_ld_i(&rp->direct)) {  // its own kernels write its result
+        if (!s_have) {  // the launch is closing: the host looks at its event from now on
+            if (lane == 0) __hip_atomic_store(a.left, a.gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            break;
+        }
+        const Req rq = s_req;
+        if (rq.direct) {  // its own kernels write its result
             if (lane == 0) atomicSub(a.ctrl + CT_BUSY, 1u);
-            __syncthreads();        // every lane has read s_ticket before lane 0 claims again
+            __syncthreads();        // every lane has read the claim before wave 0 claims again
             continue;
         }
         const uint64_t tstart = dev_clock_100mhz();
         // ---- wait for the graph version this request needs (bounded)
         const uint32_t need = rq.type == DDP_REQ_UPDATE ? (uint32_t)rq.version - 1 : (uint32_t)rq.version;
         if (lane == 0) {
-            while (__hip_atomic_load(a.ctrl + CT_APPLIED, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < need) {
+            while (ld_u32(a.ctrl + CT_APPLIED) < need) {
                 if (dev_clock_100mhz() - tstart > a.wait_ticks) {
                     s_uerr = SERR_WAIT;
                     break;
@@ -353,8 +452,16 @@ __global__ void __launch_bounds__(B) serve_kernel(ServeArgs a)
         // every later request reports it instead of running.
         if (lane == 0) s_uerr |= ld_u32(a.ctrl + CT_ERR);
         __syncthreads();
-        // every wave acquires the applied version before reading graph data
-        (void)__hip_atomic_load(a.ctrl + CT_APPLIED, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+        // A query reads graph data through its CU's L1: one wave acquires the
+        // applied version for the workgroup, unless an earlier query of this
+        // slot needed as new a one.  (apply_update reads past L1.)
+        if (rq.type != DDP_REQ_UPDATE && (!any_seen || need > seen)) {
+            if (threadIdx.x < 64)
+                (void)__hip_atomic_load(a.ctrl + CT_APPLIED, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            seen = need;
+            any_seen = true;
+        }
         int32_t cost = DDP_INF_COST;
         uint32_t status = s_uerr;
         if (rq.type == DDP_REQ_UPDATE) {
@@ -363,7 +470,7 @@ __global__ void __launch_bounds__(B) serve_kernel(ServeArgs a)
             status = s_uerr;
             if (lane == 0) {
                 if (status) atomicOr(a.ctrl + CT_ERR, status);
-                __threadfence();
+                wait_vmem();  // every wave's writes are in place: apply_update ended with such a wait and a barrier
                 // published even after a failure (later requests then report the
                 // sticky error instead of stalling); atomicMax keeps it from
                 // moving backwards when an earlier version finishes late
@@ -405,7 +512,11 @@ __global__ void __launch_bounds__(B) serve_kernel(ServeArgs a)
             __hip_atomic_store(&r->version, rq.version, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             __hip_atomic_store(&r->t0, tstart, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             __hip_atomic_store(&r->t1, dev_clock_100mhz(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            __hip_atomic_store(&r->seq, ticket + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+            // the stores above go straight to host memory: waiting for them
+            // orders the sequence word after them, where a system-scope release
+            // would also write back the L2 that 32 CUs search in
+            wait_vmem();
+            __hip_atomic_store(&r->seq, ticket + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             atomicSub(a.ctrl + CT_BUSY, 1u);
         }
         __syncthreads();
@@ -559,13 +670,14 @@ struct ddp_server {
     int32_t *rdver = nullptr, *lu = nullptr, *rltail = nullptr;  // bidirectional engine
     uint64_t *rlhead = nullptr, *rlnext = nullptr;
     uint32_t *lw = nullptr, *ctrl = nullptr;
+    Req *mirror = nullptr;  // device copy of the ring
     uint64_t *lhead = nullptr, *lnext = nullptr, *gp = nullptr, *home = nullptr;
     unsigned long long *stats = nullptr;
     // pinned
     Req *ring_h = nullptr;
     Res *res_h = nullptr;
     int32_t *arena_h = nullptr;
-    uint32_t *flags_h = nullptr;  // [0] tail, [1] stop
+    uint32_t *flags_h = nullptr;  // kFlagWords
     Req *ring_d = nullptr;
     Res *res_d = nullptr;
     int32_t *arena_d = nullptr;
@@ -584,6 +696,7 @@ struct ddp_server {
     clk::time_point t_create;
     hipEvent_t done_ev = nullptr;
     bool running = false;
+    double event_seen_ms = 0;      // when done_ev was last looked at
     uint32_t gen = 0;              // number of the newest launch
     // grid mode for low-load queries (server_route_grid)
     bool grid_on = false;
@@ -604,7 +717,7 @@ static double ms_now(const ddp_server *sv)
 static void server_free(ddp_server *sv)
 {
     void *dev[] = {sv->dver, sv->lv, sv->ldel, sv->ltail, sv->touched, sv->lw, sv->ctrl, sv->lhead,
-                   sv->lnext, sv->gp, sv->home, sv->stats, sv->rdver, sv->lu, sv->rltail, sv->rlhead, sv->rlnext};
+                   sv->lnext, sv->gp, sv->home, sv->stats, sv->mirror, sv->rdver, sv->lu, sv->rltail, sv->rlhead, sv->rlnext};
     for (void *p : dev)
         if (p) hipFree(p);
     ddp_merged_free(&sv->own);
@@ -664,10 +777,12 @@ static ServeArgs server_args(const ddp_server *sv)
     a.ltail = sv->ltail;
     a.log_cap = sv->log_cap;
     a.ring = sv->ring_d;
+    a.mirror = sv->mirror;
     a.res = sv->res_d;
     a.arena = sv->arena_d;
     a.tail = sv->flags_d;
     a.stop = sv->flags_d + 1;
+    a.left = sv->flags_d + kLeftWord;
     a.ring_mask = sv->ring - 1;
     a.ctrl = sv->ctrl;
     a.gp = sv->gp;
@@ -702,9 +817,16 @@ static int server_launch(ddp_server *sv)
 }
 
 // Relaunches the kernel if every workgroup has exited while requests wait.
+// An event query takes about 5 us, more than everything else a submission
+// does, so the event is looked at once the launch has said that it is leaving
+// (and every millisecond, in case it cannot say so any more).
 static int server_ensure(ddp_server *sv)
 {
     if (sv->running) {
+        const double now = ms_now(sv);
+        if (__atomic_load_n(&sv->flags_h[kLeftWord], __ATOMIC_ACQUIRE) != sv->gen && now - sv->event_seen_ms < 1.0)
+            return DDP_OK;
+        sv->event_seen_ms = now;
         const hipError_t q = hipEventQuery(sv->done_ev);
         if (q == hipErrorNotReady) return DDP_OK;
         if (q != hipSuccess) return ddp_hip_err(sv->ctx, q, "serve kernel", __FILE__, __LINE__);
@@ -843,6 +965,7 @@ extern "C" int ddp_server_create(ddp_ctx *ctx, const ddp_graph *g, ddp_heur_t h,
     size_t fr = 0, tot = 0;
     e = hipMemGetInfo(&fr, &tot);
     const size_t fixed = (size_t)g->E * 4 + (size_t)g->N * 12 + (size_t)sv->log_cap * 24 + (1 << 20) +
+                         (size_t)sv->ring * sizeof(Req) +
                          (DIRS == 2 ? (size_t)g->RE * 4 + (size_t)g->N * 12 + (size_t)sv->log_cap * 12 : 0);
     const size_t per_slot = DIRS * ((size_t)g->N * 12 + (size_t)sv->cap * sv->B * 8);
     const size_t budget = fr > fixed ? (size_t)((fr - fixed) * 0.9) : 0;
@@ -861,6 +984,7 @@ extern "C" int ddp_server_create(ddp_ctx *ctx, const ddp_graph *g, ddp_heur_t h,
     al((void **)&sv->lw, (size_t)sv->log_cap * 4);
     al((void **)&sv->ldel, (size_t)sv->log_cap * 4);
     al((void **)&sv->ctrl, CT_WORDS * 4);
+    al((void **)&sv->mirror, (size_t)sv->ring * sizeof(Req));
     al((void **)&sv->stats, 64);
     al((void **)&sv->gp, (size_t)slots * DIRS * g->N * 8);
     al((void **)&sv->touched, (size_t)slots * DIRS * g->N * 4);
@@ -881,7 +1005,7 @@ extern "C" int ddp_server_create(ddp_ctx *ctx, const ddp_graph *g, ddp_heur_t h,
     hal((void **)&sv->ring_h, (void **)&sv->ring_d, sizeof(Req) * sv->ring);
     hal((void **)&sv->res_h, (void **)&sv->res_d, sizeof(Res) * sv->ring);
     hal((void **)&sv->arena_h, (void **)&sv->arena_d, sv->arena_cap * 4);
-    hal((void **)&sv->flags_h, (void **)&sv->flags_d, 64);
+    hal((void **)&sv->flags_h, (void **)&sv->flags_d, kFlagWords * 4);
     sv->delivered.assign(sv->ring, 0);
     sv->direct_of.assign(sv->ring, 0);
     sv->tags.assign(sv->ring, 0);
