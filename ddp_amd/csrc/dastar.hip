@@ -1055,7 +1055,7 @@ extern "C" int ddp_dastar_open(ddp_ctx *ctx, int32_t N, int32_t E, const int32_t
     d->hv.kind = DDP_H_ARRAY;
     d->hv.scale = 1;
     d->hv.h = d->d_h;
-    if ((rc = ddp_ga_plan(ctx, d->g, opts, &d->P, 2 * (int64_t)N + 65536)) ||
+    if ((rc = ddp_ga_plan(ctx, d->g, opts, &d->P, 2 * (int64_t)N + 65536, false, true)) ||
         (rc = ddp_ga_alloc_owned(ctx, N, d->P, &d->S)) || (rc = log_reserve(d, 1))) {
         dastar_free(d);
         delete d;

@@ -13,7 +13,7 @@ enum : int {
     GA_S_PUSHCNT = 0, GA_S_TOPMIN = 1, GA_S_PUSHMIN = 2, GA_S_TMIN = 3, GA_S_ERR = 4,
     GA_RES_IT = 32, GA_RES_RR = 33, GA_RES_F = 34, GA_RES_ERR = 35, GA_RES_PLEN = 36,
     GA_BAR = 64,
-    GA_CTRL_WORDS = 96,
+    GA_CTRL_WORDS = 1024,  // grid_piles.h keeps its counters behind these
 };
 
 // Error bits of GA_RES_ERR.
@@ -25,15 +25,20 @@ struct GaGridPlan {
     bool piles = false;
     bool bidi = false;   // piles from both ends: two (f, parent) arrays, touched logs and pile sets
     uint32_t ncap = 0, fcap = 0, delta0 = 1;  // pile mode: near ring, far buffers, first window
+    // grid mode on piles (grid_piles.h; otherwise lane heaps, which DA* resumes):
+    // a graph with enough edges for a workgroup per CU, and the segments one
+    // round's long rows can be cut into
+    bool pg = false, pg_wide = false;
+    uint32_t hubcap = 0;
 };
 
 // Device buffers of one GA* search state.
 struct GaGridState {
     uint64_t *gp = nullptr;      // N packed (f << 32 | parent); bidirectional: 2N, forward then backward
-    uint64_t *home = nullptr;    // cap * K heap entries (bidirectional: twice)
+    uint64_t *home = nullptr;    // cap * K heap entries (bidirectional: twice; grid mode on piles: ga_pg_sizes)
     int32_t *hsize = nullptr;    // K
     int32_t *touched = nullptr;  // N, workgroup mode only (bidirectional: 2N)
-    uint64_t *pbuf = nullptr;    // 2 * pcap push entries
+    uint64_t *pbuf = nullptr;    // 2 * pcap push entries; grid mode on piles: hubcap segments of 2 words
     uint32_t *ctrl = nullptr;    // GA_CTRL_WORDS
     unsigned long long *stats = nullptr;  // 8 counters after ctrl
     bool owned = false;          // allocated by ddp_ga_alloc_owned (freed by ddp_ga_free)
@@ -41,8 +46,9 @@ struct GaGridState {
 
 // min_pcap: lower bound on the push buffer (DA* repairs push before a launch).
 // allow_wg: honour opts->mode and plan the workgroup mode when it applies.
+// heaps: plan grid mode on lane heaps, whose queues a later search can resume.
 int ddp_ga_plan(ddp_ctx *ctx, const ddp_graph *g, const ddp_astar_opts_t *o, GaGridPlan *p,
-                int64_t min_pcap = 0, bool allow_wg = false);
+                int64_t min_pcap = 0, bool allow_wg = false, bool heaps = false);
 // State in the context's reusable scratch (valid until the next ddp_astar on ctx).
 int ddp_ga_alloc(ddp_ctx *ctx, const ddp_graph *g, const GaGridPlan &P, GaGridState *S);
 // State owned by the caller (DA*), freed by ddp_ga_free.
@@ -57,7 +63,10 @@ int ddp_ga_prepare_resume(ddp_ctx *ctx, const GaGridState &S);
 int ddp_ga_run(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P,
                const GaGridState &S, int32_t t, uint32_t F0, int32_t rr0, uint32_t *F_out,
                int32_t *rr_out, int32_t *iters_out, float *kernel_ms);
-// Grid mode, asynchronous: resets the state, seeds s and enqueues the grid
+// Grid mode on piles: a fresh search from s to completion (ddp_ga_reset before; no seed needed).
+int ddp_ga_run_piles(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P, const GaGridState &S,
+                     int32_t s, uint32_t hs, int32_t t, uint32_t *F_out, int32_t *iters_out, float *kernel_ms);
+// Grid mode on piles, asynchronous: resets the state, seeds s and enqueues the grid
 // kernel on ctx->stream without waiting.  Stream-ordered work after it reads
 // the outcome from S.ctrl (GA_RES_F: f of t, DDP_INF_F if unreachable;
 // GA_RES_ERR: GA_ERR_* bits).

@@ -1,5 +1,7 @@
-// Single-query GA*: K priority queues over one persistent grid (grid mode),
-// or all of them inside one workgroup (workgroup mode, further down).
+// Single-query GA*.  Fresh grid-mode searches run on piles over the whole GPU
+// (grid_piles.h); the K priority queues over one persistent grid below are
+// what DA* resumes in grid mode; workgroup mode keeps all queues inside one
+// workgroup (further down).
 //
 // Reference loop (GA_star/GA_v2.cu:488-559): per iteration the host launches
 // extractMin, A_star_expand, keepHeapPQ, setNV (an O(N) flag scan), insertPQ,
@@ -30,6 +32,7 @@
 
 #include "bidi_search.h"
 #include "gastar.h"
+#include "grid_piles.h"
 
 namespace {
 
@@ -251,6 +254,49 @@ __global__ void unpack_parent_kernel(const uint64_t *gp, int32_t *par, int32_t N
         par[i] = (int32_t)(uint32_t)gp[i];
 }
 
+// Fresh search on piles: gp[s], s alone in the near ring, the control words.
+__global__ void pg_seed_kernel(uint64_t *gp, uint64_t *near, uint32_t *ctrl, int32_t s, uint32_t hs)
+{
+    for (int k = threadIdx.x; k < PG_WORDS; k += blockDim.x) {
+        const int w = k >= PG_SLOTS && k < PG_BAR ? (k - PG_SLOTS) % PG_SLOT_WORDS : -1;
+        ctrl[k] = w == PG_TMIN || w == PG_FMIN ? 0xFFFFFFFFu : 0u;
+    }
+    if (threadIdx.x == 0) {
+        gp[s] = ((uint64_t)hs << 32) | 0xFFFFFFFFull;
+        near[0] = ((uint64_t)hs << 32) | (uint32_t)s;
+    }
+}
+
+using PgFn = void (*)(PgArgs);
+
+PgFn pick_pg(int hk)
+{
+    switch (hk) {
+    case DDP_H_ZERO: return ga_piles_kernel<kPgBlock, DDP_H_ZERO>;
+    case DDP_H_ARRAY: return ga_piles_kernel<kPgBlock, DDP_H_ARRAY>;
+    case DDP_H_MANHATTAN: return ga_piles_kernel<kPgBlock, DDP_H_MANHATTAN>;
+    default: return ga_piles_kernel<kPgBlock, DDP_H_EUCLID>;
+    }
+}
+
+// Workgroups of a grid search on piles (see kPgBlocks).
+int32_t pg_blocks(const ddp_ctx *ctx, const GaGridPlan &P, int hk)
+{
+    const int32_t cus = ctx->prop.multiProcessorCount;
+    return P.pg_wide && (hk == DDP_H_ZERO || hk == DDP_H_ARRAY) ? cus : std::min(kPgBlocks, cus);
+}
+
+// Entries of the near ring (a power of two) and of each far buffer: either
+// holds the K * cap entries that K queues of cap would.
+void ga_pg_sizes(const GaGridPlan &P, uint64_t *ring, uint64_t *far)
+{
+    const uint64_t total = std::min<uint64_t>((uint64_t)P.K * P.cap, 1ull << 31);
+    uint64_t r = 1024;
+    while (r < total) r *= 2;
+    *ring = r;
+    *far = std::max<uint64_t>(total, 1024);
+}
+
 using KernelFn = void (*)(GridArgs);
 
 template <int B>
@@ -388,7 +434,7 @@ WgFn pick_wg(int B, int hk, int wm)
 }  // namespace
 
 int ddp_ga_plan(ddp_ctx *ctx, const ddp_graph *g, const ddp_astar_opts_t *o, GaGridPlan *p, int64_t min_pcap,
-                bool allow_wg)
+                bool allow_wg, bool heaps)
 {
     int32_t B = (o && o->block) ? o->block : 0;
     int32_t K = (o && o->K) ? o->K : 1024;
@@ -448,6 +494,12 @@ int ddp_ga_plan(ddp_ctx *ctx, const ddp_graph *g, const ddp_astar_opts_t *o, GaG
     DDP_CHECK(pcap < (1LL << 31), ctx, DDP_ERR_ARG, "push buffer too large");
     int32_t maxit = (o && o->max_iters) ? o->max_iters : (int32_t)std::min<int64_t>(4LL * g->N + 1024, 1 << 30);
     *p = GaGridPlan{K, B, nblocks, lcap, (int32_t)cap, (int32_t)pcap, maxit};
+    if (!heaps) {
+        p->pg = true;
+        p->pg_wide = g->E >= kPgWideEdges;
+        p->hubcap = (uint32_t)((int64_t)g->E / kPgSeg + kPgRound + 64);
+        p->delta0 = std::max<uint32_t>(1, g->meanw);
+    }
     // co-residency check for the cooperative launch
     int per_cu = 0;
     DDP_HIP(ctx, hipFuncSetAttribute((const void *)pick(B, DDP_H_ZERO), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -465,13 +517,20 @@ int ddp_ga_alloc(ddp_ctx *ctx, const ddp_graph *g, const GaGridPlan &P, GaGridSt
     void *p;
     int rc;
     const size_t dirs = P.bidi ? 2 : 1;
+    size_t queue = dirs * P.cap * P.K, push = 2 * (size_t)P.pcap;  // 8-byte entries
+    if (P.pg) {
+        uint64_t ring, far;
+        ga_pg_sizes(P, &ring, &far);
+        queue = ring + 2 * far;
+        push = 2 * (size_t)P.hubcap;
+    }
     if ((rc = ddp_ws(ctx, WS_ASTAR_GP, dirs * g->N * 8, &p))) return rc;
     S->gp = (uint64_t *)p;
-    if ((rc = ddp_ws(ctx, WS_ASTAR_HEAP, dirs * P.cap * P.K * 8, &p))) return rc;
+    if ((rc = ddp_ws(ctx, WS_ASTAR_HEAP, queue * 8, &p))) return rc;
     S->home = (uint64_t *)p;
     if ((rc = ddp_ws(ctx, WS_ASTAR_HSIZE, (size_t)P.K * 4, &p))) return rc;
     S->hsize = (int32_t *)p;
-    if ((rc = ddp_ws(ctx, WS_ASTAR_PBUF, (size_t)P.pcap * 16, &p))) return rc;
+    if ((rc = ddp_ws(ctx, WS_ASTAR_PBUF, push * 8, &p))) return rc;
     S->pbuf = (uint64_t *)p;
     if ((rc = ddp_ws(ctx, WS_ASTAR_CTRL, GA_CTRL_WORDS * 4 + 64, &p))) return rc;
     S->ctrl = (uint32_t *)p;
@@ -493,10 +552,17 @@ int ddp_ga_alloc_owned(ddp_ctx *ctx, int32_t N, const GaGridPlan &P, GaGridState
     auto al = [&](void **p, size_t bytes) {
         if (e == hipSuccess) e = hipMalloc(p, std::max<size_t>(bytes, 64));
     };
+    size_t queue = (size_t)P.cap * P.K, push = 2 * (size_t)P.pcap;
+    if (P.pg) {
+        uint64_t ring, far;
+        ga_pg_sizes(P, &ring, &far);
+        queue = ring + 2 * far;
+        push = 2 * (size_t)P.hubcap;
+    }
     al((void **)&S->gp, (size_t)N * 8);
-    al((void **)&S->home, (size_t)P.cap * P.K * 8);
+    al((void **)&S->home, queue * 8);
     al((void **)&S->hsize, (size_t)P.K * 4);
-    al((void **)&S->pbuf, (size_t)P.pcap * 16);
+    al((void **)&S->pbuf, push * 8);
     al((void **)&S->ctrl, GA_CTRL_WORDS * 4 + 64);
     if (e != hipSuccess) {
         ddp_ga_free(S);
@@ -519,8 +585,9 @@ int ddp_ga_reset(ddp_ctx *ctx, int32_t N, const GaGridPlan &P, const GaGridState
 {
     hipLaunchKernelGGL(fill_u64_kernel, dim3(1024), dim3(256), 0, ctx->stream, S.gp, (int64_t)N * (P.bidi ? 2 : 1),
                        (uint64_t)DDP_GP_INF);
-    hipLaunchKernelGGL(fill_i32_kernel, dim3(std::max(1, std::min(1024, P.K / 256 + 1))), dim3(256), 0,
-                       ctx->stream, S.hsize, (int64_t)P.K, 0);
+    if (!P.pg)
+        hipLaunchKernelGGL(fill_i32_kernel, dim3(std::max(1, std::min(1024, P.K / 256 + 1))), dim3(256), 0,
+                           ctx->stream, S.hsize, (int64_t)P.K, 0);
     DDP_HIP(ctx, hipMemsetAsync(S.stats, 0, 64, ctx->stream));
     DDP_HIP(ctx, hipGetLastError());
     return DDP_OK;
@@ -600,32 +667,43 @@ int grid_enqueue(ddp_ctx *ctx, GridArgs &a, const GaGridPlan &P, int hk)
     return DDP_OK;
 }
 
-}  // namespace
-
-int ddp_ga_launch(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P,
-                  const GaGridState &S, int32_t N, int32_t s, uint32_t hs, int32_t t)
+// Grid mode on piles: seeds s and enqueues the search.  Ordinary launch, as
+// grid_enqueue's; at most one workgroup per CU, so all are resident at once.
+int pg_enqueue(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P, const GaGridState &S,
+               int32_t s, uint32_t hs, int32_t t)
 {
-    DDP_CHECK(!P.wg, ctx, DDP_ERR_STATE, "GA*: not a grid plan");
-    int rc;
-    if ((rc = ddp_ga_reset(ctx, N, P, S))) return rc;
-    if ((rc = ddp_ga_seed(ctx, P, S, s, hs))) return rc;  // also clears the barrier and the result words
-    GridArgs a = grid_args(gv, hv, P, S, t, DDP_INF_F, 0);
-    return grid_enqueue(ctx, a, P, hv.kind);
+    uint64_t ring, far;
+    ga_pg_sizes(P, &ring, &far);
+    PgArgs a{};
+    a.g = gv;
+    a.h = hv;
+    a.gp = S.gp;
+    a.near = S.home;
+    a.far0 = S.home + ring;
+    a.far1 = a.far0 + far;
+    a.hubs = S.pbuf;
+    a.nmask = (uint32_t)(ring - 1);
+    a.fcap = (uint32_t)far;
+    a.hubcap = P.hubcap;
+    a.ctrl = S.ctrl;
+    a.stats = S.stats;
+    a.grow = (uint32_t)P.K;
+    a.t = t;
+    a.maxit = P.maxit;
+    a.delta0 = P.delta0;
+    a.thr0 = hs > 0xFFFFFFFFu - P.delta0 ? 0xFFFFFFFFu : hs + P.delta0;
+    a.barrier_ticks = 100ull * 1000 * 1000 * 20;  // 20 s of the 100 MHz clock
+    hipLaunchKernelGGL(pg_seed_kernel, dim3(1), dim3(256), 0, ctx->stream, S.gp, S.home, S.ctrl, s, hs);
+    void *args[] = {&a};
+    DDP_HIP(ctx, hipLaunchKernel((const void *)pick_pg(hv.kind), dim3(pg_blocks(ctx, P, hv.kind)), dim3(kPgBlock), args,
+                                 0, ctx->stream));
+    return DDP_OK;
 }
 
-// Runs the GA* loop from the current state (fresh or resumed).
-int ddp_ga_run(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P,
-               const GaGridState &S, int32_t t, uint32_t F0, int32_t rr0, uint32_t *F_out,
-               int32_t *rr_out, int32_t *iters_out, float *kernel_ms)
+// Waits for a grid search (its events recorded) and reads its outcome.
+int grid_finish(ddp_ctx *ctx, const GaGridPlan &P, const GaGridState &S, uint32_t *F_out, int32_t *rr_out,
+                int32_t *iters_out, float *kernel_ms)
 {
-    GridArgs a = grid_args(gv, hv, P, S, t, F0, rr0);
-    // a previous launch that timed out may have left the barrier mid-count
-    DDP_HIP(ctx, hipMemsetAsync(S.ctrl + GA_BAR, 0, 8, ctx->stream));
-    DDP_HIP(ctx, hipMemsetAsync(S.ctrl + GA_RES_ERR, 0, 4, ctx->stream));
-    DDP_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-    int rc = grid_enqueue(ctx, a, P, hv.kind);
-    if (rc) return rc;
-    DDP_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
     uint32_t res[4];
     DDP_HIP(ctx, hipMemcpyAsync(res, S.ctrl + GA_RES_IT, 16, hipMemcpyDeviceToHost, ctx->stream));
     DDP_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -642,6 +720,44 @@ int ddp_ga_run(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGr
               "GA*: a queue exceeded heap_cap=%d entries; raise heap_cap", P.cap);
     DDP_CHECK(!(err & ERR_PBUF), ctx, DDP_ERR_OVERFLOW, "GA*: push buffer (%d entries) overflowed", P.pcap);
     return DDP_OK;
+}
+
+}  // namespace
+
+int ddp_ga_launch(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P,
+                  const GaGridState &S, int32_t N, int32_t s, uint32_t hs, int32_t t)
+{
+    DDP_CHECK(P.pg, ctx, DDP_ERR_STATE, "GA*: not a grid plan");
+    int rc;
+    if ((rc = ddp_ga_reset(ctx, N, P, S))) return rc;
+    return pg_enqueue(ctx, gv, hv, P, S, s, hs, t);
+}
+
+// Runs the GA* loop from the current state (fresh or resumed).
+int ddp_ga_run(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P,
+               const GaGridState &S, int32_t t, uint32_t F0, int32_t rr0, uint32_t *F_out,
+               int32_t *rr_out, int32_t *iters_out, float *kernel_ms)
+{
+    GridArgs a = grid_args(gv, hv, P, S, t, F0, rr0);
+    // a previous launch that timed out may have left the barrier mid-count
+    DDP_HIP(ctx, hipMemsetAsync(S.ctrl + GA_BAR, 0, 8, ctx->stream));
+    DDP_HIP(ctx, hipMemsetAsync(S.ctrl + GA_RES_ERR, 0, 4, ctx->stream));
+    DDP_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
+    int rc = grid_enqueue(ctx, a, P, hv.kind);
+    if (rc) return rc;
+    DDP_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
+    return grid_finish(ctx, P, S, F_out, rr_out, iters_out, kernel_ms);
+}
+
+// Grid mode on piles: a fresh search (ddp_ga_reset before).
+int ddp_ga_run_piles(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P, const GaGridState &S,
+                     int32_t s, uint32_t hs, int32_t t, uint32_t *F_out, int32_t *iters_out, float *kernel_ms)
+{
+    DDP_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
+    int rc = pg_enqueue(ctx, gv, hv, P, S, s, hs, t);
+    if (rc) return rc;
+    DDP_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
+    return grid_finish(ctx, P, S, F_out, nullptr, iters_out, kernel_ms);
 }
 
 int ddp_ga_run_wg(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P,
@@ -727,8 +843,8 @@ extern "C" int ddp_astar(ddp_ctx *ctx, const ddp_graph *g, ddp_heur_t h, int32_t
     if (stats) {
         std::memset(stats, 0, sizeof *stats);
         stats->K = P.K;
-        stats->block = P.B;
-        stats->blocks = P.nblocks;
+        stats->block = P.pg ? kPgBlock : P.B;
+        stats->blocks = P.pg ? pg_blocks(ctx, P, hv.kind) : P.nblocks;
     }
     if ((rc = ddp_ga_reset(ctx, g->N, P, S))) return rc;
     if (hv.kind == DDP_H_ARRAY && hs < 0) {
@@ -775,8 +891,9 @@ extern "C" int ddp_astar(ddp_ctx *ctx, const ddp_graph *g, ddp_heur_t h, int32_t
             gv.relax_min = g->minw >= 1;
             rc = ddp_ga_run_wg(ctx, gv, hv, P, S, g->N, s, t, &F, &iters, &kms);
         } else {
-            if ((rc = ddp_ga_seed(ctx, P, S, s, (uint32_t)hs))) return rc;
-            rc = ddp_ga_run(ctx, ddp_view(g), hv, P, S, t, DDP_INF_F, 0, &F, nullptr, &iters, &kms);
+            GraphView gv = ddp_view(g);
+            gv.relax_min = g->minw >= 1;
+            rc = ddp_ga_run_piles(ctx, gv, hv, P, S, s, (uint32_t)hs, t, &F, &iters, &kms);
         }
         if (rc) return rc;
         *cost = (int32_t)F;
@@ -812,7 +929,7 @@ extern "C" int ddp_astar(ddp_ctx *ctx, const ddp_graph *g, ddp_heur_t h, int32_t
         int32_t *dpar = nullptr;
         void *p;
         // reuse the push buffer region as a staging area when large enough
-        if ((size_t)P.pcap * 16 >= (size_t)g->N * 4) dpar = (int32_t *)S.pbuf;
+        if (!P.pg && (size_t)P.pcap * 16 >= (size_t)g->N * 4) dpar = (int32_t *)S.pbuf;
         else {
             if ((rc = ddp_ws(ctx, WS_PATH, (size_t)g->N * 4 + 256, &p))) return rc;
             dpar = (int32_t *)p;

@@ -1,0 +1,449 @@
+// One query searched by the whole GPU (grid mode): the near/far piles of
+// slot_search.h shared by a persistent grid.
+//
+// Open entries (f << 32 | node) sit in a near ring (f below a threshold) and
+// a far pile.  A round takes the near entries (up to kPgRound); eight lanes
+// expand one, and the chunks of eight entries a wave takes are dealt over the
+// workgroups.  Rows longer than kPgSeg edges are
+// cut into segments that the round's second step spreads over the whole grid:
+// a power-law hub would otherwise keep one workgroup busy while the others
+// wait at the barrier.  When the near ring is empty the threshold moves to the
+// far pile's lower bound plus a window width, and one pass sends the entries
+// under it to the near ring and compacts the other live ones into the second
+// far buffer (which gives the next lower bound; it is exact up to entries that
+// have gone stale since).  As in the slots this is a label-correcting search:
+// an entry is dropped only when it is stale or cannot lead to anything below
+// F(t), so the cost is exact for an admissible heuristic.  K sets the window:
+// a width that fed fewer than K entries doubles, one that fed more than 8K
+// halves.
+//
+// Why piles and not the K lane heaps this replaced: a heap pop is a chain of
+// dependent LDS and HBM accesses (8 us an iteration on the 100,000-node random
+// graph, 41 us on R-MAT scale 20), an entry was expanded by its own lane's
+// wave however long its row (R-MAT: 135 us, and 94 us of waiting for the
+// workgroup with the hub), and K lanes were all the parallelism there was.
+// Measured, whole call, heaps and piles: random graph of 100,000 nodes, K = 1,024,
+// 1.5-3.1 and 0.39-0.43 ms; R-MAT scale 20, K = 16,384, 9.8-11.2 and 2.0-2.9 ms;
+// 2,048 x 2,048 maze, K = 512, 49.1 and 26.0 ms.  What is left is latency: a
+// round is seven dependent round trips and a barrier, 6 us.
+//
+// Everything workgroups share -- the (f, parent) words, the piles, the control
+// words -- is accessed through agent-scope atomics only, as grid_sync needs.
+// A round's steps each end with grid_sync; what a step appended is counted in
+// one of three rotating slots, read by everybody after the barrier and cleared
+// two steps later, so all workgroups take every decision from the same values.
+#pragma once
+
+#include "gastar.h"
+#include "search_expand.h"
+
+// Control words behind the result words of gastar.h (a 128-byte line each).
+enum : int {
+    PG_NEAR = 0, PG_FAR = 32, PG_TMIN = 64, PG_FMIN = 96, PG_HUBS = 128, PG_ERR = 129, PG_SLOT_WORDS = 160,
+    PG_SLOTS = 128, PG_BAR = PG_SLOTS + 3 * PG_SLOT_WORDS, PG_WORDS = PG_BAR + GRID_SYNC_WORDS
+};
+static_assert(PG_WORDS <= GA_CTRL_WORDS, "control block too small");
+
+constexpr int32_t kPgSeg = 64;    // edges per hub segment
+constexpr int kPgLanes = 8;       // lanes per entry
+constexpr int kPgUnroll = 2;      // edges per lane and step
+constexpr int kPgBlock = 1024;
+// Workgroups: 64 (a barrier of 1.9 us), or one per CU (2.6 us) where a round
+// scans hundreds of thousands of edges -- searches without a geometric
+// heuristic on graphs of kPgWideEdges edges and more.  Measured with 64 and
+// 256 workgroups (ms): R-MAT of 16.8M edges 3.1 and 2.0; R-MAT of 0.8M edges
+// 0.53 and 0.72; random graph of 0.6M edges 0.32 and 0.53; 1,024 x 1,024 maze
+// 12.6 and 14.3; geometric graph of 2M edges, Euclidean heuristic, 1.45 and
+// 1.79.  (64 workgroups of 256 lanes: 6.8, 0.73, 0.40, 12.5, 1.40.)
+constexpr int kPgBlocks = 64;
+constexpr int64_t kPgWideEdges = 1 << 22;
+// Near entries a round takes at most.  Taking the whole window at once saves
+// rounds and costs little order, which the window's width keeps: 8,192 against
+// 65,536 entries took 0.39 and 0.32 ms on the random graph (K = 1,024), 0.68
+// and 0.36 ms on one of 300,000 nodes at K = 256.
+constexpr uint32_t kPgRound = 65536;
+// Near entries that count as stragglers: with 256 the split ran ahead of f
+// order on mazes (703,000 expansions against 56,000 without early splits).
+constexpr uint32_t kPgThin = 64;
+
+struct PgArgs {
+    GraphView g;
+    HeurView h;
+    uint64_t *gp;
+    uint64_t *near;       // ring of nmask + 1 entries
+    uint64_t *far0, *far1;
+    uint64_t *hubs;       // 2 words per segment: start | length << 32, node | g << 32
+    uint32_t nmask, fcap, hubcap;
+    uint32_t *ctrl;
+    unsigned long long *stats;
+    int32_t t, maxit;
+    uint32_t grow;        // K: a window that fed fewer entries doubles, one that fed 8 times as many halves
+    uint32_t thr0, delta0;
+    uint64_t barrier_ticks;
+};
+
+// Where a step's improvements go: staged in LDS, and placed with one atomic
+// per workgroup and pile when the step ends; what LDS cannot hold is placed
+// by its wave at once.
+template <int B>
+struct PgStage {
+    static constexpr uint32_t kCap = 2 * B;
+    uint64_t near[kCap], far[kCap];
+    uint32_t n[2], base[2];  // near, far
+    uint32_t tmin, fmin, err;
+};
+
+template <int B>
+struct PgPush {
+    PgStage<B> *S;
+    const PgArgs *a;
+    uint32_t *slot;       // this step's counters
+    uint32_t nbase, head; // ring positions where this step's appends start, and of the oldest entry
+    uint64_t *far;
+    uint32_t fbase;
+    uint32_t thr, F;
+    uint32_t fmin = 0xFFFFFFFFu;  // smallest f this lane sent to the far pile
+
+    __device__ __forceinline__ void put_near(uint32_t k, uint64_t key) const
+    {
+        const uint32_t pos = nbase + k;
+        if (pos - head <= a->nmask) st_u64(a->near + (pos & a->nmask), key);
+        else atomicOr(&S->err, (uint32_t)GA_ERR_HEAP);
+    }
+    __device__ __forceinline__ void put_far(uint32_t k, uint64_t key) const
+    {
+        const uint64_t pos = (uint64_t)fbase + k;
+        if (pos < a->fcap) st_u64(far + pos, key);
+        else atomicOr(&S->err, (uint32_t)GA_ERR_HEAP);
+    }
+    __device__ __forceinline__ void target(uint32_t f) const { atomicMin(&S->tmin, f); }
+    __device__ __forceinline__ void touch(int32_t, uint64_t) const {}
+    template <int R>
+    __device__ __forceinline__ void touch_all(const bool (&)[R], const int32_t (&)[R]) const {}
+    // wave-collective
+    template <int R>
+    __device__ __forceinline__ void all(const bool (&has)[R], const uint64_t (&key)[R])
+    {
+#pragma unroll
+        for (int pile = 0; pile < 2; ++pile) {
+            bool sel[R];
+            uint32_t pos[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const uint32_t f = (uint32_t)(key[r] >> 32);
+                sel[r] = has[r] && f < F && (f < thr) == (pile == 0);
+                if (pile == 1 && sel[r] && f < fmin) fmin = f;
+            }
+            wave_append<R>(sel, &S->n[pile], pos);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                if (sel[r] && pos[r] < PgStage<B>::kCap) (pile == 0 ? S->near : S->far)[pos[r]] = key[r];
+                const bool over[1] = {sel[r] && pos[r] >= PgStage<B>::kCap};
+                if (__any(over[0])) {
+                    uint32_t k[1];
+                    wave_append<1>(over, slot + (pile == 0 ? PG_NEAR : PG_FAR), k);
+                    if (over[0]) {
+                        if (pile == 0) put_near(k[0], key[r]);
+                        else put_far(k[0], key[r]);
+                    }
+                }
+            }
+        }
+    }
+    // block-collective: the staged entries to their piles
+    __device__ __forceinline__ void flush()
+    {
+        const int lane = threadIdx.x;
+        if (__any(fmin != 0xFFFFFFFFu)) {
+            const uint32_t m = wave_min_u32(fmin);
+            if ((lane & 63) == 0) atomicMin(&S->fmin, m);
+        }
+        __syncthreads();
+        if (lane == 0 || lane == 64) {
+            const int pile = lane >> 6;
+            const uint32_t m = S->n[pile] < PgStage<B>::kCap ? S->n[pile] : PgStage<B>::kCap;
+            S->base[pile] = m ? add_u32(slot + (pile == 0 ? PG_NEAR : PG_FAR), m) : 0;
+        } else if (lane == 192) {
+            if (S->fmin != 0xFFFFFFFFu)
+                (void)__hip_atomic_fetch_min(slot + PG_FMIN, S->fmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else if (lane == 128) {
+            if (S->tmin != 0xFFFFFFFFu)
+                (void)__hip_atomic_fetch_min(slot + PG_TMIN, S->tmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        const uint32_t m0 = S->n[0] < PgStage<B>::kCap ? S->n[0] : PgStage<B>::kCap;
+        const uint32_t m1 = S->n[1] < PgStage<B>::kCap ? S->n[1] : PgStage<B>::kCap;
+        for (uint32_t k = lane; k < m0; k += B) put_near(S->base[0] + k, S->near[k]);
+        for (uint32_t k = lane; k < m1; k += B) put_far(S->base[1] + k, S->far[k]);
+        __syncthreads();
+        if (lane == 0) {
+            if (S->err) (void)__hip_atomic_fetch_or(slot + PG_ERR, S->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            S->n[0] = S->n[1] = 0;
+            S->tmin = S->fmin = 0xFFFFFFFFu;
+        }
+    }
+};
+
+// The edges [start, start + len) of node u (g value gu) by the eight lanes of
+// a group; every lane of the wave calls it (len = 0: nothing to do).
+template <int B, int HK>
+__device__ __forceinline__ void pg_expand(const PgArgs &a, uint32_t start, uint32_t len, int32_t u, uint32_t gu,
+                                          uint32_t F, ExpandCounters &C, PgPush<B> &push)
+{
+    constexpr int U = kPgUnroll;
+    const uint32_t sub = threadIdx.x % kPgLanes;
+    for (uint32_t j = 0; __any(j < len); j += kPgLanes * U) {
+        int32_t c[U], dv[U];
+        uint32_t wt[U];
+#pragma unroll
+        for (int r = 0; r < U; ++r) {
+            const uint32_t k = j + r * kPgLanes + sub;
+            c[r] = -1;
+            wt[r] = 0;
+            dv[r] = INT32_MAX;
+            if (k < len) {
+                c[r] = a.g.col[start + k];
+                wt[r] = a.g.w[start + k];
+                if (a.g.dver) dv[r] = a.g.dver[start + k];
+                C.edges++;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < U; ++r)
+            if (a.g.dver && dv[r] <= a.g.ver) c[r] = -1;  // deleted at or before this version
+        relax_window<U, HK>(a.g, a.h, a.gp, a.t, c, wt, [&](int) { return gu; }, [&](int) { return u; }, F, C, push);
+    }
+}
+
+template <int B, int HK>
+__global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
+{
+    __shared__ PgStage<B> S;
+    __shared__ int32_t s_flag;
+    constexpr uint32_t kPerWave = 64 / kPgLanes, kWaves = B / 64;
+    const int lane = threadIdx.x;
+    const uint32_t wl = lane & 63, sub = lane % kPgLanes;
+    uint32_t *ctrl = a.ctrl;
+    uint32_t gen = ld_u32(ctrl + PG_BAR + 32);
+    // ring positions and far entries as of the last barrier, the same in every workgroup
+    uint32_t head = 0, tail = 1, fn = 0, F = DDP_INF_F, thr = a.thr0, delta = a.delta0, phase_n = 0;
+    uint32_t low = 0xFFFFFFFFu;  // no live far entry is below this
+    uint64_t *far = a.far0, *far2 = a.far1;
+    uint32_t step = 0, err = 0;
+    int32_t it = 0;
+    bool timeout = false;
+    ExpandCounters C;
+    uint32_t stale = 0;
+    if (lane == 0) {
+        S.n[0] = S.n[1] = 0;
+        S.tmin = S.fmin = 0xFFFFFFFFu;
+        S.err = 0;
+    }
+    __syncthreads();
+    // a step: its counters' slot; the next step's (last read two barriers ago) is cleared meanwhile
+    auto begin = [&]() {
+        if (blockIdx.x == 0 && lane < 6) {
+            uint32_t *ns = ctrl + PG_SLOTS + ((step + 1) % 3) * PG_SLOT_WORDS;
+            if (lane < 5) st_u32(ns + 32 * lane, lane == 2 || lane == 3 ? 0xFFFFFFFFu : 0u);
+            else st_u32(ns + PG_ERR, 0u);
+        }
+        return ctrl + PG_SLOTS + (step % 3) * PG_SLOT_WORDS;
+    };
+    auto add_sat = [](uint32_t x, uint32_t y) { return x > 0xFFFFFFFFu - y ? 0xFFFFFFFFu : x + y; };
+    for (;;) {
+        const uint32_t avail = tail - head;
+        if (avail == 0 && (fn == 0 || low >= F)) break;  // nothing open can improve t
+        // The far pile is split when the near ring is empty, or when all but
+        // stragglers of a window that has fed its K entries are done and the
+        // next window adjoins it (entries further out would run ahead of f
+        // order): the stragglers' round and the split then share a barrier.
+        const bool split = fn > 0 && (avail == 0 || (avail < kPgThin && phase_n >= a.grow && low < add_sat(thr, delta)));
+        if (split) {
+            if (avail == 0) {
+                if (it > 0) {
+                    if (phase_n < a.grow) delta = add_sat(delta, delta);
+                    else if (phase_n > 8 * a.grow && delta > 1) delta >>= 1;
+                }
+                phase_n = 0;
+            }
+            const uint32_t nt = add_sat(low, delta);
+            thr = nt > thr ? nt : thr;
+            if (blockIdx.x == 0 && lane == 0) C.refills++;
+        }
+        if (avail && it >= a.maxit) {
+            err |= GA_ERR_ITERS;
+            break;
+        }
+        if (avail) ++it;
+        const uint32_t n = avail < kPgRound ? avail : kPgRound;
+        phase_n += n;
+        // ---- step 1: the round's entries, hub rows cut into segments, and the split
+        uint32_t *slot = begin();
+        {
+            PgPush<B> push{&S, &a, slot, tail, head, split ? far2 : far, split ? 0u : fn, thr, F};
+            const uint32_t chunks = (n + kPerWave - 1) / kPerWave;
+            for (uint32_t ch = (lane >> 6) * gridDim.x + blockIdx.x; ch < chunks; ch += kWaves * gridDim.x) {
+                const uint32_t i = ch * kPerWave + wl / kPgLanes;
+                int32_t u = -1;
+                uint32_t gu = 0, start = 0, deg = 0;
+                if (i < n) {
+                    const uint64_t key = ld_gp(a.near + ((head + i) & a.nmask));
+                    const uint32_t f = (uint32_t)(key >> 32);
+                    const int32_t node = (int32_t)(uint32_t)key;
+                    // the node's word, row and heuristic input in one round trip
+                    const uint64_t word = ld_gp(a.gp + node);
+                    const int32_t rb = a.g.off[node], re = a.g.off[node + 1];
+                    const int32_t hn = heur_eval<HK>(a.h, node);
+                    if (f < F && (uint32_t)(word >> 32) == f) {
+                        u = node;
+                        gu = f - (uint32_t)hn;
+                        start = (uint32_t)rb;
+                        deg = (uint32_t)(re - rb);
+                        if (sub == 0) C.expanded++;
+                    } else if (sub == 0) {
+                        ++stale;
+                    }
+                }
+                if (__any(deg > (uint32_t)kPgSeg)) {
+                    uint32_t at = 0;
+                    const uint32_t parts = (deg + kPgSeg - 1) / kPgSeg;
+                    if (deg > (uint32_t)kPgSeg && sub == 0) at = add_u32(slot + PG_HUBS, parts);
+                    at = __shfl(at, wl - sub, 64);
+                    if (deg > (uint32_t)kPgSeg) {
+                        // (a row the list has no room for stays with its group, its places empty)
+                        const bool fits = at + parts <= a.hubcap;
+                        for (uint32_t k = sub; k < parts && at + k < a.hubcap; k += kPgLanes) {
+                            const uint32_t o = k * kPgSeg, len = deg - o < (uint32_t)kPgSeg ? deg - o : kPgSeg;
+                            st_u64(a.hubs + 2 * (uint64_t)(at + k), (uint64_t)(fits ? len : 0) << 32 | (start + o));
+                            st_u64(a.hubs + 2 * (uint64_t)(at + k) + 1, (uint64_t)gu << 32 | (uint32_t)u);
+                        }
+                        if (fits) deg = 0;
+                    }
+                }
+                pg_expand<B, HK>(a, start, deg, u, gu, F, C, push);
+                if (a.g.lhead) {
+                    // Versioned inserts: the group's first lane walks the node's
+                    // list, oldest first, up to the first entry newer than this
+                    // version (links carry the inserting version).
+                    uint64_t link = u >= 0 && sub == 0 ? ld_gp(a.g.lhead + u) : ~0ull;
+                    for (;;) {
+                        bool active = false;
+                        int32_t x = -1;
+                        while ((uint32_t)link <= (uint32_t)a.g.ver) {
+                            x = (int32_t)(link >> 32);
+                            link = ld_gp(a.g.lnext + x);
+                            if (a.g.ldel[x] > a.g.ver) {
+                                active = true;
+                                break;
+                            }
+                        }
+                        if (!__any(active)) break;
+                        bool has[1] = {false};
+                        uint64_t key[1] = {0};
+                        if (active) {
+                            C.edges++;
+                            const int32_t cn = a.g.lv[x];
+                            const int32_t hcn = heur_eval<HK>(a.h, cn);
+                            if (HK != DDP_H_ARRAY || hcn >= 0) {
+                                const uint32_t cand = gu + a.g.lw[x] + (uint32_t)hcn;
+                                uint64_t prev;
+                                if (relax_gp(a.gp, cn, cand, (uint32_t)u, &prev)) {
+                                    C.improved++;
+                                    if (cn == a.t) {
+                                        push.target(cand);
+                                    } else {
+                                        has[0] = true;
+                                        key[0] = (uint64_t)cand << 32 | (uint32_t)cn;
+                                    }
+                                }
+                            }
+                        }
+                        push.template all<1>(has, key);
+                    }
+                }
+            }
+            if (split) {
+                const uint32_t stride = gridDim.x * B, trips = (fn + stride - 1) / stride;
+                for (uint32_t r = 0; r < trips; ++r) {  // uniform: the appends are wave-wide
+                    const uint64_t i = (uint64_t)r * stride + (uint64_t)blockIdx.x * B + lane;
+                    uint64_t key[1] = {0};
+                    bool live[1] = {false};
+                    if (i < fn) {
+                        key[0] = ld_gp(far + i);
+                        const uint32_t f = (uint32_t)(key[0] >> 32);
+                        live[0] = f < F && (uint32_t)(ld_gp(a.gp + (uint32_t)key[0]) >> 32) == f;
+                        C.scanned++;
+                    }
+                    push.template all<1>(live, key);
+                }
+            }
+            push.flush();
+        }
+        if (!grid_sync(ctrl + PG_BAR, gridDim.x, gen, a.barrier_ticks, &s_flag)) {
+            timeout = true;
+            break;
+        }
+        ++step;
+        const uint32_t hubs0 = ld_u32(slot + PG_HUBS), hubs = hubs0 < a.hubcap ? hubs0 : a.hubcap;
+        {
+            const uint32_t tm = ld_u32(slot + PG_TMIN);
+            F = tm < F ? tm : F;
+            head += n;
+            tail += ld_u32(slot + PG_NEAR);
+            fn = (split ? 0 : fn) + ld_u32(slot + PG_FAR);
+            const uint32_t fm = ld_u32(slot + PG_FMIN);
+            low = !split && low < fm ? low : fm;
+            err |= ld_u32(slot + PG_ERR);
+        }
+        if (split) {
+            uint64_t *tmp = far;
+            far = far2;
+            far2 = tmp;
+        }
+        if (err) break;
+        if (hubs) {
+            // ---- step 2: the segments of long rows
+            slot = begin();
+            PgPush<B> push{&S, &a, slot, tail, head, far, fn, thr, F};
+            const uint32_t chunks = (hubs + kPerWave - 1) / kPerWave;
+            for (uint32_t ch = (lane >> 6) * gridDim.x + blockIdx.x; ch < chunks; ch += kWaves * gridDim.x) {
+                const uint32_t i = ch * kPerWave + wl / kPgLanes;
+                uint64_t row = 0, from = 0;
+                if (i < hubs) {
+                    row = ld_gp(a.hubs + 2 * (uint64_t)i);
+                    from = ld_gp(a.hubs + 2 * (uint64_t)i + 1);
+                }
+                pg_expand<B, HK>(a, (uint32_t)row, (uint32_t)(row >> 32), (int32_t)(uint32_t)from,
+                                 (uint32_t)(from >> 32), F, C, push);
+            }
+            push.flush();
+            if (!grid_sync(ctrl + PG_BAR, gridDim.x, gen, a.barrier_ticks, &s_flag)) {
+                timeout = true;
+                break;
+            }
+            ++step;
+            const uint32_t tm = ld_u32(slot + PG_TMIN);
+            F = tm < F ? tm : F;
+            const uint32_t fm = ld_u32(slot + PG_FMIN);
+            low = low < fm ? low : fm;
+            tail += ld_u32(slot + PG_NEAR);
+            fn += ld_u32(slot + PG_FAR);
+            err |= ld_u32(slot + PG_ERR);
+            if (err) break;
+        }
+    }
+    if (timeout && lane == 0) atomicOr(ctrl + GA_RES_ERR, (uint32_t)GA_ERR_BARRIER);
+    if (blockIdx.x == 0 && lane == 0) {
+        if (err) atomicOr(ctrl + GA_RES_ERR, err);
+        ctrl[GA_RES_IT] = (uint32_t)it;
+        ctrl[GA_RES_F] = F;
+    }
+    const uint64_t v0 = wave_sum_u64(C.expanded), v1 = wave_sum_u64(C.edges), v2 = wave_sum_u64(C.improved),
+                   v3 = wave_sum_u64(stale);
+    if (wl == 0) {
+        atomicAdd(a.stats + 0, (unsigned long long)v0);
+        atomicAdd(a.stats + 1, (unsigned long long)v1);
+        atomicAdd(a.stats + 2, (unsigned long long)v2);
+        atomicAdd(a.stats + 3, (unsigned long long)v3);
+    }
+}

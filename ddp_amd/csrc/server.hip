@@ -22,8 +22,8 @@
 //
 // Grid mode at low load (opts.grid_k): a query that server_route_grid sends
 // there (nothing else in flight, or arrivals slow enough for grid mode to
-// keep up) is searched by the single-query GA* grid kernel (K lane heaps over
-// the whole GPU, gastar.hip) instead of one slot.  Its ring entry is marked
+// keep up) is searched by the single-query grid mode (piles over the whole
+// GPU, grid_piles.h) instead of one slot.  Its ring entry is marked
 // so that the serve kernel skips it, and its search runs on the server's
 // stream after any serve kernel (which is told to stop: its running slots
 // finish their requests and claim nothing published after the entry) and

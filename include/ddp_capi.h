@@ -162,18 +162,21 @@ int ddp_bfs_hops_noalloc(ddp_ctx *ctx, const ddp_graph *g, int32_t t,
 /* ------------------------------------------------------ single-query GA* */
 
 typedef struct {
-    int32_t K;          /* number of priority queues (one per lane); 0 = 1024 */
-    int32_t block;      /* lanes per workgroup; grid mode: 64, 256 or 1024; 0 = auto
+    int32_t K;          /* number of priority queues (one per lane; grid mode: entries a
+                           window feeds at least); 0 = 1024 */
+    int32_t block;      /* lanes per workgroup; grid mode: 64, 256 or 1024 (rounds K up to a
+                           multiple; the grid's own workgroups have 1,024 lanes); 0 = auto
                            (grid mode: 64 below K = 4096, 256 below 65536, 1024 from there) */
-    int32_t heap_cap;   /* entries per queue (LDS part + HBM spill); 0 = auto */
+    int32_t heap_cap;   /* entries per queue (grid mode: K * heap_cap in all); 0 = auto */
     int32_t lds_cap;    /* heap entries per queue kept in LDS; 0 = auto */
     int32_t max_iters;  /* iteration limit; 0 = auto (bounded) */
     int32_t mode;       /* DDP_ASTAR_AUTO / _GRID / _WORKGROUP / _PILES / _BIDI */
     int32_t reserved[2];
 } ddp_astar_opts_t;
 
-/* Execution modes of the single-query search.  GRID spreads the K queues over
- * K/block workgroups that meet at a device-wide barrier every iteration.
+/* Execution modes of the single-query search.  GRID runs near/far piles over
+ * the whole GPU: 64 workgroups, or one per CU on large graphs without a
+ * geometric heuristic, that meet at a device-wide barrier every round.
  * WORKGROUP keeps all K <= 1024 queues in one workgroup (block = K rounded up
  * to a power of two >= 64): no device-wide barrier, but one CU's worth of
  * memory parallelism.  PILES runs the search on one workgroup of K <= 1024
