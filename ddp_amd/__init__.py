@@ -7,6 +7,7 @@ LIB/include/a_star.cuh:12-51).
 """
 import ctypes
 import os
+import struct
 import weakref
 from ctypes import byref, c_int32, c_uint32, c_void_p
 
@@ -247,8 +248,11 @@ class HostGraph:
 
 
 def _updates_array(lines):
+    from ._hostconv import fill  # built with the library
     arr = (Update * max(1, len(lines)))()
-    for i, l in enumerate(lines):
+    if fill(lines, arr):
+        return arr
+    for i, l in enumerate(lines):  # other sequences and number types
         arr[i].flag, arr[i].u, arr[i].v, arr[i].w = int(l[0]), int(l[1]), int(l[2]), int(l[3])
     return arr
 
@@ -562,8 +566,13 @@ def alternative_paths(ctx, hg, s, t, num_paths, h=None, K=0):
         d.close()
 
 
-def _result_dict(r):
-    return {f: getattr(r, f) for f, _ in _capi.ServerResult._fields_}
+_RESULT_FIELDS = [f for f, _ in _capi.ServerResult._fields_]
+
+
+def _result_dicts(results, n):
+    """The first n of a ServerResult array as dicts."""
+    raw = ctypes.string_at(results, n * ctypes.sizeof(_capi.ServerResult))
+    return [dict(zip(_RESULT_FIELDS, t)) for t in struct.iter_unpack(_capi.SERVER_RESULT_FORMAT, raw)]
 
 
 class Server:
@@ -602,7 +611,7 @@ class Server:
         buf = (_capi.ServerResult * max_results)()
         n = c_int32()
         _check(_capi.lib().ddp_server_poll(self._h, buf, max_results, byref(n)), self.ctx.handle)
-        return [_result_dict(buf[i]) for i in range(n.value)]
+        return _result_dicts(buf, n.value)
 
     def drain(self, timeout_ms=600000):
         _check(_capi.lib().ddp_server_drain(self._h, timeout_ms), self.ctx.handle)
@@ -630,7 +639,7 @@ class Server:
         out = (_capi.ServerResult * max(1, n))()
         _check(_capi.lib().ddp_server_replay(self._h, n, ptr_f64(arr), ptr_i32(ty), ptr_i32(s), ptr_i32(t),
                                              ptr_i32(uo), ua, out), self.ctx.handle)
-        return [_result_dict(out[i]) for i in range(n)]
+        return _result_dicts(out, n)
 
     def close(self):
         if getattr(self, "_h", None):

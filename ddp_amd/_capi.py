@@ -94,6 +94,9 @@ class ServerResult(ctypes.Structure):
                 ("submit_ms", c_double), ("done_ms", c_double), ("device_ms", c_double)]
 
 
+SERVER_RESULT_FORMAT = "Q4i3d"  # the struct module's name for ServerResult
+
+
 P_I32 = POINTER(c_int32)
 P_U32 = POINTER(c_uint32)
 P_F64 = POINTER(c_double)

@@ -269,7 +269,7 @@ __device__ void apply_update(const ServeArgs &a, const Req &rq, uint32_t *s_err)
 // 0.5 us each) and neither host reads nor system-scope cache invalidations,
 // which it took per claim while entries were read from host memory: a burst of
 // 1,024 requests, every twentieth an update batch, on a 200,000-node map took
-// 62 ms, one claim every 60 us; it takes 13 ms now (5 ms without updates, 3 of
+// 62 ms, one claim every 60 us; it takes 11 ms now (5 ms without updates, 3 of
 // them its longest query).
 //
 // A slot counts itself busy once it has claimed, and the launch closes (every
