@@ -21,7 +21,7 @@
 // narrow one (32 workgroups of 256 lanes, a cheap barrier) runs levels of up
 // to kNarrowMax segments, the wide one (a workgroup of 1,024 lanes per CU) the
 // others; each returns when the next level is not its own.
-// Measured against one grid of 512 workgroups, node queue, grid_barrier (whole
+// Measured against one grid of 512 workgroups, node queue, fenced barrier (whole
 // call, result on the host): random graph of 100,000 nodes 0.87 -> 0.125 ms,
 // R-MAT scale 20 (1M nodes, 16.8M edges) 21.8 -> 1.24 ms, 2048 x 2048 maze (4,600
 // levels of about 640 nodes) 273 -> 18.9 ms (4.0 us a level).

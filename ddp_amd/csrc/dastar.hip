@@ -1,7 +1,6 @@
 // Dynamic A* (DA*): repair one query's search state after a batch of edge
-// inserts and deletes, then resume the search from its retained open set --
-// the GA* grid kernel's queues, or the one-workgroup pile engine's dormant
-// pile (DDP_ASTAR_PILES).
+// inserts and deletes, then resume the search from its retained open set (the
+// dormant pile of grid_piles.h).
 //
 // Invariant kept between batches (the one A* itself maintains): every finite
 // g is the cost of a real path, and every node that is not in a queue has
@@ -34,9 +33,8 @@
 
 #include "../../include/ddp_dastar.h"
 #include "compact.h"
-#include "gastar.h"
+#include "grid_piles.h"
 #include "host_sort.h"
-#include "slot_search.h"
 
 namespace {
 
@@ -48,9 +46,33 @@ using clk = std::chrono::steady_clock;
 // order, which the insert lists rely on.
 float ms_since(clk::time_point t0) { return std::chrono::duration<float, std::milli>(clk::now() - t0).count(); }
 
-enum : int { RC_NEXT = 0, RC_MARKED = 1, RC_ROOTS = 2, RC_REPULLED = 3, RC_PUSHES = 4, RC_WORDS = 16 };
+// Two batches of 20,000 lines on the 1,000,000-node graph and the path between,
+// from Python: 3.8 ms with one workgroup resuming the search, fences in the
+// walk's barrier and five more launches and copies a batch, 2.2 ms now; a full
+// recompute on 100,000 nodes 4.3 ms (one workgroup) and 0.77 ms (lane heaps)
+// before, 0.36 ms now.
+//
+// One device block holds every small word of a batch, cleared by one kernel
+// and read back in one copy: the search's control words (grid_piles.h), the
+// search counters, the repair's counters, open_split's, the walk's barrier.
+enum : int {
+    DC_STATS = GA_CTRL_WORDS, DC_REPAIR = DC_STATS + 16, DC_SPLIT = DC_REPAIR + 16, DC_WALK = DC_SPLIT + 32,
+    DC_WORDS = DC_WALK + 96
+};
+enum : int {
+    RC_MARKED = 0, RC_ROOTS = 1, RC_REPULLED = 2, RC_PUSHES = 3, RC_DEL_BASE = 4, RC_DEL_LOG = 5, RC_WALKED = 6,
+    RC_WALK_ERR = 7
+};
+// open_split: live and kept entries, overflow, smallest live f
+enum : int { SP_LIVE = 0, SP_KEEP = 1, SP_OVF = 2, SP_MIN = 3 };
 
-enum : int { RC_DEL_BASE = 5, RC_DEL_LOG = 6, RC_WALKED = 7, RC_WALK_ERR = 8 };
+__global__ void da_begin(uint32_t *ctl)
+{
+    for (int k = threadIdx.x; k < DC_WORDS; k += blockDim.x) {
+        const int w = k >= PG_SLOTS && k < PG_BAR ? (k - PG_SLOTS) % PG_SLOT_WORDS : -1;
+        ctl[k] = w == PG_TMIN || w == PG_FMIN || k == DC_SPLIT + SP_MIN ? 0xFFFFFFFFu : 0u;
+    }
+}
 
 // The log of inserted edges: entry x is u -> v with weight w, live while
 // del[x] == INT32_MAX.  head/next links pack (entry << 32 | 0); the end of a
@@ -66,27 +88,22 @@ struct InsLog {
 
 __device__ __forceinline__ bool link_end(uint64_t link) { return (uint32_t)link != 0u; }
 
-// Appends the children claimed in one group to the next level (nxt[k - base]
-// for draw k of *next_cnt) and to the marked list: wave-collective (every
-// lane of the wave calls it), one counter atomic per wave and list.  Per-node
-// atomics on two shared counters serialised in L2 and made the walk of a C3
-// batch (12,500 invalidated nodes) take about 340 us.  Both lists hold at
-// most cap (N) entries, as each node is claimed once per epoch; a store past
-// that is dropped rather than written out of bounds.
+// Appends claimed nodes to the marked list: wave-collective (every lane of the
+// wave calls it), one counter atomic per wave.  (Per-node atomics on a shared
+// counter serialised in L2 and made the walk of a C3 batch, 12,500 invalidated
+// nodes, take about 340 us.)  The list holds at most cap (N) entries, as each
+// node is claimed once per epoch; a store past that is dropped rather than
+// written out of bounds.  Stores are agent-scope: other workgroups of the walk
+// read the list after a barrier without fences.
 template <int K>
-__device__ __forceinline__ void append_claims(const bool (&sel)[K], const int32_t (&y)[K], uint32_t *next_cnt,
-                                              uint32_t base, int32_t *nxt, uint32_t *marked_cnt, int32_t *marked,
-                                              uint32_t cap)
+__device__ __forceinline__ void append_claims(const bool (&sel)[K], const int32_t (&y)[K], uint32_t *count,
+                                              int32_t *marked, uint32_t cap)
 {
     uint32_t pos[K];
-    wave_append<K>(sel, next_cnt, pos);
+    wave_append<K>(sel, count, pos);
 #pragma unroll
     for (int k = 0; k < K; ++k)
-        if (sel[k] && pos[k] - base < cap) nxt[pos[k] - base] = y[k];
-    wave_append<K>(sel, marked_cnt, pos);
-#pragma unroll
-    for (int k = 0; k < K; ++k)
-        if (sel[k] && pos[k] < cap) marked[pos[k]] = y[k];
+        if (sel[k] && pos[k] < cap) st_u32((uint32_t *)marked + pos[k], (uint32_t)y[k]);
 }
 
 // Deletes, one thread per line: the first live instance of u -> v, base row
@@ -98,7 +115,7 @@ __device__ __forceinline__ void append_claims(const bool (&sel)[K], const int32_
 // each wave adds its counts with one atomic per counter.
 __global__ void apply_deletes(const int32_t *pairs, int32_t n, GraphView F, int32_t *col, int32_t *rcol,
                               const int32_t *roff, const int32_t *reid, InsLog L, const uint64_t *gp, int32_t *mark,
-                              int32_t epoch, int32_t *front, int32_t *marked, uint32_t *rctrl)
+                              int32_t epoch, int32_t *marked, uint32_t *rctrl)
 {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     int32_t u = -1, v = -1;
@@ -155,39 +172,41 @@ __global__ void apply_deletes(const int32_t *pairs, int32_t n, GraphView F, int3
         if (ml) atomicAdd(rctrl + RC_DEL_LOG, (uint32_t)__popcll(ml));
         if (mr) atomicAdd(rctrl + RC_ROOTS, (uint32_t)__popcll(mr));
     }
-    append_claims<1>(root, rv, rctrl + RC_NEXT, 0u, front, rctrl + RC_MARKED, marked, (uint32_t)F.N);
+    append_claims<1>(root, rv, rctrl + RC_MARKED, marked, (uint32_t)F.N);
 }
 
-// New log entries: one thread per group of equal keys (entries arrive sorted
-// by key, stably, so a group keeps insert order) appends the group to the
-// key's list.  grp holds (key, entry) pairs.
-__global__ void log_append(const int32_t *grp, int32_t n, uint64_t *head, uint64_t *next, int32_t *tail)
+// A batch's inserts, one launch: row 0 of the grid fills the new log entries at
+// + k from the uploaded (u, v, w) triples, live (del = INT32_MAX) until a later
+// batch deletes them; rows 1 and 2 thread them onto the lists by source and by
+// target.  fg and rg hold (key, entry) pairs sorted by key, stably, so a group
+// keeps insert order; the first thread of a group appends it.
+__global__ void log_insert(const int32_t *ins, const int32_t *fg, const int32_t *rg, int32_t n, InsLog L, int64_t at)
 {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
+    if (blockIdx.y == 0) {
+        L.u[at + i] = ins[3 * i];
+        L.v[at + i] = ins[3 * i + 1];
+        L.w[at + i] = (uint32_t)ins[3 * i + 2];
+        L.del[at + i] = INT32_MAX;
+        return;
+    }
+    const bool by_source = blockIdx.y == 1;
+    const int32_t *grp = by_source ? fg : rg;
+    uint64_t *head = by_source ? L.fhead : L.rhead, *next = by_source ? L.fnext : L.rnext;
+    int32_t *tail = by_source ? L.ftail : L.rtail;
     const int32_t key = grp[2 * i];
     if (i > 0 && grp[2 * (i - 1)] == key) return;
+    int32_t last = tail[key];
     for (int32_t k = i; k < n && grp[2 * k] == key; ++k) {
         const int32_t x = grp[2 * k + 1];
         next[x] = ~0ull;
         const uint64_t link = (uint64_t)(uint32_t)x << 32;
-        const int32_t last = tail[key];
         if (last < 0) head[key] = link;
         else next[last] = link;
-        tail[key] = x;
+        last = x;
     }
-}
-
-// New log entries at + k from the uploaded (u, v, w) triples, live (del =
-// INT32_MAX) until a later batch deletes them.
-__global__ void log_fill(const int32_t *ins, int32_t n, InsLog L, int64_t at)
-{
-    const int32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    L.u[at + k] = ins[3 * k];
-    L.v[at + k] = ins[3 * k + 1];
-    L.w[at + k] = (uint32_t)ins[3 * k + 2];
-    L.del[at + k] = INT32_MAX;
+    tail[key] = last;
 }
 
 __global__ void fill_i32(int32_t *p, int64_t n, int32_t v)
@@ -202,32 +221,14 @@ __global__ void fill_u64(uint64_t *p, int64_t n, uint64_t v)
         p[i] = v;
 }
 
-// Where the children claimed in a level go (wave-collective append<K>):
-// GlobalSink lists them in nxt[k - base] for draw k of a device counter (the
-// wide levels, one launch over the grid each); WalkSink keeps a level in LDS
-// and sends what does not fit to the device buffer `out` (the narrow levels
-// of subtree_walk).  Both add each claimed node to the marked list.
-struct GlobalSink {
-    uint32_t *next_cnt, *marked_cnt;
-    uint32_t base;
-    int32_t *nxt, *marked;
-    uint32_t cap;  // entries of nxt and marked (N)
-    template <int K>
-    __device__ void append(const bool (&sel)[K], const int32_t (&y)[K])
-    {
-        append_claims<K>(sel, y, next_cnt, base, nxt, marked_cnt, marked, cap);
-    }
-};
-
 // One node x of a level of the parent-subtree walk (x < 0: none): its
 // children are its live out-neighbours y whose parent is x.  A node has one
 // parent and every root is marked before the walk, so a child is reached
 // from one lane only (its parent's) once per epoch: reading its mark with
 // its word and storing the epoch claims it without an atomic round trip.
 // Wave-collective: the loop runs while any lane of the wave has work.
-template <class Sink>
 __device__ __forceinline__ void claim_children(const GraphView &G, const InsLog &L, int32_t x, const uint64_t *gp,
-                                               int32_t *mark, int32_t epoch, Sink &sink)
+                                               int32_t *mark, int32_t epoch, uint32_t *count, int32_t *marked)
 {
     // Each step takes a group of 8 row entries and one entry of the inserted
     // list together: their columns and list fields in one round trip, then
@@ -275,33 +276,32 @@ __device__ __forceinline__ void claim_children(const GraphView &G, const InsLog 
             for (int q = 0; q < k; ++q) sel[k] = sel[k] && y[q] != y[k];
             if (sel[k]) mark[y[k]] = epoch;
         }
-        sink.template append<kG + 1>(sel, y);
+        append_claims<kG + 1>(sel, y, count, marked, (uint32_t)G.N);
     }
 }
 
-// Device-wide barrier of the subtree walk over nblocks co-resident
-// workgroups (bar[0] arrivals, bar[1] generation, bar[2] published count):
-// the last workgroup to arrive reads *cnt -- every workgroup's draws of the
-// level are in by then -- and publishes it with the new generation, so each
-// workgroup learns the level's total without racing the next level's draws.
-// Waits are bounded by limit_ticks of the 100 MHz clock (false on timeout).
+// Device-wide barrier of the subtree walk over nblocks co-resident workgroups
+// (bar[0] arrivals, bar[32] generation, bar[64] published count): the last
+// workgroup to arrive reads *cnt -- every workgroup's draws of the level are
+// in by then -- and publishes it with the new generation, so each workgroup
+// learns the level's total without racing the next level's draws.  No fences
+// (see grid_sync): the walk shares its list, the marks and the counters
+// through agent-scope accesses.  Waits are bounded by limit_ticks of the
+// 100 MHz clock (false on timeout).
 __device__ __forceinline__ bool walk_barrier(uint32_t *bar, uint32_t nblocks, uint32_t &gen, const uint32_t *cnt,
                                              uint64_t limit_ticks, int32_t *s_flag, uint32_t *s_total)
 {
     block_sync_global();  // every wave's draws and stores reach L2 first
     if (threadIdx.x == 0) {
         bool ok = true;
-        __threadfence();
-        const uint32_t arrived = atomicAdd(&bar[0], 1u);
-        if (arrived == nblocks - 1) {
-            __threadfence();
-            const uint32_t total = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&bar[2], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&bar[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&bar[1], gen + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        if (add_u32(bar, 1u) == nblocks - 1) {
+            st_u32(bar + 64, ld_u32(cnt));
+            st_u32(bar, 0u);
+            wait_vmem();
+            st_u32(bar + 32, gen + 1);
         } else {
             const uint64_t t0 = dev_clock_100mhz();
-            while (__hip_atomic_load(&bar[1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) == gen) {
+            while (ld_u32(bar + 32) == gen) {
                 __builtin_amdgcn_s_sleep(1);
                 if (dev_clock_100mhz() - t0 > limit_ticks) {
                     ok = false;
@@ -309,8 +309,7 @@ __device__ __forceinline__ bool walk_barrier(uint32_t *bar, uint32_t nblocks, ui
                 }
             }
         }
-        __threadfence();
-        *s_total = __hip_atomic_load(&bar[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *s_total = ld_u32(bar + 64);
         *s_flag = ok ? 1 : 0;
     }
     gen += 1;
@@ -319,84 +318,61 @@ __device__ __forceinline__ bool walk_barrier(uint32_t *bar, uint32_t nblocks, ui
 }
 
 // The parent-subtree walk in one launch over kWalkGrid co-resident
-// workgroups: level after level, each ended by walk_barrier.  Node i of a
+// workgroups: level after level, each ended by walk_barrier.  The marked list
+// is the walk's queue: apply_deletes put the roots there, and a level is what
+// the one before appended (each node is claimed once per epoch).  Node i of a
 // level goes to workgroup i % kWalkGrid, so even a level of a few hundred
 // nodes spreads over kWalkGrid CUs: one workgroup walking alone was bound
 // by its CU's gather rate (about 35 ns per node, 42 us for a level of 1,200
 // nodes).  Sixteen workgroups (4,096 lanes) still take a C3 level in one
 // pass and their barrier is cheaper than 32's or 64's: the repair's device
-// time per C3 batch was 0.250, 0.259 and 0.296 ms with 16, 32 and 64.  The
-// roots are the rctrl[RC_NEXT] draws apply_deletes made into buf0; later
-// levels alternate between buf1 and buf0 (each at most N nodes: every node is
-// claimed once per epoch).  On exit rctrl[RC_WALKED] holds the number of
-// levels, and RC_WALK_ERR is set if a barrier timed out.
+// time per C3 batch was 0.250, 0.259 and 0.296 ms with 16, 32 and 64.  On exit
+// rctrl[RC_WALKED] holds the number of levels, and RC_WALK_ERR is set if a
+// barrier timed out.
 constexpr int kWalkGrid = 16, kWalkGridBlock = 256;
 
 __global__ void __launch_bounds__(kWalkGridBlock)
-    subtree_walk(GraphView G, InsLog L, const uint64_t *gp, int32_t *mark, int32_t epoch, int32_t *buf0,
-                 int32_t *buf1, int32_t *marked, uint32_t *rctrl, uint32_t *bar, uint64_t limit_ticks)
+    subtree_walk(GraphView G, InsLog L, const uint64_t *gp, int32_t *mark, int32_t epoch, int32_t *marked,
+                 uint32_t *rctrl, uint32_t *bar, uint64_t limit_ticks)
 {
     __shared__ int32_t s_flag;
     __shared__ uint32_t s_total;
     const uint32_t N = (uint32_t)G.N;
-    uint32_t gen = 0;
-    int32_t *cur = buf0, *nxt = buf1;
-    uint32_t base = __hip_atomic_load(rctrl + RC_NEXT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    uint32_t ncur = base < N ? base : N;
-    uint32_t levels = 0;
-    while (ncur > 0) {
-        GlobalSink sink{rctrl + RC_NEXT, rctrl + RC_MARKED, base, nxt, marked, N};
-        const uint32_t per = (ncur + kWalkGrid - 1) / kWalkGrid;  // this workgroup's share, at most
-        for (uint32_t s0 = 0; s0 < per; s0 += kWalkGridBlock) {   // uniform trips: the appends are wave-wide
+    uint32_t gen = 0, base = 0, end = ld_u32(rctrl + RC_MARKED), levels = 0;
+    end = end < N ? end : N;
+    while (base < end) {
+        const uint32_t ncur = end - base, per = (ncur + kWalkGrid - 1) / kWalkGrid;  // this workgroup's share, at most
+        for (uint32_t s0 = 0; s0 < per; s0 += kWalkGridBlock) {  // uniform trips: the appends are wave-wide
             const uint32_t slot = s0 + threadIdx.x;
             const uint32_t i = slot * kWalkGrid + blockIdx.x;
-            claim_children(G, L, (slot < per && i < ncur) ? cur[i] : -1, gp, mark, epoch, sink);
+            const int32_t x = slot < per && i < ncur ? (int32_t)ld_u32((const uint32_t *)marked + base + i) : -1;
+            claim_children(G, L, x, gp, mark, epoch, rctrl + RC_MARKED, marked);
         }
-        if (!walk_barrier(bar, gridDim.x, gen, rctrl + RC_NEXT, limit_ticks, &s_flag, &s_total)) {
+        if (!walk_barrier(bar, gridDim.x, gen, rctrl + RC_MARKED, limit_ticks, &s_flag, &s_total)) {
             if (threadIdx.x == 0) atomicOr(rctrl + RC_WALK_ERR, 1u);
             break;
         }
-        const uint32_t total = s_total;
-        ncur = total - base < N ? total - base : N;
-        base = total;
-        int32_t *tmp = cur;
-        cur = nxt;
-        nxt = tmp;
+        base = end;
+        end = s_total < N ? s_total : N;
         ++levels;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) rctrl[RC_WALKED] = levels;
 }
 
+// Nodes the repair gave a new value: open entries for the search (rctrl's
+// RC_PUSHES of them).  The target is never queued; its value is in its word.
 struct RepairPush {
-    uint64_t *buf;     // push buffer of "iteration -1"
-    uint32_t *slot;    // control slot 2
-    int32_t pcap;
+    uint64_t *buf;
+    uint32_t cap;
     uint32_t *rctrl;
     int32_t t;
 
     __device__ void push(bool has, int32_t v, uint32_t f)
     {
-        if (has && v == t) {
-            atomicMin(slot + GA_S_TMIN, f);  // the target is never queued
-            has = false;
-        }
-        const uint64_t mask = __ballot(has);
-        if (!mask) return;
-        const int lane = threadIdx.x & 63;
-        const int leader = __builtin_ctzll(mask);
-        const uint32_t fmin = wave_min_u32(has ? f : 0xFFFFFFFFu);  // one atomicMin per wave
-        uint32_t base = 0;
-        if (lane == leader) {
-            base = atomicAdd(slot + GA_S_PUSHCNT, (uint32_t)__popcll(mask));
-            atomicAdd(rctrl + RC_PUSHES, (uint32_t)__popcll(mask));
-            atomicMin(slot + GA_S_PUSHMIN, fmin);
-        }
-        base = __shfl(base, leader, 64);
-        if (has) {
-            const uint32_t idx = base + lane_rank(mask);
-            if (idx < (uint32_t)pcap) buf[idx] = ((uint64_t)f << 32) | (uint32_t)v;
-            else atomicOr(slot + GA_S_ERR, 2u);
-        }
+        const bool sel[1] = {has && v != t};
+        uint32_t pos[1];
+        wave_append<1>(sel, rctrl + RC_PUSHES, pos);
+        if (sel[0] && pos[0] < cap) buf[pos[0]] = ((uint64_t)f << 32) | (uint32_t)v;  // open_split reports the rest
     }
 };
 
@@ -501,26 +477,13 @@ __global__ void relax_inserts(const int32_t *ins, int32_t n, const int32_t *h, u
     P.push(has, v, cand);
 }
 
-// The search behind DA* in pile mode: one workgroup runs the pile engine of
-// the batched slots (slot_search.h) resumed from the retained open set -- the
-// dormant pile of the previous search plus this batch's repair pushes -- with
-// F(t) read from the target's word.  Its rounds synchronise through LDS
-// barriers only, where the grid mode pays a device-wide barrier per
-// iteration; a repair's few-hop propagation is bound by that per-round
-// latency.  Entries that cannot beat F(t) now are kept (dormant) for later
-// batches, which may raise F(t) again.
-constexpr int kPileBlock = 1024;
-
-// open_split counters
-enum { SP_LIVE = 0, SP_KEEP = 1, SP_OVF = 2, SP_WORDS = 4 };
-
-// Ahead of the one-workgroup search, the whole GPU splits the retained open
+// Ahead of the search, the whole GPU splits the retained open
 // set and this batch's repair pushes around F(t): current entries below it
 // (live) seed the search, current entries at or above it stay dormant
 // (keep), and stale ones -- the node's word has moved on, so an entry with
 // its current f exists elsewhere -- are dropped.  The search then scans only
-// the live entries, where it used to scan the whole retained set (1.3M+
-// entries on the 1M-node graph of 8 out-edges) on its one CU every batch.
+// the live entries and not the whole retained set (1.3M+ entries on the 1M-node
+// graph of 8 out-edges) every time it splits its far pile.
 // Live entries are always checked; kept ones only with check_all (a random
 // word read each: the caller asks for it when the retained set has grown),
 // since a stale kept entry costs room, not correctness.
@@ -531,7 +494,7 @@ __global__ void __launch_bounds__(kSplitBlock)
                const uint64_t *gp, int32_t t, uint64_t *live, uint64_t *keep, uint32_t cap, uint32_t *cnt,
                int32_t check_all)
 {
-    __shared__ uint32_t s_wc[2][kSplitBlock / 64], s_base[2];
+    __shared__ uint32_t s_wc[2][kSplitBlock / 64], s_base[2], s_min;
     const uint32_t np0 = __hip_atomic_load(push_n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint32_t np = np0 < pcap ? np0 : pcap;
     if (np0 > pcap && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(cnt + SP_OVF, 1u);
@@ -557,7 +520,8 @@ __global__ void __launch_bounds__(kSplitBlock)
         const bool need = i < n && v != t && ((uint32_t)(key[k] >> 32) < F0 || check_all);
         word[k] = need ? ld_gp(gp + v) : 0;
     }
-    uint32_t mine[2] = {0, 0};
+    uint32_t mine[2] = {0, 0}, mymin = 0xFFFFFFFFu;  // the smallest live f is the search's first window
+    if (threadIdx.x == 0) s_min = 0xFFFFFFFFu;
 #pragma unroll
     for (int k = 0; k < kSplitPer; ++k) {
         const uint64_t i = b0 + (uint64_t)k * kSplitBlock + threadIdx.x;
@@ -569,6 +533,7 @@ __global__ void __launch_bounds__(kSplitBlock)
         }
         mine[0] += sel[0][k];
         mine[1] += sel[1][k];
+        if (sel[0][k] && f < mymin) mymin = f;
     }
     // one reservation per workgroup and list: prefix over the threads
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -579,13 +544,16 @@ __global__ void __launch_bounds__(kSplitBlock)
         pre[l] = x - mine[l];
         if (lane == 63) s_wc[l][wid] = x;
     }
+    mymin = wave_min_u32(mymin);
     __syncthreads();
+    if (lane == 0 && mymin != 0xFFFFFFFFu) atomicMin(&s_min, mymin);
     if (threadIdx.x < 2) {
         uint32_t tot = 0;
         for (int w = 0; w < kSplitBlock / 64; ++w) tot += s_wc[threadIdx.x][w];
         s_base[threadIdx.x] = tot ? atomicAdd(cnt + threadIdx.x, tot) : 0u;
     }
     __syncthreads();
+    if (threadIdx.x == 64 && s_min != 0xFFFFFFFFu) atomicMin(cnt + SP_MIN, s_min);
 #pragma unroll
     for (int l = 0; l < 2; ++l) {
         uint32_t pos = s_base[l] + pre[l];
@@ -601,41 +569,13 @@ __global__ void __launch_bounds__(kSplitBlock)
     }
 }
 
-struct DaPileArgs {
-    GraphView g;
-    HeurView h;
-    uint64_t *gp;
-    uint64_t *live, *alt, *dorm;  // live entries in, far-pile partner, dormant pile (kept entries first)
-    uint64_t *near;               // ncap entries
-    uint32_t cap, ncap, lring, delta0;
-    const uint32_t *split;        // open_split counters
-    int32_t N, t, maxit;
-    uint32_t *res;                // iterations, F(t), error flags, dormant entries
-    unsigned long long *stats;
-};
-
-__global__ void __launch_bounds__(kPileBlock) dastar_pile_kernel(DaPileArgs a)
+// A fresh search: every word infinite but s's (fill_u64 before), s the whole open set.
+__global__ void da_seed(uint64_t *gp, uint64_t *open, const int32_t *h, int32_t s)
 {
-    extern __shared__ uint64_t s_ring[];
-    __shared__ SlotLds<kPileBlock, kPileBlock> S;
-    const int lane = threadIdx.x;
-    const uint32_t n_live = __hip_atomic_load(a.split + SP_LIVE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t n_keep = __hip_atomic_load(a.split + SP_KEEP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const bool fits = __hip_atomic_load(a.split + SP_OVF, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
-    const uint32_t F0 = (uint32_t)(ld_gp(a.gp + a.t) >> 32);
-    const PilePtrs P{a.near, a.live, a.alt, a.ncap, a.cap, s_ring, a.lring};
-    const PileResume Z{a.dorm, a.cap, fits ? n_live : 0u, F0, fits ? n_keep : 0u};
-    ExpandCounters C;
-    uint32_t stale = 0;
-    slot_search_piles<kPileBlock, DDP_H_ARRAY, 1, true>(a.g, a.h, a.gp, nullptr, P, a.N, -1, a.t, a.maxit, a.delta0, S,
-                                                        C, stale, &Z);
-    if (lane == 0) {
-        a.res[0] = (uint32_t)S.iters;
-        a.res[1] = S.F;
-        a.res[2] = S.err | (fits ? 0u : (uint32_t)QERR_HEAP);
-        a.res[3] = S.dorm_n;
-    }
-    slot_flush_stats<kPileBlock>(a.stats, C, stale);
+    if (threadIdx.x != 0) return;
+    const uint64_t hs = (uint64_t)(uint32_t)h[s] << 32;
+    gp[s] = hs | 0xFFFFFFFFull;
+    open[0] = hs | (uint32_t)s;
 }
 
 __global__ void map_h(const int32_t *in, int32_t *out, int32_t N)
@@ -677,9 +617,9 @@ struct ddp_dastar {
     int64_t compact_at = 0;     // log entries that trigger a compaction after a batch (0 = never)
     int32_t compactions = 0;
     int32_t *d_h = nullptr;
-    int32_t *d_mark = nullptr, *d_front = nullptr, *d_marked = nullptr;
-    uint32_t *d_rctrl = nullptr;
-    uint32_t *d_walkbar = nullptr;  // subtree_walk's device-wide barrier words
+    int32_t *d_mark = nullptr, *d_marked = nullptr;
+    uint32_t *d_ctl = nullptr;  // DC_WORDS
+    uint32_t *h_ctl = nullptr;  // pinned copy
     hipEvent_t ev_r0 = nullptr, ev_r1 = nullptr;  // around the repair's device work
     int32_t *d_work = nullptr;  // per-batch lines: delete pairs, insert triples, list groups
     size_t c_work = 0;
@@ -687,22 +627,19 @@ struct ddp_dastar {
     size_t c_hwork = 0;
     std::vector<int32_t> ku, kv, kx, tk, tv;  // host scratch of a batch's insert grouping
     int32_t epoch = 0;
-    // search
+    // search: the (f, parent) words, the repair's pushes, three rotating open-set
+    // buffers (open set in, far-pile partner, dormant pile out), the near ring
+    // and the segments of long rows
     GaGridPlan P{};
-    GaGridState S{};
     HeurView hv{};
-    int32_t rr = 0;
     uint32_t F = DDP_INF_F;
-    // pile mode (DDP_ASTAR_PILES): three rotating buffers (open set in,
-    // far-pile partner, dormant pile out), the HBM near ring and result words
-    bool piles = false;
+    uint64_t *gp = nullptr, *push = nullptr;
     uint64_t *pbuf[3] = {nullptr, nullptr, nullptr};
-    uint64_t *pnear = nullptr;
-    uint32_t *pres = nullptr;
-    uint32_t *d_split = nullptr;  // open_split counters
-    uint32_t pcap_open = 0, pncap = 0;
-    int32_t open_at = 0;   // which buffer holds the open set
-    uint32_t open_n = 0;   // its entries
+    uint64_t *pnear = nullptr, *phubs = nullptr;
+    uint32_t pcap_open = 0, pncap = 0, hubcap = 0;
+    bool rebuild = true;        // piles that overflow are rebuilt (no heap_cap was asked for)
+    int32_t open_at = 0;        // which buffer holds the open set
+    uint32_t open_n = 0;        // its entries
     uint32_t open_checked = 0;  // open_n after the last split that checked every entry
 };
 
@@ -721,11 +658,11 @@ static void dastar_free(ddp_dastar *d)
     if (d->h_work) hipHostFree(d->h_work);
     if (d->ev_r0) hipEventDestroy(d->ev_r0);
     if (d->ev_r1) hipEventDestroy(d->ev_r1);
-    ddp_ga_free(&d->S);
+    if (d->h_ctl) hipHostFree(d->h_ctl);
     log_free(d->L);
     void *ptrs[] = {d->L.fhead, d->L.rhead, d->L.ftail, d->L.rtail, d->d_reid, d->d_h,
-                    d->d_mark, d->d_front, d->d_marked, d->d_rctrl, d->d_walkbar, d->d_work,
-                    d->pbuf[0], d->pbuf[1], d->pbuf[2], d->pnear, d->pres, d->d_split};
+                    d->d_mark, d->d_marked, d->d_ctl, d->d_work, d->gp, d->push,
+                    d->pbuf[0], d->pbuf[1], d->pbuf[2], d->pnear, d->phubs};
     for (void *p : ptrs)
         if (p) hipFree(p);
     if (d->g) ddp_graph_destroy(d->g);
@@ -859,104 +796,98 @@ static int dastar_compact(ddp_dastar *d)
     return DDP_OK;
 }
 
-// One pile-mode search over the open set d->pbuf[open_at] (open_n entries)
-// plus the repair pushes counted in control slot 2; the dormant pile it leaves
-// becomes the next open set.
-// rctrl_out: also copies the repair counters back, in the same host round trip.
-static int pile_run(ddp_dastar *d, int32_t *iters, float *kms, uint32_t *rctrl_out = nullptr,
-                    unsigned long long *stats_out = nullptr)
+// One search over the open set d->pbuf[open_at] (open_n entries) plus the
+// repair pushes counted on the device; the dormant pile it leaves becomes the
+// next open set.  Waits for it; d->h_ctl then holds every small word.
+static int search_run(ddp_dastar *d, bool fresh, int32_t *iters, float *kms)
 {
     ddp_ctx *ctx = d->ctx;
-    DaPileArgs a{};
+    uint32_t *split = d->d_ctl + DC_SPLIT;
+    PgArgs a{};
     a.g = fwd_view(d);
     a.g.relax_min = d->g->minw >= 1;
     a.h = d->hv;
-    a.gp = d->S.gp;
+    a.gp = d->gp;
+    a.near = d->pnear;
+    a.nmask = d->pncap - 1;
     // the open set (pbuf[open_at]) is split into live (the next buffer) and
     // kept entries (the one after, which the search's dormant pile extends);
     // the open set's own buffer is free then and serves as the far-pile partner
     uint64_t *open = d->pbuf[d->open_at];
     // kept entries are re-checked once the retained set has grown by a quarter
     const bool check_all = d->open_n > d->open_checked + d->open_checked / 4 + 65536;
-    a.live = d->pbuf[(d->open_at + 1) % 3];
-    a.alt = open;
+    a.far0 = d->pbuf[(d->open_at + 1) % 3];
+    a.far1 = open;
     a.dorm = d->pbuf[(d->open_at + 2) % 3];
-    a.near = d->pnear;
-    a.cap = d->pcap_open;
-    a.ncap = d->pncap;
-    a.lring = 8u * kPileBlock;
+    a.fcap = a.dcap = d->pcap_open;
+    a.hubs = d->phubs;
+    a.hubcap = d->hubcap;
+    a.ctrl = d->d_ctl;
+    a.stats = (unsigned long long *)(d->d_ctl + DC_STATS);
+    a.live_n = split + SP_LIVE;
+    a.live_min = split + SP_MIN;
+    a.live_ovf = split + SP_OVF;
+    a.dorm_n = split + SP_KEEP;
+    a.N = d->N;
+    a.rebuild = d->rebuild;
+    a.t = d->t;
+    a.maxit = d->P.maxit;
+    a.grow = (uint32_t)d->P.K;
+    a.thr0 = 0;
     a.delta0 = std::max<uint32_t>(1, d->g->meanw);
-    a.split = d->d_split;
-    hipLaunchKernelGGL(fill_i32, dim3(1), dim3(64), 0, ctx->stream, (int32_t *)d->d_split, (int64_t)SP_WORDS, 0);
+    a.barrier_ticks = 100ull * 1000 * 1000 * 20;  // 20 s of the 100 MHz clock
     const uint64_t nsplit = (uint64_t)d->open_n + (uint64_t)d->P.pcap;  // the pushes' count is on the device
     const uint32_t gsplit = (uint32_t)std::max<uint64_t>(1, (nsplit + kSplitBlock * kSplitPer - 1) /
                                                                 (kSplitBlock * kSplitPer));
     hipLaunchKernelGGL(open_split, dim3(gsplit), dim3(kSplitBlock), 0, ctx->stream, (const uint64_t *)open, d->open_n,
-                       (const uint64_t *)(d->S.pbuf + d->P.pcap),
-                       (const uint32_t *)(d->S.ctrl + 2 * GA_SLOT_WORDS + GA_S_PUSHCNT), (uint32_t)d->P.pcap,
-                       (const uint64_t *)d->S.gp, d->t, a.live, a.dorm, d->pcap_open, d->d_split, (int32_t)check_all);
-    a.N = d->N;
-    a.t = d->t;
-    a.maxit = d->P.maxit;
-    a.res = d->pres;
-    a.stats = d->S.stats;
-    const size_t lds = (size_t)a.lring * 8;
-    DDP_HIP(ctx, hipFuncSetAttribute((const void *)dastar_pile_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)lds));
+                       (const uint64_t *)d->push, (const uint32_t *)(d->d_ctl + DC_REPAIR + RC_PUSHES),
+                       (uint32_t)d->P.pcap, (const uint64_t *)d->gp, d->t, a.far0, a.dorm, d->pcap_open, split,
+                       (int32_t)check_all);
     DDP_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-    hipLaunchKernelGGL(dastar_pile_kernel, dim3(1), dim3(kPileBlock), lds, ctx->stream, a);
+    // An ordinary launch of at most one workgroup per CU (see pg_enqueue).  A
+    // repair's rounds are a few hundred entries: 8, 16, 32 and 64 workgroups
+    // took 186, 178, 186 and 208 us on the 1,000,000-node graph (20,000 lines a
+    // batch) and 67, 73, 85 and 110 us on one of 100,000 nodes (200 lines).
+    const int cus = ctx->prop.multiProcessorCount;
+    const int blocks = std::min(cus, !fresh ? 16 : d->P.pg_wide ? cus : kPgBlocks);
+    hipLaunchKernelGGL((ga_piles_kernel<kPgBlock, DDP_H_ARRAY, true>),
+                       dim3(blocks), dim3(kPgBlock), 0, ctx->stream, a);
     DDP_HIP(ctx, hipGetLastError());
     DDP_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
-    uint32_t res[4];
-    DDP_HIP(ctx, hipMemcpyAsync(res, d->pres, 16, hipMemcpyDeviceToHost, ctx->stream));
-    if (rctrl_out)
-        DDP_HIP(ctx, hipMemcpyAsync(rctrl_out, d->d_rctrl, RC_WORDS * 4, hipMemcpyDeviceToHost, ctx->stream));
-    if (stats_out)  // the search counters in the same round trip
-        DDP_HIP(ctx, hipMemcpyAsync(stats_out, d->S.stats, 64, hipMemcpyDeviceToHost, ctx->stream));
+    DDP_HIP(ctx, hipMemcpyAsync(d->h_ctl, d->d_ctl, DC_WORDS * 4, hipMemcpyDeviceToHost, ctx->stream));
     DDP_HIP(ctx, hipStreamSynchronize(ctx->stream));
     float ms = 0;
     DDP_HIP(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
     *kms = ms;
-    *iters = (int32_t)res[0];
-    DDP_CHECK(!(res[2] & QERR_ITERS), ctx, DDP_ERR_TIMEOUT, "DA*: iteration limit %d reached", d->P.maxit);
-    DDP_CHECK(!(res[2] & QERR_HEAP), ctx, DDP_ERR_OVERFLOW,
-              "DA*: the pile-mode open set outgrew its %u entries", d->pcap_open);
-    d->F = res[1];
+    *iters = (int32_t)d->h_ctl[GA_RES_IT];
+    const uint32_t err = d->h_ctl[GA_RES_ERR];
+    DDP_CHECK(!(err & GA_ERR_BARRIER), ctx, DDP_ERR_TIMEOUT, "DA*: grid barrier wait timed out");
+    DDP_CHECK(!(err & GA_ERR_ITERS), ctx, DDP_ERR_TIMEOUT, "DA*: iteration limit %d reached", d->P.maxit);
+    DDP_CHECK(!(err & GA_ERR_HEAP), ctx, DDP_ERR_OVERFLOW, "DA*: the open set outgrew its %u entries", d->pcap_open);
+    d->F = d->h_ctl[GA_RES_F];
     d->open_at = (d->open_at + 2) % 3;
-    d->open_n = res[3];
+    d->open_n = d->h_ctl[GA_RES_PLEN];
     if (check_all) d->open_checked = d->open_n;
     return DDP_OK;
 }
 
+// A search from s alone (da_begin before it: no repair pushes).
 static int fresh_search(ddp_dastar *d, int32_t *iters, float *kms)
 {
     ddp_ctx *ctx = d->ctx;
-    int rc;
-    if ((rc = ddp_ga_reset(ctx, d->N, d->P, d->S))) return rc;
-    int32_t hs = 0;
-    DDP_HIP(ctx, hipMemcpyAsync(&hs, d->d_h + d->s, 4, hipMemcpyDeviceToHost, ctx->stream));
+    hipLaunchKernelGGL(fill_u64, dim3(1024), dim3(256), 0, ctx->stream, d->gp, (int64_t)d->N, (uint64_t)DDP_GP_INF);
+    hipLaunchKernelGGL(da_seed, dim3(1), dim3(64), 0, ctx->stream, d->gp, d->pbuf[d->open_at],
+                       (const int32_t *)d->d_h, d->s);
+    DDP_HIP(ctx, hipGetLastError());
+    d->open_n = 1;
+    d->open_checked = 0;
+    if (d->s != d->t) return search_run(d, true, iters, kms);
+    uint64_t word = 0;
+    DDP_HIP(ctx, hipMemcpyAsync(&word, d->gp + d->s, 8, hipMemcpyDeviceToHost, ctx->stream));
+    DDP_HIP(ctx, hipMemcpyAsync(d->h_ctl, d->d_ctl, DC_WORDS * 4, hipMemcpyDeviceToHost, ctx->stream));
     DDP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    d->rr = 0;
-    if (d->s == d->t) {
-        d->F = (uint32_t)hs;
-        uint64_t word = ((uint64_t)(uint32_t)hs << 32) | 0xFFFFFFFFull;
-        DDP_HIP(ctx, hipMemcpyAsync(d->S.gp + d->s, &word, 8, hipMemcpyHostToDevice, ctx->stream));
-        DDP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        return DDP_OK;
-    }
-    if (d->piles) {
-        // the open set is s alone; no repair pushes
-        const uint64_t word = ((uint64_t)(uint32_t)hs << 32) | 0xFFFFFFFFull;
-        const uint64_t key = ((uint64_t)(uint32_t)hs << 32) | (uint32_t)d->s;
-        DDP_HIP(ctx, hipMemcpyAsync(d->S.gp + d->s, &word, 8, hipMemcpyHostToDevice, ctx->stream));
-        DDP_HIP(ctx, hipMemcpyAsync(d->pbuf[d->open_at], &key, 8, hipMemcpyHostToDevice, ctx->stream));
-        if ((rc = ddp_ga_prepare_resume(ctx, d->S))) return rc;
-        d->open_n = 1;
-        d->open_checked = 0;
-        return pile_run(d, iters, kms);
-    }
-    if ((rc = ddp_ga_seed(ctx, d->P, d->S, d->s, (uint32_t)hs))) return rc;
-    return ddp_ga_run(ctx, fwd_view(d), d->hv, d->P, d->S, d->t, DDP_INF_F, 0, &d->F, &d->rr, iters, kms);
+    d->F = (uint32_t)(word >> 32);
+    return DDP_OK;
 }
 
 extern "C" int ddp_dastar_open(ddp_ctx *ctx, int32_t N, int32_t E, const int32_t *off, const int32_t *col,
@@ -1040,10 +971,9 @@ extern "C" int ddp_dastar_open(ddp_ctx *ctx, int32_t N, int32_t E, const int32_t
     if (h_tmp) hipFree(h_tmp);
     if (e == hipSuccess) e = hipMalloc((void **)&d->d_mark, (size_t)N * 4);
     if (e == hipSuccess) e = hipMemsetAsync(d->d_mark, 0, (size_t)N * 4, ctx->stream);
-    if (e == hipSuccess) e = hipMalloc((void **)&d->d_front, (size_t)N * 8 + 64);
     if (e == hipSuccess) e = hipMalloc((void **)&d->d_marked, (size_t)N * 4 + 64);
-    if (e == hipSuccess) e = hipMalloc((void **)&d->d_rctrl, RC_WORDS * 4);
-    if (e == hipSuccess) e = hipMalloc((void **)&d->d_walkbar, 16);
+    if (e == hipSuccess) e = hipMalloc((void **)&d->d_ctl, DC_WORDS * 4);
+    if (e == hipSuccess) e = hipHostMalloc((void **)&d->h_ctl, DC_WORDS * 4);
     if (e == hipSuccess) e = hipEventCreate(&d->ev_r0);
     if (e == hipSuccess) e = hipEventCreate(&d->ev_r1);
     if (e != hipSuccess) {
@@ -1055,31 +985,41 @@ extern "C" int ddp_dastar_open(ddp_ctx *ctx, int32_t N, int32_t E, const int32_t
     d->hv.kind = DDP_H_ARRAY;
     d->hv.scale = 1;
     d->hv.h = d->d_h;
-    if ((rc = ddp_ga_plan(ctx, d->g, opts, &d->P, 2 * (int64_t)N + 65536, false, true)) ||
-        (rc = ddp_ga_alloc_owned(ctx, N, d->P, &d->S)) || (rc = log_reserve(d, 1))) {
+    if ((rc = ddp_ga_plan(ctx, d->g, opts, &d->P, 2 * (int64_t)N + 65536)) || (rc = log_reserve(d, 1))) {
         dastar_free(d);
         delete d;
         return rc;
     }
-    d->piles = opts && opts->mode == DDP_ASTAR_PILES;
-    if (d->piles) {
-        // room for three open sets of an exhaustive search each; the near ring
-        // a power of two of about a quarter of that
+    {
+        // room for the open set of an exhaustive search in each buffer, or for
+        // the K * heap_cap entries that were asked for (which are then a
+        // limit); any node may be near once a rebuild queues them all
+        const bool piles = opts && opts->mode == DDP_ASTAR_PILES;
         d->pcap_open = (uint32_t)std::min<int64_t>(std::max<int64_t>(1 << 20, 3LL * N), 1LL << 31);
-        uint32_t nc = 1;
-        while (nc * 2 <= std::max<uint32_t>(d->pcap_open / 4, 1u << 16)) nc *= 2;
+        if (!piles && opts && opts->heap_cap > 0) {
+            d->pcap_open = (uint32_t)std::min<int64_t>(std::max<int64_t>(1024, (int64_t)d->P.K * d->P.cap), 1LL << 31);
+            d->rebuild = false;
+        }
+        uint32_t nc = 1u << 16;
+        while (nc < (uint32_t)N) nc *= 2;
         d->pncap = nc;
+        d->hubcap = d->P.hubcap;
         hipError_t e2 = hipSuccess;
-        for (int k = 0; k < 3 && e2 == hipSuccess; ++k) e2 = hipMalloc((void **)&d->pbuf[k], (size_t)d->pcap_open * 8);
-        if (e2 == hipSuccess) e2 = hipMalloc((void **)&d->pnear, (size_t)nc * 8);
-        if (e2 == hipSuccess) e2 = hipMalloc((void **)&d->pres, 64);
-        if (e2 == hipSuccess) e2 = hipMalloc((void **)&d->d_split, SP_WORDS * 4);
+        auto al2 = [&](uint64_t **p, size_t entries) {
+            if (e2 == hipSuccess) e2 = hipMalloc((void **)p, entries * 8);
+        };
+        for (int k = 0; k < 3; ++k) al2(&d->pbuf[k], d->pcap_open);
+        al2(&d->pnear, nc);
+        al2(&d->phubs, 2 * (size_t)d->hubcap);
+        al2(&d->gp, N);
+        al2(&d->push, d->P.pcap);
         if (e2 != hipSuccess) {
             dastar_free(d);
             delete d;
-            return ddp_hip_err(ctx, e2, "DA* pile state", __FILE__, __LINE__);
+            return ddp_hip_err(ctx, e2, "DA* search state", __FILE__, __LINE__);
         }
     }
+    hipLaunchKernelGGL(da_begin, dim3(1), dim3(256), 0, ctx->stream, d->d_ctl);
     int32_t iters = 0;
     float kms = 0;
     if ((rc = fresh_search(d, &iters, &kms))) {
@@ -1161,90 +1101,73 @@ extern "C" int ddp_dastar_apply(ddp_dastar *d, const ddp_update_t *lines, int32_
     auto grid = [&](size_t k) { return dim3((unsigned)std::max<size_t>(1, (k + T - 1) / T)); };
     // ---- 2. device: deletes (they never see this batch's inserts), then the appends
     d->epoch += 1;
-    uint32_t rctrl[RC_WORDS] = {0};
+    uint32_t *rctrl = d->d_ctl + DC_REPAIR;
     DDP_HIP(ctx, hipEventRecord(d->ev_r0, ctx->stream));
-    DDP_HIP(ctx, hipMemsetAsync(d->d_rctrl, 0, RC_WORDS * 4, ctx->stream));
+    hipLaunchKernelGGL(da_begin, dim3(1), dim3(256), 0, ctx->stream, d->d_ctl);
     const int32_t npairs = nd, nins = ni;
     if (npairs)
         hipLaunchKernelGGL(apply_deletes, grid(npairs), dim3(T), 0, ctx->stream, w_pairs, npairs, fwd_view(d),
                            d->g->col, d->g->rcol, (const int32_t *)d->g->roff, (const int32_t *)d->d_reid, d->L,
-                           (const uint64_t *)d->S.gp, d->d_mark, d->epoch, d->d_front, d->d_marked, d->d_rctrl);
-    if (nins) {
-        hipLaunchKernelGGL(log_fill, grid(nins), dim3(T), 0, ctx->stream, w_ins, nins, d->L, (int64_t)d->log_used);
-        hipLaunchKernelGGL(log_append, grid(nins), dim3(T), 0, ctx->stream, w_fg, nins, d->L.fhead, d->L.fnext,
-                           d->L.ftail);
-        hipLaunchKernelGGL(log_append, grid(nins), dim3(T), 0, ctx->stream, w_rg, nins, d->L.rhead, d->L.rnext,
-                           d->L.rtail);
-    }
+                           (const uint64_t *)d->gp, d->d_mark, d->epoch, d->d_marked, rctrl);
+    if (nins)
+        hipLaunchKernelGGL(log_insert, dim3(grid(nins).x, 3), dim3(T), 0, ctx->stream, w_ins, w_fg, w_rg, nins, d->L,
+                           (int64_t)d->log_used);
     DDP_HIP(ctx, hipGetLastError());
     d->log_used += nins;
     // host preparation only: the device work below follows without a host
-    // round trip until the repair's counters are read
+    // round trip until the search has ended
     S.host_ms = ms_since(t0);
     int32_t iters = 0;
     float kms = 0;
-    unsigned long long cnt[8] = {0};  // the search counters (expanded, edges, improved, stale, rebuilds, refills, scanned)
-    bool have_cnt = false;
     if (mode == DDP_DASTAR_RECOMPUTE) {
         if ((rc = fresh_search(d, &iters, &kms))) return rc;
-        DDP_HIP(ctx, hipMemcpyAsync(rctrl, d->d_rctrl, RC_WORDS * 4, hipMemcpyDeviceToHost, ctx->stream));
-        DDP_HIP(ctx, hipStreamSynchronize(ctx->stream));
     } else {
-        if ((rc = ddp_ga_prepare_resume(ctx, d->S))) return rc;
         const GraphView F = fwd_view(d), R = rev_view(d);
         // ---- 3. invalidate the parent subtrees of deleted tree edges (roots
         // seeded by apply_deletes): every level in one launch
-        DDP_HIP(ctx, hipMemsetAsync(d->d_walkbar, 0, 16, ctx->stream));
-        hipLaunchKernelGGL(subtree_walk, dim3(kWalkGrid), dim3(kWalkGridBlock), 0, ctx->stream, F, d->L, d->S.gp,
-                           d->d_mark, d->epoch, d->d_front, d->d_front + N, d->d_marked, d->d_rctrl, d->d_walkbar,
-                           (uint64_t)100 * 1000 * 1000 * 5);  // 5 s of the 100 MHz clock per barrier
+        if (npairs)
+            hipLaunchKernelGGL(subtree_walk, dim3(kWalkGrid), dim3(kWalkGridBlock), 0, ctx->stream, F, d->L, d->gp,
+                               d->d_mark, d->epoch, d->d_marked, rctrl, d->d_ctl + DC_WALK,
+                               (uint64_t)100 * 1000 * 1000 * 5);  // 5 s of the 100 MHz clock per barrier
         // ---- 4. re-pull invalidated nodes (their count is read on the device), 5. relax inserted edges
-        RepairPush P{d->S.pbuf + d->P.pcap, d->S.ctrl + 2 * GA_SLOT_WORDS, d->P.pcap, d->d_rctrl, d->t};
-        hipLaunchKernelGGL(repull, dim3(256), dim3(T), 0, ctx->stream, R, d->L, d->d_h, d->S.gp, d->d_mark, d->epoch,
-                           (const int32_t *)d->d_marked, (const uint32_t *)d->d_rctrl, P);
+        RepairPush P{d->push, (uint32_t)d->P.pcap, rctrl, d->t};
+        if (npairs)
+            hipLaunchKernelGGL(repull, dim3(256), dim3(T), 0, ctx->stream, R, d->L, d->d_h, d->gp, d->d_mark, d->epoch,
+                               (const int32_t *)d->d_marked, (const uint32_t *)rctrl, P);
         if (nins)
-            hipLaunchKernelGGL(relax_inserts, grid(nins), dim3(T), 0, ctx->stream, w_ins, nins, d->d_h, d->S.gp, P);
+            hipLaunchKernelGGL(relax_inserts, grid(nins), dim3(T), 0, ctx->stream, w_ins, nins, d->d_h, d->gp, P);
         DDP_HIP(ctx, hipGetLastError());
         DDP_HIP(ctx, hipEventRecord(d->ev_r1, ctx->stream));
-        DDP_HIP(ctx, hipMemsetAsync(d->S.stats, 0, 64, ctx->stream));
-        // ---- 6. resume GA* from the retained queues plus the repair pushes
-        if (d->piles && d->s != d->t) {
-            // the pile search reads F(t) on the device: one host round trip
-            // for the repair counters, the search and its counters together
-            if ((rc = pile_run(d, &iters, &kms, rctrl, cnt))) return rc;
-            have_cnt = true;
+        // ---- 6. resume the search from the retained open set plus the repair
+        // pushes; it reads F(t) on the device, and one host round trip brings
+        // its outcome and every counter
+        if (d->s != d->t) {
+            if ((rc = search_run(d, false, &iters, &kms))) return rc;
         } else {
             uint64_t tword = 0;
-            DDP_HIP(ctx, hipMemcpyAsync(&tword, d->S.gp + d->t, 8, hipMemcpyDeviceToHost, ctx->stream));
-            DDP_HIP(ctx, hipMemcpyAsync(rctrl, d->d_rctrl, RC_WORDS * 4, hipMemcpyDeviceToHost, ctx->stream));
+            DDP_HIP(ctx, hipMemcpyAsync(&tword, d->gp + d->t, 8, hipMemcpyDeviceToHost, ctx->stream));
+            DDP_HIP(ctx, hipMemcpyAsync(d->h_ctl, d->d_ctl, DC_WORDS * 4, hipMemcpyDeviceToHost, ctx->stream));
             DDP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-            if (d->s == d->t) {
-                d->F = (uint32_t)(tword >> 32);
-            } else if (d->piles) {
-                if ((rc = pile_run(d, &iters, &kms))) return rc;
-            } else if ((rc = ddp_ga_run(ctx, F, d->hv, d->P, d->S, d->t, (uint32_t)(tword >> 32), d->rr, &d->F,
-                                        &d->rr, &iters, &kms))) {
-                return rc;
-            }
+            d->F = (uint32_t)(tword >> 32);
         }
-        DDP_CHECK(rctrl[RC_WALK_ERR] == 0, ctx, DDP_ERR_TIMEOUT,
+        const uint32_t *rc_h = d->h_ctl + DC_REPAIR;
+        DDP_CHECK(rc_h[RC_WALK_ERR] == 0, ctx, DDP_ERR_TIMEOUT,
                   "DA*: a device-wide barrier of the subtree walk timed out (are %d workgroups co-resident?)",
                   kWalkGrid);
-        S.roots = (int32_t)rctrl[RC_ROOTS];
-        S.invalidated = (int32_t)std::min<uint32_t>(rctrl[RC_MARKED], (uint32_t)N);
-        S.repulled = (int32_t)rctrl[RC_REPULLED];
-        S.pushes = (int32_t)rctrl[RC_PUSHES];
+        S.roots = (int32_t)rc_h[RC_ROOTS];
+        S.invalidated = (int32_t)std::min<uint32_t>(rc_h[RC_MARKED], (uint32_t)N);
+        S.repulled = (int32_t)rc_h[RC_REPULLED];
+        S.pushes = (int32_t)rc_h[RC_PUSHES];
         DDP_HIP(ctx, hipEventElapsedTime(&S.repair_ms, d->ev_r0, d->ev_r1));
     }
-    S.deletes_effective = (int32_t)(rctrl[RC_DEL_BASE] + rctrl[RC_DEL_LOG]);
-    d->live_base -= rctrl[RC_DEL_BASE];
-    d->live_log += nins - (int64_t)rctrl[RC_DEL_LOG];
+    const uint32_t del_base = d->h_ctl[DC_REPAIR + RC_DEL_BASE], del_log = d->h_ctl[DC_REPAIR + RC_DEL_LOG];
+    S.deletes_effective = (int32_t)(del_base + del_log);
+    d->live_base -= del_base;
+    d->live_log += nins - (int64_t)del_log;
     S.iterations = iters;
     S.search_ms = kms;
-    if (!have_cnt) {
-        DDP_HIP(ctx, hipMemcpyAsync(cnt, d->S.stats, 64, hipMemcpyDeviceToHost, ctx->stream));
-        DDP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    }
+    unsigned long long cnt[8];  // the search counters (expanded, edges, improved, stale, rebuilds, refills, scanned)
+    std::memcpy(cnt, d->h_ctl + DC_STATS, sizeof cnt);
     S.expansions = (int64_t)cnt[0];
     S.edges = (int64_t)cnt[1];
     S.improvements = (int64_t)cnt[2];
@@ -1286,7 +1209,7 @@ extern "C" int ddp_dastar_path(ddp_dastar *d, int32_t *path, int32_t cap, int32_
         *len = 0;
         return DDP_OK;
     }
-    return ddp_extract_path(d->ctx, d->S.gp, d->N, d->s, d->t, path, cap, len);
+    return ddp_extract_path(d->ctx, d->gp, d->N, d->s, d->t, path, cap, len);
 }
 
 extern "C" int ddp_dastar_num_edges(const ddp_dastar *d, int32_t *E)

@@ -78,7 +78,6 @@ int ddp_ws(ddp_ctx *ctx, int slot, size_t bytes, void **out);
 enum {
     WS_ASTAR_GP = 0,
     WS_ASTAR_HEAP,
-    WS_ASTAR_HSIZE,
     WS_ASTAR_PBUF,
     WS_ASTAR_CTRL,
     WS_ASTAR_TOUCH,

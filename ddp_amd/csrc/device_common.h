@@ -287,42 +287,12 @@ __device__ __forceinline__ uint64_t dev_clock_100mhz()
     return __builtin_amdgcn_s_memrealtime();
 }
 
-// Sense-counting grid barrier over `nblocks` co-resident workgroups.
-// bar[0] = arrival count, bar[1] = generation.  Every wait is bounded by
-// `limit_ticks` of the 100 MHz clock; returns false if the wait timed out.
-__device__ __forceinline__ bool grid_barrier(uint32_t *bar, uint32_t nblocks, uint32_t &gen,
-                                             uint64_t limit_ticks, int32_t *s_flag)
-{
-    // every wave's stores reach L2 before thread 0's agent-scope release
-    block_sync_global();
-    if (threadIdx.x == 0) {
-        bool ok = true;
-        __threadfence();
-        uint32_t arrived = atomicAdd(&bar[0], 1u);
-        if (arrived == nblocks - 1) {
-            __hip_atomic_store(&bar[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&bar[1], gen + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            const uint64_t t0 = dev_clock_100mhz();
-            while (__hip_atomic_load(&bar[1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) == gen) {
-                __builtin_amdgcn_s_sleep(2);
-                if (dev_clock_100mhz() - t0 > limit_ticks) { ok = false; break; }
-            }
-        }
-        __threadfence();
-        *s_flag = ok ? 1 : 0;
-    }
-    gen += 1;
-    __syncthreads();
-    return *s_flag != 0;
-}
-
 // Grid barrier without cache maintenance, for kernels whose workgroups share
 // data only through agent-scope atomics (loads and stores included: ld_gp,
 // ld_u32, st_u64, ...): those go past L1 and are kept coherent between the
 // XCDs' L2s, so a wave's vmcnt(0) is all the release that is needed and a
-// relaxed poll all the acquire.  The fences of grid_barrier (an L2 write-back
-// and invalidate by every workgroup) were most of its cost: 1.9 us with 16
+// relaxed poll all the acquire.  With agent-scope fences and acquire polls (an
+// L2 write-back and invalidate by every workgroup) it cost 1.9 us with 16
 // workgroups of 64, 4.0 with 64, 14.4 with 256, 28.6 with 512, against 1.4,
 // 1.9, 4.0 and 6.9 us here.  Beyond 64 workgroups the arrivals, which one
 // counter takes at about 11 ns each, are counted in eight groups first (a

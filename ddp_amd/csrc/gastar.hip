@@ -41,211 +41,10 @@ enum : uint32_t {
     ERR_PATH = 16
 };
 
-struct GridArgs {
-    GraphView g;
-    HeurView h;
-    uint64_t *gp;
-    uint64_t *home;      // heap spill / home: entry i of queue q at home[i*K + q]
-    int32_t *hsize;      // K
-    uint64_t *pbuf;      // 2 * pcap
-    uint32_t *ctrl;      // GA_CTRL_WORDS
-    unsigned long long *stats;  // expanded, edges, improved, stale
-    int32_t K, lcap, cap, pcap, t, maxit;
-    uint32_t F0;
-    int32_t rr0;
-    uint64_t barrier_ticks;
-};
-
-template <int B>
-struct GridPush {
-    uint64_t *buf;
-    uint32_t *pushcnt;
-    int32_t pcap;
-    uint32_t tmin = 0xFFFFFFFFu, pushmin = 0xFFFFFFFFu;
-    uint32_t err = 0;
-
-    __device__ void target(uint32_t f) { tmin = f < tmin ? f : tmin; }
-    __device__ void touch(int32_t, uint64_t) {}
-    __device__ void operator()(bool has, uint64_t key)
-    {
-        const uint64_t mask = __ballot(has);
-        if (mask == 0) return;
-        const int lane = threadIdx.x & 63;
-        const int leader = __builtin_ctzll(mask);
-        uint32_t base = 0;
-        if (lane == leader) base = atomicAdd(pushcnt, (uint32_t)__popcll(mask));
-        base = __shfl(base, leader, 64);
-        if (has) {
-            const uint32_t idx = base + lane_rank(mask);
-            if (idx < (uint32_t)pcap) buf[idx] = key;
-            else err |= ERR_PBUF;
-            const uint32_t f = (uint32_t)(key >> 32);
-            pushmin = f < pushmin ? f : pushmin;
-        }
-    }
-    template <int R>
-    __device__ void touch_all(const bool (&)[R], const int32_t (&)[R]) {}
-    template <int R>
-    __device__ void all(const bool (&has)[R], const uint64_t (&key)[R])
-    {
-        uint32_t pos[R];
-        wave_append<R>(has, pushcnt, pos);
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (!has[r]) continue;
-            if (pos[r] < (uint32_t)pcap) buf[pos[r]] = key[r];
-            else err |= ERR_PBUF;
-            const uint32_t f = (uint32_t)(key[r] >> 32);
-            pushmin = f < pushmin ? f : pushmin;
-        }
-    }
-};
-
-template <int B, int HK>
-__global__ void __launch_bounds__(B) ga_grid_kernel(GridArgs a)
-{
-    extern __shared__ uint64_t s_heap[];  // lcap * B
-    __shared__ ExpandLds<B> L;
-    __shared__ uint32_t s_red[16];
-    __shared__ int32_t s_flag;
-
-    const int lane = threadIdx.x;
-    const int32_t K = a.K;
-    const int32_t q = blockIdx.x * B + lane;
-    uint32_t *ctrl = a.ctrl;
-    const LaneHeap H{s_heap + lane, a.home + q, B, a.lcap, (int64_t)K, a.cap};
-    int32_t size = a.hsize[q];
-    for (int32_t i = 0; i < size && i < a.lcap; ++i) s_heap[i * B + lane] = a.home[(int64_t)i * K + q];
-
-    uint32_t gen = ld_u32(ctrl + GA_BAR + 1);
-    uint32_t F = a.F0;
-    int32_t rr = a.rr0;
-    uint32_t err_local = 0, err_seen = 0;
-    ExpandCounters C;
-    uint32_t stale = 0;
-    int32_t it = 0;
-    for (;; ++it) {
-        // -- drain the previous iteration's pushes into this lane's queue
-        const int ps = (it + 2) % 3;
-        const uint32_t n = ld_u32(ctrl + ps * GA_SLOT_WORDS + GA_S_PUSHCNT);
-        const uint32_t topm = ld_u32(ctrl + ps * GA_SLOT_WORDS + GA_S_TOPMIN);
-        const uint32_t pm = ld_u32(ctrl + ps * GA_SLOT_WORDS + GA_S_PUSHMIN);
-        const uint32_t tm = ld_u32(ctrl + ps * GA_SLOT_WORDS + GA_S_TMIN);
-        err_seen |= ld_u32(ctrl + ps * GA_SLOT_WORDS + GA_S_ERR);
-        F = tm < F ? tm : F;
-        const uint32_t navail = n < (uint32_t)a.pcap ? n : (uint32_t)a.pcap;
-        const uint64_t *buf = a.pbuf + (int64_t)((it + 1) & 1) * a.pcap;
-        for (int64_t p = ((int64_t)q - rr) % K + (q < rr ? K : 0); p < (int64_t)navail; p += K) {
-            const uint64_t e = __hip_atomic_load(buf + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (!heap_push(H, size, e)) err_local |= ERR_HEAP;
-        }
-        rr = (int32_t)(((int64_t)rr + n) % K);
-        // -- termination (uniform: every input was frozen by the last barrier)
-        const uint32_t open_min = topm < pm ? topm : pm;
-        if (it > 0 && F <= open_min) break;
-        if (err_seen) break;
-        if (it >= a.maxit) {
-            err_local |= ERR_ITERS;
-            break;
-        }
-        const int cs = it % 3;
-        if (blockIdx.x == 0 && lane == 0) {
-            uint32_t *ns = ctrl + ((it + 1) % 3) * GA_SLOT_WORDS;
-            st_u32(ns + GA_S_PUSHCNT, 0);
-            st_u32(ns + GA_S_TOPMIN, 0xFFFFFFFFu);
-            st_u32(ns + GA_S_PUSHMIN, 0xFFFFFFFFu);
-            st_u32(ns + GA_S_TMIN, 0xFFFFFFFFu);
-            st_u32(ns + GA_S_ERR, 0);
-        }
-        // -- publish the smallest queue top (stale tops only make this smaller)
-        const uint32_t mytop = size > 0 ? (uint32_t)(s_heap[lane] >> 32) : 0xFFFFFFFFu;
-        const uint32_t bmin = block_min_u32<B>(mytop, s_red);
-        if (lane == 0 && bmin != 0xFFFFFFFFu) atomicMin(ctrl + cs * GA_SLOT_WORDS + GA_S_TOPMIN, bmin);
-        // -- pop the best entry whose f is still current
-        int32_t u = -1;
-        uint32_t fu = 0;
-        while (size > 0) {
-            uint64_t key;
-            heap_pop(H, size, key);
-            const int32_t node = (int32_t)(uint32_t)key;
-            const uint32_t f = (uint32_t)(key >> 32);
-            if ((uint32_t)(ld_gp(a.gp + node) >> 32) == f) {
-                u = node;
-                fu = f;
-                break;
-            }
-            ++stale;
-        }
-        // -- expand and push
-        GridPush<B> push{a.pbuf + (int64_t)(it & 1) * a.pcap, ctrl + cs * GA_SLOT_WORDS + GA_S_PUSHCNT, a.pcap};
-        expand_block<B, HK>(a.g, a.h, a.gp, a.t, u, fu, L, C, push);
-        err_local |= push.err;
-        const uint32_t wt = wave_min_u32(push.tmin);
-        const uint32_t wp = wave_min_u32(push.pushmin);
-        if ((lane & 63) == 0) {
-            if (wt != 0xFFFFFFFFu) atomicMin(ctrl + cs * GA_SLOT_WORDS + GA_S_TMIN, wt);
-            if (wp != 0xFFFFFFFFu) atomicMin(ctrl + cs * GA_SLOT_WORDS + GA_S_PUSHMIN, wp);
-        }
-        if (err_local) atomicOr(ctrl + cs * GA_SLOT_WORDS + GA_S_ERR, err_local);
-        if (!grid_barrier(ctrl + GA_BAR, gridDim.x, gen, a.barrier_ticks, &s_flag)) {
-            atomicOr(ctrl + GA_RES_ERR, (uint32_t)ERR_BARRIER);
-            break;
-        }
-    }
-    // -- persist queues for a later resume (DA*) and report
-    for (int32_t i = 0; i < size && i < a.lcap; ++i) a.home[(int64_t)i * K + q] = s_heap[i * B + lane];
-    a.hsize[q] = size;
-    if (err_local) atomicOr(ctrl + GA_RES_ERR, err_local);
-    if (err_seen) atomicOr(ctrl + GA_RES_ERR, err_seen);
-    if (blockIdx.x == 0 && lane == 0) {
-        ctrl[GA_RES_IT] = (uint32_t)it;
-        ctrl[GA_RES_RR] = (uint32_t)rr;
-        ctrl[GA_RES_F] = F;
-    }
-    uint64_t v0 = wave_sum_u64(C.expanded), v1 = wave_sum_u64(C.edges), v2 = wave_sum_u64(C.improved),
-             v3 = wave_sum_u64(stale);
-    if ((lane & 63) == 0) {
-        atomicAdd(a.stats + 0, (unsigned long long)v0);
-        atomicAdd(a.stats + 1, (unsigned long long)v1);
-        atomicAdd(a.stats + 2, (unsigned long long)v2);
-        atomicAdd(a.stats + 3, (unsigned long long)v3);
-    }
-}
-
 __global__ void fill_u64_kernel(uint64_t *p, int64_t n, uint64_t v)
 {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         p[i] = v;
-}
-
-__global__ void fill_i32_kernel(int32_t *p, int64_t n, int32_t v)
-{
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = v;
-}
-
-// Fresh search: gp[s] = (h(s), parent -1); s is the only push of "iteration -1".
-__global__ void seed_kernel(uint64_t *gp, uint64_t *pbuf1, uint32_t *ctrl, int32_t s, uint32_t hs)
-{
-    if (threadIdx.x != 0) return;
-    gp[s] = ((uint64_t)hs << 32) | 0xFFFFFFFFull;
-    pbuf1[0] = ((uint64_t)hs << 32) | (uint32_t)s;
-    for (int k = 0; k < 3; ++k) {
-        uint32_t *sl = ctrl + k * GA_SLOT_WORDS;
-        sl[GA_S_PUSHCNT] = 0;
-        sl[GA_S_TOPMIN] = 0xFFFFFFFFu;
-        sl[GA_S_PUSHMIN] = 0xFFFFFFFFu;
-        sl[GA_S_TMIN] = 0xFFFFFFFFu;
-        sl[GA_S_ERR] = 0;
-    }
-    ctrl[2 * GA_SLOT_WORDS + GA_S_PUSHCNT] = 1;
-    ctrl[2 * GA_SLOT_WORDS + GA_S_PUSHMIN] = hs;
-    ctrl[GA_RES_IT] = 0;
-    ctrl[GA_RES_RR] = 0;
-    ctrl[GA_RES_F] = DDP_INF_F;
-    ctrl[GA_RES_ERR] = 0;
-    ctrl[GA_BAR] = 0;
-    ctrl[GA_BAR + 1] = 0;
 }
 
 __global__ void unpack_parent_kernel(const uint64_t *gp, int32_t *par, int32_t N)
@@ -295,28 +94,6 @@ void ga_pg_sizes(const GaGridPlan &P, uint64_t *ring, uint64_t *far)
     while (r < total) r *= 2;
     *ring = r;
     *far = std::max<uint64_t>(total, 1024);
-}
-
-using KernelFn = void (*)(GridArgs);
-
-template <int B>
-KernelFn pick_kernel(int hk)
-{
-    switch (hk) {
-    case DDP_H_ZERO: return ga_grid_kernel<B, DDP_H_ZERO>;
-    case DDP_H_ARRAY: return ga_grid_kernel<B, DDP_H_ARRAY>;
-    case DDP_H_MANHATTAN: return ga_grid_kernel<B, DDP_H_MANHATTAN>;
-    default: return ga_grid_kernel<B, DDP_H_EUCLID>;
-    }
-}
-
-KernelFn pick(int B, int hk)
-{
-    switch (B) {
-    case 64: return pick_kernel<64>(hk);
-    case 256: return pick_kernel<256>(hk);
-    default: return pick_kernel<1024>(hk);
-    }
 }
 
 // Workgroup mode: all K <= 1024 queues live in one workgroup, one per lane,
@@ -375,7 +152,7 @@ __global__ void __launch_bounds__(B) ga_wg_kernel(WgArgs a)
     } else {
         if constexpr (WM == WM_PILES) {
             const PilePtrs P{a.home, a.home + a.ncap, a.home + a.ncap + a.fcap, a.ncap, a.fcap, s_heap, a.lring};
-            slot_search_piles<B, HK, pile_entries_per_lane<B>(), false, true>(a.g, a.h, a.gp, a.touched, P, a.N, a.s,
+            slot_search_piles<B, HK, pile_entries_per_lane<B>(), true>(a.g, a.h, a.gp, a.touched, P, a.N, a.s,
                                                                               a.t, a.maxit, a.delta0, S, C, stale);
         } else {
             slot_search<B, HK>(a.g, a.h, a.gp, a.touched, H, s_heap, a.N, a.s, a.t, a.maxit, S, C, stale);
@@ -434,7 +211,7 @@ WgFn pick_wg(int B, int hk, int wm)
 }  // namespace
 
 int ddp_ga_plan(ddp_ctx *ctx, const ddp_graph *g, const ddp_astar_opts_t *o, GaGridPlan *p, int64_t min_pcap,
-                bool allow_wg, bool heaps)
+                bool allow_wg)
 {
     int32_t B = (o && o->block) ? o->block : 0;
     int32_t K = (o && o->K) ? o->K : 1024;
@@ -494,18 +271,15 @@ int ddp_ga_plan(ddp_ctx *ctx, const ddp_graph *g, const ddp_astar_opts_t *o, GaG
     DDP_CHECK(pcap < (1LL << 31), ctx, DDP_ERR_ARG, "push buffer too large");
     int32_t maxit = (o && o->max_iters) ? o->max_iters : (int32_t)std::min<int64_t>(4LL * g->N + 1024, 1 << 30);
     *p = GaGridPlan{K, B, nblocks, lcap, (int32_t)cap, (int32_t)pcap, maxit};
-    if (!heaps) {
-        p->pg = true;
-        p->pg_wide = g->E >= kPgWideEdges;
-        p->hubcap = (uint32_t)((int64_t)g->E / kPgSeg + kPgRound + 64);
-        p->delta0 = std::max<uint32_t>(1, g->meanw);
-    }
-    // co-residency check for the cooperative launch
-    int per_cu = 0;
-    DDP_HIP(ctx, hipFuncSetAttribute((const void *)pick(B, DDP_H_ZERO), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)((size_t)lcap * B * 8)));
-    DDP_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)pick(B, DDP_H_ZERO), B,
-                                                             (size_t)lcap * B * 8));
+    p->pg = true;
+    p->pg_wide = g->E >= kPgWideEdges;
+    p->hubcap = (uint32_t)((int64_t)g->E / kPgSeg + kPgRound + 64);
+    p->delta0 = std::max<uint32_t>(1, g->meanw);
+    // K is bounded by the queues whose tops and expansion tables the device
+    // could hold at once, as callers know it (the piles themselves need no LDS
+    // per queue): workgroups of B lanes per CU by LDS and by 20 waves.
+    const size_t lds = (size_t)lcap * B * 8 + 48 * (size_t)B + 392;
+    const int per_cu = (int)std::min<size_t>(ctx->prop.maxSharedMemoryPerMultiProcessor / lds, 20 * 64 / B);
     DDP_CHECK((int64_t)per_cu * ctx->prop.multiProcessorCount >= nblocks, ctx, DDP_ERR_ARG,
               "K=%d needs %d co-resident workgroups of %d lanes; the device holds %d", K, nblocks, B,
               per_cu * ctx->prop.multiProcessorCount);
@@ -517,7 +291,7 @@ int ddp_ga_alloc(ddp_ctx *ctx, const ddp_graph *g, const GaGridPlan &P, GaGridSt
     void *p;
     int rc;
     const size_t dirs = P.bidi ? 2 : 1;
-    size_t queue = dirs * P.cap * P.K, push = 2 * (size_t)P.pcap;  // 8-byte entries
+    size_t queue = dirs * P.cap * P.K, push = 0;  // 8-byte entries
     if (P.pg) {
         uint64_t ring, far;
         ga_pg_sizes(P, &ring, &far);
@@ -528,9 +302,7 @@ int ddp_ga_alloc(ddp_ctx *ctx, const ddp_graph *g, const GaGridPlan &P, GaGridSt
     S->gp = (uint64_t *)p;
     if ((rc = ddp_ws(ctx, WS_ASTAR_HEAP, queue * 8, &p))) return rc;
     S->home = (uint64_t *)p;
-    if ((rc = ddp_ws(ctx, WS_ASTAR_HSIZE, (size_t)P.K * 4, &p))) return rc;
-    S->hsize = (int32_t *)p;
-    if ((rc = ddp_ws(ctx, WS_ASTAR_PBUF, push * 8, &p))) return rc;
+    if ((rc = ddp_ws(ctx, WS_ASTAR_PBUF, push * 8 + 64, &p))) return rc;
     S->pbuf = (uint64_t *)p;
     if ((rc = ddp_ws(ctx, WS_ASTAR_CTRL, GA_CTRL_WORDS * 4 + 64, &p))) return rc;
     S->ctrl = (uint32_t *)p;
@@ -552,17 +324,12 @@ int ddp_ga_alloc_owned(ddp_ctx *ctx, int32_t N, const GaGridPlan &P, GaGridState
     auto al = [&](void **p, size_t bytes) {
         if (e == hipSuccess) e = hipMalloc(p, std::max<size_t>(bytes, 64));
     };
-    size_t queue = (size_t)P.cap * P.K, push = 2 * (size_t)P.pcap;
-    if (P.pg) {
-        uint64_t ring, far;
-        ga_pg_sizes(P, &ring, &far);
-        queue = ring + 2 * far;
-        push = 2 * (size_t)P.hubcap;
-    }
+    DDP_CHECK(P.pg, ctx, DDP_ERR_STATE, "GA*: not a grid plan");
+    uint64_t ring, far;
+    ga_pg_sizes(P, &ring, &far);
     al((void **)&S->gp, (size_t)N * 8);
-    al((void **)&S->home, queue * 8);
-    al((void **)&S->hsize, (size_t)P.K * 4);
-    al((void **)&S->pbuf, push * 8);
+    al((void **)&S->home, (ring + 2 * far) * 8);
+    al((void **)&S->pbuf, 16 * (size_t)P.hubcap);
     al((void **)&S->ctrl, GA_CTRL_WORDS * 4 + 64);
     if (e != hipSuccess) {
         ddp_ga_free(S);
@@ -575,7 +342,7 @@ int ddp_ga_alloc_owned(ddp_ctx *ctx, int32_t N, const GaGridPlan &P, GaGridState
 void ddp_ga_free(GaGridState *S)
 {
     if (!S->owned) return;
-    void *ptrs[] = {S->gp, S->home, S->hsize, S->pbuf, S->ctrl};
+    void *ptrs[] = {S->gp, S->home, S->pbuf, S->ctrl};
     for (void *p : ptrs)
         if (p) hipFree(p);
     *S = GaGridState{};
@@ -585,37 +352,7 @@ int ddp_ga_reset(ddp_ctx *ctx, int32_t N, const GaGridPlan &P, const GaGridState
 {
     hipLaunchKernelGGL(fill_u64_kernel, dim3(1024), dim3(256), 0, ctx->stream, S.gp, (int64_t)N * (P.bidi ? 2 : 1),
                        (uint64_t)DDP_GP_INF);
-    if (!P.pg)
-        hipLaunchKernelGGL(fill_i32_kernel, dim3(std::max(1, std::min(1024, P.K / 256 + 1))), dim3(256), 0,
-                           ctx->stream, S.hsize, (int64_t)P.K, 0);
     DDP_HIP(ctx, hipMemsetAsync(S.stats, 0, 64, ctx->stream));
-    DDP_HIP(ctx, hipGetLastError());
-    return DDP_OK;
-}
-
-int ddp_ga_seed(ddp_ctx *ctx, const GaGridPlan &P, const GaGridState &S, int32_t s, uint32_t hs)
-{
-    hipLaunchKernelGGL(seed_kernel, dim3(1), dim3(64), 0, ctx->stream, S.gp, S.pbuf + P.pcap, S.ctrl, s, hs);
-    DDP_HIP(ctx, hipGetLastError());
-    return DDP_OK;
-}
-
-__global__ void prepare_resume_kernel(uint32_t *ctrl)
-{
-    if (threadIdx.x != 0) return;
-    for (int k = 0; k < 3; ++k) {
-        uint32_t *sl = ctrl + k * GA_SLOT_WORDS;
-        sl[GA_S_PUSHCNT] = 0;
-        sl[GA_S_TOPMIN] = 0xFFFFFFFFu;
-        sl[GA_S_PUSHMIN] = 0xFFFFFFFFu;
-        sl[GA_S_TMIN] = 0xFFFFFFFFu;
-        sl[GA_S_ERR] = 0;
-    }
-}
-
-int ddp_ga_prepare_resume(ddp_ctx *ctx, const GaGridState &S)
-{
-    hipLaunchKernelGGL(prepare_resume_kernel, dim3(1), dim3(64), 0, ctx->stream, S.ctrl);
     DDP_HIP(ctx, hipGetLastError());
     return DDP_OK;
 }
@@ -629,46 +366,10 @@ int ddp_ga_stats(ddp_ctx *ctx, const GaGridState &S, unsigned long long out[4])
 
 namespace {
 
-GridArgs grid_args(const GraphView &gv, const HeurView &hv, const GaGridPlan &P, const GaGridState &S, int32_t t,
-                   uint32_t F0, int32_t rr0)
-{
-    GridArgs a{};
-    a.g = gv;
-    a.h = hv;
-    a.gp = S.gp;
-    a.home = S.home;
-    a.hsize = S.hsize;
-    a.pbuf = S.pbuf;
-    a.ctrl = S.ctrl;
-    a.stats = S.stats;
-    a.K = P.K;
-    a.lcap = P.lcap;
-    a.cap = P.cap;
-    a.pcap = P.pcap;
-    a.t = t;
-    a.maxit = P.maxit;
-    a.F0 = F0;
-    a.rr0 = rr0;
-    a.barrier_ticks = 100ull * 1000 * 1000 * 20;  // 20 s of the 100 MHz clock
-    return a;
-}
-
-// Ordinary launch: ddp_ga_plan sized the grid to what the device holds at
-// once and the grid barrier is software with bounded waits (a cooperative
-// launch would also reserve the global wave-sync unit, one process only).
-int grid_enqueue(ddp_ctx *ctx, GridArgs &a, const GaGridPlan &P, int hk)
-{
-    void *args[] = {&a};
-    KernelFn fn = pick(P.B, hk);
-    DDP_HIP(ctx, hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)((size_t)P.lcap * P.B * 8)));
-    DDP_HIP(ctx, hipLaunchKernel((const void *)fn, dim3(P.nblocks), dim3(P.B), args, (size_t)P.lcap * P.B * 8,
-                                 ctx->stream));
-    return DDP_OK;
-}
-
-// Grid mode on piles: seeds s and enqueues the search.  Ordinary launch, as
-// grid_enqueue's; at most one workgroup per CU, so all are resident at once.
+// Seeds s and enqueues the grid search.  Ordinary launch of at most one
+// workgroup per CU, so all are resident at once, and the grid barrier is
+// software with bounded waits (a cooperative launch would also reserve the
+// global wave-sync unit, one process only).
 int pg_enqueue(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P, const GaGridState &S,
                int32_t s, uint32_t hs, int32_t t)
 {
@@ -701,8 +402,8 @@ int pg_enqueue(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGr
 }
 
 // Waits for a grid search (its events recorded) and reads its outcome.
-int grid_finish(ddp_ctx *ctx, const GaGridPlan &P, const GaGridState &S, uint32_t *F_out, int32_t *rr_out,
-                int32_t *iters_out, float *kernel_ms)
+int grid_finish(ddp_ctx *ctx, const GaGridPlan &P, const GaGridState &S, uint32_t *F_out, int32_t *iters_out,
+                float *kernel_ms)
 {
     uint32_t res[4];
     DDP_HIP(ctx, hipMemcpyAsync(res, S.ctrl + GA_RES_IT, 16, hipMemcpyDeviceToHost, ctx->stream));
@@ -711,7 +412,6 @@ int grid_finish(ddp_ctx *ctx, const GaGridPlan &P, const GaGridState &S, uint32_
     DDP_HIP(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
     if (kernel_ms) *kernel_ms = ms;
     if (iters_out) *iters_out = (int32_t)res[0];
-    if (rr_out) *rr_out = (int32_t)res[1];
     if (F_out) *F_out = res[2];
     const uint32_t err = res[3];
     DDP_CHECK(!(err & ERR_BARRIER), ctx, DDP_ERR_TIMEOUT, "GA*: grid barrier wait timed out");
@@ -733,22 +433,6 @@ int ddp_ga_launch(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const G
     return pg_enqueue(ctx, gv, hv, P, S, s, hs, t);
 }
 
-// Runs the GA* loop from the current state (fresh or resumed).
-int ddp_ga_run(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P,
-               const GaGridState &S, int32_t t, uint32_t F0, int32_t rr0, uint32_t *F_out,
-               int32_t *rr_out, int32_t *iters_out, float *kernel_ms)
-{
-    GridArgs a = grid_args(gv, hv, P, S, t, F0, rr0);
-    // a previous launch that timed out may have left the barrier mid-count
-    DDP_HIP(ctx, hipMemsetAsync(S.ctrl + GA_BAR, 0, 8, ctx->stream));
-    DDP_HIP(ctx, hipMemsetAsync(S.ctrl + GA_RES_ERR, 0, 4, ctx->stream));
-    DDP_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-    int rc = grid_enqueue(ctx, a, P, hv.kind);
-    if (rc) return rc;
-    DDP_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
-    return grid_finish(ctx, P, S, F_out, rr_out, iters_out, kernel_ms);
-}
-
 // Grid mode on piles: a fresh search (ddp_ga_reset before).
 int ddp_ga_run_piles(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P, const GaGridState &S,
                      int32_t s, uint32_t hs, int32_t t, uint32_t *F_out, int32_t *iters_out, float *kernel_ms)
@@ -757,7 +441,7 @@ int ddp_ga_run_piles(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, cons
     int rc = pg_enqueue(ctx, gv, hv, P, S, s, hs, t);
     if (rc) return rc;
     DDP_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
-    return grid_finish(ctx, P, S, F_out, nullptr, iters_out, kernel_ms);
+    return grid_finish(ctx, P, S, F_out, iters_out, kernel_ms);
 }
 
 int ddp_ga_run_wg(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P,
@@ -926,14 +610,9 @@ extern "C" int ddp_astar(ddp_ctx *ctx, const ddp_graph *g, ddp_heur_t h, int32_t
         }
     }
     if (parent_out) {
-        int32_t *dpar = nullptr;
         void *p;
-        // reuse the push buffer region as a staging area when large enough
-        if (!P.pg && (size_t)P.pcap * 16 >= (size_t)g->N * 4) dpar = (int32_t *)S.pbuf;
-        else {
-            if ((rc = ddp_ws(ctx, WS_PATH, (size_t)g->N * 4 + 256, &p))) return rc;
-            dpar = (int32_t *)p;
-        }
+        if ((rc = ddp_ws(ctx, WS_PATH, (size_t)g->N * 4 + 256, &p))) return rc;
+        int32_t *dpar = (int32_t *)p;
         hipLaunchKernelGGL(unpack_parent_kernel, dim3(1024), dim3(256), 0, ctx->stream, S.gp, dpar, g->N);
         DDP_HIP(ctx, hipMemcpyAsync(parent_out, dpar, (size_t)g->N * 4, hipMemcpyDeviceToHost, ctx->stream));
         DDP_HIP(ctx, hipStreamSynchronize(ctx->stream));

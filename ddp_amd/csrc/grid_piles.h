@@ -27,6 +27,12 @@
 // 2,048 x 2,048 maze, K = 512, 49.1 and 26.0 ms.  What is left is latency: a
 // round is seven dependent round trips and a barrier, 6 us.
 //
+// RESUME (DA*): the search starts from an open set -- the first entries of far0,
+// counted on the device -- with F(t) read from the target's word, and a current
+// entry that cannot beat F(t) goes to a dormant pile instead of being dropped:
+// a later batch may raise F(t) again. On return the dormant pile holds the open
+// set for the next resume.  Every relaxation is kept, whatever F(t) is.
+//
 // Everything workgroups share -- the (f, parent) words, the piles, the control
 // words -- is accessed through agent-scope atomics only, as grid_sync needs.
 // A round's steps each end with grid_sync; what a step appended is counted in
@@ -76,6 +82,14 @@ struct PgArgs {
     uint32_t nmask, fcap, hubcap;
     uint32_t *ctrl;
     unsigned long long *stats;
+    // RESUME: the dormant pile (dcap entries) and its count, the live entries'
+    // count and smallest f, and whether counting them overflowed; with
+    // `rebuild`, piles that overflow are rebuilt from the N nodes' words
+    uint64_t *dorm;
+    uint32_t dcap;
+    uint32_t *dorm_n;
+    const uint32_t *live_n, *live_min, *live_ovf;
+    int32_t N, rebuild;
     int32_t t, maxit;
     uint32_t grow;        // K: a window that fed fewer entries doubles, one that fed 8 times as many halves
     uint32_t thr0, delta0;
@@ -85,17 +99,22 @@ struct PgArgs {
 // Where a step's improvements go: staged in LDS, and placed with one atomic
 // per workgroup and pile when the step ends; what LDS cannot hold is placed
 // by its wave at once.
-template <int B>
+template <int B, bool RESUME>
 struct PgStage {
     static constexpr uint32_t kCap = 2 * B;
-    uint64_t near[kCap], far[kCap];
-    uint32_t n[2], base[2];  // near, far
+    static constexpr int kPiles = RESUME ? 3 : 2;
+    uint64_t q[kPiles][kCap];            // near, far, dormant
+    uint32_t n[kPiles], base[kPiles];
     uint32_t tmin, fmin, err;
 };
 
-template <int B>
+// Error bits beside GA_ERR_*: a resumed search's piles overflowed and are to be rebuilt.
+constexpr uint32_t PG_ERR_REBUILD = 0x100;
+
+template <int B, bool RESUME>
 struct PgPush {
-    PgStage<B> *S;
+    using Stage = PgStage<B, RESUME>;
+    Stage *S;
     const PgArgs *a;
     uint32_t *slot;       // this step's counters
     uint32_t nbase, head; // ring positions where this step's appends start, and of the oldest entry
@@ -104,17 +123,27 @@ struct PgPush {
     uint32_t thr, F;
     uint32_t fmin = 0xFFFFFFFFu;  // smallest f this lane sent to the far pile
 
-    __device__ __forceinline__ void put_near(uint32_t k, uint64_t key) const
+    __device__ __forceinline__ uint32_t *counter(int pile) const
     {
-        const uint32_t pos = nbase + k;
-        if (pos - head <= a->nmask) st_u64(a->near + (pos & a->nmask), key);
-        else atomicOr(&S->err, (uint32_t)GA_ERR_HEAP);
+        return pile == 0 ? slot + PG_NEAR : pile == 1 ? slot + PG_FAR : a->dorm_n;
     }
-    __device__ __forceinline__ void put_far(uint32_t k, uint64_t key) const
+    // entry k of what this step appends to the pile (of the dormant pile: entry k)
+    __device__ __forceinline__ void put(int pile, uint32_t k, uint64_t key) const
     {
-        const uint64_t pos = (uint64_t)fbase + k;
-        if (pos < a->fcap) st_u64(far + pos, key);
-        else atomicOr(&S->err, (uint32_t)GA_ERR_HEAP);
+        bool ok;
+        if (pile == 0) {
+            const uint32_t pos = nbase + k;
+            ok = pos - head <= a->nmask;
+            if (ok) st_u64(a->near + (pos & a->nmask), key);
+        } else if (pile == 1) {
+            const uint64_t pos = (uint64_t)fbase + k;
+            ok = pos < a->fcap;
+            if (ok) st_u64(far + pos, key);
+        } else {
+            ok = k < a->dcap;
+            if (ok) st_u64(a->dorm + k, key);
+        }
+        if (!ok) atomicOr(&S->err, RESUME && a->rebuild ? PG_ERR_REBUILD : (uint32_t)GA_ERR_HEAP);
     }
     __device__ __forceinline__ void target(uint32_t f) const { atomicMin(&S->tmin, f); }
     __device__ __forceinline__ void touch(int32_t, uint64_t) const {}
@@ -125,27 +154,24 @@ struct PgPush {
     __device__ __forceinline__ void all(const bool (&has)[R], const uint64_t (&key)[R])
     {
 #pragma unroll
-        for (int pile = 0; pile < 2; ++pile) {
+        for (int pile = 0; pile < Stage::kPiles; ++pile) {
             bool sel[R];
             uint32_t pos[R];
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 const uint32_t f = (uint32_t)(key[r] >> 32);
-                sel[r] = has[r] && f < F && (f < thr) == (pile == 0);
+                sel[r] = has[r] && (f < F ? (f < thr ? 0 : 1) : 2) == pile;
                 if (pile == 1 && sel[r] && f < fmin) fmin = f;
             }
             wave_append<R>(sel, &S->n[pile], pos);
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                if (sel[r] && pos[r] < PgStage<B>::kCap) (pile == 0 ? S->near : S->far)[pos[r]] = key[r];
-                const bool over[1] = {sel[r] && pos[r] >= PgStage<B>::kCap};
+                if (sel[r] && pos[r] < Stage::kCap) S->q[pile][pos[r]] = key[r];
+                const bool over[1] = {sel[r] && pos[r] >= Stage::kCap};
                 if (__any(over[0])) {
                     uint32_t k[1];
-                    wave_append<1>(over, slot + (pile == 0 ? PG_NEAR : PG_FAR), k);
-                    if (over[0]) {
-                        if (pile == 0) put_near(k[0], key[r]);
-                        else put_far(k[0], key[r]);
-                    }
+                    wave_append<1>(over, counter(pile), k);
+                    if (over[0]) put(pile, k[0], key[r]);
                 }
             }
         }
@@ -159,36 +185,38 @@ struct PgPush {
             if ((lane & 63) == 0) atomicMin(&S->fmin, m);
         }
         __syncthreads();
-        if (lane == 0 || lane == 64) {
+        if ((lane & 63) == 0 && lane < 64 * Stage::kPiles) {  // a wave per pile, so that the round trips overlap
             const int pile = lane >> 6;
-            const uint32_t m = S->n[pile] < PgStage<B>::kCap ? S->n[pile] : PgStage<B>::kCap;
-            S->base[pile] = m ? add_u32(slot + (pile == 0 ? PG_NEAR : PG_FAR), m) : 0;
+            const uint32_t m = S->n[pile] < Stage::kCap ? S->n[pile] : Stage::kCap;
+            S->base[pile] = m ? add_u32(counter(pile), m) : 0;
         } else if (lane == 192) {
             if (S->fmin != 0xFFFFFFFFu)
                 (void)__hip_atomic_fetch_min(slot + PG_FMIN, S->fmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } else if (lane == 128) {
             if (S->tmin != 0xFFFFFFFFu)
                 (void)__hip_atomic_fetch_min(slot + PG_TMIN, S->tmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         __syncthreads();
-        const uint32_t m0 = S->n[0] < PgStage<B>::kCap ? S->n[0] : PgStage<B>::kCap;
-        const uint32_t m1 = S->n[1] < PgStage<B>::kCap ? S->n[1] : PgStage<B>::kCap;
-        for (uint32_t k = lane; k < m0; k += B) put_near(S->base[0] + k, S->near[k]);
-        for (uint32_t k = lane; k < m1; k += B) put_far(S->base[1] + k, S->far[k]);
+#pragma unroll
+        for (int pile = 0; pile < Stage::kPiles; ++pile) {
+            const uint32_t m = S->n[pile] < Stage::kCap ? S->n[pile] : Stage::kCap;
+            for (uint32_t k = lane; k < m; k += B) put(pile, S->base[pile] + k, S->q[pile][k]);
+        }
         __syncthreads();
         if (lane == 0) {
             if (S->err) (void)__hip_atomic_fetch_or(slot + PG_ERR, S->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            S->n[0] = S->n[1] = 0;
+#pragma unroll
+            for (int pile = 0; pile < Stage::kPiles; ++pile) S->n[pile] = 0;
             S->tmin = S->fmin = 0xFFFFFFFFu;
+            S->err = 0;
         }
     }
 };
 
 // The edges [start, start + len) of node u (g value gu) by the eight lanes of
 // a group; every lane of the wave calls it (len = 0: nothing to do).
-template <int B, int HK>
+template <int B, int HK, bool RESUME>
 __device__ __forceinline__ void pg_expand(const PgArgs &a, uint32_t start, uint32_t len, int32_t u, uint32_t gu,
-                                          uint32_t F, ExpandCounters &C, PgPush<B> &push)
+                                          uint32_t Fb, ExpandCounters &C, PgPush<B, RESUME> &push)
 {
     constexpr int U = kPgUnroll;
     const uint32_t sub = threadIdx.x % kPgLanes;
@@ -211,14 +239,15 @@ __device__ __forceinline__ void pg_expand(const PgArgs &a, uint32_t start, uint3
 #pragma unroll
         for (int r = 0; r < U; ++r)
             if (a.g.dver && dv[r] <= a.g.ver) c[r] = -1;  // deleted at or before this version
-        relax_window<U, HK>(a.g, a.h, a.gp, a.t, c, wt, [&](int) { return gu; }, [&](int) { return u; }, F, C, push);
+        relax_window<U, HK>(a.g, a.h, a.gp, a.t, c, wt, [&](int) { return gu; }, [&](int) { return u; }, Fb, C, push);
     }
 }
 
-template <int B, int HK>
+template <int B, int HK, bool RESUME = false>
 __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
 {
-    __shared__ PgStage<B> S;
+    static_assert(B >= 256, "flush uses four waves");
+    __shared__ PgStage<B, RESUME> S;
     __shared__ int32_t s_flag;
     constexpr uint32_t kPerWave = 64 / kPgLanes, kWaves = B / 64;
     const int lane = threadIdx.x;
@@ -229,13 +258,23 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
     uint32_t head = 0, tail = 1, fn = 0, F = DDP_INF_F, thr = a.thr0, delta = a.delta0, phase_n = 0;
     uint32_t low = 0xFFFFFFFFu;  // no live far entry is below this
     uint64_t *far = a.far0, *far2 = a.far1;
-    uint32_t step = 0, err = 0;
+    uint32_t step = 0, err = 0, err_seen = 0;
     int32_t it = 0;
     bool timeout = false;
     ExpandCounters C;
     uint32_t stale = 0;
+    if constexpr (RESUME) {
+        tail = 0;
+        fn = ld_u32(a.live_n);
+        low = ld_u32(a.live_min);
+        F = (uint32_t)(ld_gp(a.gp + a.t) >> 32);
+        if (ld_u32(a.live_ovf) || fn > a.fcap) {
+            fn = 0;
+            err = GA_ERR_HEAP;
+        }
+    }
     if (lane == 0) {
-        S.n[0] = S.n[1] = 0;
+        for (int pile = 0; pile < PgStage<B, RESUME>::kPiles; ++pile) S.n[pile] = 0;
         S.tmin = S.fmin = 0xFFFFFFFFu;
         S.err = 0;
     }
@@ -250,7 +289,52 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
         return ctrl + PG_SLOTS + (step % 3) * PG_SLOT_WORDS;
     };
     auto add_sat = [](uint32_t x, uint32_t y) { return x > 0xFFFFFFFFu - y ? 0xFFFFFFFFu : x + y; };
-    for (;;) {
+    while (!err) {
+        if constexpr (RESUME) {
+            if (err_seen & PG_ERR_REBUILD) {
+                // entries were lost: the piles start again from every node with a
+                // finite word (nodes that were expanded at that value already are
+                // expanded again, which is harmless)
+                err_seen = 0;
+                if (blockIdx.x == 0 && lane == 0) {
+                    st_u32(a.dorm_n, 0u);
+                    C.rebuilds++;
+                }
+                uint32_t *slot = begin();
+                if (!grid_sync(ctrl + PG_BAR, gridDim.x, gen, a.barrier_ticks, &s_flag)) {
+                    timeout = true;
+                    break;
+                }
+                ++step;
+                slot = begin();
+                head = tail;
+                PgPush<B, RESUME> push{&S, &a, slot, tail, head, far, 0u, thr, F};
+                const uint32_t stride = gridDim.x * B, trips = ((uint32_t)a.N + stride - 1) / stride;
+                for (uint32_t r = 0; r < trips; ++r) {
+                    const uint32_t v = r * stride + blockIdx.x * B + lane;
+                    uint64_t key[1] = {0};
+                    bool live[1] = {false};
+                    if (v < (uint32_t)a.N && v != (uint32_t)a.t) {
+                        const uint32_t f = (uint32_t)(ld_gp(a.gp + v) >> 32);
+                        live[0] = f != DDP_INF_F;
+                        key[0] = (uint64_t)f << 32 | v;
+                    }
+                    push.template all<1>(live, key);
+                }
+                push.flush();
+                if (!grid_sync(ctrl + PG_BAR, gridDim.x, gen, a.barrier_ticks, &s_flag)) {
+                    timeout = true;
+                    break;
+                }
+                ++step;
+                tail += ld_u32(slot + PG_NEAR);
+                fn = ld_u32(slot + PG_FAR);
+                low = ld_u32(slot + PG_FMIN);
+                err_seen = ld_u32(slot + PG_ERR);
+                err = err_seen & ~PG_ERR_REBUILD;
+                continue;
+            }
+        }
         const uint32_t avail = tail - head;
         if (avail == 0 && (fn == 0 || low >= F)) break;  // nothing open can improve t
         // The far pile is split when the near ring is empty, or when all but
@@ -280,12 +364,15 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
         // ---- step 1: the round's entries, hub rows cut into segments, and the split
         uint32_t *slot = begin();
         {
-            PgPush<B> push{&S, &a, slot, tail, head, split ? far2 : far, split ? 0u : fn, thr, F};
+            PgPush<B, RESUME> push{&S, &a, slot, tail, head, split ? far2 : far, split ? 0u : fn, thr, F};
             const uint32_t chunks = (n + kPerWave - 1) / kPerWave;
             for (uint32_t ch = (lane >> 6) * gridDim.x + blockIdx.x; ch < chunks; ch += kWaves * gridDim.x) {
                 const uint32_t i = ch * kPerWave + wl / kPgLanes;
                 int32_t u = -1;
                 uint32_t gu = 0, start = 0, deg = 0;
+                uint64_t link = ~0ull;  // head of the node's list of inserted edges
+                bool dz[1] = {false};   // current, but hopeless now
+                uint64_t dkey[1] = {0};
                 if (i < n) {
                     const uint64_t key = ld_gp(a.near + ((head + i) & a.nmask));
                     const uint32_t f = (uint32_t)(key >> 32);
@@ -294,6 +381,9 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
                     const uint64_t word = ld_gp(a.gp + node);
                     const int32_t rb = a.g.off[node], re = a.g.off[node + 1];
                     const int32_t hn = heur_eval<HK>(a.h, node);
+                    if (a.g.lhead && sub == 0) link = ld_gp(a.g.lhead + node);
+                    dz[0] = RESUME && f >= F && (uint32_t)(word >> 32) == f && node != a.t && sub == 0;
+                    dkey[0] = key;
                     if (f < F && (uint32_t)(word >> 32) == f) {
                         u = node;
                         gu = f - (uint32_t)hn;
@@ -304,6 +394,8 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
                         ++stale;
                     }
                 }
+                if constexpr (RESUME)
+                    if (__any(dz[0])) push.template all<1>(dz, dkey);
                 if (__any(deg > (uint32_t)kPgSeg)) {
                     uint32_t at = 0;
                     const uint32_t parts = (deg + kPgSeg - 1) / kPgSeg;
@@ -320,12 +412,12 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
                         if (fits) deg = 0;
                     }
                 }
-                pg_expand<B, HK>(a, start, deg, u, gu, F, C, push);
+                pg_expand<B, HK>(a, start, deg, u, gu, RESUME ? 0xFFFFFFFFu : F, C, push);
                 if (a.g.lhead) {
                     // Versioned inserts: the group's first lane walks the node's
                     // list, oldest first, up to the first entry newer than this
                     // version (links carry the inserting version).
-                    uint64_t link = u >= 0 && sub == 0 ? ld_gp(a.g.lhead + u) : ~0ull;
+                    if (u < 0) link = ~0ull;
                     for (;;) {
                         bool active = false;
                         int32_t x = -1;
@@ -371,7 +463,8 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
                     if (i < fn) {
                         key[0] = ld_gp(far + i);
                         const uint32_t f = (uint32_t)(key[0] >> 32);
-                        live[0] = f < F && (uint32_t)(ld_gp(a.gp + (uint32_t)key[0]) >> 32) == f;
+                        live[0] = (RESUME ? (int32_t)(uint32_t)key[0] != a.t : f < F) &&
+                                  (uint32_t)(ld_gp(a.gp + (uint32_t)key[0]) >> 32) == f;
                         C.scanned++;
                     }
                     push.template all<1>(live, key);
@@ -393,18 +486,18 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
             fn = (split ? 0 : fn) + ld_u32(slot + PG_FAR);
             const uint32_t fm = ld_u32(slot + PG_FMIN);
             low = !split && low < fm ? low : fm;
-            err |= ld_u32(slot + PG_ERR);
+            err_seen |= ld_u32(slot + PG_ERR);
+            err = err_seen & ~PG_ERR_REBUILD;
         }
         if (split) {
             uint64_t *tmp = far;
             far = far2;
             far2 = tmp;
         }
-        if (err) break;
-        if (hubs) {
+        if (hubs && !err) {
             // ---- step 2: the segments of long rows
             slot = begin();
-            PgPush<B> push{&S, &a, slot, tail, head, far, fn, thr, F};
+            PgPush<B, RESUME> push{&S, &a, slot, tail, head, far, fn, thr, F};
             const uint32_t chunks = (hubs + kPerWave - 1) / kPerWave;
             for (uint32_t ch = (lane >> 6) * gridDim.x + blockIdx.x; ch < chunks; ch += kWaves * gridDim.x) {
                 const uint32_t i = ch * kPerWave + wl / kPgLanes;
@@ -414,7 +507,7 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
                     from = ld_gp(a.hubs + 2 * (uint64_t)i + 1);
                 }
                 pg_expand<B, HK>(a, (uint32_t)row, (uint32_t)(row >> 32), (int32_t)(uint32_t)from,
-                                 (uint32_t)(from >> 32), F, C, push);
+                                 (uint32_t)(from >> 32), RESUME ? 0xFFFFFFFFu : F, C, push);
             }
             push.flush();
             if (!grid_sync(ctrl + PG_BAR, gridDim.x, gen, a.barrier_ticks, &s_flag)) {
@@ -428,9 +521,18 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
             low = low < fm ? low : fm;
             tail += ld_u32(slot + PG_NEAR);
             fn += ld_u32(slot + PG_FAR);
-            err |= ld_u32(slot + PG_ERR);
-            if (err) break;
+            err_seen |= ld_u32(slot + PG_ERR);
+            err = err_seen & ~PG_ERR_REBUILD;
         }
+    }
+    if constexpr (RESUME) {
+        // what is left of the far pile cannot beat F(t): dormant.  Nobody
+        // appends any more, so every workgroup reads the same count.
+        const uint32_t dn = ld_u32(a.dorm_n);
+        if ((uint64_t)dn + fn > a.dcap) err |= GA_ERR_HEAP;
+        else
+            for (uint32_t i = blockIdx.x * B + lane; i < fn; i += gridDim.x * B) st_u64(a.dorm + dn + i, ld_gp(far + i));
+        if (blockIdx.x == 0 && lane == 0) ctrl[GA_RES_PLEN] = dn + fn;
     }
     if (timeout && lane == 0) atomicOr(ctrl + GA_RES_ERR, (uint32_t)GA_ERR_BARRIER);
     if (blockIdx.x == 0 && lane == 0) {
@@ -439,11 +541,15 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
         ctrl[GA_RES_F] = F;
     }
     const uint64_t v0 = wave_sum_u64(C.expanded), v1 = wave_sum_u64(C.edges), v2 = wave_sum_u64(C.improved),
-                   v3 = wave_sum_u64(stale);
+                   v3 = wave_sum_u64(stale), v4 = wave_sum_u64(C.rebuilds), v5 = wave_sum_u64(C.refills),
+                   v6 = wave_sum_u64(C.scanned);
     if (wl == 0) {
         atomicAdd(a.stats + 0, (unsigned long long)v0);
         atomicAdd(a.stats + 1, (unsigned long long)v1);
         atomicAdd(a.stats + 2, (unsigned long long)v2);
         atomicAdd(a.stats + 3, (unsigned long long)v3);
+        if (v4) atomicAdd(a.stats + 4, (unsigned long long)v4);
+        if (v5) atomicAdd(a.stats + 5, (unsigned long long)v5);
+        if (v6) atomicAdd(a.stats + 6, (unsigned long long)v6);
     }
 }
