@@ -82,7 +82,7 @@ __global__ void __launch_bounds__(B) batch_kernel(BatchArgs a)
                              {touched, touched + N}, {PF, PB}};
             slot_search_bidi<B, HK>(D, a.h, a.g.relax_min != 0, N, s, t, a.maxit, a.delta0, S, C, stale);
             if (a.path_cap > 0) {
-                slot_path_bidi(gp, gp + N, N, s, t, a.path + (int64_t)q * a.path_cap, a.path_cap, S);
+                slot_path_bidi(D, N, s, t, a.path + (int64_t)q * a.path_cap, a.path_cap, S);
                 if (lane == 0) a.plen[q] = S.plen;
             }
             slot_reset_bidi(gp, gp + N, touched, touched + N, S);

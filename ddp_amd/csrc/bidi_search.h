@@ -96,6 +96,8 @@ struct BidiLds {
     uint32_t err;
     int32_t plen;
     int32_t iters;
+    uint32_t wide;            // thin rounds: rows were left for the block
+    int32_t chain[2];         // path walk: nodes of the chain from the meeting node to either root
     BidiDir d[2];
 };
 
@@ -149,6 +151,10 @@ __device__ __forceinline__ void bidi_settle(const BidiSide &D, int32_t s, int32_
                                             uint64_t *const (&far)[2], BidiLds<B> &S)
 {
     wait_vmem();
+    bool any = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) any |= ok[r];
+    if (!__any(any)) return;
     uint64_t oth[R];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -372,6 +378,158 @@ __device__ __forceinline__ void expand_bidi(const BidiSide &D, const HeurView &H
     }
 }
 
+// A thin round: every entry gets kThinLanes lanes, which read its row together,
+// so there is no prefix scan, no owner map and no barrier between taking an
+// entry and relaxing its edges; and each direction has half of the waves to
+// itself, so a wave's pointers and limits are uniform and its pushes take one
+// LDS round trip (three counters in one instruction) where bidi_settle takes
+// six or more per direction.  A round of tens of entries is bound by what its
+// waves issue, by LDS round trips and by barriers: on a 64 x 64 maze (12
+// entries a round, everything in L2) a round took 6.4 us through expand_bidi
+// and 3.7 us here; on the 4,096 x 4,096 one (122 entries) 6.5 and 5.4.
+// Rows longer than kThinRow are left to expand_bidi (u, rs; S.wide says that
+// some lane has one).  For heuristics without loads, the atomicMin relaxation,
+// empty HBM rings and LDS rings with room for every row (the caller's rule).
+// An edge whose key cannot beat F is skipped before its atomic: its end would
+// be dropped and no meeting through it can be shorter.  No closing barrier.
+constexpr int kThinLanes = 2, kThinEdges = 2, kThinRow = 8;
+
+template <int B, int HK>
+__device__ __forceinline__ void expand_bidi_thin(const BidiSide &D, const HeurView &H, int32_t s, int32_t t,
+                                                 const uint32_t (&n)[2], const uint32_t (&lh)[2],
+                                                 const uint32_t (&thr)[2], const uint32_t (&F)[2],
+                                                 uint64_t *const (&far)[2], BidiLds<B> &S, ExpandCounters &C,
+                                                 uint32_t &stale, int32_t &u, RowSpan &rs)
+{
+    constexpr int R = kThinEdges, G = kThinLanes;
+    const bool one = __builtin_amdgcn_readfirstlane(threadIdx.x >= B / 2 ? 1 : 0) != 0;
+    const uint32_t l = threadIdx.x % (B / 2), me = l / G, sub = l % G;
+    const uint32_t nd = pick2(n, one);
+    u = -1;
+    if (__builtin_amdgcn_readfirstlane(me) >= nd) return;  // no entry for this wave
+    uint64_t *gp = pick2(D.gp, one), *go = pick2(D.gp, !one);
+    const int32_t *col = pick2(D.col, one);
+    const uint32_t *w = pick2(D.w, one);
+    uint64_t *lring = one ? D.P[1].lring : D.P[0].lring;
+    const uint32_t lmask = (one ? D.P[1].lcap : D.P[0].lcap) - 1, fcap = one ? D.P[1].fcap : D.P[0].fcap;
+    const uint32_t Fd = pick2(F, one), td = pick2(thr, one);
+    int32_t node = -1, deg = 0, b = 0;
+    uint32_t gu = 0;
+    if (me < nd) {
+        const uint64_t key = lring[(pick2(lh, one) + me) & lmask];
+        const uint32_t f = (uint32_t)(key >> 32);
+        node = (int32_t)(uint32_t)key;
+        const uint64_t word = ld_gp(gp + node);
+        const int32_t *off = pick2(D.off, one);
+        const int32_t rb = off[node], re = off[node + 1];
+        const int32_t pn = pot_from<HK>(H, node, HeurIn{0, 0});
+        if (f < Fd && (uint32_t)(word >> 32) == f) {
+            gu = f - (uint32_t)(one ? -pn : pn);
+            b = rb;
+            deg = re - rb;
+            if (deg > kThinRow) {
+                if (sub == 0) {
+                    u = node;
+                    rs.b = rb;
+                    rs.deg = deg;
+                    rs.gu = gu;
+                    S.wide = 1;
+                }
+                deg = 0;
+            } else if (sub == 0) {
+                C.expanded++;
+            }
+        } else if (sub == 0) {
+            ++stale;
+        }
+    }
+    for (int32_t j = 0; __any(j < deg); j += G * R) {
+        int32_t c[R];
+        uint32_t wt[R], cand[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            c[r] = -1;
+            wt[r] = 0;
+            const int32_t k = j + r * G + (int32_t)sub;
+            if (k < deg) {
+                c[r] = col[b + k];
+                wt[r] = w[b + k];
+                C.edges++;
+            }
+        }
+        uint64_t got[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int32_t pc = c[r] >= 0 ? pot_from<HK>(H, c[r], HeurIn{0, 0}) : 0;
+            cand[r] = gu + wt[r] + (uint32_t)(one ? -pc : pc);
+            if (cand[r] >= Fd) c[r] = -1;
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): every load above was consumed
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (c[r] >= 0)
+                got[r] = (uint64_t)atomicMin((unsigned long long *)(gp + c[r]),
+                                             ((unsigned long long)cand[r] << 32) | (uint32_t)node);
+        bool ok[R];
+        uint64_t oth[R], mp[R], mf[R], mt[R];
+        uint32_t cnt[3] = {0, 0, 0};
+        wait_vmem();  // the other side's words are read after this lane's atomics have completed
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            ok[r] = c[r] >= 0 && (uint32_t)(got[r] >> 32) > cand[r];
+            if (ok[r]) {
+                oth[r] = ld_gp(go + c[r]);
+                C.improved++;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const bool put = ok[r] && c[r] != (one ? s : t);  // the other search's root is never queued
+            mp[r] = __ballot(put && cand[r] < td);
+            mf[r] = __ballot(put && cand[r] >= td);
+            mt[r] = __ballot(ok[r] && (uint32_t)(got[r] >> 32) == DDP_INF_F);
+            cnt[0] += (uint32_t)__popcll(mp[r]);
+            cnt[1] += (uint32_t)__popcll(mf[r]);
+            cnt[2] += (uint32_t)__popcll(mt[r]);
+        }
+        if ((cnt[0] | cnt[1] | cnt[2]) != 0) {
+            // near ring, far pile and touched log reserved by three lanes at once
+            constexpr uint32_t kTail = offsetof(BidiDir, lring_tail) / 4, kFar = offsetof(BidiDir, far_n) / 4,
+                               kTouch = offsetof(BidiDir, ntouch) / 4;
+            const uint32_t wl = threadIdx.x & 63;
+            uint32_t *q = (uint32_t *)&S.d[one ? 1 : 0];
+            uint32_t base = 0;
+            if (wl < 3)
+                base = atomicAdd(q + (wl == 0 ? kTail : wl == 1 ? kFar : kTouch),
+                                 wl == 0 ? cnt[0] : wl == 1 ? cnt[1] : cnt[2]);
+            uint32_t bp = __builtin_amdgcn_readlane(base, 0), bf = __builtin_amdgcn_readlane(base, 1),
+                     bt = __builtin_amdgcn_readlane(base, 2);
+            const uint64_t bit = 1ull << wl;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const uint64_t key = ((uint64_t)cand[r] << 32) | (uint32_t)c[r];
+                if (mp[r] & bit) lring[(bp + lane_rank(mp[r])) & lmask] = key;
+                if (mf[r] & bit) {
+                    const uint32_t pos = bf + lane_rank(mf[r]);
+                    if (pos < fcap) pick2(far, one)[pos] = key;
+                    else S.d[one ? 1 : 0].ovf = 1;  // dropped: the next refill rebuilds the far pile
+                }
+                if (mt[r] & bit) pick2(D.touched, one)[bt + lane_rank(mt[r])] = c[r];
+                bp += (uint32_t)__popcll(mp[r]);
+                bf += (uint32_t)__popcll(mf[r]);
+                bt += (uint32_t)__popcll(mt[r]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (ok[r] && (uint32_t)(oth[r] >> 32) != DDP_INF_F) {
+                const uint64_t mu = (uint64_t)cand[r] + (oth[r] >> 32);
+                if (mu < DDP_INF_F) atomicMin(&S.meet, (unsigned long long)((mu << 32) | (uint32_t)c[r]));
+            }
+        }
+    }
+}
+
 // Refill of direction d's near rings from its far pile (the refill of
 // slot_search_piles); a full refill (near rings empty) publishes the
 // direction's bound.  Block-collective; ends with a barrier.  The direction
@@ -504,7 +662,11 @@ __device__ __forceinline__ void slot_search_bidi(const BidiSide &D, HeurView hv,
 {
     constexpr uint32_t Vd = B / 2;
     const int lane = threadIdx.x;
+    // thin rounds: where registers allow the second expansion (1,024 lanes have
+    // 128 each, and the wide one takes them all)
+    constexpr bool kThin = B <= 512 && !VERS && (HK == DDP_H_ZERO || HK == DDP_H_MANHATTAN);
     if (lane == 0) {
+        S.wide = 0;
         S.meet = kNoMeet;
         S.bound[0] = S.bound[1] = 0;
         S.err = 0;
@@ -553,6 +715,9 @@ __device__ __forceinline__ void slot_search_bidi(const BidiSide &D, HeurView hv,
     uint64_t *far[2] = {D.P[0].far0, D.P[1].far0}, *far2[2] = {D.P[0].far1, D.P[1].far1};
     uint32_t lh[2] = {0, 0}, hh[2] = {0, 0};  // ring heads (uniform)
     int32_t it = 0;
+    int32_t u = -1;
+    RowSpan rs;
+    uint32_t wide_F[2] = {0, 0};  // bounds of the thin round whose long rows are still to be expanded
     while (run) {
         // Every LDS word the round's decisions need, read together: they are
         // independent, so one wait covers them (read one by one between the
@@ -561,8 +726,8 @@ __device__ __forceinline__ void slot_search_bidi(const BidiSide &D, HeurView hv,
         // which its closing barrier ordered; only HBM ring contents need the
         // store drain below.
         const uint64_t meet = S.meet;
-        const uint32_t b0 = S.bound[0], b1 = S.bound[1];
-        uint32_t lt[2], nt[2], fn[2], ov[2], ne[2];
+        const uint32_t b0 = S.bound[0], b1 = S.bound[1], wide = kThin ? S.wide : 0;
+        uint32_t lt[2], nt[2], fn[2], ov[2], ne[2], tr[2];
 #pragma unroll
         for (int d = 0; d < 2; ++d) {
             lt[d] = S.d[d].lring_tail;
@@ -570,6 +735,24 @@ __device__ __forceinline__ void slot_search_bidi(const BidiSide &D, HeurView hv,
             fn[d] = S.d[d].far_n;
             ov[d] = S.d[d].ovf;
             ne[d] = S.d[d].no_early;
+            tr[d] = S.d[d].thr;
+        }
+        if constexpr (kThin) {
+            if (lane == 0) {  // a thin round leaves the heads to the next one
+#pragma unroll
+                for (int d = 0; d < 2; ++d) {
+                    S.d[d].lring_head = lh[d];
+                    S.d[d].near_head = hh[d];
+                }
+            }
+            if (wide) {  // long rows of the thin round just done
+                __syncthreads();
+                if (lane == 0) S.wide = 0;
+                expand_bidi<B, HK, VERS>(D, hv, relax_min, s, t, u, rs, B / 2, wide_F, far, S, C);
+                __syncthreads();
+                if (S.err) break;
+                continue;
+            }
         }
         const uint32_t mu = (uint32_t)(meet >> 32);
         if ((uint64_t)b0 + b1 >= mu) break;  // no open entry on either side can shorten mu
@@ -610,8 +793,33 @@ __device__ __forceinline__ void slot_search_bidi(const BidiSide &D, HeurView hv,
         // lanes: each side gets at least half when it has that many
         const uint32_t n0 = min(avail[0], (uint32_t)B - min(avail[1], Vd));
         const uint32_t n1 = min(avail[1], (uint32_t)B - n0);
-        int32_t u = -1;
-        RowSpan rs;
+        if constexpr (kThin) {
+            constexpr uint32_t kMost = B / 2 / kThinLanes;  // entries a direction's waves take at once
+            bool thin = relax_min;
+#pragma unroll
+            for (int d = 0; d < 2; ++d)
+                thin = thin && from_lds[d] && nt[d] == hh[d] && avail[d] <= kMost &&
+                       avail[d] * (kThinRow + 1) <= (d ? D.P[1].lcap : D.P[0].lcap);
+            if (thin) {
+                // every wave has read the words above before a fast one changes them
+                __syncthreads();
+                expand_bidi_thin<B, HK>(D, hv, s, t, avail, lh, tr, F, far, S, C, stale, u, rs);
+                // the heads move on in registers only: a slower wave may still
+                // be reading its entries when a faster one pushes
+                lh[0] += avail[0];
+                lh[1] += avail[1];
+                if (lane == 0) {
+                    S.d[0].phase_n += avail[0];
+                    S.d[1].phase_n += avail[1];
+                }
+                wide_F[0] = F[0];
+                wide_F[1] = F[1];
+                __syncthreads();
+                if (S.err) break;
+                continue;
+            }
+        }
+        u = -1;
         if ((uint32_t)lane < n0 + n1) {
             const int d = (uint32_t)lane >= n0 ? 1 : 0;
             const uint32_t idx = d ? lane - n0 : lane;
@@ -665,55 +873,67 @@ __device__ __forceinline__ void slot_search_bidi(const BidiSide &D, HeurView hv,
     block_sync_global();
 }
 
-// Lane 0 writes the path s..t through the meeting node into out[0..cap) and
-// its length into S.plen (0 if unreachable, -len if longer than cap).
+// Writes the path s..t through the meeting node into out[0..cap) and its length
+// into S.plen (0 if unreachable, -len if longer than cap).  Two lanes walk the
+// two chains at the same time, one dependent read a hop, into the far piles
+// (free now); the block then copies them out.  A chain longer than its far
+// pile (a small heap_cap) is walked again, into out.  Block-collective.
 template <int B>
-__device__ void slot_path_bidi(const uint64_t *gpf, const uint64_t *gpb, int32_t N, int32_t s, int32_t t,
-                               int32_t *out, int32_t cap, BidiLds<B> &S)
+__device__ void slot_path_bidi(const BidiSide &D, int32_t N, int32_t s, int32_t t, int32_t *out, int32_t cap,
+                               BidiLds<B> &S)
 {
-    if (threadIdx.x != 0) return;
+    const int lane = threadIdx.x;
     const uint64_t meet = S.meet;
-    int32_t n = 0;
-    if ((uint32_t)(meet >> 32) != DDP_INF_F) {
-        const int32_t m = (int32_t)(uint32_t)meet;
-        // m back to s along forward parents
-        int32_t v = m;
-        for (int32_t step = 0; step <= N; ++step) {
-            if (n < cap) out[n] = v;
-            ++n;
-            if (v == s) break;
-            const uint32_t p = (uint32_t)ld_gp(gpf + v);
-            if (p >= (uint32_t)N) {
-                n = -1;
-                break;
-            }
+    if ((uint32_t)(meet >> 32) == DDP_INF_F) {
+        if (lane == 0) S.plen = 0;
+        __syncthreads();
+        return;
+    }
+    const int32_t m = (int32_t)(uint32_t)meet;
+    const uint32_t room = D.P[0].fcap < 0x3FFFFFFFu ? 2 * D.P[0].fcap : 0x7FFFFFFFu;  // both piles are as large
+    auto walk = [&](const uint64_t *gp, int32_t root, auto keep) {  // nodes from m (not kept) to the root
+        int32_t v = m, n = 0;
+        while (v != root) {
+            const uint32_t p = (uint32_t)ld_gp(gp + v);
+            if (p >= (uint32_t)N || n > N) return (int32_t)-1;
             v = (int32_t)p;
+            keep(n++, v);
         }
-        if (n > 0 && n <= cap)
-            for (int32_t i = 0; i < n / 2; ++i) {  // m..s -> s..m
-                const int32_t x = out[i];
-                out[i] = out[n - 1 - i];
-                out[n - 1 - i] = x;
-            }
-        // m on to t along backward parents
-        v = m;
-        for (int32_t step = 0; n > 0 && v != t && step <= N; ++step) {
-            const uint32_t p = (uint32_t)ld_gp(gpb + v);
-            if (p >= (uint32_t)N) {
-                n = -1;
-                break;
-            }
-            v = (int32_t)p;
-            if (n < cap) out[n] = v;
-            ++n;
-        }
-        if (n > 0 && v != t) n = -1;
-        if (n < 0) {
-            n = 0;
+        return n;
+    };
+    if (lane == 0 || lane == 64) {
+        const bool one = lane != 0;
+        int32_t *chain = (int32_t *)(one ? D.P[1].far0 : D.P[0].far0);
+        S.chain[one] = walk(one ? D.gp[1] : D.gp[0], one ? t : s, [&](int32_t k, int32_t v) {
+            if ((uint32_t)k < room) chain[k] = v;
+        });
+    }
+    block_sync_global();
+    const int32_t n0 = S.chain[0], n1 = S.chain[1];
+    const int32_t n = n0 + n1 + 1;
+    if (n0 < 0 || n1 < 0) {
+        if (lane == 0) {
+            S.plen = 0;
             atomicOr(&S.err, (uint32_t)QERR_PATH);
         }
+    } else {
+        if (lane == 0) S.plen = n > cap ? -n : n;
+        if (n <= cap) {
+            if (lane == 0) out[n0] = m;
+            const int32_t *c0 = (const int32_t *)D.P[0].far0, *c1 = (const int32_t *)D.P[1].far0;
+            if ((uint32_t)n0 <= room) {
+                for (int32_t i = lane; i < n0; i += B) out[n0 - 1 - i] = c0[i];
+            } else if (lane == 0) {
+                (void)walk(D.gp[0], s, [&](int32_t k, int32_t v) { out[n0 - 1 - k] = v; });
+            }
+            if ((uint32_t)n1 <= room) {
+                for (int32_t i = lane; i < n1; i += B) out[n0 + 1 + i] = c1[i];
+            } else if (lane == 0) {
+                (void)walk(D.gp[1], t, [&](int32_t k, int32_t v) { out[n0 + 1 + k] = v; });
+            }
+        }
     }
-    S.plen = (n > cap) ? -n : n;
+    __syncthreads();
 }
 
 // Clears every word either direction touched (barriers on both ends, as slot_reset).

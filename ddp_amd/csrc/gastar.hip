@@ -140,7 +140,7 @@ __global__ void __launch_bounds__(B) ga_wg_kernel(WgArgs a)
         const BidiSide D{{a.g.off, a.gr.off}, {a.g.col, a.gr.col}, {a.g.w, a.gr.w}, {a.gp, a.gp + N},
                          {a.touched, a.touched + N}, {PF, PB}};
         slot_search_bidi<B, HK>(D, a.h, a.g.relax_min != 0, N, a.s, a.t, a.maxit, a.delta0, S, C, stale);
-        if (a.path) slot_path_bidi(a.gp, a.gp + N, N, a.s, a.t, a.path, a.path_cap, S);
+        if (a.path) slot_path_bidi(D, N, a.s, a.t, a.path, a.path_cap, S);
         if (lane == 0) {
             const uint32_t e = S.err;
             a.ctrl[GA_RES_IT] = (uint32_t)S.iters;

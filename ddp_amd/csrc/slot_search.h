@@ -592,8 +592,9 @@ __device__ void slot_search_piles(const GraphView &G, HeurView hv, uint64_t *gp,
     block_sync_global();
 }
 
-// Lane 0 writes the path s..t into out[0..cap) and returns its length in
-// S.plen (0 if unreachable, -len if longer than cap).
+// Writes the path s..t into out[0..cap) and its length into S.plen (0 if
+// unreachable, -len if longer than cap): lane 0 walks t..s, one dependent read
+// a hop, and the block turns the path round.  Block-collective.
 template <int B, int V>
 __device__ void slot_path(const uint64_t *gp, int32_t N, int32_t s, int32_t t, int32_t *out, int32_t cap,
                           SlotLds<B, V> &S)
@@ -614,14 +615,15 @@ __device__ void slot_path(const uint64_t *gp, int32_t N, int32_t s, int32_t t, i
                 }
                 v = (int32_t)p;
             }
-            if (n > 0 && n <= cap)
-                for (int32_t i = 0; i < n / 2; ++i) {  // t..s -> s..t (this lane wrote every entry)
-                    const int32_t x = out[i];
-                    out[i] = out[n - 1 - i];
-                    out[n - 1 - i] = x;
-                }
         }
         S.plen = (n > cap) ? -n : n;
+    }
+    block_sync_global();
+    const int32_t n = S.plen;
+    for (int32_t i = threadIdx.x; i < n / 2; i += B) {
+        const int32_t x = __hip_atomic_load(out + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        out[i] = __hip_atomic_load(out + n - 1 - i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        out[n - 1 - i] = x;
     }
 }
 
