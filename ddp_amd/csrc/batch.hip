@@ -49,8 +49,7 @@ template <int B, int HK, int ENG>
 __global__ void __launch_bounds__(B) batch_kernel(BatchArgs a)
 {
     extern __shared__ uint64_t s_heap[];  // lcap * B (heap engine), near rings (pile engines)
-    constexpr int SV = (ENG == ENG_PILES) ? B * pile_entries_per_lane<B>() : B;  // expansion width
-    __shared__ std::conditional_t<ENG == ENG_BIDI, BidiLds<B>, SlotLds<B, SV>> S;
+    __shared__ std::conditional_t<ENG == ENG_BIDI, BidiLds<B>, SlotLds<B, ENG == ENG_PILES>> S;
     __shared__ int32_t s_q;
 
     const int lane = threadIdx.x;

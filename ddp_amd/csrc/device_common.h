@@ -174,6 +174,16 @@ __device__ __forceinline__ int32_t wave_incl_scan(int32_t v)
     return v;
 }
 
+// The same within every 16 lanes.
+__device__ __forceinline__ int32_t row16_incl_scan(int32_t v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    return v;
+}
+
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v)
 {
 #pragma unroll

@@ -126,8 +126,7 @@ template <int B, int HK, int WM>
 __global__ void __launch_bounds__(B) ga_wg_kernel(WgArgs a)
 {
     extern __shared__ uint64_t s_heap[];  // lcap * B (heaps), near rings (piles)
-    constexpr int SV = (WM == WM_PILES) ? B * pile_entries_per_lane<B>() : B;  // expansion width
-    __shared__ std::conditional_t<WM == WM_BIDI, BidiLds<B>, SlotLds<B, SV>> S;
+    __shared__ std::conditional_t<WM == WM_BIDI, BidiLds<B>, SlotLds<B, WM == WM_PILES>> S;
     const int lane = threadIdx.x;
     const LaneHeap H{s_heap + lane, a.home + lane, B, a.lcap, (int64_t)B, a.cap};
     ExpandCounters C;
@@ -152,7 +151,7 @@ __global__ void __launch_bounds__(B) ga_wg_kernel(WgArgs a)
     } else {
         if constexpr (WM == WM_PILES) {
             const PilePtrs P{a.home, a.home + a.ncap, a.home + a.ncap + a.fcap, a.ncap, a.fcap, s_heap, a.lring};
-            slot_search_piles<B, HK, pile_entries_per_lane<B>(), true>(a.g, a.h, a.gp, a.touched, P, a.N, a.s,
+            slot_search_piles<B, HK, true>(a.g, a.h, a.gp, a.touched, P, a.N, a.s,
                                                                               a.t, a.maxit, a.delta0, S, C, stale);
         } else {
             slot_search<B, HK>(a.g, a.h, a.gp, a.touched, H, s_heap, a.N, a.s, a.t, a.maxit, S, C, stale);

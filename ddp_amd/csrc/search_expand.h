@@ -2,17 +2,31 @@
 //
 // Each lane of the block brings at most one popped node u (its queue's pop).
 // Out-degrees are prefix-summed across the block and the union of all rows is
-// walked R*B edges per round, so lanes read consecutive CSR entries and a long
-// row is split across the whole block instead of serialising one lane (the
-// reference gives each thread its own row: GA_star/GA_v2.cu:109-167).
-// Within a window every lane owns R edges and issues their loads stage by
-// stage (row entries, then heuristic inputs and (f, parent) words, then the
-// CAS or atomicMin attempts), so R independent memory round trips overlap
-// instead of running back to back.
+// cut into one range of consecutive edges per wave, so lanes read consecutive
+// CSR entries and a long row is split across the whole block instead of
+// serialising one lane (the reference gives each thread its own row:
+// GA_star/GA_v2.cu:109-167).  A wave takes its range R windows of 64 edges at
+// a time and issues their loads stage by stage (row entries, then heuristic
+// inputs and (f, parent) words), so R independent memory round trips overlap.
+//
+// Edges that beat their node's word are few (5% on R-MAT, a fifth on a road
+// map), so a wave collects them in LDS and relaxes and queues 64 at a time.
+// Not for the lane-owned heaps: their pushes have to stay spread over the
+// lanes (collected, the C4 batch overflowed heaps of 2,048 entries, and with
+// the lanes taking turns it took 96-117 ms instead of 79).
+//
+// What a wave issues bounds a round, not what it waits for: with every stage
+// run for all R windows and the rows located by a binary search per edge (or by
+// owner hints in small rounds), a 1,024-lane workgroup spent 10.1 us on 4,096
+// edges in a batch of 256 queries on R-MAT (scale 20; a query 105 ms on
+// average), now 7.1 us (74 ms); the C4 batch went from 19.3 to 16.1 ms.
 #pragma once
 
 #include "device_common.h"
 
+// Owner hints of expand_bidi: edge slot of the round -> lane, written for rows
+// up to kOwnRun edges (every row of a road or geometric graph); the rest of a
+// longer row falls back to a binary search over the prefix.
 template <int V>
 struct ExpandLds {
     static_assert(V <= 65536, "owner entries are 16-bit");
@@ -21,13 +35,33 @@ struct ExpandLds {
     uint32_t gu[V];      // g(u) = f(u) - h(u), unsigned as GA_v2.cu:137
     int32_t node[V];
     int32_t tmp[16];
-    uint16_t own[16 * V];  // edge slot of the round -> virtual lane (a hint)
+    uint16_t own[16 * V];
 };
 
-// Owner entries a lane writes per row and window: rows up to this long (every
-// row of a road or geometric graph) are located with one LDS read per edge;
-// the rest of a longer row falls back to a binary search over the prefix.
 constexpr int32_t kOwnRun = 32;
+
+// Edges handled per lane and trip (memory requests a lane keeps in flight
+// per stage).  At 1,024 lanes two, three, four and six took 80, 78, 73 and 73
+// ms a query on R-MAT (scale 20) and 16.1, 16.2, 16.2 and 16.7 ms for C4.
+template <int B>
+constexpr int expand_unroll()
+{
+    return B == 512 ? 2 : 4;
+}
+
+// Rows of a round and its collected edges (expand_rows; COLLECT, else none).
+// Only rows that have edges are listed, so incl ascends strictly.
+template <int B, bool COLLECT>
+struct RowsLds {
+    static constexpr int CAP = COLLECT ? 64 * expand_unroll<B>() + 64 : 1;  // collected edges of a wave
+    int32_t incl[B];        // inclusive prefix of degrees
+    int32_t rowb[B];        // row start - edges before the row
+    uint32_t gu[B];         // g(u) = f(u) - h(u), unsigned as GA_v2.cu:137
+    int32_t node[B];
+    int2 tmp[B / 64];       // edges and rows of each wave
+    uint64_t key[B / 64 * CAP];  // candidate f << 32 | node
+    uint16_t row[B / 64 * CAP];
+};
 
 // What expanding u needs besides u itself: its row and g(u).
 struct RowSpan {
@@ -58,33 +92,70 @@ struct ExpandCounters {
     uint32_t scanned = 0;   // pile engine: far-pile entries read by refills
 };
 
-// Edges handled per lane and window (memory requests a lane keeps in flight
-// per stage).  Four where registers allow it without lowering occupancy (the
-// 1,024-lane pile kernel fits 128 VGPRs at four); two and three measured no
-// faster on the C4 batch.
-template <int B>
-constexpr int expand_unroll()
+// Rows of 64 consecutive edges, found by a wave at once: lane i reads the end
+// of row row + i and marks the lane of the edge after it; an edge's row is row
+// plus the marks up to it.  row: the row of edge e0, moved on to that of
+// e0 + 64.  Every lane of the wave calls it, with e0 below the last row's end.
+template <int B, bool COLLECT>
+__device__ __forceinline__ int32_t wave_rows(const RowsLds<B, COLLECT> &L, int32_t nrows, int32_t e0, int32_t &row)
 {
-    return B == 512 ? 2 : 4;
+    const int32_t wl = (int32_t)(threadIdx.x & 63), at = row + wl;
+    const int32_t p = at < nrows ? L.incl[at] - e0 : INT32_MAX;  // >= 1: row holds e0
+    const int32_t r0 = row;
+    const int32_t p0 = __builtin_amdgcn_readfirstlane(p);
+    if (p0 >= 64) {  // one row holds the window
+        row += p0 == 64 ? 1 : 0;
+        return r0;
+    }
+    row += (int32_t)__popcll(__ballot(p <= 64));
+    // lane 0, which no mark is for, takes what the other lanes push
+    const int32_t mark = __builtin_amdgcn_ds_permute((p < 64 ? p : 0) << 2, p < 64 ? 1 : 0);
+    const uint64_t m = __ballot(wl != 0 && mark != 0);
+    return r0 + (int32_t)lane_rank(m) + (int32_t)(m >> wl & 1);
 }
 
-// Stages 2-4 of one window of R edges per lane: edge r leads to c[r] (< 0:
+// Relaxes one candidate per lane (key: f << 32 | node, of a node at which it
+// can improve the word) and hands the improvements to the push policy.  Every
+// lane of the wave calls it.
+template <class Push>
+__device__ __forceinline__ void relax_collected(const GraphView &G, uint64_t *gp, int32_t t, bool have, uint64_t key,
+                                                int32_t par, ExpandCounters &C, Push &push)
+{
+    const uint32_t cand = (uint32_t)(key >> 32);
+    const int32_t c[1] = {(int32_t)(uint32_t)key};
+    bool ok = false;
+    uint64_t prev = 0;
+    if (G.relax_min != 0) {  // uniform
+        // one atomicMin: the smallest (f, parent) of the round wins with no
+        // retry round trips
+        if (have) {
+            prev = (uint64_t)atomicMin((unsigned long long *)(gp + c[0]),
+                                       ((unsigned long long)cand << 32) | (uint32_t)par);
+            ok = (uint32_t)(prev >> 32) > cand;
+        }
+    } else if (have) {
+        ok = relax_gp(gp, c[0], cand, (uint32_t)par, &prev);
+    }
+    if (ok) {
+        C.improved++;
+        if (c[0] == t) push.target(cand);
+    }
+    const bool first[1] = {ok && (uint32_t)(prev >> 32) == DDP_INF_F}, has[1] = {ok && c[0] != t};
+    const uint64_t k[1] = {key};
+    push.template touch_all<1>(first, c);
+    push.template all<1>(has, k);
+}
+
+// Relaxes R edges per lane (grid engine, lane heaps): edge r leads to c[r] (< 0:
 // none) with weight wt[r] from the node par(r), whose g is gu(r).  Loads are
 // issued stage by stage (heuristic inputs and (f, parent) words, then one
 // atomic per improving edge), and improvements go to the push policy.  Fb
 // as in expand_rows.
-//
-// DIRECT (atomicMin relaxation, heuristics that need no load): no word is
-// read first; every edge that can still beat Fb issues its atomicMin, whose
-// returned word says whether it improved.  A small round is a chain of
-// dependent round trips, and this takes one out of it; a large round keeps the
-// read, which spares the atomics of the many edges that cannot improve.
-template <int R, int HK, bool DIRECT = false, class GuOf, class ParOf, class Push>
+template <int R, int HK, class GuOf, class ParOf, class Push>
 __device__ __forceinline__ void relax_window(const GraphView &G, const HeurView &H, uint64_t *gp, int32_t t,
                                              int32_t (&c)[R], const uint32_t (&wt)[R], GuOf gu_of, ParOf par_of,
                                              uint32_t Fb, ExpandCounters &C, Push &push)
 {
-    static_assert(!DIRECT || HK == DDP_H_ZERO || HK == DDP_H_MANHATTAN, "DIRECT: heuristics without loads only");
     // stage 2: heuristic inputs and the current (f, parent) words, all
     // loads issued before the first heuristic is computed.  hin, cur and
     // got below are only written and read by lanes whose edge takes part:
@@ -99,7 +170,7 @@ __device__ __forceinline__ void relax_window(const GraphView &G, const HeurView 
                 c[r] = -1;  // cannot beat the bound: no word read
         if (c[r] >= 0) {  // negative id = deleted edge
             hin[r] = heur_load<HK>(H, c[r]);
-            if constexpr (!DIRECT) cur[r] = ld_gp(gp + c[r]);
+            cur[r] = ld_gp(gp + c[r]);
         }
     }
     int32_t hc[R];
@@ -115,14 +186,13 @@ __device__ __forceinline__ void relax_window(const GraphView &G, const HeurView 
         if (c[r] >= 0 && (HK != DDP_H_ARRAY || hc[r] >= 0)) {  // h = -1: cannot reach t
             const uint32_t cand = gu_of(r) + wt[r] + (uint32_t)hc[r];
             want[r] = ((uint64_t)cand << 32) | (uint32_t)par_of(r);
-            if constexpr (DIRECT) tried[r] = true;
-            else tried[r] = (uint32_t)(cur[r] >> 32) > cand;
+            tried[r] = (uint32_t)(cur[r] >> 32) > cand;
         }
     }
     // Every load above has returned by now (the comparisons used them);
     // saying so keeps the compiler from waiting again before each CAS.
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    const bool by_min = DIRECT || G.relax_min != 0;  // uniform
+    const bool by_min = G.relax_min != 0;  // uniform
     if (by_min) {
         // one atomicMin per improving edge: the smallest (f, parent) of
         // the round wins with no retry round trips
@@ -130,7 +200,7 @@ __device__ __forceinline__ void relax_window(const GraphView &G, const HeurView 
         for (int r = 0; r < R; ++r)
             if (tried[r]) got[r] = (uint64_t)atomicMin((unsigned long long *)(gp + c[r]),
                                                        (unsigned long long)want[r]);
-    } else if constexpr (!DIRECT) {
+    } else {
 #pragma unroll
         for (int r = 0; r < R; ++r)
             if (tried[r])
@@ -147,16 +217,9 @@ __device__ __forceinline__ void relax_window(const GraphView &G, const HeurView 
         key[r] = 0;
         if (tried[r]) {
             const uint32_t cand = (uint32_t)(want[r] >> 32);
-            bool ok;
-            uint64_t prev;
-            if constexpr (DIRECT) {
-                ok = (uint32_t)(got[r] >> 32) > cand;
-                prev = got[r];
-            } else {
-                ok = by_min ? (uint32_t)(got[r] >> 32) > cand : got[r] == cur[r];
-                prev = by_min ? got[r] : cur[r];
-            }
-            if (!DIRECT && !ok && !by_min) {
+            bool ok = by_min ? (uint32_t)(got[r] >> 32) > cand : got[r] == cur[r];
+            uint64_t prev = by_min ? got[r] : cur[r];
+            if (!ok && !by_min) {
                 uint64_t now = got[r];
                 while ((uint32_t)(now >> 32) > cand) {
                     const uint64_t old = atomicCAS((unsigned long long *)(gp + c[r]), (unsigned long long)now,
@@ -185,17 +248,16 @@ __device__ __forceinline__ void relax_window(const GraphView &G, const HeurView 
     push.template all<R>(has, key);
 }
 
-// Push policy interface (block-collective members: every lane calls them):
+// Push policy interface (kCollect: edges may reach it from any lane of their wave;
+// members marked wave-wide: every lane of the wave calls them):
 //   void target(uint32_t f)                    -- t improved to f (t is never queued)
 //   void touch(int32_t c, uint64_t prev)       -- c's word was prev before the update
-//   void operator()(bool has, uint64_t key)    -- block-collective
-//   void touch_all<R>(first[R], c[R])          -- block-collective: touch() of R edges
+//   void operator()(bool has, uint64_t key)    -- wave-wide
+//   void touch_all<R>(first[R], c[R])          -- wave-wide: touch() of R edges
 //                                                 whose previous f was infinite
-//   void all<R>(has[R], key[R])                -- block-collective: operator() of R edges
-// Each lane brings up to P nodes u[p] (or -1) and their row spans (row_span,
-// or the same values loaded earlier by the caller); node p of lane l is
-// "virtual lane" l*P + p of a B*P-wide expansion, so a wide round pays the
-// scan and barriers once for B*P rows.
+//   void all<R>(has[R], key[R])                -- wave-wide: operator() of R edges
+// Each lane brings a node u (or -1) and its row span (row_span, or the same
+// values loaded earlier by the caller).
 //
 // Without FINAL_SYNC the function returns without its closing barrier; the
 // caller must pass a barrier before the next expand_rows (or before reading
@@ -207,149 +269,190 @@ __device__ __forceinline__ void relax_window(const GraphView &G, const HeurView 
 // (f, parent) word is read: it cannot lead to a cheaper path to t, and the
 // word's random 8-byte read costs a whole cache line.  Callers that keep
 // searching for a later, larger bound (a resumed DA* search) pass UINT32_MAX.
-template <int B, int HK, int P, class Push, bool FINAL_SYNC = true, bool DIRECT_OK = false>
+//
+// DIRECT_OK (heuristics without loads, atomicMin relaxation): in a round of at
+// most one edge per lane no word is read first; every edge that can still beat
+// Fb issues its atomicMin, whose returned word says whether it improved.  A
+// small round is a chain of dependent round trips, and this takes one out of
+// it; a large round keeps the read, which spares the atomics of the many edges
+// that cannot improve.
+template <int B, int HK, class Push, bool FINAL_SYNC = true, bool DIRECT_OK = false>
 __device__ __forceinline__ void expand_rows(const GraphView &G, const HeurView &H, uint64_t *gp, int32_t t,
-                                            const int32_t (&u)[P], const RowSpan (&rs)[P], ExpandLds<B * P> &L,
+                                            int32_t u, const RowSpan &rs, RowsLds<B, Push::kCollect> &L,
                                             ExpandCounters &C, Push &push, uint32_t Fb = 0xFFFFFFFFu)
 {
-    constexpr int R = expand_unroll<B>();
-    constexpr int V = B * P;
-    const int lane = threadIdx.x;
-    int32_t deg[P], lsum = 0;
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-        deg[p] = u[p] >= 0 ? rs[p].deg : 0;
-        lsum += deg[p];
-        if (u[p] >= 0) C.expanded++;
-    }
-    int32_t total;
-    // no barrier after the scan: the next write to L.tmp comes after the
-    // barrier that publishes L below
-    const int32_t run0 = block_incl_scan<B, false>(lsum, L.tmp, total) - lsum;
-    int32_t ends[P];
-    {
-        int32_t run = run0;
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            run += deg[p];
-            ends[p] = run;
-            L.incl[lane * P + p] = run;
-            L.rowb[lane * P + p] = rs[p].b;
-            L.gu[lane * P + p] = rs[p].gu;
-            L.node[lane * P + p] = u[p];
-        }
-    }
-    // Owner hints, when the round's edges fit in four windows of B*R slots
-    // (16V): each row writes its virtual lane into the slots of its first
-    // kOwnRun edges.  A hint is checked against the prefix before use, so a
-    // stale one only costs the binary search.  Larger rounds (hub rows of
-    // power-law graphs) skip the hints: refilling them per window cost two
-    // barriers each and measured slower than searching.
-    const bool use_own = total <= 4 * B * R;
-    // a round of at most one edge per lane is latency-bound: relax without the
-    // word read (atomicMin relaxation, heuristics without loads; relax_window).
-    // Only where the caller allows it (DIRECT_OK): the second copy of the
-    // relaxation costs registers that the 1,024-lane batch and serve kernels
-    // do not have to spare, and their rounds are mostly large.
-    const bool direct = DIRECT_OK && G.relax_min != 0 && total <= B;
-    if (use_own) {
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            const int32_t st = ends[p] - deg[p];
-            const int32_t to = ends[p] < st + kOwnRun ? ends[p] : st + kOwnRun;
-            for (int32_t x = st; x < to; ++x) L.own[x] = (uint16_t)(lane * P + p);
-        }
+    constexpr int R = expand_unroll<B>(), W = B / 64;
+    constexpr bool kNoLoad = HK == DDP_H_ZERO || HK == DDP_H_MANHATTAN;
+    const int lane = threadIdx.x, wl = lane & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(lane >> 6);
+    const int32_t deg = u >= 0 ? rs.deg : 0;
+    if (u >= 0) C.expanded++;
+    // edges and non-empty rows before this lane's row: within the wave, then
+    // over the waves, whose sums every 16 lanes scan
+    const int32_t x = wave_incl_scan(deg);
+    const uint64_t full = __ballot(deg > 0);
+    if (wl == 63) L.tmp[wid] = make_int2(x, (int32_t)__popcll(full));
+    __syncthreads();
+    int2 ws = make_int2(0, 0);
+    if ((wl & 15) < W) ws = L.tmp[wl & 15];
+    const int32_t we_sum = row16_incl_scan(ws.x), wr_sum = row16_incl_scan(ws.y);
+    const int32_t total = __builtin_amdgcn_readlane(we_sum, 15), nrows = __builtin_amdgcn_readlane(wr_sum, 15);
+    if (deg > 0) {
+        const int32_t i = (wid ? __builtin_amdgcn_readlane(wr_sum, wid - 1) : 0) + (int32_t)lane_rank(full);
+        const int32_t end = (wid ? __builtin_amdgcn_readlane(we_sum, wid - 1) : 0) + x;
+        L.incl[i] = end;
+        L.rowb[i] = rs.b - (end - deg);
+        L.gu[i] = rs.gu;
+        L.node[i] = u;
     }
     __syncthreads();
-    int32_t prow = 0;  // row of this lane's previous edge (edges are visited in increasing order)
-    for (int32_t base = 0; base < total; base += B * R) {
-        int32_t c[R], jj[R];
-        uint32_t wt[R];
-        // stage 1: locate each edge (LDS only), then issue its column and
-        // weight loads for all R edges before any of them is used
-        int32_t pos[R];
+    // This wave's windows of 64 edges: consecutive ones, dealt out evenly, or
+    // (lane heaps) every W-th, which mixes the rows over the heaps: with
+    // consecutive ones the C4 batch's heaps kept each other's offspring and
+    // expanded 20% more nodes.
+    constexpr int STEP = Push::kCollect ? 64 : B;
+    const int32_t nw = (int32_t)(((uint32_t)total + 63) / 64);
+    int32_t we = Push::kCollect ? nw * wid / W * 64 : wid * 64, wend = total;
+    if constexpr (Push::kCollect) {
+        const int32_t we1 = nw * (wid + 1) / W * 64;
+        wend = we1 < total ? we1 : total;
+    }
+    auto row_of = [&](int32_t e) {  // every lane of the wave, e < total
+        const int g = (int)__popcll(__ballot(wl < W && we_sum <= e));  // waves whose rows all end before
+        const int32_t at = (g ? __builtin_amdgcn_readlane(wr_sum, g - 1) : 0) + wl;
+        return at - wl + (int32_t)__popcll(__ballot(at < nrows && L.incl[at < nrows ? at : 0] <= e));
+    };
+    const bool direct = DIRECT_OK && kNoLoad && G.relax_min != 0 && total <= B;
+    if (we < wend) {
+        int32_t row = row_of(we);
+        uint64_t *const ck = L.key + wid * RowsLds<B, Push::kCollect>::CAP;
+        uint16_t *const cr = L.row + wid * RowsLds<B, Push::kCollect>::CAP;
+        int32_t cn = 0;  // collected edges
+        while (we < wend) {
+            int32_t c[R], jj[R], pos[R];
+            uint32_t wt[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int32_t e = base + r * B + lane;
-            pos[r] = -1;
-            jj[r] = 0;
-            if (e < total) {
-                // the owner hint, else the row of this lane's previous edge
-                // (a lane's edges only move forward, so that row or a later
-                // one holds e: hub rows keep it for many windows), else a
-                // binary search from that row on
-                int32_t lo = use_own ? L.own[e] : prow;
-                int32_t ex = 0;
-                if (lo < V) ex = lo ? L.incl[lo - 1] : 0;
-                if (!(lo < V && ex <= e && e < L.incl[lo])) {
-                    int32_t a = prow, hi = V - 1;
-                    while (a < hi) {
-                        const int32_t mid = (a + hi) >> 1;
-                        if (L.incl[mid] > e) hi = mid;
-                        else a = mid + 1;
-                    }
-                    lo = a;
-                    ex = lo ? L.incl[lo - 1] : 0;
+            for (int r = 0; r < R; ++r) {
+                pos[r] = -1;
+                jj[r] = 0;
+                const int32_t e0 = we + r * STEP;
+                if (e0 >= wend) continue;
+                if (STEP != 64) row = row_of(e0);
+                jj[r] = wave_rows(L, nrows, e0, row);
+                if (e0 + wl < wend) {
+                    pos[r] = L.rowb[jj[r]] + e0 + wl;
+                    C.edges++;
                 }
-                prow = lo;
-                jj[r] = lo;
-                pos[r] = L.rowb[lo] + (e - ex);
-                C.edges++;
             }
-        }
-        int32_t dv[R];
+            int32_t dv[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            c[r] = -1;
-            wt[r] = 0;
-            dv[r] = INT32_MAX;
-            if (pos[r] >= 0) {
-                c[r] = G.col[pos[r]];
-                wt[r] = G.w[pos[r]];
-                if (G.dver) dv[r] = G.dver[pos[r]];
+            for (int r = 0; r < R; ++r) {
+                c[r] = -1;
+                wt[r] = 0;
+                dv[r] = INT32_MAX;
+                if (pos[r] >= 0) {
+                    c[r] = G.col[pos[r]];
+                    wt[r] = G.w[pos[r]];
+                    if (G.dver) dv[r] = G.dver[pos[r]];
+                }
             }
-        }
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-            if (G.dver && dv[r] <= G.ver) c[r] = -1;  // deleted at or before this version
-        auto gu_of = [&](int r) { return L.gu[jj[r]]; };
-        auto par_of = [&](int r) { return L.node[jj[r]]; };
-        if constexpr (DIRECT_OK && (HK == DDP_H_ZERO || HK == DDP_H_MANHATTAN)) {
-            if (direct) relax_window<R, HK, true>(G, H, gp, t, c, wt, gu_of, par_of, Fb, C, push);
-            else relax_window<R, HK>(G, H, gp, t, c, wt, gu_of, par_of, Fb, C, push);
-        } else {
-            relax_window<R, HK>(G, H, gp, t, c, wt, gu_of, par_of, Fb, C, push);
+            for (int r = 0; r < R; ++r)
+                if (G.dver && dv[r] <= G.ver) c[r] = -1;  // deleted at or before this version
+            if constexpr (!Push::kCollect) {
+                we += STEP * R;
+                relax_window<R, HK>(G, H, gp, t, c, wt, [&](int r) { return L.gu[jj[r]]; },
+                                    [&](int r) { return L.node[jj[r]]; }, Fb, C, push);
+                continue;
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r) wt[r] += pos[r] >= 0 ? L.gu[jj[r]] : 0;  // g of the edge's end
+            // heuristic inputs and current (f, parent) words, all loads issued
+            // before the first heuristic is computed.  hin and cur are only
+            // written and read by lanes whose edge takes part: giving the
+            // others a value would make the compiler merge the two and wait
+            // for each load before issuing the next.
+            HeurIn hin[R];
+            uint64_t cur[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                if constexpr (kNoLoad)
+                    if (c[r] >= 0 && wt[r] + (uint32_t)heur_from<HK>(H, c[r], HeurIn{0, 0}) >= Fb)
+                        c[r] = -1;  // cannot beat the bound: no word read
+                if (c[r] >= 0) {  // negative id = deleted edge
+                    hin[r] = heur_load<HK>(H, c[r]);
+                    if (!direct) cur[r] = ld_gp(gp + c[r]);
+                }
+            }
+            uint64_t key[R];
+            bool tried[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                tried[r] = false;
+                key[r] = 0;
+                if (c[r] >= 0) {
+                    const int32_t hc = heur_from<HK>(H, c[r], hin[r]);
+                    if (HK != DDP_H_ARRAY || hc >= 0) {  // h = -1: cannot reach t
+                        const uint32_t cand = wt[r] + (uint32_t)hc;
+                        key[r] = ((uint64_t)cand << 32) | (uint32_t)c[r];
+                        tried[r] = direct || (uint32_t)(cur[r] >> 32) > cand;
+                    }
+                }
+            }
+            we += STEP * R;
+            if (total <= B) {  // at most one edge per lane: nothing to collect
+                relax_collected(G, gp, t, tried[0], key[0], tried[0] ? L.node[jj[0]] : 0, C, push);
+                break;
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const uint64_t m = __ballot(tried[r]);
+                if (tried[r]) {
+                    const int32_t at = cn + (int32_t)lane_rank(m);
+                    ck[at] = key[r];
+                    cr[at] = (uint16_t)jj[r];
+                }
+                cn += (int32_t)__popcll(m);
+            }
+            while (cn >= 64 || (cn > 0 && we >= wend)) {  // the last ones first, so the rest stays where it is
+                const int32_t n = cn < 64 ? cn : 64, at = cn - n + wl;
+                uint64_t k = 0;
+                int32_t par = 0;
+                if (wl < n) {
+                    k = ck[at];
+                    par = L.node[cr[at]];
+                }
+                relax_collected(G, gp, t, wl < n, k, par, C, push);
+                cn -= n;
+            }
         }
     }
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-        if (!G.lhead) break;
+    if (G.lhead) {
         // Versioned inserts: each lane walks its own node's list, oldest
         // first, stopping at the first entry newer than this version (links
         // carry the inserting version, so newer entries are never read).
-        const uint32_t gu = rs[p].gu;
-        uint64_t link = u[p] >= 0 ? __hip_atomic_load(G.lhead + u[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                  : ~0ull;
+        const uint32_t gu = rs.gu;
+        uint64_t link = u >= 0 ? __hip_atomic_load(G.lhead + u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : ~0ull;
         for (;;) {
             bool active = false, has = false;
             uint64_t key = 0;
-            int32_t x = -1;
+            int32_t xe = -1;
             while ((uint32_t)link <= (uint32_t)G.ver) {
-                x = (int32_t)(link >> 32);
-                link = __hip_atomic_load(G.lnext + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (G.ldel[x] > G.ver) {
+                xe = (int32_t)(link >> 32);
+                link = __hip_atomic_load(G.lnext + xe, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (G.ldel[xe] > G.ver) {
                     active = true;
                     break;
                 }
             }
             if (active) {
                 C.edges++;
-                const int32_t cn = G.lv[x];
+                const int32_t cn = G.lv[xe];
                 const int32_t hcn = heur_eval<HK>(H, cn);
                 if (HK != DDP_H_ARRAY || hcn >= 0) {
-                    const uint32_t cand = gu + G.lw[x] + (uint32_t)hcn;
+                    const uint32_t cand = gu + G.lw[xe] + (uint32_t)hcn;
                     uint64_t prev;
-                    if (relax_gp(gp, cn, cand, (uint32_t)u[p], &prev)) {
+                    if (relax_gp(gp, cn, cand, (uint32_t)u, &prev)) {
                         C.improved++;
                         push.touch(cn, prev);
                         if (cn == t) {
@@ -370,10 +473,8 @@ __device__ __forceinline__ void expand_rows(const GraphView &G, const HeurView &
 
 template <int B, int HK, bool DIRECT_OK = false, class Push>
 __device__ __forceinline__ void expand_block(const GraphView &G, const HeurView &H, uint64_t *gp, int32_t t,
-                                             int32_t u, uint32_t fu, ExpandLds<B> &L, ExpandCounters &C,
-                                             Push &push)
+                                             int32_t u, uint32_t fu, RowsLds<B, Push::kCollect> &L,
+                                             ExpandCounters &C, Push &push)
 {
-    const int32_t uu[1] = {u};
-    const RowSpan rs[1] = {row_span<HK>(G, H, u, fu)};
-    expand_rows<B, HK, 1, Push, true, DIRECT_OK>(G, H, gp, t, uu, rs, L, C, push);
+    expand_rows<B, HK, Push, true, DIRECT_OK>(G, H, gp, t, u, row_span<HK>(G, H, u, fu), L, C, push);
 }

@@ -390,8 +390,7 @@ template <int B, int HK, int ENG>
 __global__ void __launch_bounds__(B) serve_kernel(ServeArgs a)
 {
     extern __shared__ uint64_t s_heap[];
-    constexpr int SV = (ENG == SENG_PILES) ? B * pile_entries_per_lane<B>() : B;  // expansion width
-    __shared__ std::conditional_t<ENG == SENG_BIDI, BidiLds<B>, SlotLds<B, SV>> S;
+    __shared__ std::conditional_t<ENG == SENG_BIDI, BidiLds<B>, SlotLds<B, ENG == SENG_PILES>> S;
     __shared__ uint32_t s_ticket;
     __shared__ int32_t s_have;
     __shared__ uint32_t s_uerr;

@@ -10,11 +10,9 @@
 
 enum : uint32_t { QERR_HEAP = 1, QERR_ITERS = 2, QERR_BADQ = 4, QERR_PATH = 8 };
 
-// V: expansion width (B lanes x entries per lane; the pile engine can take
-// more than one entry per lane and round).
-template <int B, int V = B>
+template <int B, bool COLLECT>
 struct SlotLds {
-    ExpandLds<V> L;
+    RowsLds<B, COLLECT> L;
     uint32_t red[16];
     uint32_t F;        // best f of the target so far
     uint32_t err;
@@ -33,6 +31,7 @@ struct SlotLds {
 
 template <int B>
 struct SlotPush {
+    static constexpr bool kCollect = false;
     const LaneHeap *H;
     int32_t *size;
     uint32_t *s_F;
@@ -83,7 +82,7 @@ __device__ __forceinline__ void set_target(HeurView &hv, int32_t t)
 // touched still describe the search so the caller can walk the path.
 template <int B, int HK>
 __device__ void slot_search(const GraphView &G, HeurView hv, uint64_t *gp, int32_t *touched, const LaneHeap &H,
-                            uint64_t *s_heap, int32_t N, int32_t s, int32_t t, int32_t maxit, SlotLds<B> &S,
+                            uint64_t *s_heap, int32_t N, int32_t s, int32_t t, int32_t maxit, SlotLds<B, false> &S,
                             ExpandCounters &C, uint32_t &stale)
 {
     const int lane = threadIdx.x;
@@ -271,11 +270,12 @@ __device__ __forceinline__ bool pile_place(const PilePtrs &P, uint32_t thr, bool
     return dropped;
 }
 
-template <int B, int V>
+template <int B>
 struct PilePush {
+    static constexpr bool kCollect = true;
     const PilePtrs *P;
     uint64_t *far;
-    SlotLds<B, V> *S;
+    SlotLds<B, true> *S;
     int32_t *touched;
     uint32_t err = 0;
 
@@ -324,19 +324,13 @@ __device__ __forceinline__ uint32_t sat_add_u32(uint32_t a, uint32_t b)
     return a > 0xFFFFFFFFu - b ? 0xFFFFFFFFu : a + b;
 }
 
-// Entries each lane takes from the near ring per round.  One: two per lane
-// (2,048 per round at 1,024 lanes) measured slower on the C4 batch (139k
-// against 148k queries/s) -- wider rounds expand more nodes out of f order
-// (80M against 63M) and do not shorten the longest searches, whose rounds are
-// bound by the memory requests one CU keeps in flight, not by per-round costs.
-template <int B>
-constexpr int pile_entries_per_lane()
-{
-    return 1;
-}
-
 // Same contract as slot_search (S.F, S.err, gp and touched describe the search
-// on return).  delta0 is the first window width.  W entries per lane per round.
+// on return).  delta0 is the first window width.
+//
+// A round takes one entry per lane.  Two (2,048 per round at 1,024 lanes)
+// measured slower on the C4 batch (139k against 148k queries/s): wider rounds
+// expand more nodes out of f order (80M against 63M) and do not shorten the
+// longest searches.
 //
 // The near ring has two levels: P.lring in LDS (P.lcap entries) and P.near in
 // HBM for what does not fit, kept in FIFO order together (see PilePush).
@@ -354,12 +348,12 @@ constexpr int pile_entries_per_lane()
 // 256 (three or fewer entries) refilled so often that it was slower.
 constexpr uint32_t kThinRing = 64;
 
-template <int B, int HK, int W = pile_entries_per_lane<B>(), bool DIRECT_OK = false>
+template <int B, int HK, bool DIRECT_OK = false>
 __device__ void slot_search_piles(const GraphView &G, HeurView hv, uint64_t *gp, int32_t *touched,
                                   const PilePtrs &P, int32_t N, int32_t s, int32_t t, int32_t maxit,
-                                  uint32_t delta0, SlotLds<B, B * W> &S, ExpandCounters &C, uint32_t &stale)
+                                  uint32_t delta0, SlotLds<B, true> &S, ExpandCounters &C, uint32_t &stale)
 {
-    constexpr uint32_t V = (uint32_t)B * W;
+    constexpr uint32_t V = B;
     const int lane = threadIdx.x;
     const uint32_t nmask = P.ncap - 1, lmask = P.lcap ? P.lcap - 1 : 0;
     if (lane == 0) {
@@ -546,31 +540,26 @@ __device__ void slot_search_piles(const GraphView &G, HeurView hv, uint64_t *gp,
             break;
         }
         ++it;
-        // ---- take up to V entries from one ring, W per lane (coalesced: entry w*B + lane)
+        // ---- take up to V entries from one ring (coalesced)
         const uint32_t n = avail < V ? avail : V;
-        int32_t u[W];
-        RowSpan rs[W];
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            u[w] = -1;
-            const uint32_t idx = (uint32_t)(w * B + lane);
-            if (idx < n) {
-                const uint64_t key = from_lds ? P.lring[(lh + idx) & lmask] : P.near[(hh + idx) & nmask];
-                const uint32_t f = (uint32_t)(key >> 32);
-                const int32_t node = (int32_t)(uint32_t)key;
-                // the node's word, row and heuristic input in one round trip:
-                // the row is loaded before the entry is known to be current
-                const uint64_t word = ld_gp(gp + node);
-                const int32_t rb = G.off[node], re = G.off[node + 1];
-                const int32_t hn = heur_eval<HK>(hv, node);
-                if (f < F && (uint32_t)(word >> 32) == f) {
-                    u[w] = node;
-                    rs[w].b = rb;
-                    rs[w].deg = re - rb;
-                    rs[w].gu = f - (uint32_t)hn;
-                } else {
-                    ++stale;
-                }
+        int32_t u = -1;
+        RowSpan rs;
+        if ((uint32_t)lane < n) {
+            const uint64_t key = from_lds ? P.lring[(lh + lane) & lmask] : P.near[(hh + lane) & nmask];
+            const uint32_t f = (uint32_t)(key >> 32);
+            const int32_t node = (int32_t)(uint32_t)key;
+            // the node's word, row and heuristic input in one round trip:
+            // the row is loaded before the entry is known to be current
+            const uint64_t word = ld_gp(gp + node);
+            const int32_t rb = G.off[node], re = G.off[node + 1];
+            const int32_t hn = heur_eval<HK>(hv, node);
+            if (f < F && (uint32_t)(word >> 32) == f) {
+                u = node;
+                rs.b = rb;
+                rs.deg = re - rb;
+                rs.gu = f - (uint32_t)hn;
+            } else {
+                ++stale;
             }
         }
         // Pushes of this round start after expand_rows' first barrier, when
@@ -582,8 +571,8 @@ __device__ void slot_search_piles(const GraphView &G, HeurView hv, uint64_t *gp,
             S.near_head = hh;
             S.phase_n += n;
         }
-        PilePush<B, B * W> push{&P, far, &S, touched};
-        expand_rows<B, HK, W, PilePush<B, B * W>, false, DIRECT_OK>(G, hv, gp, t, u, rs, S.L, C, push, F);
+        PilePush<B> push{&P, far, &S, touched};
+        expand_rows<B, HK, PilePush<B>, false, DIRECT_OK>(G, hv, gp, t, u, rs, S.L, C, push, F);
         if (push.err) atomicOr(&S.err, push.err);
         __syncthreads();  // the round's pushes and errors are visible to the next round
         if (S.err) break;
@@ -595,9 +584,9 @@ __device__ void slot_search_piles(const GraphView &G, HeurView hv, uint64_t *gp,
 // Writes the path s..t into out[0..cap) and its length into S.plen (0 if
 // unreachable, -len if longer than cap): lane 0 walks t..s, one dependent read
 // a hop, and the block turns the path round.  Block-collective.
-template <int B, int V>
+template <int B, bool COLLECT>
 __device__ void slot_path(const uint64_t *gp, int32_t N, int32_t s, int32_t t, int32_t *out, int32_t cap,
-                          SlotLds<B, V> &S)
+                          SlotLds<B, COLLECT> &S)
 {
     if (threadIdx.x == 0) {
         int32_t n = 0;
@@ -630,8 +619,8 @@ __device__ void slot_path(const uint64_t *gp, int32_t N, int32_t s, int32_t t, i
 // Clears every (f, parent) word the query touched.  Starts with a barrier so
 // lane 0's path walk has finished reading parents; ends with one so the next
 // query's atomics see the cleared words.
-template <int B, int V>
-__device__ void slot_reset(uint64_t *gp, const int32_t *touched, SlotLds<B, V> &S)
+template <int B, bool COLLECT>
+__device__ void slot_reset(uint64_t *gp, const int32_t *touched, SlotLds<B, COLLECT> &S)
 {
     __syncthreads();
     const int32_t nt = S.ntouch;
