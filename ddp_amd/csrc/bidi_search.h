@@ -89,7 +89,7 @@ struct BidiDir {
 
 template <int B>
 struct BidiLds {
-    ExpandLds<B> L;
+    RowsLds<B, true> L;
     uint32_t red[16];
     unsigned long long meet;  // mu << 32 | meeting node
     uint32_t bound[2];        // L_d: lower bound of direction d's open keys (UINT32_MAX: none left)
@@ -193,63 +193,74 @@ __device__ __forceinline__ void bidi_settle(const BidiSide &D, int32_t s, int32_
 }
 
 // One cooperative pass over the rows of the entries taken this round: lanes
-// below n0 hold forward nodes, the others backward nodes.  Loads are issued
-// stage by stage as in expand_rows.  With VERS, deleted base entries are
-// skipped and each lane then walks its node's inserted-edge list.  No closing
-// barrier.
+// below n0 hold forward nodes, the others backward nodes.  Rows, windows and
+// collected edges as in expand_rows (rows below L.split are forward ones), and
+// for the same reason: a round is bound by what its waves issue.  With a
+// binary search per edge and every stage run for every window, at 1,024 lanes:
+// 128 queries on R-MAT (scale 18) 67.7 ms, now 26.1; the C4 batch 57.6, now
+// 42.5; the 4,096 x 4,096 maze 30.6, now 24.6.  With VERS, deleted base entries
+// are skipped and each lane then walks its node's inserted-edge list.  No
+// closing barrier.
 template <int B, int HK, bool VERS>
 __device__ __forceinline__ void expand_bidi(const BidiSide &D, const HeurView &H, bool relax_min, int32_t s,
                                             int32_t t, int32_t u, RowSpan rs, int32_t n0, const uint32_t (&F)[2],
                                             uint64_t *const (&far)[2], BidiLds<B> &S, ExpandCounters &C)
 {
-    constexpr int R = expand_unroll<B>();
-    const int lane = threadIdx.x;
-    ExpandLds<B> &L = S.L;
-    const int32_t deg = u >= 0 ? rs.deg : 0;
+    constexpr int R = expand_unroll<B>(), W = B / 64, CAP = RowsLds<B, true>::CAP;
+    constexpr bool kNoLoad = HK == DDP_H_ZERO || HK == DDP_H_MANHATTAN;
+    const int lane = threadIdx.x, wl = lane & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(lane >> 6);
+    RowsLds<B, true> &L = S.L;
     if (u >= 0) C.expanded++;
-    int32_t total;
-    const int32_t run0 = block_incl_scan<B, false>(deg, L.tmp, total) - deg;
-    L.incl[lane] = run0 + deg;
-    L.rowb[lane] = rs.b;
-    L.gu[lane] = rs.gu;
-    L.node[lane] = u;
-    const bool use_own = total <= 4 * B * R;
+    const RoundRows rr = list_rows<B>(L, u >= 0 ? rs.deg : 0, rs.b, rs.gu, u, n0);
+    const int32_t total = rr.total, split = n0 < B ? L.split : rr.nrows;
     // a round of at most one edge per lane is latency-bound: relax without the
     // word read, the atomicMin's returned word telling whether it improved
-    // (heuristics without loads; as relax_window's DIRECT)
-    const bool direct = (HK == DDP_H_ZERO || HK == DDP_H_MANHATTAN) && relax_min && total <= B;
-    if (use_own) {
-        const int32_t to = deg < kOwnRun ? run0 + deg : run0 + kOwnRun;
-        for (int32_t x = run0; x < to; ++x) L.own[x] = (uint16_t)lane;
-    }
-    __syncthreads();
-    int32_t prow = 0;
-    for (int32_t base = 0; base < total; base += B * R) {
+    // (heuristics without loads; as expand_rows)
+    const bool direct = kNoLoad && relax_min && total <= B;
+    const int32_t nw = (int32_t)(((uint32_t)total + 63) / 64);
+    const int32_t we1 = nw * (wid + 1) / W * 64, wend = we1 < total ? we1 : total;
+    int32_t we = nw * wid / W * 64;
+    int32_t row = we < wend ? first_row(L, rr, we) : 0;
+    uint64_t *const ck = L.key + wid * CAP;
+    uint16_t *const cr = L.row + wid * CAP;
+    int32_t cn = 0;  // collected edges
+    // relaxes one candidate per lane and settles the improvements
+    auto relax = [&](bool have, uint64_t key, int32_t j) {
+        bool ok[1] = {false}, first[1] = {false}, dr[1] = {j >= split};
+        const int32_t c[1] = {(int32_t)(uint32_t)key};
+        const uint32_t cand = (uint32_t)(key >> 32);
+        uint64_t want[1] = {0};
+        if (have) {
+            want[0] = ((uint64_t)cand << 32) | (uint32_t)L.node[j];
+            uint64_t *word = pick2(D.gp, dr[0]) + c[0];
+            uint64_t prev = 0;
+            if (relax_min) {
+                prev = (uint64_t)atomicMin((unsigned long long *)word, (unsigned long long)want[0]);
+                ok[0] = (uint32_t)(prev >> 32) > cand;
+            } else {
+                ok[0] = relax_gp(pick2(D.gp, dr[0]), c[0], cand, (uint32_t)want[0], &prev);
+            }
+            if (ok[0]) {
+                C.improved++;
+                first[0] = (uint32_t)(prev >> 32) == DDP_INF_F;
+            }
+        }
+        bidi_settle<B, 1>(D, s, t, ok, first, dr, c, want, F, far, S);
+    };
+    while (we < wend) {
         int32_t pos[R], jj[R], c[R];
         bool dr[R];
         uint32_t wt[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const int32_t e = base + r * B + lane;
             pos[r] = -1;
             jj[r] = 0;
-            if (e < total) {
-                int32_t lo = use_own ? L.own[e] : prow;
-                int32_t ex = 0;
-                if (lo < B) ex = lo ? L.incl[lo - 1] : 0;
-                if (!(lo < B && ex <= e && e < L.incl[lo])) {
-                    int32_t a = prow, hi = B - 1;
-                    while (a < hi) {
-                        const int32_t mid = (a + hi) >> 1;
-                        if (L.incl[mid] > e) hi = mid;
-                        else a = mid + 1;
-                    }
-                    lo = a;
-                    ex = lo ? L.incl[lo - 1] : 0;
-                }
-                prow = lo;
-                jj[r] = lo;
-                pos[r] = L.rowb[lo] + (e - ex);
+            const int32_t e0 = we + r * 64;
+            if (e0 >= wend) continue;
+            jj[r] = wave_rows(L, rr.nrows, e0, row);
+            if (e0 + wl < wend) {
+                pos[r] = L.rowb[jj[r]] + e0 + wl;
                 C.edges++;
             }
         }
@@ -259,7 +270,7 @@ __device__ __forceinline__ void expand_bidi(const BidiSide &D, const HeurView &H
             c[r] = -1;
             wt[r] = 0;
             dv[r] = INT32_MAX;
-            dr[r] = jj[r] >= n0;
+            dr[r] = jj[r] >= split;
             if (pos[r] >= 0) {
                 const int k = dr[r] ? 1 : 0;
                 c[r] = pick2(D.col, k != 0)[pos[r]];
@@ -267,77 +278,67 @@ __device__ __forceinline__ void expand_bidi(const BidiSide &D, const HeurView &H
                 if constexpr (VERS) dv[r] = pick2(D.dver, k != 0)[pos[r]];
             }
         }
-        // stage 2: heuristic inputs and current words (written only by lanes that take part)
+        // heuristic inputs and current words (written only by lanes that take
+        // part).  An edge whose key cannot beat F is skipped first where that
+        // needs no load: its end would be dropped, and no meeting through it
+        // can be shorter.
         HeurIn hin[R];
         uint64_t cur[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             if (VERS && dv[r] <= D.ver) c[r] = -1;  // deleted at or before this version
+            if (c[r] >= 0) wt[r] += L.gu[jj[r]];
+            if constexpr (kNoLoad) {
+                if (c[r] >= 0) {
+                    const int32_t pc = pot_from<HK>(H, c[r], HeurIn{0, 0});
+                    wt[r] += (uint32_t)(dr[r] ? -pc : pc);
+                    if (wt[r] >= pick2(F, dr[r])) c[r] = -1;
+                }
+            }
             if (c[r] >= 0) {
-                hin[r] = heur_load<HK>(H, c[r]);
+                if constexpr (!kNoLoad) hin[r] = heur_load<HK>(H, c[r]);
                 if (!direct) cur[r] = ld_gp(pick2(D.gp, dr[r]) + c[r]);
             }
         }
-        // stage 3: candidates and one atomic per improving edge
-        uint64_t want[R], got[R];
+        uint64_t key[R];
         bool tried[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             tried[r] = false;
-            want[r] = 0;
+            key[r] = 0;
             if (c[r] >= 0) {
-                const int32_t pc = pot_from<HK>(H, c[r], hin[r]);
-                const uint32_t cand = L.gu[jj[r]] + wt[r] + (uint32_t)(dr[r] ? -pc : pc);
-                want[r] = ((uint64_t)cand << 32) | (uint32_t)L.node[jj[r]];
+                const int32_t pc = kNoLoad ? 0 : pot_from<HK>(H, c[r], hin[r]);
+                const uint32_t cand = wt[r] + (uint32_t)(dr[r] ? -pc : pc);
+                key[r] = ((uint64_t)cand << 32) | (uint32_t)c[r];
                 tried[r] = direct || (uint32_t)(cur[r] >> 32) > cand;
             }
         }
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): every load above was consumed
-        if (relax_min) {
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-                if (tried[r])
-                    got[r] = (uint64_t)atomicMin((unsigned long long *)(pick2(D.gp, dr[r]) + c[r]),
-                                                 (unsigned long long)want[r]);
-        } else {
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-                if (tried[r])
-                    got[r] = (uint64_t)atomicCAS((unsigned long long *)(pick2(D.gp, dr[r]) + c[r]),
-                                                 (unsigned long long)cur[r], (unsigned long long)want[r]);
+        we += 64 * R;
+        if (total <= B) {  // at most one edge per lane: nothing to collect
+            relax(tried[0], key[0], jj[0]);
+            break;
         }
-        // stage 4: settle contended CASes
-        bool ok[R], first[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            ok[r] = false;
-            first[r] = false;
+            const uint64_t m = __ballot(tried[r]);
             if (tried[r]) {
-                const uint32_t cand = (uint32_t)(want[r] >> 32);
-                bool good = relax_min ? (uint32_t)(got[r] >> 32) > cand : got[r] == cur[r];
-                uint64_t prev = relax_min ? got[r] : cur[r];
-                if (!good && !relax_min) {
-                    uint64_t now = got[r];
-                    while ((uint32_t)(now >> 32) > cand) {
-                        const uint64_t old =
-                            atomicCAS((unsigned long long *)(pick2(D.gp, dr[r]) + c[r]), (unsigned long long)now,
-                                      (unsigned long long)want[r]);
-                        if (old == now) {
-                            good = true;
-                            prev = now;
-                            break;
-                        }
-                        now = old;
-                    }
-                }
-                ok[r] = good;
-                if (good) {
-                    C.improved++;
-                    first[r] = (uint32_t)(prev >> 32) == DDP_INF_F;
-                }
+                const int32_t at = cn + (int32_t)lane_rank(m);
+                ck[at] = key[r];
+                cr[at] = (uint16_t)jj[r];
             }
+            cn += (int32_t)__popcll(m);
         }
-        bidi_settle<B, R>(D, s, t, ok, first, dr, c, want, F, far, S);
+        while (cn >= 64 || (cn > 0 && we >= wend)) {  // the last ones first, so the rest stays where it is
+            const int32_t n = cn < 64 ? cn : 64, at = cn - n + wl;
+            uint64_t k = 0;
+            int32_t j = 0;
+            if (wl < n) {
+                k = ck[at];
+                j = cr[at];
+            }
+            relax(wl < n, k, j);
+            cn -= n;
+        }
     }
     if constexpr (VERS) {
         // Inserted edges: each lane walks its own node's list, oldest first,
@@ -379,7 +380,7 @@ __device__ __forceinline__ void expand_bidi(const BidiSide &D, const HeurView &H
 }
 
 // A thin round: every entry gets kThinLanes lanes, which read its row together,
-// so there is no prefix scan, no owner map and no barrier between taking an
+// so there is no prefix scan, no row search and no barrier between taking an
 // entry and relaxing its edges; and each direction has half of the waves to
 // itself, so a wave's pointers and limits are uniform and its pushes take one
 // LDS round trip (three counters in one instruction) where bidi_settle takes

@@ -201,34 +201,6 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v)
     return v;
 }
 
-// Block-wide inclusive scan; `tmp` must hold B/64 ints of LDS.  Returns the
-// block total too.  With TAIL_SYNC it ends with a barrier, so `tmp` may be
-// reused right after; without, the caller must pass another barrier before
-// anything writes `tmp` again.
-template <int B, bool TAIL_SYNC = true>
-__device__ __forceinline__ int32_t block_incl_scan(int32_t v, int32_t *tmp, int32_t &total)
-{
-    int32_t x = wave_incl_scan(v);
-    if constexpr (B == 64) {
-        total = __builtin_amdgcn_readlane(x, 63);
-        return x;
-    } else {
-        const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-        if (lane == 63) tmp[wid] = x;
-        __syncthreads();
-        int32_t add = 0, tot = 0;
-#pragma unroll
-        for (int k = 0; k < B / 64; ++k) {
-            int32_t s = tmp[k];
-            if (k < wid) add += s;
-            tot += s;
-        }
-        total = tot;
-        if constexpr (TAIL_SYNC) __syncthreads();
-        return x + add;
-    }
-}
-
 template <int B>
 __device__ __forceinline__ uint32_t block_min_u32(uint32_t v, uint32_t *tmp)
 {

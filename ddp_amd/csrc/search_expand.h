@@ -24,22 +24,6 @@
 
 #include "device_common.h"
 
-// Owner hints of expand_bidi: edge slot of the round -> lane, written for rows
-// up to kOwnRun edges (every row of a road or geometric graph); the rest of a
-// longer row falls back to a binary search over the prefix.
-template <int V>
-struct ExpandLds {
-    static_assert(V <= 65536, "owner entries are 16-bit");
-    int32_t incl[V];     // inclusive prefix of degrees
-    int32_t rowb[V];     // row start
-    uint32_t gu[V];      // g(u) = f(u) - h(u), unsigned as GA_v2.cu:137
-    int32_t node[V];
-    int32_t tmp[16];
-    uint16_t own[16 * V];
-};
-
-constexpr int32_t kOwnRun = 32;
-
 // Edges handled per lane and trip (memory requests a lane keeps in flight
 // per stage).  At 1,024 lanes two, three, four and six took 80, 78, 73 and 73
 // ms a query on R-MAT (scale 20) and 16.1, 16.2, 16.2 and 16.7 ms for C4.
@@ -59,6 +43,7 @@ struct RowsLds {
     uint32_t gu[B];         // g(u) = f(u) - h(u), unsigned as GA_v2.cu:137
     int32_t node[B];
     int2 tmp[B / 64];       // edges and rows of each wave
+    int32_t split;          // rows of the lanes below n0 (list_rows)
     uint64_t key[B / 64 * CAP];  // candidate f << 32 | node
     uint16_t row[B / 64 * CAP];
 };
@@ -91,6 +76,58 @@ struct ExpandCounters {
     uint32_t refills = 0;   // pile engine: near-ring refills from the far pile (lane 0 counts)
     uint32_t scanned = 0;   // pile engine: far-pile entries read by refills
 };
+
+// A round's rows: edges and rows in all, and (in every 16 lanes) up to and with
+// each wave.
+struct RoundRows {
+    int32_t total, nrows, we_sum, wr_sum;
+};
+
+// Lists the rows that the block's lanes bring (deg edges from row start b, of
+// node u with g(u) = gu).  Every lane of the block calls it; it begins with
+// L free and ends with a barrier.  L.split: the rows of lanes below n0.
+template <int B, bool COLLECT>
+__device__ __forceinline__ RoundRows list_rows(RowsLds<B, COLLECT> &L, int32_t deg, int32_t b, uint32_t gu, int32_t u,
+                                               int32_t n0 = -1)
+{
+    constexpr int W = B / 64;
+    const int lane = threadIdx.x, wl = lane & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(lane >> 6);
+    // edges and non-empty rows before this lane's row: within the wave, then
+    // over the waves, whose sums every 16 lanes scan
+    const int32_t x = wave_incl_scan(deg);
+    const uint64_t full = __ballot(deg > 0);
+    if (wl == 63) L.tmp[wid] = make_int2(x, (int32_t)__popcll(full));
+    __syncthreads();
+    int2 ws = make_int2(0, 0);
+    if ((wl & 15) < W) ws = L.tmp[wl & 15];
+    RoundRows rr;
+    rr.we_sum = row16_incl_scan(ws.x);
+    rr.wr_sum = row16_incl_scan(ws.y);
+    rr.total = __builtin_amdgcn_readlane(rr.we_sum, 15);
+    rr.nrows = __builtin_amdgcn_readlane(rr.wr_sum, 15);
+    const int32_t i = (wid ? __builtin_amdgcn_readlane(rr.wr_sum, wid - 1) : 0) + (int32_t)lane_rank(full);
+    if (deg > 0) {
+        const int32_t end = (wid ? __builtin_amdgcn_readlane(rr.we_sum, wid - 1) : 0) + x;
+        L.incl[i] = end;
+        L.rowb[i] = b - (end - deg);
+        L.gu[i] = gu;
+        L.node[i] = u;
+    }
+    if (lane == n0) L.split = i;
+    __syncthreads();
+    return rr;
+}
+
+// The row of edge e < total.  Every lane of the wave calls it.
+template <int B, bool COLLECT>
+__device__ __forceinline__ int32_t first_row(const RowsLds<B, COLLECT> &L, const RoundRows &rr, int32_t e)
+{
+    const int wl = threadIdx.x & 63;
+    const int g = (int)__popcll(__ballot(wl < B / 64 && rr.we_sum <= e));  // waves whose rows all end before
+    const int32_t at = (g ? __builtin_amdgcn_readlane(rr.wr_sum, g - 1) : 0) + wl;
+    return at - wl + (int32_t)__popcll(__ballot(at < rr.nrows && L.incl[at < rr.nrows ? at : 0] <= e));
+}
 
 // Rows of 64 consecutive edges, found by a wave at once: lane i reads the end
 // of row row + i and marks the lane of the edge after it; an edge's row is row
@@ -285,27 +322,9 @@ __device__ __forceinline__ void expand_rows(const GraphView &G, const HeurView &
     constexpr bool kNoLoad = HK == DDP_H_ZERO || HK == DDP_H_MANHATTAN;
     const int lane = threadIdx.x, wl = lane & 63;
     const int wid = __builtin_amdgcn_readfirstlane(lane >> 6);
-    const int32_t deg = u >= 0 ? rs.deg : 0;
     if (u >= 0) C.expanded++;
-    // edges and non-empty rows before this lane's row: within the wave, then
-    // over the waves, whose sums every 16 lanes scan
-    const int32_t x = wave_incl_scan(deg);
-    const uint64_t full = __ballot(deg > 0);
-    if (wl == 63) L.tmp[wid] = make_int2(x, (int32_t)__popcll(full));
-    __syncthreads();
-    int2 ws = make_int2(0, 0);
-    if ((wl & 15) < W) ws = L.tmp[wl & 15];
-    const int32_t we_sum = row16_incl_scan(ws.x), wr_sum = row16_incl_scan(ws.y);
-    const int32_t total = __builtin_amdgcn_readlane(we_sum, 15), nrows = __builtin_amdgcn_readlane(wr_sum, 15);
-    if (deg > 0) {
-        const int32_t i = (wid ? __builtin_amdgcn_readlane(wr_sum, wid - 1) : 0) + (int32_t)lane_rank(full);
-        const int32_t end = (wid ? __builtin_amdgcn_readlane(we_sum, wid - 1) : 0) + x;
-        L.incl[i] = end;
-        L.rowb[i] = rs.b - (end - deg);
-        L.gu[i] = rs.gu;
-        L.node[i] = u;
-    }
-    __syncthreads();
+    const RoundRows rr = list_rows<B>(L, u >= 0 ? rs.deg : 0, rs.b, rs.gu, u);
+    const int32_t total = rr.total, nrows = rr.nrows;
     // This wave's windows of 64 edges: consecutive ones, dealt out evenly, or
     // (lane heaps) every W-th, which mixes the rows over the heaps: with
     // consecutive ones the C4 batch's heaps kept each other's offspring and
@@ -317,14 +336,9 @@ __device__ __forceinline__ void expand_rows(const GraphView &G, const HeurView &
         const int32_t we1 = nw * (wid + 1) / W * 64;
         wend = we1 < total ? we1 : total;
     }
-    auto row_of = [&](int32_t e) {  // every lane of the wave, e < total
-        const int g = (int)__popcll(__ballot(wl < W && we_sum <= e));  // waves whose rows all end before
-        const int32_t at = (g ? __builtin_amdgcn_readlane(wr_sum, g - 1) : 0) + wl;
-        return at - wl + (int32_t)__popcll(__ballot(at < nrows && L.incl[at < nrows ? at : 0] <= e));
-    };
     const bool direct = DIRECT_OK && kNoLoad && G.relax_min != 0 && total <= B;
     if (we < wend) {
-        int32_t row = row_of(we);
+        int32_t row = first_row(L, rr, we);
         uint64_t *const ck = L.key + wid * RowsLds<B, Push::kCollect>::CAP;
         uint16_t *const cr = L.row + wid * RowsLds<B, Push::kCollect>::CAP;
         int32_t cn = 0;  // collected edges
@@ -337,7 +351,7 @@ __device__ __forceinline__ void expand_rows(const GraphView &G, const HeurView &
                 jj[r] = 0;
                 const int32_t e0 = we + r * STEP;
                 if (e0 >= wend) continue;
-                if (STEP != 64) row = row_of(e0);
+                if (STEP != 64) row = first_row(L, rr, e0);
                 jj[r] = wave_rows(L, nrows, e0, row);
                 if (e0 + wl < wend) {
                     pos[r] = L.rowb[jj[r]] + e0 + wl;
@@ -376,11 +390,14 @@ __device__ __forceinline__ void expand_rows(const GraphView &G, const HeurView &
             uint64_t cur[R];
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                if constexpr (kNoLoad)
-                    if (c[r] >= 0 && wt[r] + (uint32_t)heur_from<HK>(H, c[r], HeurIn{0, 0}) >= Fb)
-                        c[r] = -1;  // cannot beat the bound: no word read
+                if constexpr (kNoLoad) {
+                    if (c[r] >= 0) {
+                        wt[r] += (uint32_t)heur_from<HK>(H, c[r], HeurIn{0, 0});
+                        if (wt[r] >= Fb) c[r] = -1;  // cannot beat the bound: no word read
+                    }
+                }
                 if (c[r] >= 0) {  // negative id = deleted edge
-                    hin[r] = heur_load<HK>(H, c[r]);
+                    if constexpr (!kNoLoad) hin[r] = heur_load<HK>(H, c[r]);
                     if (!direct) cur[r] = ld_gp(gp + c[r]);
                 }
             }
@@ -391,7 +408,7 @@ __device__ __forceinline__ void expand_rows(const GraphView &G, const HeurView &
                 tried[r] = false;
                 key[r] = 0;
                 if (c[r] >= 0) {
-                    const int32_t hc = heur_from<HK>(H, c[r], hin[r]);
+                    const int32_t hc = kNoLoad ? 0 : heur_from<HK>(H, c[r], hin[r]);
                     if (HK != DDP_H_ARRAY || hc >= 0) {  // h = -1: cannot reach t
                         const uint32_t cand = wt[r] + (uint32_t)hc;
                         key[r] = ((uint64_t)cand << 32) | (uint32_t)c[r];
