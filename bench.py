@@ -393,7 +393,7 @@ def run_c2(args):
             raise SystemExit(f"C2 cost differs across K: {r.cost} vs {cost}")
         cost = r.cost
         abytes = 8 * st["expansions"] + 12 * st["edges"] + 8 * st["improvements"]  # closed-form h reads nothing
-        kern = "ga_grid_kernel" if mode == ddp_amd.MODE_GRID else "ga_wg_kernel"  # one-workgroup modes
+        kern = "ga_piles_kernel" if mode == ddp_amd.MODE_GRID else "ga_wg_kernel"  # one-workgroup modes
         sweep[name] = {"K": K, "wall_ms": round(wall, 3), "kernel_ms": round(kms, 3), "iterations": st["iterations"],
                        "expansions": st["expansions"], "edges": st["edges"], "block": st["block"],
                        "blocks": st["blocks"], "roofline": roofline(abytes, kms, kern)}
@@ -445,8 +445,7 @@ def run_c3(args):
     ug = ddp_amd.DeviceGraph(ctx, ddp_amd.HostGraph(uoff, vs[order], ws[order]), reverse=True)
     h, _ = ug.bfs_hops(t, reverse=True, scale=int(ws.min()))
     ug.close()
-    # repair and full recompute, each with the GA* grid kernel (K queues) and
-    # with one workgroup's pile engine
+    # repair and full recompute, each opened in grid and in pile mode
     sessions = {
         "repair_grid": (ddp_amd.DAStar.REPAIR, ddp_amd.MODE_AUTO),
         "repair_piles": (ddp_amd.DAStar.REPAIR, ddp_amd.MODE_PILES),

@@ -490,8 +490,8 @@ class DAStar:
     REPAIR, RECOMPUTE = 0, 1
 
     def __init__(self, ctx, hg, s, t, h=None, K=0, block=0, heap_cap=0, lds_cap=0, mode=MODE_AUTO):
-        """mode: MODE_PILES runs every search (initial, resumed, recomputed) on
-        one workgroup's pile engine; anything else the GA* grid kernel."""
+        """mode: as ddp_astar's; every search (initial, resumed, recomputed) runs
+        on near/far piles over the whole GPU in either mode."""
         self.ctx, self.N, self.s, self.t = ctx, hg.N, s, t
         o = AstarOpts(K, block, heap_cap, lds_cap, 0, mode)
         hh = None if h is None else as_i32(h)

@@ -200,7 +200,7 @@ typedef struct {
     int64_t edges;          /* edges scanned (tombstones included) */
     int64_t improvements;   /* successful relaxations */
     int64_t stale_pops;     /* popped entries superseded by a better one */
-    int32_t iterations;     /* GA* iterations (one pop per queue each) */
+    int32_t iterations;     /* rounds: one pop per queue, or up to K (lanes) near entries */
     int32_t K;              /* queues used */
     int32_t block;          /* lanes per workgroup used */
     int32_t blocks;         /* workgroups used */

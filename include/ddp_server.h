@@ -46,7 +46,7 @@ typedef struct {
                                while no slot runs a request; 0 = 2000 */
     int32_t engine;         /* DDP_SERVER_AUTO / _HEAPS / _PILES (as DDP_BATCH_*) */
     int32_t grid_k;         /* 0 = off.  K > 0: low-load queries are searched in grid mode
-                               (ddp_astar's DDP_ASTAR_GRID, K lane heaps over the whole GPU)
+                               (ddp_astar's DDP_ASTAR_GRID: near/far piles over the whole GPU)
                                instead of one slot: a query goes there while no update is
                                in flight on the slot path, if nothing else is in flight,
                                or, while grid mode alone keeps up with submissions (a
