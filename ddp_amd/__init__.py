@@ -247,10 +247,15 @@ class HostGraph:
         return Updates._from_handle(u)
 
 
+try:
+    from ._hostconv import fill as _fill
+except ImportError:  # no Python headers where the library was built, or another interpreter
+    _fill = None
+
+
 def _updates_array(lines):
-    from ._hostconv import fill  # built with the library
     arr = (Update * max(1, len(lines)))()
-    if fill(lines, arr):
+    if _fill is not None and _fill(lines, arr):
         return arr
     for i, l in enumerate(lines):  # other sequences and number types
         arr[i].flag, arr[i].u, arr[i].v, arr[i].w = int(l[0]), int(l[1]), int(l[2]), int(l[3])
