@@ -641,6 +641,10 @@ struct ddp_dastar {
     int32_t open_at = 0;        // which buffer holds the open set
     uint32_t open_n = 0;        // its entries
     uint32_t open_checked = 0;  // open_n after the last split that checked every entry
+    // a batch's device work has begun and its search has not ended well: the
+    // words and the open set say nothing (a search overwrites the buffer of the
+    // open set it started from), and only a search from s mends them
+    bool lost = false;
 };
 
 static void log_free(InsLog &L)
@@ -1101,6 +1105,8 @@ extern "C" int ddp_dastar_apply(ddp_dastar *d, const ddp_update_t *lines, int32_
     auto grid = [&](size_t k) { return dim3((unsigned)std::max<size_t>(1, (k + T - 1) / T)); };
     // ---- 2. device: deletes (they never see this batch's inserts), then the appends
     d->epoch += 1;
+    const bool fresh = mode == DDP_DASTAR_RECOMPUTE || d->lost;
+    d->lost = true;  // until this batch's search has ended well
     uint32_t *rctrl = d->d_ctl + DC_REPAIR;
     DDP_HIP(ctx, hipEventRecord(d->ev_r0, ctx->stream));
     hipLaunchKernelGGL(da_begin, dim3(1), dim3(256), 0, ctx->stream, d->d_ctl);
@@ -1119,8 +1125,19 @@ extern "C" int ddp_dastar_apply(ddp_dastar *d, const ddp_update_t *lines, int32_
     S.host_ms = ms_since(t0);
     int32_t iters = 0;
     float kms = 0;
-    if (mode == DDP_DASTAR_RECOMPUTE) {
-        if ((rc = fresh_search(d, &iters, &kms))) return rc;
+    // The batch is part of the graph however its search ends (the counters are
+    // read back with the outcome, unless the GPU itself failed).
+    auto account = [&](int code) {
+        if (code == DDP_ERR_HIP) return;
+        const uint32_t *rc_h = d->h_ctl + DC_REPAIR;
+        S.deletes_effective = (int32_t)(rc_h[RC_DEL_BASE] + rc_h[RC_DEL_LOG]);
+        d->live_base -= rc_h[RC_DEL_BASE];
+        d->live_log += nins - (int64_t)rc_h[RC_DEL_LOG];
+    };
+    if (fresh) {
+        rc = fresh_search(d, &iters, &kms);
+        account(rc);
+        if (rc) return rc;
     } else {
         const GraphView F = fwd_view(d), R = rev_view(d);
         // ---- 3. invalidate the parent subtrees of deleted tree edges (roots
@@ -1142,13 +1159,16 @@ extern "C" int ddp_dastar_apply(ddp_dastar *d, const ddp_update_t *lines, int32_
         // pushes; it reads F(t) on the device, and one host round trip brings
         // its outcome and every counter
         if (d->s != d->t) {
-            if ((rc = search_run(d, false, &iters, &kms))) return rc;
+            rc = search_run(d, false, &iters, &kms);
+            account(rc);
+            if (rc) return rc;
         } else {
             uint64_t tword = 0;
             DDP_HIP(ctx, hipMemcpyAsync(&tword, d->gp + d->t, 8, hipMemcpyDeviceToHost, ctx->stream));
             DDP_HIP(ctx, hipMemcpyAsync(d->h_ctl, d->d_ctl, DC_WORDS * 4, hipMemcpyDeviceToHost, ctx->stream));
             DDP_HIP(ctx, hipStreamSynchronize(ctx->stream));
             d->F = (uint32_t)(tword >> 32);
+            account(DDP_OK);
         }
         const uint32_t *rc_h = d->h_ctl + DC_REPAIR;
         DDP_CHECK(rc_h[RC_WALK_ERR] == 0, ctx, DDP_ERR_TIMEOUT,
@@ -1160,10 +1180,7 @@ extern "C" int ddp_dastar_apply(ddp_dastar *d, const ddp_update_t *lines, int32_
         S.pushes = (int32_t)rc_h[RC_PUSHES];
         DDP_HIP(ctx, hipEventElapsedTime(&S.repair_ms, d->ev_r0, d->ev_r1));
     }
-    const uint32_t del_base = d->h_ctl[DC_REPAIR + RC_DEL_BASE], del_log = d->h_ctl[DC_REPAIR + RC_DEL_LOG];
-    S.deletes_effective = (int32_t)(del_base + del_log);
-    d->live_base -= del_base;
-    d->live_log += nins - (int64_t)del_log;
+    d->lost = false;
     S.iterations = iters;
     S.search_ms = kms;
     unsigned long long cnt[8];  // the search counters (expanded, edges, improved, stale, rebuilds, refills, scanned)
@@ -1205,6 +1222,7 @@ extern "C" int ddp_dastar_path(ddp_dastar *d, int32_t *path, int32_t cap, int32_
 {
     if (!d || !path || !len) return DDP_ERR_ARG;
     DDP_HIP(d->ctx, hipSetDevice(d->ctx->device));
+    DDP_CHECK(!d->lost, d->ctx, DDP_ERR_STATE, "DA*: the last batch's search failed, so there is no path; apply again");
     if (d->F == DDP_INF_F) {
         *len = 0;
         return DDP_OK;

@@ -58,7 +58,10 @@ typedef struct {
 int ddp_dastar_open(ddp_ctx *ctx, int32_t N, int32_t E, const int32_t *off, const int32_t *col,
                     const uint32_t *w, const int32_t *h, int32_t s, int32_t t,
                     const ddp_astar_opts_t *opts, ddp_dastar **out, int32_t *cost);
-/* Applies one update batch and returns the new cost of t. */
+/* Applies one update batch and returns the new cost of t.  If the search
+ * fails (DDP_ERR_TIMEOUT, DDP_ERR_OVERFLOW) the batch is part of the graph all
+ * the same; the next apply, in either mode and with any number of lines,
+ * searches from s, and until one succeeds there is no path. */
 int ddp_dastar_apply(ddp_dastar *d, const ddp_update_t *lines, int32_t n, int32_t mode,
                      int32_t *cost, ddp_dastar_stats_t *stats);
 /* Current path s..t (*len = 0 if unreachable, -len if cap is too small). */
