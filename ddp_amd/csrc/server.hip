@@ -319,9 +319,13 @@ __device__ __forceinline__ bool serve_claim(const ServeArgs &a, uint32_t &ticket
                 uint32_t got = 0;
                 if (lane == 0) {
                     got = atomicCAS(a.ctrl + CT_HEAD, h, h + 1) == h;
-                    if (got) add_u32(a.ctrl + CT_BUSY, 1u);
+                    if (got && !d) add_u32(a.ctrl + CT_BUSY, 1u);
                 }
                 if (__builtin_amdgcn_readfirstlane(got)) {
+                    // an entry with kernels of its own is passed over here and
+                    // not read again: it may have its result, and its place in
+                    // the ring a later entry
+                    if (d) continue;
                     ticket = h;
                     have = true;
                     break;
@@ -429,11 +433,6 @@ __global__ void __launch_bounds__(B) serve_kernel(ServeArgs a)
             break;
         }
         const Req rq = s_req;
-        if (rq.direct) {  // its own kernels write its result
-            if (lane == 0) atomicSub(a.ctrl + CT_BUSY, 1u);
-            __syncthreads();        // every lane has read the claim before wave 0 claims again
-            continue;
-        }
         const uint64_t tstart = dev_clock_100mhz();
         // ---- wait for the graph version this request needs (bounded)
         const uint32_t need = rq.type == DDP_REQ_UPDATE ? (uint32_t)rq.version - 1 : (uint32_t)rq.version;
@@ -521,6 +520,17 @@ __global__ void __launch_bounds__(B) serve_kernel(ServeArgs a)
         __syncthreads();
     }
     slot_flush_stats<B>(a.stats, C, stale);
+}
+
+// Before a launch: the last one's closing is undone, and the counts move past
+// what has been delivered already (entries with kernels of their own, which no
+// launch passed over).  Their places in the ring may hold later entries.
+__global__ void serve_begin(uint32_t *ctrl, uint32_t collected)
+{
+    if (threadIdx.x != 0) return;
+    ctrl[CT_BUSY] = 0;
+    if ((int32_t)(collected - ctrl[CT_HEAD]) > 0) ctrl[CT_HEAD] = collected;
+    if ((int32_t)(collected - ctrl[CT_TAIL]) > 0) ctrl[CT_TAIL] = collected;
 }
 
 __global__ void serve_fill_u64(uint64_t *p, int64_t n, uint64_t v)
@@ -807,7 +817,7 @@ static int server_launch(ddp_server *sv)
     ServeArgs a = server_args(sv);
     a.gen = ++sv->gen;
     void *args[] = {&a};
-    DDP_HIP(ctx, hipMemsetAsync(sv->ctrl + CT_BUSY, 0, 4, ctx->stream));  // the last launch closed it
+    hipLaunchKernelGGL(serve_begin, dim3(1), dim3(64), 0, ctx->stream, sv->ctrl, sv->collected);
     DDP_HIP(ctx, hipLaunchKernel((const void *)pick_serve(sv->B, sv->hv.kind, sv->eng), dim3(sv->slots), dim3(sv->B),
                                  args, sv->lds, ctx->stream));
     DDP_HIP(ctx, hipEventRecord(sv->done_ev, ctx->stream));
