@@ -72,16 +72,19 @@ struct Res {       // pinned, written by the device
 };
 
 enum : uint32_t { SERR_WAIT = 16, SERR_LOG = 32 };
-// ctrl words, one 64-byte line apart: claimed count, device copy of the host's
-// published count, applied version, poller lease, sticky error, copy of the
-// host's stop word, busy word.  Launches are numbered (gen) and the stop word
-// holds the newest launch told to stop, so a launch exits once it is >= its
-// own number and no flag is ever cleared while a kernel might still read it.
+// ctrl words: claimed count, applied version, sticky error and busy word on
+// 64-byte lines of their own, and one line for everything that ends an idle
+// slot's wait: the device copy of the host's published count, the copy of its
+// stop word, the poller lease and the newest launch that has closed.  Launches
+// are numbered (gen) and the stop word holds the newest launch told to stop,
+// so a launch exits once it is >= its own number and no flag is ever cleared
+// while a kernel might still read it.
 // The busy word counts slots running a request, plus kClosed once the launch
 // closes for lack of work (cleared by the host before each launch).
 // Counts are unsigned and compared by difference, so they may wrap.
 enum : int {
-    CT_HEAD = 0, CT_TAIL = 16, CT_APPLIED = 32, CT_POLL = 48, CT_ERR = 64, CT_STOP = 80, CT_BUSY = 96, CT_WORDS = 112
+    CT_HEAD = 0, CT_TAIL = 16, CT_STOP = 17, CT_POLL = 18, CT_DONE = 19, CT_APPLIED = 32, CT_ERR = 48, CT_BUSY = 64,
+    CT_WORDS = 80
 };
 constexpr uint32_t kClosed = 0x80000000u;
 constexpr int kLeftWord = 16, kFlagWords = 32;  // pinned flag words: [0] tail, [1] stop, [kLeftWord] left (a line of its own)
@@ -287,34 +290,44 @@ __device__ void apply_update(const ServeArgs &a, const Req &rq, uint32_t *s_err)
 // launch stopped for such an entry (its stop_gen) claims nothing from there
 // on: requests published after it run after its kernels, in the next launch,
 // instead of keeping this one alive while that entry's kernels wait behind it.
-__device__ __forceinline__ bool serve_claim(const ServeArgs &a, uint32_t &ticket)
+//
+// Idle slots wait with four lanes reading one line about every 15 us, and look
+// at the other words only when that line has changed (or every sixteenth time,
+// for the idle time).  Hundreds of them may wait beside the last searches of a
+// burst, on the same memory: with four words read by whole waves and an atomic
+// on the lease per look (one takes 11 ns), a Dijkstra-order search on R-MAT
+// scale 15 took 252 ms beside 1,023 idle slots of 128 lanes (lane heaps) and
+// 14.1 beside 15; 512 such requests at scale 14 took 148 ms, now 14.
+__device__ __forceinline__ bool serve_claim(const ServeArgs &a, uint32_t &ticket, Req *req)
 {
     const uint32_t lane = threadIdx.x;
     constexpr int kWords = sizeof(Req) / 8;
     static_assert(sizeof(Req) % 8 == 0, "entries are copied as 8-byte words");
     const uint64_t t0 = dev_clock_100mhz();
     bool poller = false, have = false;
-    int backoff = 0;  // idle non-pollers back off to ~15 us
+    uint32_t backoff = 0;  // idle non-pollers back off to ~15 us
     uint32_t contended = 0;
     for (;;) {
-        const uint32_t h = __builtin_amdgcn_readfirstlane(ld_u32(a.ctrl + CT_HEAD));
-        const uint32_t tail = __builtin_amdgcn_readfirstlane(ld_u32(a.ctrl + CT_TAIL));
-        const uint32_t bw = __builtin_amdgcn_readfirstlane(ld_u32(a.ctrl + CT_BUSY));
-        const uint32_t applied = __builtin_amdgcn_readfirstlane(ld_u32(a.ctrl + CT_APPLIED));
+        // one look at every word, a lane each
+        const uint32_t at = lane == 0 ? CT_HEAD : lane < 5 ? CT_TAIL - 1 + lane : lane == 5 ? CT_APPLIED : CT_BUSY;
+        uint32_t word = 0;
+        if (lane < 7) word = ld_u32(a.ctrl + at);
+        const uint32_t h = __builtin_amdgcn_readlane(word, 0), tail = __builtin_amdgcn_readlane(word, 1);
+        const uint32_t stop = __builtin_amdgcn_readlane(word, 2), lease = __builtin_amdgcn_readlane(word, 3);
+        const uint32_t applied = __builtin_amdgcn_readlane(word, 5), bw = __builtin_amdgcn_readlane(word, 6);
         if (bw & kClosed) break;
         const bool waiting = (int32_t)(tail - h) > 0;
         if (waiting) {
             // a stale h reads an entry that its failed claim below ignores
-            const uint32_t *e = (const uint32_t *)(a.mirror + (h & a.ring_mask));
-            const uint32_t type = ld_u32(e + offsetof(Req, type) / 4), ver = ld_u32(e + offsetof(Req, version) / 4),
-                           direct = ld_u32(e + offsetof(Req, direct) / 4),
-                           stop_gen = ld_u32(e + offsetof(Req, stop_gen) / 4);
-            const bool d = __builtin_amdgcn_readfirstlane(direct) != 0;
+            uint32_t e = 0;
+            if (lane < sizeof(Req) / 4) e = ld_u32((const uint32_t *)(a.mirror + (h & a.ring_mask)) + lane);
+            auto field = [&](size_t off) { return (uint32_t)__builtin_amdgcn_readlane(e, (int)(off / 4)); };
+            const bool d = field(offsetof(Req, direct)) != 0;
             // this launch was stopped for this entry: what follows it starts
             // after the entry's own kernels, in a later launch
-            if (d && __builtin_amdgcn_readfirstlane(stop_gen) == a.gen) break;
-            const uint32_t v = __builtin_amdgcn_readfirstlane(ver);
-            const uint32_t need = __builtin_amdgcn_readfirstlane(type) == DDP_REQ_UPDATE ? v - 1 : v;
+            if (d && field(offsetof(Req, stop_gen)) == a.gen) break;
+            const uint32_t v = field(offsetof(Req, version));
+            const uint32_t need = field(offsetof(Req, type)) == DDP_REQ_UPDATE ? v - 1 : v;
             if (d || applied >= need) {
                 uint32_t got = 0;
                 if (lane == 0) {
@@ -322,10 +335,9 @@ __device__ __forceinline__ bool serve_claim(const ServeArgs &a, uint32_t &ticket
                     if (got && !d) add_u32(a.ctrl + CT_BUSY, 1u);
                 }
                 if (__builtin_amdgcn_readfirstlane(got)) {
-                    // an entry with kernels of its own is passed over here and
-                    // not read again: it may have its result, and its place in
-                    // the ring a later entry
+                    // an entry with kernels of its own is passed over
                     if (d) continue;
+                    if (lane < sizeof(Req) / 4) ((uint32_t *)req)[lane] = e;
                     ticket = h;
                     have = true;
                     break;
@@ -339,15 +351,18 @@ __device__ __forceinline__ bool serve_claim(const ServeArgs &a, uint32_t &ticket
                 continue;
             }
         }
-        if ((int32_t)(__builtin_amdgcn_readfirstlane(ld_u32(a.ctrl + CT_STOP)) - a.gen) >= 0) break;
+        if ((int32_t)(stop - a.gen) >= 0) break;
         uint32_t won = 0;
         if (lane == 0) {
             if (dev_clock_100mhz() - t0 > a.idle_ticks && bw == 0 && atomicCAS(a.ctrl + CT_BUSY, 0u, kClosed) == 0u)
                 won = 2;
-            else if (!poller) won = atomicCAS(a.ctrl + CT_POLL, 0u, 1u) == 0u;
+            else if (!poller && lease == 0) won = atomicCAS(a.ctrl + CT_POLL, 0u, 1u) == 0u;
         }
         won = __builtin_amdgcn_readfirstlane(won);
-        if (won == 2) break;
+        if (won == 2) {
+            if (lane == 0) st_u32(a.ctrl + CT_DONE, a.gen);
+            break;
+        }
         poller = poller || won == 1;
         if (poller) {
             // the lease holder is the only writer of the tail copy and the mirror
@@ -378,12 +393,22 @@ __device__ __forceinline__ bool serve_claim(const ServeArgs &a, uint32_t &ticket
                 if ((int32_t)(sg - a.gen) >= 0 && lane == 0) atomicExch(a.ctrl + CT_STOP, sg);
                 __builtin_amdgcn_s_sleep(16);
             }
-        } else {
-            // waiting for a version, which comes within tens of microseconds: 1.7 us
+        } else if (waiting) {
+            // for a version, which comes within tens of microseconds: 1.7 us
             // between looks (0.2 us kept the words they look at so busy that the
-            // update itself took twice as long)
-            backoff = waiting ? 1 : backoff < 8 ? backoff + 1 : 8;
-            for (int k = 0; k < backoff; ++k) __builtin_amdgcn_s_sleep(64);
+            // update itself took twice as long), longer where more slots look
+            for (uint32_t k = 0; k <= gridDim.x / 512; ++k) __builtin_amdgcn_s_sleep(64);
+        } else {
+            for (int quiet = 0; quiet < 16; ++quiet) {
+                backoff = backoff < 8 ? backoff + 1 : 8;
+                for (uint32_t k = 0; k < backoff; ++k) __builtin_amdgcn_s_sleep(64);
+                uint32_t line = 0;
+                if (lane < 4) line = ld_u32(a.ctrl + CT_TAIL + lane);
+                if (__builtin_amdgcn_readlane(line, 0) != tail || __builtin_amdgcn_readlane(line, 2) == 0 ||
+                    (int32_t)(__builtin_amdgcn_readlane(line, 1) - a.gen) >= 0 ||
+                    __builtin_amdgcn_readlane(line, 3) == a.gen)
+                    break;
+            }
         }
     }
     if (poller && lane == 0) atomicExch(a.ctrl + CT_POLL, 0u);
@@ -415,11 +440,7 @@ __global__ void __launch_bounds__(B) serve_kernel(ServeArgs a)
     for (;;) {
         if (threadIdx.x < 64) {
             uint32_t ticket = 0;
-            const bool have = serve_claim(a, ticket);
-            constexpr uint32_t kWords = sizeof(Req) / 4;
-            if (have && threadIdx.x < kWords)
-                ((uint32_t *)&s_req)[threadIdx.x] =
-                    ld_u32((const uint32_t *)(a.mirror + (ticket & a.ring_mask)) + threadIdx.x);
+            const bool have = serve_claim(a, ticket, &s_req);
             if (lane == 0) {
                 s_ticket = ticket;
                 s_have = have ? 1 : 0;
