@@ -268,9 +268,10 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
         fn = ld_u32(a.live_n);
         low = ld_u32(a.live_min);
         F = (uint32_t)(ld_gp(a.gp + a.t) >> 32);
-        if (ld_u32(a.live_ovf) || fn > a.fcap) {
+        if (ld_u32(a.live_ovf) || fn > a.fcap) {  // the open set did not fit its buffers
             fn = 0;
-            err = GA_ERR_HEAP;
+            if (a.rebuild) err_seen = PG_ERR_REBUILD;
+            else err = GA_ERR_HEAP;
         }
     }
     if (lane == 0) {
@@ -336,7 +337,22 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
             }
         }
         const uint32_t avail = tail - head;
-        if (avail == 0 && (fn == 0 || low >= F)) break;  // nothing open can improve t
+        if (avail == 0 && (fn == 0 || low >= F)) {  // nothing open can improve t
+            if constexpr (RESUME) {
+                // What is left of the far pile joins the dormant pile below.  If
+                // they do not fit together (stale entries count too), a rebuild
+                // leaves every node in one of them once.
+                if (a.rebuild && (uint64_t)ld_u32(a.dorm_n) + fn > a.dcap) {
+                    if (!grid_sync(ctrl + PG_BAR, gridDim.x, gen, a.barrier_ticks, &s_flag)) {
+                        timeout = true;
+                        break;
+                    }  // everybody has read the count
+                    err_seen |= PG_ERR_REBUILD;
+                    continue;
+                }
+            }
+            break;
+        }
         // The far pile is split when the near ring is empty, or when all but
         // stragglers of a window that has fed its K entries are done and the
         // next window adjoins it (entries further out would run ahead of f
