@@ -614,6 +614,7 @@ struct ddp_dastar {
     // ... and the log of inserted edges
     InsLog L{};
     int32_t log_cap = 0, log_used = 0;
+    bool zero_w = false;        // an edge of weight 0 was inserted (minw is of the graph as opened)
     int64_t compact_at = 0;     // log entries that trigger a compaction after a batch (0 = never)
     int32_t compactions = 0;
     int32_t *d_h = nullptr;
@@ -809,7 +810,9 @@ static int search_run(ddp_dastar *d, bool fresh, int32_t *iters, float *kms)
     uint32_t *split = d->d_ctl + DC_SPLIT;
     PgArgs a{};
     a.g = fwd_view(d);
-    a.g.relax_min = d->g->minw >= 1;
+    // atomicMin only while every weight is at least 1, wherever an edge lives
+    // (a compaction turns inserts into base rows)
+    a.g.relax_min = d->g->minw >= 1 && !d->zero_w;
     a.h = d->hv;
     a.gp = d->gp;
     a.near = d->pnear;
@@ -1090,6 +1093,7 @@ extern "C" int ddp_dastar_apply(ddp_dastar *d, const ddp_update_t *lines, int32_
             o_ins[3 * b] = l.u;
             o_ins[3 * b + 1] = l.v;
             o_ins[3 * b + 2] = (int32_t)l.w;
+            d->zero_w = d->zero_w || l.w == 0;
             d->ku[b] = l.u;
             d->kv[b] = l.v;
             d->kx[b] = d->log_used + b;
