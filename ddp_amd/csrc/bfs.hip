@@ -35,7 +35,8 @@ namespace {
 // control words, a line apart where workgroups update them
 enum : int {
     BC_CNT = 0,  // three rotating level sizes, 32 words apart
-    BC_LEVEL = 96, BC_HEAD = 97, BC_ERR = 98, BC_NEXT = 99, BC_BAR = 128, BC_WORDS = BC_BAR + GRID_SYNC_WORDS
+    BC_LEVEL = 96, BC_HEAD = 97, BC_ERR = 98, BC_NEXT = 99, BC_BAR = 128, BC_TEAM = BC_BAR + GRID_SYNC_WORDS,
+    BC_WORDS = BC_TEAM + TEAM_WORDS
 };
 
 struct BfsArgs {
@@ -76,22 +77,34 @@ __device__ __forceinline__ void bfs_split(const BfsArgs &a, bool is_new, uint32_
 // mostly visited nodes, and a load costs less than an atomic (one CU: 0.86
 // random loads against 0.59 atomics per ns, 2.4 when they hit L2); a narrow
 // level is a chain of round trips and does without that one.
-template <int B, int U, bool CHECK>
+// TEAM: the workgroups that are resident together do the work (grid_team.h);
+// the narrow grid, 32 workgroups of four waves, takes up to four CUs and is
+// launched as a whole.
+template <int B, int U, bool CHECK, bool TEAM>
 __global__ void __launch_bounds__(B) bfs_kernel(BfsArgs a)
 {
     constexpr uint32_t kLanes = 8, kPerWave = 64 / kLanes, kWaves = B / 64, kLocal = 4 * B;
     __shared__ uint64_t s_q[kLocal];
     __shared__ uint32_t s_n, s_base;
     __shared__ int32_t s_flag;
+    __shared__ Team s_team;
     const uint32_t wl = threadIdx.x & 63, sub = wl % kLanes;
     uint32_t *ctrl = a.ctrl;
+    const uint32_t rank = TEAM ? grid_arrive(ctrl + BC_TEAM) : 0u;
     uint32_t gen = ld_u32(ctrl + BC_BAR + 32);
     uint32_t level = ctrl[BC_LEVEL], head = ctrl[BC_HEAD];
-    uint32_t n;
-    for (;;) {
-        n = ld_u32(ctrl + BC_CNT + 32 * (level % 3));
-        if (n <= a.lo || n > a.hi) break;  // lo >= 0: an empty level ends every grid
-        if (blockIdx.x == 0 && threadIdx.x == 0) st_u32(ctrl + BC_CNT + 32 * ((level + 2) % 3), 0);
+    uint32_t n = ld_u32(ctrl + BC_CNT + 32 * (level % 3));
+    Team tm{blockIdx.x, gridDim.x};
+    if constexpr (TEAM) {
+        bool timeout;
+        tm = grid_team(ctrl + BC_TEAM, rank, a.barrier_ticks, &s_team, timeout, n <= a.lo || n > a.hi);
+        if (tm.n == 0) {  // not this grid's level, or the team was complete before this workgroup started
+            if (timeout && threadIdx.x == 0) atomicOr(ctrl + BC_ERR, 1u);
+            return;
+        }
+    }
+    while (n > a.lo && n <= a.hi) {  // lo >= 0: an empty level ends every grid
+        if (tm.me == 0 && threadIdx.x == 0) st_u32(ctrl + BC_CNT + 32 * ((level + 2) % 3), 0);
         uint32_t *ncnt = ctrl + BC_CNT + 32 * ((level + 1) % 3);
         const uint32_t base = head + n;
         const int32_t nl = (int32_t)level + 1;
@@ -100,8 +113,8 @@ __global__ void __launch_bounds__(B) bfs_kernel(BfsArgs a)
         // chunk of kPerWave segments per wave, dealt over the workgroups first
         // so that the segments of one hub go to different CUs
         const uint64_t chunks = ((uint64_t)n + kPerWave - 1) / kPerWave;
-        for (uint64_t ch = (threadIdx.x >> 6) * (uint64_t)gridDim.x + blockIdx.x; ch < chunks;
-             ch += (uint64_t)kWaves * gridDim.x) {
+        for (uint64_t ch = (threadIdx.x >> 6) * (uint64_t)tm.n + tm.me; ch < chunks;
+             ch += (uint64_t)kWaves * tm.n) {
             const uint32_t i = (uint32_t)ch * kPerWave + wl / kLanes;
             uint64_t e = 0;
             if (i < n) e = ld_gp(a.queue + head + i);
@@ -159,18 +172,21 @@ __global__ void __launch_bounds__(B) bfs_kernel(BfsArgs a)
         __syncthreads();
         for (uint32_t k = threadIdx.x; k < mine; k += B)
             if (s_base + k < a.cap) st_u64(a.queue + s_base + k, s_q[k]);
-        if (!grid_sync(ctrl + BC_BAR, gridDim.x, gen, a.barrier_ticks, &s_flag)) {
+        if (!grid_sync(ctrl + BC_BAR, tm, gen, a.barrier_ticks, &s_flag)) {
             if (threadIdx.x == 0) atomicOr(ctrl + BC_ERR, 1u);
             break;
         }
         head = base;
         ++level;
+        n = ld_u32(ctrl + BC_CNT + 32 * (level % 3));
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (tm.me == 0 && threadIdx.x == 0) {
         ctrl[BC_LEVEL] = level;
         ctrl[BC_HEAD] = head;
         ctrl[BC_NEXT] = n;
     }
+    if (!TEAM && blockIdx.x == 0)  // for the wide launch behind this one
+        for (uint32_t k = threadIdx.x; k < TEAM_WORDS; k += B) st_u32(ctrl + BC_TEAM + k, 0u);
 }
 
 // Every distance to -1 but t's, t's row in front of the queue and the control words.
@@ -229,19 +245,19 @@ int bfs_run(ddp_ctx *ctx, const ddp_graph *g, int32_t t, int32_t reverse, int32_
     hipLaunchKernelGGL(bfs_init, dim3(std::min(1024, (N + 255) / 256)), dim3(256), 0, ctx->stream, off, dist, N,
                        queue, cap, seg, ctrl, t);
     BfsArgs a{off, reverse ? g->rcol : g->col, dist, queue, cap, seg, 0, 0, ctrl, 100ull * 1000 * 1000 * 20};
-    // Ordinary launches: the grid barrier is software and only needs every
-    // workgroup resident at once, which one workgroup per CU gives on an idle
-    // device (a cooperative launch would also reserve the GPU's global
-    // wave-sync unit, which only one process may hold).  Every barrier wait is
-    // bounded, so a non-resident grid ends with DDP_ERR_TIMEOUT, not a hang.
+    // Ordinary launches: the grid barrier is software and only needs its
+    // workgroups resident at once (a cooperative launch would also reserve the
+    // GPU's global wave-sync unit, which only one process may hold).  Every
+    // barrier wait is bounded, so a narrow grid without room for its 32
+    // workgroups ends with DDP_ERR_TIMEOUT, not a hang.
     const bool wide = bfs_entries(N, reverse ? g->RE : g->E, seg) > kNarrowMax;  // some level may be
     auto run = [&](bool w) {
         a.lo = w ? kNarrowMax / 2 : 0;  // the wide grid keeps a level until it is clearly narrow
         a.hi = w ? 0xFFFFFFFFu : kNarrowMax;
         void *args[] = {&a};
-        return w ? hipLaunchKernel((const void *)bfs_kernel<kWideBlock, 2, true>, dim3(wide_blocks), dim3(kWideBlock),
-                                   args, 0, ctx->stream)
-                 : hipLaunchKernel((const void *)bfs_kernel<kNarrowBlock, 1, false>, dim3(kNarrowBlocks),
+        return w ? hipLaunchKernel((const void *)bfs_kernel<kWideBlock, 2, true, true>, dim3(wide_blocks),
+                                   dim3(kWideBlock), args, 0, ctx->stream)
+                 : hipLaunchKernel((const void *)bfs_kernel<kNarrowBlock, 1, false, false>, dim3(kNarrowBlocks),
                                    dim3(kNarrowBlock), args, 0, ctx->stream);
     };
     uint32_t res[4];

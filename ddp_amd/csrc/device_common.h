@@ -5,6 +5,7 @@
 #include <cstdint>
 
 #include "ddp_internal.h"
+#include "grid_team.h"
 #include "isqrt.h"
 
 #define DDP_INF_F 0x7FFFFFFFu                      // Cx "infinity" (INT_MAX)
@@ -293,9 +294,15 @@ __device__ __forceinline__ void st_u64(uint64_t *p, uint64_t v)
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ bool grid_sync(uint32_t *bar, uint32_t nblocks, uint32_t &gen, uint64_t limit_ticks,
-                                          int32_t *s_flag)
+// The barrier's workgroups: a launch's members (grid_team.h) and this one's
+// number among them, or the whole grid.
+struct Team {
+    uint32_t me, n;
+};
+
+__device__ __forceinline__ bool grid_sync(uint32_t *bar, Team tm, uint32_t &gen, uint64_t limit_ticks, int32_t *s_flag)
 {
+    const uint32_t nblocks = tm.n;
     block_sync_global();
     if (threadIdx.x == 0) {
         constexpr uint32_t kGroups = 8;
@@ -303,7 +310,7 @@ __device__ __forceinline__ bool grid_sync(uint32_t *bar, uint32_t nblocks, uint3
         if (nblocks <= 64) {
             last = add_u32(bar, 1u) == nblocks - 1;
         } else {
-            const uint32_t g = blockIdx.x % kGroups, members = (nblocks - g + kGroups - 1) / kGroups;
+            const uint32_t g = tm.me % kGroups, members = (nblocks - g + kGroups - 1) / kGroups;
             uint32_t *grp = bar + 32 * (2 + g);
             last = add_u32(grp, 1u) == members - 1;
             if (last) {
@@ -331,4 +338,46 @@ __device__ __forceinline__ bool grid_sync(uint32_t *bar, uint32_t nblocks, uint3
     gen += 1;
     __syncthreads();
     return *s_flag != 0;
+}
+
+struct TeamMem {
+    using Word = uint32_t;
+    __device__ __forceinline__ uint32_t add(uint32_t *p, uint32_t v) { return add_u32(p, v); }
+    __device__ __forceinline__ uint32_t fetch_or(uint32_t *p, uint32_t v)
+    {
+        return __hip_atomic_fetch_or(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ uint32_t load(uint32_t *p) { return ld_u32(p); }
+    __device__ __forceinline__ void store(uint32_t *p, uint32_t v) { st_u32(p, v); }
+    __device__ __forceinline__ void fence() { wait_vmem(); }
+    __device__ __forceinline__ uint64_t clock() { return dev_clock_100mhz(); }
+    __device__ __forceinline__ void pause() { __builtin_amdgcn_s_sleep(1); }
+};
+
+// Lane 0's arrival at the launch's team (grid_team.h; other lanes: nothing).
+__device__ __forceinline__ uint32_t grid_arrive(uint32_t *words)
+{
+    TeamMem m;
+    return threadIdx.x == 0 ? team_arrive(m, words, blockIdx.x) : 0u;
+}
+
+// The launch's team; block-collective.  n = 0: the workgroup leaves, with an
+// error if timeout is set.  skip (of lane 0): the launch has nothing to do,
+// leave without waiting.
+__device__ __forceinline__ Team grid_team(uint32_t *words, uint32_t rank, uint64_t limit_ticks, Team *s_team,
+                                          bool &timeout, bool skip = false)
+{
+    if (threadIdx.x == 0) {
+        TeamMem m;
+        Team t{0, 0};
+        const int got =
+            skip ? TEAM_CLOSED : team_settle(m, words, rank, blockIdx.x, gridDim.x, limit_ticks, t.me, t.n);
+        if (got != TEAM_MEMBER) t = Team{got == TEAM_TIMEOUT ? 1u : 0u, 0};
+        *s_team = t;
+    }
+    __syncthreads();
+    const Team t{(uint32_t)__builtin_amdgcn_readfirstlane(s_team->me),
+                 (uint32_t)__builtin_amdgcn_readfirstlane(s_team->n)};
+    timeout = t.n == 0 && t.me != 0;
+    return t;
 }

@@ -8,7 +8,7 @@
 // counters behind them.
 enum : int {
     GA_RES_IT = 32, GA_RES_F = 34, GA_RES_ERR = 35, GA_RES_PLEN = 36,
-    GA_CTRL_WORDS = 1024,
+    GA_CTRL_WORDS = 1280,
 };
 
 // Error bits of GA_RES_ERR.

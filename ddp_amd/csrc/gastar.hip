@@ -366,9 +366,10 @@ int ddp_ga_stats(ddp_ctx *ctx, const GaGridState &S, unsigned long long out[4])
 namespace {
 
 // Seeds s and enqueues the grid search.  Ordinary launch of at most one
-// workgroup per CU, so all are resident at once, and the grid barrier is
-// software with bounded waits (a cooperative launch would also reserve the
-// global wave-sync unit, one process only).
+// workgroup per CU; those that find room at once are the search's team
+// (grid_team.h), and the grid barrier is software with bounded waits (a
+// cooperative launch would also reserve the global wave-sync unit, one process
+// only).
 int pg_enqueue(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P, const GaGridState &S,
                int32_t s, uint32_t hs, int32_t t)
 {

@@ -35,7 +35,8 @@
 //
 // Everything workgroups share -- the (f, parent) words, the piles, the control
 // words -- is accessed through agent-scope atomics only, as grid_sync needs.
-// A round's steps each end with grid_sync; what a step appended is counted in
+// The workgroups are a team (grid_team.h): those of the launch that are resident
+// together.  A round's steps each end with grid_sync; what a step appended is counted in
 // one of three rotating slots, read by everybody after the barrier and cleared
 // two steps later, so all workgroups take every decision from the same values.
 #pragma once
@@ -46,7 +47,8 @@
 // Control words behind the result words of gastar.h (a 128-byte line each).
 enum : int {
     PG_NEAR = 0, PG_FAR = 32, PG_TMIN = 64, PG_FMIN = 96, PG_HUBS = 128, PG_ERR = 129, PG_SLOT_WORDS = 160,
-    PG_SLOTS = 128, PG_BAR = PG_SLOTS + 3 * PG_SLOT_WORDS, PG_WORDS = PG_BAR + GRID_SYNC_WORDS
+    PG_SLOTS = 128, PG_BAR = PG_SLOTS + 3 * PG_SLOT_WORDS, PG_TEAM = PG_BAR + GRID_SYNC_WORDS,
+    PG_WORDS = PG_TEAM + TEAM_WORDS
 };
 static_assert(PG_WORDS <= GA_CTRL_WORDS, "control block too small");
 
@@ -249,10 +251,12 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
     static_assert(B >= 256, "flush uses four waves");
     __shared__ PgStage<B, RESUME> S;
     __shared__ int32_t s_flag;
+    __shared__ Team s_team;
     constexpr uint32_t kPerWave = 64 / kPgLanes, kWaves = B / 64;
     const int lane = threadIdx.x;
     const uint32_t wl = lane & 63, sub = lane % kPgLanes;
     uint32_t *ctrl = a.ctrl;
+    const uint32_t rank = grid_arrive(ctrl + PG_TEAM);
     uint32_t gen = ld_u32(ctrl + PG_BAR + 32);
     // ring positions and far entries as of the last barrier, the same in every workgroup
     uint32_t head = 0, tail = 1, fn = 0, F = DDP_INF_F, thr = a.thr0, delta = a.delta0, phase_n = 0;
@@ -261,6 +265,11 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
     uint32_t step = 0, err = 0, err_seen = 0;
     int32_t it = 0;
     bool timeout = false;
+    const Team tm = grid_team(ctrl + PG_TEAM, rank, a.barrier_ticks, &s_team, timeout);
+    if (tm.n == 0) {  // the team was complete before this workgroup started
+        if (timeout && lane == 0) atomicOr(ctrl + GA_RES_ERR, (uint32_t)GA_ERR_BARRIER);
+        return;
+    }
     ExpandCounters C;
     uint32_t stale = 0;
     if constexpr (RESUME) {
@@ -282,7 +291,7 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
     __syncthreads();
     // a step: its counters' slot; the next step's (last read two barriers ago) is cleared meanwhile
     auto begin = [&]() {
-        if (blockIdx.x == 0 && lane < 6) {
+        if (tm.me == 0 && lane < 6) {
             uint32_t *ns = ctrl + PG_SLOTS + ((step + 1) % 3) * PG_SLOT_WORDS;
             if (lane < 5) st_u32(ns + 32 * lane, lane == 2 || lane == 3 ? 0xFFFFFFFFu : 0u);
             else st_u32(ns + PG_ERR, 0u);
@@ -297,12 +306,12 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
                 // finite word (nodes that were expanded at that value already are
                 // expanded again, which is harmless)
                 err_seen = 0;
-                if (blockIdx.x == 0 && lane == 0) {
+                if (tm.me == 0 && lane == 0) {
                     st_u32(a.dorm_n, 0u);
                     C.rebuilds++;
                 }
                 uint32_t *slot = begin();
-                if (!grid_sync(ctrl + PG_BAR, gridDim.x, gen, a.barrier_ticks, &s_flag)) {
+                if (!grid_sync(ctrl + PG_BAR, tm, gen, a.barrier_ticks, &s_flag)) {
                     timeout = true;
                     break;
                 }
@@ -310,9 +319,9 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
                 slot = begin();
                 head = tail;
                 PgPush<B, RESUME> push{&S, &a, slot, tail, head, far, 0u, thr, F};
-                const uint32_t stride = gridDim.x * B, trips = ((uint32_t)a.N + stride - 1) / stride;
+                const uint32_t stride = tm.n * B, trips = ((uint32_t)a.N + stride - 1) / stride;
                 for (uint32_t r = 0; r < trips; ++r) {
-                    const uint32_t v = r * stride + blockIdx.x * B + lane;
+                    const uint32_t v = r * stride + tm.me * B + lane;
                     uint64_t key[1] = {0};
                     bool live[1] = {false};
                     if (v < (uint32_t)a.N && v != (uint32_t)a.t) {
@@ -323,7 +332,7 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
                     push.template all<1>(live, key);
                 }
                 push.flush();
-                if (!grid_sync(ctrl + PG_BAR, gridDim.x, gen, a.barrier_ticks, &s_flag)) {
+                if (!grid_sync(ctrl + PG_BAR, tm, gen, a.barrier_ticks, &s_flag)) {
                     timeout = true;
                     break;
                 }
@@ -343,7 +352,7 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
                 // they do not fit together (stale entries count too), a rebuild
                 // leaves every node in one of them once.
                 if (a.rebuild && (uint64_t)ld_u32(a.dorm_n) + fn > a.dcap) {
-                    if (!grid_sync(ctrl + PG_BAR, gridDim.x, gen, a.barrier_ticks, &s_flag)) {
+                    if (!grid_sync(ctrl + PG_BAR, tm, gen, a.barrier_ticks, &s_flag)) {
                         timeout = true;
                         break;
                     }  // everybody has read the count
@@ -368,7 +377,7 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
             }
             const uint32_t nt = add_sat(low, delta);
             thr = nt > thr ? nt : thr;
-            if (blockIdx.x == 0 && lane == 0) C.refills++;
+            if (tm.me == 0 && lane == 0) C.refills++;
         }
         if (avail && it >= a.maxit) {
             err |= GA_ERR_ITERS;
@@ -382,7 +391,7 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
         {
             PgPush<B, RESUME> push{&S, &a, slot, tail, head, split ? far2 : far, split ? 0u : fn, thr, F};
             const uint32_t chunks = (n + kPerWave - 1) / kPerWave;
-            for (uint32_t ch = (lane >> 6) * gridDim.x + blockIdx.x; ch < chunks; ch += kWaves * gridDim.x) {
+            for (uint32_t ch = (lane >> 6) * tm.n + tm.me; ch < chunks; ch += kWaves * tm.n) {
                 const uint32_t i = ch * kPerWave + wl / kPgLanes;
                 int32_t u = -1;
                 uint32_t gu = 0, start = 0, deg = 0;
@@ -471,9 +480,9 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
                 }
             }
             if (split) {
-                const uint32_t stride = gridDim.x * B, trips = (fn + stride - 1) / stride;
+                const uint32_t stride = tm.n * B, trips = (fn + stride - 1) / stride;
                 for (uint32_t r = 0; r < trips; ++r) {  // uniform: the appends are wave-wide
-                    const uint64_t i = (uint64_t)r * stride + (uint64_t)blockIdx.x * B + lane;
+                    const uint64_t i = (uint64_t)r * stride + (uint64_t)tm.me * B + lane;
                     uint64_t key[1] = {0};
                     bool live[1] = {false};
                     if (i < fn) {
@@ -488,7 +497,7 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
             }
             push.flush();
         }
-        if (!grid_sync(ctrl + PG_BAR, gridDim.x, gen, a.barrier_ticks, &s_flag)) {
+        if (!grid_sync(ctrl + PG_BAR, tm, gen, a.barrier_ticks, &s_flag)) {
             timeout = true;
             break;
         }
@@ -515,7 +524,7 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
             slot = begin();
             PgPush<B, RESUME> push{&S, &a, slot, tail, head, far, fn, thr, F};
             const uint32_t chunks = (hubs + kPerWave - 1) / kPerWave;
-            for (uint32_t ch = (lane >> 6) * gridDim.x + blockIdx.x; ch < chunks; ch += kWaves * gridDim.x) {
+            for (uint32_t ch = (lane >> 6) * tm.n + tm.me; ch < chunks; ch += kWaves * tm.n) {
                 const uint32_t i = ch * kPerWave + wl / kPgLanes;
                 uint64_t row = 0, from = 0;
                 if (i < hubs) {
@@ -526,7 +535,7 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
                                  (uint32_t)(from >> 32), RESUME ? 0xFFFFFFFFu : F, C, push);
             }
             push.flush();
-            if (!grid_sync(ctrl + PG_BAR, gridDim.x, gen, a.barrier_ticks, &s_flag)) {
+            if (!grid_sync(ctrl + PG_BAR, tm, gen, a.barrier_ticks, &s_flag)) {
                 timeout = true;
                 break;
             }
@@ -547,11 +556,11 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
         const uint32_t dn = ld_u32(a.dorm_n);
         if ((uint64_t)dn + fn > a.dcap) err |= GA_ERR_HEAP;
         else
-            for (uint32_t i = blockIdx.x * B + lane; i < fn; i += gridDim.x * B) st_u64(a.dorm + dn + i, ld_gp(far + i));
-        if (blockIdx.x == 0 && lane == 0) ctrl[GA_RES_PLEN] = dn + fn;
+            for (uint32_t i = tm.me * B + lane; i < fn; i += tm.n * B) st_u64(a.dorm + dn + i, ld_gp(far + i));
+        if (tm.me == 0 && lane == 0) ctrl[GA_RES_PLEN] = dn + fn;
     }
     if (timeout && lane == 0) atomicOr(ctrl + GA_RES_ERR, (uint32_t)GA_ERR_BARRIER);
-    if (blockIdx.x == 0 && lane == 0) {
+    if (tm.me == 0 && lane == 0) {
         if (err) atomicOr(ctrl + GA_RES_ERR, err);
         ctrl[GA_RES_IT] = (uint32_t)it;
         ctrl[GA_RES_F] = F;
