@@ -33,6 +33,7 @@
 #include "bidi_search.h"
 #include "gastar.h"
 #include "grid_piles.h"
+#include "pile_sizes.h"
 
 namespace {
 
@@ -85,16 +86,7 @@ int32_t pg_blocks(const ddp_ctx *ctx, const GaGridPlan &P, int hk)
     return P.pg_wide && (hk == DDP_H_ZERO || hk == DDP_H_ARRAY) ? cus : std::min(kPgBlocks, cus);
 }
 
-// Entries of the near ring (a power of two) and of each far buffer: either
-// holds the K * cap entries that K queues of cap would.
-void ga_pg_sizes(const GaGridPlan &P, uint64_t *ring, uint64_t *far)
-{
-    const uint64_t total = std::min<uint64_t>((uint64_t)P.K * P.cap, 1ull << 31);
-    uint64_t r = 1024;
-    while (r < total) r *= 2;
-    *ring = r;
-    *far = std::max<uint64_t>(total, 1024);
-}
+PgSizes ga_pg_sizes(const GaGridPlan &P, int32_t N) { return pg_sizes((uint64_t)P.K * P.cap, N); }
 
 // Workgroup mode: all K <= 1024 queues live in one workgroup, one per lane,
 // and an improved node goes to the queue of the lane that relaxed it.  An
@@ -292,9 +284,7 @@ int ddp_ga_alloc(ddp_ctx *ctx, const ddp_graph *g, const GaGridPlan &P, GaGridSt
     const size_t dirs = P.bidi ? 2 : 1;
     size_t queue = dirs * P.cap * P.K, push = 0;  // 8-byte entries
     if (P.pg) {
-        uint64_t ring, far;
-        ga_pg_sizes(P, &ring, &far);
-        queue = ring + 2 * far;
+        queue = ga_pg_sizes(P, g->N).entries();
         push = 2 * (size_t)P.hubcap;
     }
     if ((rc = ddp_ws(ctx, WS_ASTAR_GP, dirs * g->N * 8, &p))) return rc;
@@ -324,10 +314,8 @@ int ddp_ga_alloc_owned(ddp_ctx *ctx, int32_t N, const GaGridPlan &P, GaGridState
         if (e == hipSuccess) e = hipMalloc(p, std::max<size_t>(bytes, 64));
     };
     DDP_CHECK(P.pg, ctx, DDP_ERR_STATE, "GA*: not a grid plan");
-    uint64_t ring, far;
-    ga_pg_sizes(P, &ring, &far);
     al((void **)&S->gp, (size_t)N * 8);
-    al((void **)&S->home, (ring + 2 * far) * 8);
+    al((void **)&S->home, ga_pg_sizes(P, N).entries() * 8);
     al((void **)&S->pbuf, 16 * (size_t)P.hubcap);
     al((void **)&S->ctrl, GA_CTRL_WORDS * 4 + 64);
     if (e != hipSuccess) {
@@ -373,18 +361,19 @@ namespace {
 int pg_enqueue(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGridPlan &P, const GaGridState &S,
                int32_t s, uint32_t hs, int32_t t)
 {
-    uint64_t ring, far;
-    ga_pg_sizes(P, &ring, &far);
+    const PgSizes z = ga_pg_sizes(P, gv.N);
     PgArgs a{};
     a.g = gv;
     a.h = hv;
     a.gp = S.gp;
     a.near = S.home;
-    a.far0 = S.home + ring;
-    a.far1 = a.far0 + far;
+    a.far0 = S.home + z.ring;
+    a.far1 = a.far0 + z.far;
     a.hubs = S.pbuf;
-    a.nmask = (uint32_t)(ring - 1);
-    a.fcap = (uint32_t)far;
+    a.nmask = (uint32_t)(z.ring - 1);
+    a.fcap = (uint32_t)z.far;
+    a.N = gv.N;
+    a.rebuild = z.rebuild;
     a.hubcap = P.hubcap;
     a.ctrl = S.ctrl;
     a.stats = S.stats;

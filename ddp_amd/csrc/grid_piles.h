@@ -85,12 +85,13 @@ struct PgArgs {
     uint32_t *ctrl;
     unsigned long long *stats;
     // RESUME: the dormant pile (dcap entries) and its count, the live entries'
-    // count and smallest f, and whether counting them overflowed; with
-    // `rebuild`, piles that overflow are rebuilt from the N nodes' words
+    // count and smallest f, and whether counting them overflowed
     uint64_t *dorm;
     uint32_t dcap;
     uint32_t *dorm_n;
     const uint32_t *live_n, *live_min, *live_ovf;
+    // rebuild: piles that overflow are rebuilt from the N nodes' words (the ring
+    // and each far buffer hold N entries at least)
     int32_t N, rebuild;
     int32_t t, maxit;
     uint32_t grow;        // K: a window that fed fewer entries doubles, one that fed 8 times as many halves
@@ -110,7 +111,7 @@ struct PgStage {
     uint32_t tmin, fmin, err;
 };
 
-// Error bits beside GA_ERR_*: a resumed search's piles overflowed and are to be rebuilt.
+// Error bits beside GA_ERR_*: the piles overflowed and are to be rebuilt.
 constexpr uint32_t PG_ERR_REBUILD = 0x100;
 
 template <int B, bool RESUME>
@@ -145,7 +146,7 @@ struct PgPush {
             ok = k < a->dcap;
             if (ok) st_u64(a->dorm + k, key);
         }
-        if (!ok) atomicOr(&S->err, RESUME && a->rebuild ? PG_ERR_REBUILD : (uint32_t)GA_ERR_HEAP);
+        if (!ok) atomicOr(&S->err, a->rebuild ? PG_ERR_REBUILD : (uint32_t)GA_ERR_HEAP);
     }
     __device__ __forceinline__ void target(uint32_t f) const { atomicMin(&S->tmin, f); }
     __device__ __forceinline__ void touch(int32_t, uint64_t) const {}
@@ -300,50 +301,48 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
     };
     auto add_sat = [](uint32_t x, uint32_t y) { return x > 0xFFFFFFFFu - y ? 0xFFFFFFFFu : x + y; };
     while (!err) {
-        if constexpr (RESUME) {
-            if (err_seen & PG_ERR_REBUILD) {
-                // entries were lost: the piles start again from every node with a
-                // finite word (nodes that were expanded at that value already are
-                // expanded again, which is harmless)
-                err_seen = 0;
-                if (tm.me == 0 && lane == 0) {
-                    st_u32(a.dorm_n, 0u);
-                    C.rebuilds++;
-                }
-                uint32_t *slot = begin();
-                if (!grid_sync(ctrl + PG_BAR, tm, gen, a.barrier_ticks, &s_flag)) {
-                    timeout = true;
-                    break;
-                }
-                ++step;
-                slot = begin();
-                head = tail;
-                PgPush<B, RESUME> push{&S, &a, slot, tail, head, far, 0u, thr, F};
-                const uint32_t stride = tm.n * B, trips = ((uint32_t)a.N + stride - 1) / stride;
-                for (uint32_t r = 0; r < trips; ++r) {
-                    const uint32_t v = r * stride + tm.me * B + lane;
-                    uint64_t key[1] = {0};
-                    bool live[1] = {false};
-                    if (v < (uint32_t)a.N && v != (uint32_t)a.t) {
-                        const uint32_t f = (uint32_t)(ld_gp(a.gp + v) >> 32);
-                        live[0] = f != DDP_INF_F;
-                        key[0] = (uint64_t)f << 32 | v;
-                    }
-                    push.template all<1>(live, key);
-                }
-                push.flush();
-                if (!grid_sync(ctrl + PG_BAR, tm, gen, a.barrier_ticks, &s_flag)) {
-                    timeout = true;
-                    break;
-                }
-                ++step;
-                tail += ld_u32(slot + PG_NEAR);
-                fn = ld_u32(slot + PG_FAR);
-                low = ld_u32(slot + PG_FMIN);
-                err_seen = ld_u32(slot + PG_ERR);
-                err = err_seen & ~PG_ERR_REBUILD;
-                continue;
+        if (err_seen & PG_ERR_REBUILD) {
+            // entries were lost: the piles start again from every node whose
+            // word is below F(t) (RESUME: finite; nodes that were expanded at
+            // that value already are expanded again, which is harmless)
+            err_seen = 0;
+            if (tm.me == 0 && lane == 0) {
+                if constexpr (RESUME) st_u32(a.dorm_n, 0u);
+                C.rebuilds++;
             }
+            uint32_t *slot = begin();
+            if (!grid_sync(ctrl + PG_BAR, tm, gen, a.barrier_ticks, &s_flag)) {
+                timeout = true;
+                break;
+            }
+            ++step;
+            slot = begin();
+            head = tail;
+            PgPush<B, RESUME> push{&S, &a, slot, tail, head, far, 0u, thr, F};
+            const uint32_t stride = tm.n * B, trips = ((uint32_t)a.N + stride - 1) / stride;
+            for (uint32_t r = 0; r < trips; ++r) {
+                const uint32_t v = r * stride + tm.me * B + lane;
+                uint64_t key[1] = {0};
+                bool live[1] = {false};
+                if (v < (uint32_t)a.N && v != (uint32_t)a.t) {
+                    const uint32_t f = (uint32_t)(ld_gp(a.gp + v) >> 32);
+                    live[0] = f != DDP_INF_F;
+                    key[0] = (uint64_t)f << 32 | v;
+                }
+                push.template all<1>(live, key);
+            }
+            push.flush();
+            if (!grid_sync(ctrl + PG_BAR, tm, gen, a.barrier_ticks, &s_flag)) {
+                timeout = true;
+                break;
+            }
+            ++step;
+            tail += ld_u32(slot + PG_NEAR);
+            fn = ld_u32(slot + PG_FAR);
+            low = ld_u32(slot + PG_FMIN);
+            err_seen = ld_u32(slot + PG_ERR);
+            err = err_seen & ~PG_ERR_REBUILD;
+            continue;
         }
         const uint32_t avail = tail - head;
         if (avail == 0 && (fn == 0 || low >= F)) {  // nothing open can improve t

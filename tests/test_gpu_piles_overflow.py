@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import ddp_amd
+from helpers import path_cost
 from oracle import pyoracle
 
 pytestmark = pytest.mark.gpu
@@ -55,3 +56,17 @@ def test_dastar_far_and_dormant_do_not_fit_together(ctx, mode):
         cost, _ = d.apply(lines)
         assert cost == dijkstra(cur, 0, t), lines
     d.close()
+
+
+@pytest.mark.parametrize("exit_at,K", [(24, 64), (-1, 64), (-1, 1024)])
+def test_grid_search_larger_than_its_piles(ctx, exit_at, K):
+    """1.5M entries, far buffers of two entries a node: rebuilt as often as it takes."""
+    hg = fans(30000, 50, exit_at)
+    dg = ddp_amd.DeviceGraph(ctx, hg)
+    want = dijkstra((hg.off, hg.col, hg.w), 0, 50)
+    heap_cap = (2 * hg.N + K - 1) // K  # the least that is no limit
+    for kw in (dict(), dict(heap_cap=heap_cap)):
+        r = ddp_amd.astar(ctx, dg, 0, 50, heur=ddp_amd.H_ZERO, K=K, mode=ddp_amd.MODE_GRID, **kw)
+        assert r.cost == want
+        assert path_cost(hg.off, hg.col, hg.w, r.path) == want and r.path[0] == 0 and r.path[-1] == 50
+    dg.close()
