@@ -380,8 +380,8 @@ int pg_enqueue(ddp_ctx *ctx, const GraphView &gv, const HeurView &hv, const GaGr
     a.grow = (uint32_t)P.K;
     a.t = t;
     a.maxit = P.maxit;
-    a.delta0 = P.delta0;
-    a.thr0 = hs > 0xFFFFFFFFu - P.delta0 ? 0xFFFFFFFFu : hs + P.delta0;
+    a.delta0 = pg_first_window(P.delta0, hv.kind == DDP_H_MANHATTAN);
+    a.thr0 = hs > 0xFFFFFFFFu - a.delta0 ? 0xFFFFFFFFu : hs + a.delta0;
     a.barrier_ticks = 100ull * 1000 * 1000 * 20;  // 20 s of the 100 MHz clock
     hipLaunchKernelGGL(pg_seed_kernel, dim3(1), dim3(256), 0, ctx->stream, S.gp, S.home, S.ctrl, s, hs);
     void *args[] = {&a};

@@ -70,6 +70,26 @@ constexpr int64_t kPgWideEdges = 1 << 22;
 // 65,536 entries took 0.39 and 0.32 ms on the random graph (K = 1,024), 0.68
 // and 0.36 ms on one of 300,000 nodes at K = 256.
 constexpr uint32_t kPgRound = 65536;
+// Near entries a window's rounds take on average at least: a window of fewer
+// doubles too, however many it fed in all.  A round costs 6 us whatever it takes,
+// and on a maze with the Manhattan heuristic a chain of thousands of rounds of 15
+// entries passed the K test: 4,096 x 4,096 took 76 ms (12,477 rounds), now 26
+// (3,928; K = 1,024); 512 x 512 8.8 and 6.0; a map of 1M nodes without heuristic 12.6
+// and 6.5 (64 entries instead of 512: 12.6).  Random graphs, R-MAT and maps with
+// their heuristic are the same within 1%.
+constexpr uint32_t kPgFeed = 512;
+// The first window: the mean weight, or 32 of them with the Manhattan heuristic.
+// There f grows by two a detour, so windows of a few steps are chains of rounds of
+// a handful of entries until they have doubled often enough: 21 mazes of 64 x 64
+// to 1,500 x 1,500 (2 queries each, K = 1,024) took 0.74 to 1.6 times as long as on lane
+// heaps, now 0.59 to 0.87; 4,096 x 4,096 25.9 and 18.7 ms.  Other searches keep the
+// mean: wider ones make R-MAT of scale 16 0.59 -> 0.69 ms, and random graphs of
+// 500,000 nodes 0.40 -> 0.69 from 8 on.
+inline uint32_t pg_first_window(uint32_t mean, bool manhattan)
+{
+    const uint64_t d = (uint64_t)mean * (manhattan ? 32 : 1);
+    return d < 0x7FFFFFFFu ? (uint32_t)d : 0x7FFFFFFFu;
+}
 // Near entries that count as stragglers: with 256 the split ran ahead of f
 // order on mazes (703,000 expansions against 56,000 without early splits).
 constexpr uint32_t kPgThin = 64;
@@ -260,7 +280,7 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
     const uint32_t rank = grid_arrive(ctrl + PG_TEAM);
     uint32_t gen = ld_u32(ctrl + PG_BAR + 32);
     // ring positions and far entries as of the last barrier, the same in every workgroup
-    uint32_t head = 0, tail = 1, fn = 0, F = DDP_INF_F, thr = a.thr0, delta = a.delta0, phase_n = 0;
+    uint32_t head = 0, tail = 1, fn = 0, F = DDP_INF_F, thr = a.thr0, delta = a.delta0, phase_n = 0, phase_it = 0;
     uint32_t low = 0xFFFFFFFFu;  // no live far entry is below this
     uint64_t *far = a.far0, *far2 = a.far1;
     uint32_t step = 0, err = 0, err_seen = 0;
@@ -369,10 +389,11 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
         if (split) {
             if (avail == 0) {
                 if (it > 0) {
-                    if (phase_n < a.grow) delta = add_sat(delta, delta);
-                    else if (phase_n > 8 * a.grow && delta > 1) delta >>= 1;
+                    if (phase_n < a.grow || phase_n < kPgFeed * phase_it) delta = add_sat(delta, delta);
+                    else if (phase_n > 8 * a.grow && phase_n > 8 * kPgFeed * phase_it && delta > 1) delta >>= 1;
                 }
                 phase_n = 0;
+                phase_it = 0;
             }
             const uint32_t nt = add_sat(low, delta);
             thr = nt > thr ? nt : thr;
@@ -382,7 +403,10 @@ __global__ void __launch_bounds__(B) ga_piles_kernel(PgArgs a)
             err |= GA_ERR_ITERS;
             break;
         }
-        if (avail) ++it;
+        if (avail) {
+            ++it;
+            ++phase_it;
+        }
         const uint32_t n = avail < kPgRound ? avail : kPgRound;
         phase_n += n;
         // ---- step 1: the round's entries, hub rows cut into segments, and the split
