@@ -851,12 +851,12 @@ static int search_run(ddp_dastar *d, bool fresh, int32_t *iters, float *kms)
                        (uint32_t)d->P.pcap, (const uint64_t *)d->gp, d->t, a.far0, a.dorm, d->pcap_open, split,
                        (int32_t)check_all);
     DDP_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-    // An ordinary launch of at most one workgroup per CU (see pg_enqueue).  A
+    // An ordinary launch of at most one workgroup per CU (see pg_workgroups).  A
     // repair's rounds are a few hundred entries: 8, 16, 32 and 64 workgroups
     // took 186, 178, 186 and 208 us on the 1,000,000-node graph (20,000 lines a
     // batch) and 67, 73, 85 and 110 us on one of 100,000 nodes (200 lines).
     const int cus = ctx->prop.multiProcessorCount;
-    const int blocks = std::min(cus, !fresh ? 16 : d->P.pg_wide ? cus : kPgBlocks);
+    const int blocks = fresh ? pg_workgroups(d->P.edges, false, cus) : std::min(cus, 16);
     hipLaunchKernelGGL((ga_piles_kernel<kPgBlock, DDP_H_ARRAY, true>),
                        dim3(blocks), dim3(kPgBlock), 0, ctx->stream, a);
     DDP_HIP(ctx, hipGetLastError());

@@ -20,9 +20,9 @@ struct GaGridPlan {
     bool piles = false;
     bool bidi = false;   // piles from both ends: two (f, parent) arrays, touched logs and pile sets
     uint32_t ncap = 0, fcap = 0, delta0 = 1;  // pile mode: near ring, far buffers, first window
-    // grid mode (grid_piles.h): a graph with enough edges for a workgroup per CU, and the segments one
-    // round's long rows can be cut into
-    bool pg = false, pg_wide = false;
+    // grid mode (grid_piles.h): the graph's edges and the segments one round's long rows can be cut into
+    bool pg = false;
+    int64_t edges = 0;
     uint32_t hubcap = 0;
 };
 

@@ -79,11 +79,9 @@ PgFn pick_pg(int hk)
     }
 }
 
-// Workgroups of a grid search on piles (see kPgBlocks).
 int32_t pg_blocks(const ddp_ctx *ctx, const GaGridPlan &P, int hk)
 {
-    const int32_t cus = ctx->prop.multiProcessorCount;
-    return P.pg_wide && (hk == DDP_H_ZERO || hk == DDP_H_ARRAY) ? cus : std::min(kPgBlocks, cus);
+    return pg_workgroups(P.edges, hk == DDP_H_MANHATTAN || hk == DDP_H_EUCLID, ctx->prop.multiProcessorCount);
 }
 
 PgSizes ga_pg_sizes(const GaGridPlan &P, int32_t N) { return pg_sizes((uint64_t)P.K * P.cap, N); }
@@ -263,7 +261,7 @@ int ddp_ga_plan(ddp_ctx *ctx, const ddp_graph *g, const ddp_astar_opts_t *o, GaG
     int32_t maxit = (o && o->max_iters) ? o->max_iters : (int32_t)std::min<int64_t>(4LL * g->N + 1024, 1 << 30);
     *p = GaGridPlan{K, B, nblocks, lcap, (int32_t)cap, (int32_t)pcap, maxit};
     p->pg = true;
-    p->pg_wide = g->E >= kPgWideEdges;
+    p->edges = g->E;
     p->hubcap = (uint32_t)((int64_t)g->E / kPgSeg + kPgRound + 64);
     p->delta0 = std::max<uint32_t>(1, g->meanw);
     // K is bounded by the queues whose tops and expansion tables the device

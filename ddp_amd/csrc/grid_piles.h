@@ -56,15 +56,33 @@ constexpr int32_t kPgSeg = 64;    // edges per hub segment
 constexpr int kPgLanes = 8;       // lanes per entry
 constexpr int kPgUnroll = 2;      // edges per lane and step
 constexpr int kPgBlock = 1024;
-// Workgroups: 64 (a barrier of 1.9 us), or one per CU (2.6 us) where a round
-// scans hundreds of thousands of edges -- searches without a geometric
-// heuristic on graphs of kPgWideEdges edges and more.  Measured with 64 and
-// 256 workgroups (ms): R-MAT of 16.8M edges 3.1 and 2.0; R-MAT of 0.8M edges
-// 0.53 and 0.72; random graph of 0.6M edges 0.32 and 0.53; 1,024 x 1,024 maze
-// 12.6 and 14.3; geometric graph of 2M edges, Euclidean heuristic, 1.45 and
-// 1.79.  (64 workgroups of 256 lanes: 6.8, 0.73, 0.40, 12.5, 1.40.)
-constexpr int kPgBlocks = 64;
-constexpr int64_t kPgWideEdges = 1 << 22;
+// Workgroups: 64 (a barrier of 1.9 us); one per CU (2.6 us) where a round scans
+// hundreds of thousands of edges -- searches without a geometric heuristic on
+// graphs of kPgWideEdges edges and more; 16 (1.4 us, and a launch that starts in a
+// third of the time) below kPgSmallEdges edges.  A call in us with 16, 64 and 256
+// workgroups:
+//   random graph     6,000 edges   204   244   402     maze 64 x 64   198   235   397
+//                  300,000         342   323   483     maze 256^2   1,638 1,681 2,014
+//                  600,000         597   428   569     map, 200,000   589   619   818
+//   R-MAT          196,000         384   380   532          1,000,000 1,254 1,275 1,542
+//                  786,000         676   593   747
+// and in ms with 64, 128 and 256:
+//   random graph   4.0M edges  0.58 0.58 0.66   R-MAT  2.1M  0.50 0.52 0.60
+//                  8.0M        0.95 0.75 0.91          4.2M  1.10 1.02 1.05
+//                 10.0M        1.23 0.84 0.85          8.4M  2.04 1.52 1.50
+//                 16.0M        2.01 1.43 1.26         16.8M  3.75 2.23 1.70
+//                 32.0M        2.05 1.37 1.46         33.6M  8.09 6.86 5.77
+// A geometric heuristic keeps rounds small at any size (map of 20M edges, 64 and
+// 256 workgroups without heuristic 5.7 and 6.4).
+constexpr int kPgBlocks = 64, kPgSmallBlocks = 16;
+constexpr int64_t kPgWideEdges = 1 << 22, kPgSmallEdges = 1 << 18;
+
+// For a graph of E edges on a GPU of `cus` CUs.
+inline int32_t pg_workgroups(int64_t E, bool geometric, int32_t cus)
+{
+    const int32_t most = E >= kPgWideEdges && !geometric ? cus : E < kPgSmallEdges ? kPgSmallBlocks : kPgBlocks;
+    return most < cus ? most : cus;
+}
 // Near entries a round takes at most.  Taking the whole window at once saves
 // rounds and costs little order, which the window's width keeps: 8,192 against
 // 65,536 entries took 0.39 and 0.32 ms on the random graph (K = 1,024), 0.68
