@@ -63,13 +63,16 @@ __global__ void __launch_bounds__(B) batch_kernel(BatchArgs a)
     const PilePtrs P{home, home + a.ncap, home + a.ncap + a.fcap, a.ncap, a.fcap, s_heap, a.lring};
     ExpandCounters C;
     uint32_t stale = 0;
+    if (lane == 0) S.rc = RefillCounts{};
     for (;;) {
         if (lane == 0) s_q = (int32_t)atomicAdd(a.next, 1u);
         __syncthreads();
-        const int32_t qi = s_q;
+        // the same for every lane, and read as such: the search takes nearly all
+        // the registers that a slot's waves have
+        const int32_t qi = __builtin_amdgcn_readfirstlane(s_q);
         if (qi >= a.nq) break;
-        const int32_t q = a.order ? a.order[qi] : qi;
-        const int32_t s = a.qs[q], t = a.qt[q];
+        const int32_t q = a.order ? __builtin_amdgcn_readfirstlane(a.order[qi]) : qi;
+        const int32_t s = __builtin_amdgcn_readfirstlane(a.qs[q]), t = __builtin_amdgcn_readfirstlane(a.qt[q]);
         if (lane == 0) a.qtime[2 * (int64_t)q] = dev_clock_100mhz();
         if constexpr (ENG == ENG_BIDI) {
             // one half of the queue memory and of the LDS near ring per direction
@@ -106,9 +109,9 @@ __global__ void __launch_bounds__(B) batch_kernel(BatchArgs a)
                 a.qtime[2 * (int64_t)q + 1] = dev_clock_100mhz();
             }
         }
-        if (__ballot(C.edges >= (1u << 30))) slot_flush_stats<B>(a.stats, C, stale);  // before 32 bits wrap
+        if (__ballot(C.edges >= (1u << 30))) slot_flush_stats(a.stats, C, stale, S.rc);  // before 32 bits wrap
     }
-    slot_flush_stats<B>(a.stats, C, stale);
+    slot_flush_stats(a.stats, C, stale, S.rc);
 }
 
 __global__ void batch_fill_u64(uint64_t *p, int64_t n, uint64_t v)

@@ -70,8 +70,8 @@ __device__ __forceinline__ void set_source(HeurView &hv, int32_t s)
         hv.sy = s / hv.width;
         hv.sx = s - hv.sy * hv.width;
     } else if constexpr (HK == DDP_H_EUCLID) {
-        hv.sx = hv.xy[2 * s];
-        hv.sy = hv.xy[2 * s + 1];
+        hv.sx = __builtin_amdgcn_readfirstlane(hv.xy[2 * s]);  // one for the whole workgroup
+        hv.sy = __builtin_amdgcn_readfirstlane(hv.xy[2 * s + 1]);
     }
 }
 
@@ -90,6 +90,7 @@ struct BidiDir {
 template <int B>
 struct BidiLds {
     RowsLds<B, true> L;
+    RefillCounts rc;
     uint32_t red[16];
     unsigned long long meet;  // mu << 32 | meeting node
     uint32_t bound[2];        // L_d: lower bound of direction d's open keys (UINT32_MAX: none left)
@@ -206,7 +207,7 @@ __device__ __forceinline__ void expand_bidi(const BidiSide &D, const HeurView &H
                                             int32_t t, int32_t u, RowSpan rs, int32_t n0, const uint32_t (&F)[2],
                                             uint64_t *const (&far)[2], BidiLds<B> &S, ExpandCounters &C)
 {
-    constexpr int R = expand_unroll<B>(), W = B / 64, CAP = RowsLds<B, true>::CAP;
+    constexpr int R = expand_unroll<B, HK>(), W = B / 64, CAP = RowsLds<B, true>::CAP;
     constexpr bool kNoLoad = HK == DDP_H_ZERO || HK == DDP_H_MANHATTAN;
     const int lane = threadIdx.x, wl = lane & 63;
     const int wid = __builtin_amdgcn_readfirstlane(lane >> 6);
@@ -567,7 +568,7 @@ __device__ __forceinline__ void bidi_refill(const BidiSide &D, int32_t oroot, bo
         if (lane == 0) {
             Q.far_n = Q.far_n2;
             Q.ovf = 0;
-            C.rebuilds++;
+            S.rc.rebuilds++;
         }
         uint64_t *tmp = far[d];
         far[d] = far2[d];
@@ -576,8 +577,10 @@ __device__ __forceinline__ void bidi_refill(const BidiSide &D, int32_t oroot, bo
         if (S.err) return;
     }
     const uint32_t nf = Q.far_n < P.fcap ? Q.far_n : P.fcap;
-    if (lane == 0) C.refills++;
-    C.scanned += 2 * ((nf > (uint32_t)lane) ? (nf - 1 - lane) / B + 1 : 0);
+    if (lane == 0) {
+        S.rc.refills++;
+        S.rc.scanned += 2 * (uint64_t)nf;
+    }
     constexpr int KC = 2;
     uint64_t *fp = far[d];
     auto load_chunk = [&](uint32_t base, uint64_t (&k)[KC], bool (&live)[KC]) {

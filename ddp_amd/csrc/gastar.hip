@@ -121,6 +121,7 @@ __global__ void __launch_bounds__(B) ga_wg_kernel(WgArgs a)
     const LaneHeap H{s_heap + lane, a.home + lane, B, a.lcap, (int64_t)B, a.cap};
     ExpandCounters C;
     uint32_t stale = 0;
+    if (lane == 0) S.rc = RefillCounts{};
     if constexpr (WM == WM_BIDI) {
         const int32_t N = a.N;
         uint64_t *bh = a.home + (int64_t)a.cap * B;
@@ -153,7 +154,7 @@ __global__ void __launch_bounds__(B) ga_wg_kernel(WgArgs a)
             a.ctrl[GA_RES_ERR] = ((e & QERR_HEAP) ? ERR_HEAP : 0u) | ((e & QERR_ITERS) ? ERR_ITERS : 0u);
         }
     }
-    slot_flush_stats<B>(a.stats, C, stale);
+    slot_flush_stats(a.stats, C, stale, S.rc);
 }
 
 using WgFn = void (*)(WgArgs);

@@ -26,11 +26,15 @@
 
 // Edges handled per lane and trip (memory requests a lane keeps in flight
 // per stage).  At 1,024 lanes two, three, four and six took 80, 78, 73 and 73
-// ms a query on R-MAT (scale 20) and 16.1, 16.2, 16.2 and 16.7 ms for C4.
-template <int B>
+// ms a query on R-MAT (scale 20) and 16.1, 16.2, 16.2 and 16.7 ms for C4: three
+// with the Euclidean heuristic, whose kernels run out of registers with four
+// (20 bytes of scratch in the batch kernel).  At 512 lanes two: four take R-MAT
+// bursts on a server 7% further, but the kernels past the 128 registers that let
+// two workgroups share a CU.
+template <int B, int HK = DDP_H_ZERO>
 constexpr int expand_unroll()
 {
-    return B == 512 ? 2 : 4;
+    return B == 512 ? 2 : B == 1024 && HK == DDP_H_EUCLID ? 3 : 4;
 }
 
 // Rows of a round and its collected edges (expand_rows; COLLECT, else none).
@@ -68,13 +72,13 @@ __device__ __forceinline__ RowSpan row_span(const GraphView &G, const HeurView &
 
 // Per-lane statistics, 32-bit to spare registers.  Kernels add them to the
 // 64-bit device totals at exit, and slot kernels also whenever a wave's
-// edge count passes 2^30 (no counter grows faster than the edge count,
-// except rebuilds/refills/scanned, which lane 0 counts once per refill).
+// edge count passes 2^30 (no counter of theirs grows faster).
 struct ExpandCounters {
     uint32_t expanded = 0, edges = 0, improved = 0;
-    uint32_t rebuilds = 0;  // pile engine: far piles rebuilt after an overflow (lane 0 counts)
-    uint32_t refills = 0;   // pile engine: near-ring refills from the far pile (lane 0 counts)
-    uint32_t scanned = 0;   // pile engine: far-pile entries read by refills
+    // grid searches (slots count these in LDS, RefillCounts):
+    uint32_t rebuilds = 0;  // piles rebuilt after an overflow (lane 0 counts)
+    uint32_t refills = 0;   // splits of the far pile (lane 0 counts)
+    uint32_t scanned = 0;   // far-pile entries read by them
 };
 
 // A round's rows: edges and rows in all, and (in every 16 lanes) up to and with
@@ -318,7 +322,7 @@ __device__ __forceinline__ void expand_rows(const GraphView &G, const HeurView &
                                             int32_t u, const RowSpan &rs, RowsLds<B, Push::kCollect> &L,
                                             ExpandCounters &C, Push &push, uint32_t Fb = 0xFFFFFFFFu)
 {
-    constexpr int R = expand_unroll<B>(), W = B / 64;
+    constexpr int R = expand_unroll<B, HK>(), W = B / 64;
     constexpr bool kNoLoad = HK == DDP_H_ZERO || HK == DDP_H_MANHATTAN;
     const int lane = threadIdx.x, wl = lane & 63;
     const int wid = __builtin_amdgcn_readfirstlane(lane >> 6);

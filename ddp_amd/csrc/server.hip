@@ -424,6 +424,7 @@ __global__ void __launch_bounds__(B) serve_kernel(ServeArgs a)
     __shared__ int32_t s_have;
     __shared__ uint32_t s_uerr;
     __shared__ Req s_req;
+    __shared__ uint64_t s_start;
     const int lane = threadIdx.x;
     const int64_t slot = blockIdx.x;
     const int32_t N = a.N;
@@ -435,6 +436,7 @@ __global__ void __launch_bounds__(B) serve_kernel(ServeArgs a)
     const PilePtrs P{home, home + a.ncap, home + a.ncap + a.fcap, a.ncap, a.fcap, s_heap, a.lring};
     ExpandCounters C;
     uint32_t stale = 0;
+    if (lane == 0) S.rc = RefillCounts{};
     uint32_t seen = 0;  // newest version whose graph data this workgroup has acquired
     bool any_seen = false;
     for (;;) {
@@ -448,16 +450,21 @@ __global__ void __launch_bounds__(B) serve_kernel(ServeArgs a)
             }
         }
         __syncthreads();
-        const uint32_t ticket = s_ticket;
         if (!s_have) {  // the launch is closing: the host looks at its event from now on
             if (lane == 0) __hip_atomic_store(a.left, a.gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             break;
         }
-        const Req rq = s_req;
-        const uint64_t tstart = dev_clock_100mhz();
+        // What the search does not need stays in LDS (the request, its ticket and
+        // start), and what is the same for every lane is read as such: the
+        // search takes nearly all the registers that a slot's waves have.
+        const Req &rq = s_req;
+        const bool update = __builtin_amdgcn_readfirstlane(rq.type) == DDP_REQ_UPDATE;
+        const int32_t version = __builtin_amdgcn_readfirstlane(rq.version);
         // ---- wait for the graph version this request needs (bounded)
-        const uint32_t need = rq.type == DDP_REQ_UPDATE ? (uint32_t)rq.version - 1 : (uint32_t)rq.version;
+        const uint32_t need = (uint32_t)version - (update ? 1u : 0u);
         if (lane == 0) {
+            const uint64_t tstart = dev_clock_100mhz();
+            s_start = tstart;
             while (ld_u32(a.ctrl + CT_APPLIED) < need) {
                 if (dev_clock_100mhz() - tstart > a.wait_ticks) {
                     s_uerr = SERR_WAIT;
@@ -474,62 +481,65 @@ __global__ void __launch_bounds__(B) serve_kernel(ServeArgs a)
         // A query reads graph data through its CU's L1: one wave acquires the
         // applied version for the workgroup, unless an earlier query of this
         // slot needed as new a one.  (apply_update reads past L1.)
-        if (rq.type != DDP_REQ_UPDATE && (!any_seen || need > seen)) {
+        if (!update && (!any_seen || need > seen)) {
             if (threadIdx.x < 64)
                 (void)__hip_atomic_load(a.ctrl + CT_APPLIED, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
             __syncthreads();
             seen = need;
             any_seen = true;
         }
-        int32_t cost = DDP_INF_COST;
-        uint32_t status = s_uerr;
-        if (rq.type == DDP_REQ_UPDATE) {
-            if (!status) apply_update<B, ENG == SENG_BIDI>(a, rq, &s_uerr);
+        const uint32_t uerr = __builtin_amdgcn_readfirstlane(s_uerr);
+        if (update) {
+            if (!uerr) apply_update<B, ENG == SENG_BIDI>(a, rq, &s_uerr);
             __syncthreads();
-            status = s_uerr;
             if (lane == 0) {
-                if (status) atomicOr(a.ctrl + CT_ERR, status);
+                if (s_uerr) atomicOr(a.ctrl + CT_ERR, s_uerr);
                 wait_vmem();  // every wave's writes are in place: apply_update ended with such a wait and a barrier
                 // published even after a failure (later requests then report the
                 // sticky error instead of stalling); atomicMax keeps it from
                 // moving backwards when an earlier version finishes late
-                atomicMax(a.ctrl + CT_APPLIED, (uint32_t)rq.version);
+                atomicMax(a.ctrl + CT_APPLIED, (uint32_t)version);
             }
-        } else if (!status) {
+        } else if (!uerr) {
             GraphView G = a.g;
-            G.ver = rq.version;
-            G.relax_min = a.g.relax_min && rq.relax_min;
+            G.ver = version;
+            G.relax_min = a.g.relax_min && __builtin_amdgcn_readfirstlane(rq.relax_min);
+            const int32_t s = __builtin_amdgcn_readfirstlane(rq.s), t = __builtin_amdgcn_readfirstlane(rq.t);
             if constexpr (ENG == SENG_BIDI) {
                 uint64_t *bh = home + (int64_t)a.cap * B;
                 const PilePtrs PF{home, home + a.ncap, home + a.ncap + a.fcap, a.ncap, a.fcap, s_heap, a.lring / 2};
                 const PilePtrs PB{bh, bh + a.ncap, bh + a.ncap + a.fcap, a.ncap, a.fcap, s_heap + a.lring / 2,
                                   a.lring / 2};
                 const BidiSide D{{a.g.off, a.gr.off},  {a.g.col, a.gr.col}, {a.g.w, a.gr.w},     {gp, gp + N},
-                                 {touched, touched + N}, {PF, PB},          {a.dver, a.rdver}, rq.version,
+                                 {touched, touched + N}, {PF, PB},          {a.dver, a.rdver}, version,
                                  {a.lhead, a.rlhead},  {a.lnext, a.rlnext}, {a.lv, a.lu},       a.lw,
                                  a.ldel};
-                slot_search_bidi<B, HK, true>(D, a.h, G.relax_min != 0, N, rq.s, rq.t, a.maxit, a.delta0, S, C,
+                slot_search_bidi<B, HK, true>(D, a.h, G.relax_min != 0, N, s, t, a.maxit, a.delta0, S, C,
                                               stale);
-                cost = (int32_t)(uint32_t)(S.meet >> 32);
-                status = S.err;
                 slot_reset_bidi(gp, gp + N, touched, touched + N, S);
             } else {
                 if constexpr (ENG == SENG_PILES)
-                    slot_search_piles<B, HK>(G, a.h, gp, touched, P, N, rq.s, rq.t, a.maxit, a.delta0, S, C, stale);
+                    slot_search_piles<B, HK>(G, a.h, gp, touched, P, N, s, t, a.maxit, a.delta0, S, C, stale);
                 else
-                    slot_search<B, HK>(G, a.h, gp, touched, H, s_heap, N, rq.s, rq.t, a.maxit, S, C, stale);
-                cost = (int32_t)S.F;
-                status = S.err;
+                    slot_search<B, HK>(G, a.h, gp, touched, H, s_heap, N, s, t, a.maxit, S, C, stale);
                 slot_reset(gp, touched, S);
             }
-            if (__ballot(C.edges >= (1u << 30))) slot_flush_stats<B>(a.stats, C, stale);  // before 32 bits wrap
+            if (__ballot(C.edges >= (1u << 30))) slot_flush_stats(a.stats, C, stale, S.rc);  // before 32 bits wrap
         }
         if (lane == 0) {
+            const uint32_t ticket = s_ticket;
+            int32_t cost = DDP_INF_COST;
+            uint32_t status = s_uerr;
+            if (!update && !uerr) {
+                if constexpr (ENG == SENG_BIDI) cost = (int32_t)(uint32_t)(S.meet >> 32);
+                else cost = (int32_t)S.F;
+                status = S.err;
+            }
             Res *r = a.res + (ticket & a.ring_mask);
             __hip_atomic_store(&r->cost, cost, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             __hip_atomic_store(&r->status, (int32_t)status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             __hip_atomic_store(&r->version, rq.version, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            __hip_atomic_store(&r->t0, tstart, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(&r->t0, s_start, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             __hip_atomic_store(&r->t1, dev_clock_100mhz(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             // the stores above go straight to host memory: waiting for them
             // orders the sequence word after them, where a system-scope release
@@ -540,7 +550,7 @@ __global__ void __launch_bounds__(B) serve_kernel(ServeArgs a)
         }
         __syncthreads();
     }
-    slot_flush_stats<B>(a.stats, C, stale);
+    slot_flush_stats(a.stats, C, stale, S.rc);
 }
 
 // Before a launch: the last one's closing is undone, and the counts move past

@@ -10,9 +10,16 @@
 
 enum : uint32_t { QERR_HEAP = 1, QERR_ITERS = 2, QERR_BADQ = 4, QERR_PATH = 8 };
 
+// What refills count (lane 0 alone, for the launch); in LDS, as the search takes
+// nearly all the registers that its waves have.
+struct RefillCounts {
+    uint64_t rebuilds, refills, scanned;  // far piles rebuilt, refills, far entries they read
+};
+
 template <int B, bool COLLECT>
 struct SlotLds {
     RowsLds<B, COLLECT> L;
+    RefillCounts rc;
     uint32_t red[16];
     uint32_t F;        // best f of the target so far
     uint32_t err;
@@ -72,8 +79,8 @@ __device__ __forceinline__ void set_target(HeurView &hv, int32_t t)
         hv.ty = t / hv.width;
         hv.tx = t - hv.ty * hv.width;
     } else if constexpr (HK == DDP_H_EUCLID) {
-        hv.tx = hv.xy[2 * t];
-        hv.ty = hv.xy[2 * t + 1];
+        hv.tx = __builtin_amdgcn_readfirstlane(hv.xy[2 * t]);  // one for the whole workgroup
+        hv.ty = __builtin_amdgcn_readfirstlane(hv.xy[2 * t + 1]);
     }
 }
 
@@ -402,12 +409,12 @@ __device__ void slot_search_piles(const GraphView &G, HeurView hv, uint64_t *gp,
     uint32_t lh = 0, hh = 0;  // ring heads (uniform)
     int32_t it = 0;
     while (run) {
-        const uint32_t lt = S.lring_tail, F = S.F;
+        const uint32_t lt = __builtin_amdgcn_readfirstlane(S.lring_tail), F = __builtin_amdgcn_readfirstlane(S.F);
         bool from_lds = lt != lh;
         uint32_t avail = lt - lh;
         if (!from_lds) {
             block_sync_global();  // HBM entries ahead: every wave's stores have landed
-            avail = S.near_tail - hh;
+            avail = __builtin_amdgcn_readfirstlane(S.near_tail) - hh;
         }
         // Early refill: a near ring this thin holds stragglers of the window
         // while the far pile waits; move the next window in beside them.
@@ -439,7 +446,7 @@ __device__ void slot_search_piles(const GraphView &G, HeurView hv, uint64_t *gp,
                 if (lane == 0) {
                     S.far_n = S.far_n2;
                     S.ovf = 0;
-                    C.rebuilds++;
+                    S.rc.rebuilds++;
                 }
                 uint64_t *tmp = far;
                 far = far2;
@@ -448,9 +455,11 @@ __device__ void slot_search_piles(const GraphView &G, HeurView hv, uint64_t *gp,
                 if (S.err) break;
             }
             // ---- refill the near rings from the far pile
-            const uint32_t nf = S.far_n < P.fcap ? S.far_n : P.fcap;
-            if (lane == 0) C.refills++;
-            C.scanned += 2 * ((nf > (uint32_t)lane) ? (nf - 1 - lane) / B + 1 : 0);
+            const uint32_t far_n = __builtin_amdgcn_readfirstlane(S.far_n), nf = far_n < P.fcap ? far_n : P.fcap;
+            if (lane == 0) {
+                S.rc.refills++;
+                S.rc.scanned += 2 * (uint64_t)nf;
+            }
             // The far pile is read in chunks of KC*B entries, each chunk's
             // loads issued together (entries, then their (f, parent) words),
             // once for the minimum and again for the split.  (Keeping the
@@ -629,20 +638,24 @@ __device__ void slot_reset(uint64_t *gp, const int32_t *touched, SlotLds<B, COLL
     block_sync_global();
 }
 
-template <int B>
-__device__ void slot_flush_stats(unsigned long long *stats, ExpandCounters &C, uint32_t &stale)
+// Adds a wave's counts, and with the first wave what refills counted (rc, zero
+// when the kernel starts), to the launch's.
+__device__ __forceinline__ void slot_flush_stats(unsigned long long *stats, ExpandCounters &C, uint32_t &stale,
+                                                 RefillCounts &rc)
 {
     const uint64_t v0 = wave_sum_u64(C.expanded), v1 = wave_sum_u64(C.edges), v2 = wave_sum_u64(C.improved),
-                   v3 = wave_sum_u64(stale), v4 = wave_sum_u64(C.rebuilds), v5 = wave_sum_u64(C.refills),
-                   v6 = wave_sum_u64(C.scanned);
+                   v3 = wave_sum_u64(stale);
     if ((threadIdx.x & 63) == 0) {
         atomicAdd(stats + 0, (unsigned long long)v0);
         atomicAdd(stats + 1, (unsigned long long)v1);
         atomicAdd(stats + 2, (unsigned long long)v2);
         atomicAdd(stats + 3, (unsigned long long)v3);
-        if (v4) atomicAdd(stats + 4, (unsigned long long)v4);
-        if (v5) atomicAdd(stats + 5, (unsigned long long)v5);
-        if (v6) atomicAdd(stats + 6, (unsigned long long)v6);
+    }
+    if (threadIdx.x == 0) {
+        if (rc.rebuilds) atomicAdd(stats + 4, (unsigned long long)rc.rebuilds);
+        if (rc.refills) atomicAdd(stats + 5, (unsigned long long)rc.refills);
+        if (rc.scanned) atomicAdd(stats + 6, (unsigned long long)rc.scanned);
+        rc = RefillCounts{};
     }
     C = ExpandCounters{};
     stale = 0;
