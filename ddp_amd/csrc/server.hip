@@ -297,7 +297,12 @@ __device__ void apply_update(const ServeArgs &a, const Req &rq, uint32_t *s_err)
 // burst, on the same memory: with four words read by whole waves and an atomic
 // on the lease per look (one takes 11 ns), a Dijkstra-order search on R-MAT
 // scale 15 took 252 ms beside 1,023 idle slots of 128 lanes (lane heaps) and
-// 14.1 beside 15; 512 such requests at scale 14 took 148 ms, now 14.
+// 14.1 beside 15; 512 such requests at scale 14 took 148 ms, now 14.  And only as
+// many of them take note of new entries as these could need, and try to claim
+// at a pace that the count can serve: with every idle slot at each new entry
+// (41 attempts a claim) 16,384 requests on a 200,000-node map, 512 slots of 512
+// lanes, took 34 ms and a few searches four times as long as alone; now 19 ms, and
+// none does.
 __device__ __forceinline__ bool serve_claim(const ServeArgs &a, uint32_t &ticket, Req *req)
 {
     const uint32_t lane = threadIdx.x;
@@ -306,7 +311,6 @@ __device__ __forceinline__ bool serve_claim(const ServeArgs &a, uint32_t &ticket
     const uint64_t t0 = dev_clock_100mhz();
     bool poller = false, have = false;
     uint32_t backoff = 0;  // idle non-pollers back off to ~15 us
-    uint32_t contended = 0;
     for (;;) {
         // one look at every word, a lane each
         const uint32_t at = lane == 0 ? CT_HEAD : lane < 5 ? CT_TAIL - 1 + lane : lane == 5 ? CT_APPLIED : CT_BUSY;
@@ -316,8 +320,9 @@ __device__ __forceinline__ bool serve_claim(const ServeArgs &a, uint32_t &ticket
         const uint32_t stop = __builtin_amdgcn_readlane(word, 2), lease = __builtin_amdgcn_readlane(word, 3);
         const uint32_t applied = __builtin_amdgcn_readlane(word, 5), bw = __builtin_amdgcn_readlane(word, 6);
         if (bw & kClosed) break;
-        const bool waiting = (int32_t)(tail - h) > 0;
-        if (waiting) {
+        const uint32_t waits = (int32_t)(tail - h) > 0 ? tail - h : 0;  // entries to be claimed
+        bool unready = false;                                           // the next one needs a version
+        if (waits) {
             // a stale h reads an entry that its failed claim below ignores
             uint32_t e = 0;
             if (lane < sizeof(Req) / 4) e = ld_u32((const uint32_t *)(a.mirror + (h & a.ring_mask)) + lane);
@@ -342,13 +347,19 @@ __device__ __forceinline__ bool serve_claim(const ServeArgs &a, uint32_t &ticket
                     have = true;
                     break;
                 }
-                // A burst has every idle slot here, and the counter serves one
-                // attempt per 11 ns or so: waits that double with each failure,
-                // spread over the slots, keep it from serving only failures.
-                contended = contended < 7 ? contended + 1 : 7;
-                const uint32_t spread = (blockIdx.x * 2654435761u + h * 40503u) >> 25 & ((1u << contended) - 1);
-                for (uint32_t k = 0; k < spread; ++k) __builtin_amdgcn_s_sleep(1);
-                continue;
+                // Another slot was first.  The count moves on once a round trip
+                // (about 1 us) whoever tries, so idle slots try again some time
+                // within 0.4 us each (four attempts a round trip or so), and slots
+                // that the entries do not go round to wait like idle ones.
+                const uint32_t busy = bw & ~kClosed, idle = gridDim.x > busy ? gridDim.x - busy : 1;
+                const uint32_t mix = (blockIdx.x * 2654435761u + h * 40503u) >> 16;
+                if (poller || mix % idle < 4 * waits) {
+                    const uint32_t most = poller ? 16 : idle < 512 ? 16 * idle : 8192;
+                    for (uint32_t k = mix % most; k > 0; --k) __builtin_amdgcn_s_sleep(1);
+                    continue;
+                }
+            } else {
+                unready = true;
             }
         }
         if ((int32_t)(stop - a.gen) >= 0) break;
@@ -393,7 +404,7 @@ __device__ __forceinline__ bool serve_claim(const ServeArgs &a, uint32_t &ticket
                 if ((int32_t)(sg - a.gen) >= 0 && lane == 0) atomicExch(a.ctrl + CT_STOP, sg);
                 __builtin_amdgcn_s_sleep(16);
             }
-        } else if (waiting) {
+        } else if (unready) {
             // for a version, which comes within tens of microseconds: 1.7 us
             // between looks (0.2 us kept the words they look at so busy that the
             // update itself took twice as long), longer where more slots look
@@ -404,7 +415,11 @@ __device__ __forceinline__ bool serve_claim(const ServeArgs &a, uint32_t &ticket
                 for (uint32_t k = 0; k < backoff; ++k) __builtin_amdgcn_s_sleep(64);
                 uint32_t line = 0;
                 if (lane < 4) line = ld_u32(a.ctrl + CT_TAIL + lane);
-                if (__builtin_amdgcn_readlane(line, 0) != tail || __builtin_amdgcn_readlane(line, 2) == 0 ||
+                // as many slots take note of new entries as these could need,
+                // and more the longer the entries wait
+                const uint32_t fresh = __builtin_amdgcn_readlane(line, 0) - tail;
+                const uint32_t mix = (blockIdx.x * 2654435761u + (fresh + quiet) * 40503u) >> 16;
+                if ((fresh != 0 && mix % gridDim.x < 4 * fresh) || __builtin_amdgcn_readlane(line, 2) == 0 ||
                     (int32_t)(__builtin_amdgcn_readlane(line, 1) - a.gen) >= 0 ||
                     __builtin_amdgcn_readlane(line, 3) == a.gen)
                     break;
