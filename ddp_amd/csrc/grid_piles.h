@@ -66,6 +66,7 @@ constexpr int kPgBlock = 1024;
 //                  600,000         597   428   569     map, 200,000   589   619   818
 //   R-MAT          196,000         384   380   532          1,000,000 1,254 1,275 1,542
 //                  786,000         676   593   747
+// (of a server's versioned view, with its insert lists, R-MAT of 196,000: 404 and 368)
 // and in ms with 64, 128 and 256:
 //   random graph   4.0M edges  0.58 0.58 0.66   R-MAT  2.1M  0.50 0.52 0.60
 //                  8.0M        0.95 0.75 0.91          4.2M  1.10 1.02 1.05
@@ -75,7 +76,7 @@ constexpr int kPgBlock = 1024;
 // A geometric heuristic keeps rounds small at any size (map of 20M edges, 64 and
 // 256 workgroups without heuristic 5.7 and 6.4).
 constexpr int kPgBlocks = 64, kPgSmallBlocks = 16;
-constexpr int64_t kPgWideEdges = 1 << 22, kPgSmallEdges = 1 << 18;
+constexpr int64_t kPgWideEdges = 1 << 22, kPgSmallEdges = 1 << 17;
 
 // For a graph of E edges on a GPU of `cus` CUs.
 inline int32_t pg_workgroups(int64_t E, bool geometric, int32_t cus)

@@ -25,7 +25,7 @@ def test_maze_rounds(ctx, side, seed, K):
     dg.close()
 
 
-@pytest.mark.parametrize("n,deg,blocks", [(1000, 6, 16), (65535, 4, 16), (65537, 4, 64)])
+@pytest.mark.parametrize("n,deg,blocks", [(1000, 6, 16), (32767, 4, 16), (32769, 4, 64)])
 def test_small_graphs_on_few_workgroups(ctx, n, deg, blocks):
     hg = ddp_amd.HostGraph.random(n, deg, 1, 100, n)
     src, dst = hg.reachable_pairs(1, n)
