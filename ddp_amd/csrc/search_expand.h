@@ -37,11 +37,23 @@ constexpr int expand_unroll()
     return B == 512 ? 2 : B == 1024 && HK == DDP_H_EUCLID ? 3 : 4;
 }
 
+// Collected edges a lane relaxes at once (atomics it keeps in flight).  Where most
+// edges improve (a random graph with an h array) a narrow workgroup waits for
+// one atomic round trip per 64: a search of 600,000 nodes took 36.9, 18.2, 10.9 and
+// 8.2 ms with 64, 128, 256 and 512 lanes at one a lane, 32.5, 16.3, 9.9 and 7.7 at two
+// (31.3, 15.7, 9.8 and - at four, which takes a map's batch from 4.1 to 4.3 ms).  The
+// 1,024-lane kernels have no registers for a second one.
+template <int B>
+constexpr int relax_unroll()
+{
+    return B <= 512 ? 2 : 1;
+}
+
 // Rows of a round and its collected edges (expand_rows; COLLECT, else none).
 // Only rows that have edges are listed, so incl ascends strictly.
 template <int B, bool COLLECT>
 struct RowsLds {
-    static constexpr int CAP = COLLECT ? 64 * expand_unroll<B>() + 64 : 1;  // collected edges of a wave
+    static constexpr int CAP = COLLECT ? 64 * (expand_unroll<B>() + relax_unroll<B>()) : 1;  // collected edges of a wave
     int32_t incl[B];        // inclusive prefix of degrees
     int32_t rowb[B];        // row start - edges before the row
     uint32_t gu[B];         // g(u) = f(u) - h(u), unsigned as GA_v2.cu:137
@@ -155,36 +167,45 @@ __device__ __forceinline__ int32_t wave_rows(const RowsLds<B, COLLECT> &L, int32
     return r0 + (int32_t)lane_rank(m) + (int32_t)(m >> wl & 1);
 }
 
-// Relaxes one candidate per lane (key: f << 32 | node, of a node at which it
-// can improve the word) and hands the improvements to the push policy.  Every
+// Relaxes Q candidates per lane (key: f << 32 | node, of a node at which it can
+// improve the word) and hands the improvements to the push policy.  Every
 // lane of the wave calls it.
-template <class Push>
-__device__ __forceinline__ void relax_collected(const GraphView &G, uint64_t *gp, int32_t t, bool have, uint64_t key,
-                                                int32_t par, ExpandCounters &C, Push &push)
+template <int Q, class Push>
+__device__ __forceinline__ void relax_collected(const GraphView &G, uint64_t *gp, int32_t t, const bool (&have)[Q],
+                                                const uint64_t (&key)[Q], const int32_t (&par)[Q], ExpandCounters &C,
+                                                Push &push)
 {
-    const uint32_t cand = (uint32_t)(key >> 32);
-    const int32_t c[1] = {(int32_t)(uint32_t)key};
-    bool ok = false;
-    uint64_t prev = 0;
+    int32_t c[Q];
+    bool ok[Q], first[Q], has[Q];
+    uint64_t prev[Q];
     if (G.relax_min != 0) {  // uniform
         // one atomicMin: the smallest (f, parent) of the round wins with no
         // retry round trips
-        if (have) {
-            prev = (uint64_t)atomicMin((unsigned long long *)(gp + c[0]),
-                                       ((unsigned long long)cand << 32) | (uint32_t)par);
-            ok = (uint32_t)(prev >> 32) > cand;
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+            if (have[q])
+                prev[q] = (uint64_t)atomicMin((unsigned long long *)(gp + (uint32_t)key[q]),
+                                              (key[q] & 0xFFFFFFFF00000000ull) | (uint32_t)par[q]);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) ok[q] = have[q] && (uint32_t)(prev[q] >> 32) > (uint32_t)(key[q] >> 32);
+    } else {
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+            ok[q] = have[q] &&
+                    relax_gp(gp, (int32_t)(uint32_t)key[q], (uint32_t)(key[q] >> 32), (uint32_t)par[q], &prev[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        c[q] = (int32_t)(uint32_t)key[q];
+        if (ok[q]) {
+            C.improved++;
+            if (c[q] == t) push.target((uint32_t)(key[q] >> 32));
         }
-    } else if (have) {
-        ok = relax_gp(gp, c[0], cand, (uint32_t)par, &prev);
+        first[q] = ok[q] && (uint32_t)(prev[q] >> 32) == DDP_INF_F;
+        has[q] = ok[q] && c[q] != t;
     }
-    if (ok) {
-        C.improved++;
-        if (c[0] == t) push.target(cand);
-    }
-    const bool first[1] = {ok && (uint32_t)(prev >> 32) == DDP_INF_F}, has[1] = {ok && c[0] != t};
-    const uint64_t k[1] = {key};
-    push.template touch_all<1>(first, c);
-    push.template all<1>(has, k);
+    push.template touch_all<Q>(first, c);
+    push.template all<Q>(has, key);
 }
 
 // Relaxes R edges per lane (grid engine, lane heaps): edge r leads to c[r] (< 0:
@@ -322,7 +343,7 @@ __device__ __forceinline__ void expand_rows(const GraphView &G, const HeurView &
                                             int32_t u, const RowSpan &rs, RowsLds<B, Push::kCollect> &L,
                                             ExpandCounters &C, Push &push, uint32_t Fb = 0xFFFFFFFFu)
 {
-    constexpr int R = expand_unroll<B, HK>(), W = B / 64;
+    constexpr int R = expand_unroll<B, HK>(), Q = relax_unroll<B>(), W = B / 64;
     constexpr bool kNoLoad = HK == DDP_H_ZERO || HK == DDP_H_MANHATTAN;
     const int lane = threadIdx.x, wl = lane & 63;
     const int wid = __builtin_amdgcn_readfirstlane(lane >> 6);
@@ -422,7 +443,10 @@ __device__ __forceinline__ void expand_rows(const GraphView &G, const HeurView &
             }
             we += STEP * R;
             if (total <= B) {  // at most one edge per lane: nothing to collect
-                relax_collected(G, gp, t, tried[0], key[0], tried[0] ? L.node[jj[0]] : 0, C, push);
+                const bool one[1] = {tried[0]};
+                const uint64_t key1[1] = {key[0]};
+                const int32_t par1[1] = {tried[0] ? L.node[jj[0]] : 0};
+                relax_collected<1>(G, gp, t, one, key1, par1, C, push);
                 break;
             }
 #pragma unroll
@@ -435,15 +459,22 @@ __device__ __forceinline__ void expand_rows(const GraphView &G, const HeurView &
                 }
                 cn += (int32_t)__popcll(m);
             }
-            while (cn >= 64 || (cn > 0 && we >= wend)) {  // the last ones first, so the rest stays where it is
-                const int32_t n = cn < 64 ? cn : 64, at = cn - n + wl;
-                uint64_t k = 0;
-                int32_t par = 0;
-                if (wl < n) {
-                    k = ck[at];
-                    par = L.node[cr[at]];
+            while (cn >= 64 * Q || (cn > 0 && we >= wend)) {  // the last ones first, so the rest stays where it is
+                const int32_t n = cn < 64 * Q ? cn : 64 * Q, at = cn - n + wl;
+                bool have[Q];
+                uint64_t k[Q];
+                int32_t par[Q];
+#pragma unroll
+                for (int q = 0; q < Q; ++q) {
+                    have[q] = 64 * q + wl < n;
+                    k[q] = 0;
+                    par[q] = 0;
+                    if (have[q]) {
+                        k[q] = ck[at + 64 * q];
+                        par[q] = L.node[cr[at + 64 * q]];
+                    }
                 }
-                relax_collected(G, gp, t, wl < n, k, par, C, push);
+                relax_collected<Q>(G, gp, t, have, k, par, C, push);
                 cn -= n;
             }
         }
