@@ -285,8 +285,10 @@ __device__ __forceinline__ void claim_children(const GraphView &G, const InsLog 
 // workgroup to arrive reads *cnt -- every workgroup's draws of the level are
 // in by then -- and publishes it with the new generation, so each workgroup
 // learns the level's total without racing the next level's draws.  No fences
-// (see grid_sync): the walk shares its list, the marks and the counters
-// through agent-scope accesses.  Waits are bounded by limit_ticks of the
+// (see grid_sync): the walk shares its list and the counters through
+// agent-scope accesses.  The marks it stores plainly: a child is claimed by its
+// one parent's lane only, so no other workgroup acts on a mark that this launch
+// stores, and the roots' were set by the launch before.  Waits are bounded by limit_ticks of the
 // 100 MHz clock (false on timeout).
 __device__ __forceinline__ bool walk_barrier(uint32_t *bar, uint32_t nblocks, uint32_t &gen, const uint32_t *cnt,
                                              uint64_t limit_ticks, int32_t *s_flag, uint32_t *s_total)

@@ -12,7 +12,7 @@ enum : int {
 };
 
 // Error bits of GA_RES_ERR.
-enum : uint32_t { GA_ERR_HEAP = 1, GA_ERR_PBUF = 2, GA_ERR_ITERS = 4, GA_ERR_BARRIER = 8 };
+enum : uint32_t { GA_ERR_HEAP = 1, GA_ERR_ITERS = 4, GA_ERR_BARRIER = 8 };
 
 struct GaGridPlan {
     int32_t K, B, nblocks, lcap, cap, pcap, maxit;
@@ -37,7 +37,7 @@ struct GaGridState {
     bool owned = false;          // allocated by ddp_ga_alloc_owned (freed by ddp_ga_free)
 };
 
-// min_pcap: lower bound on pcap (DA* sizes its repairs' pushes by it).
+// min_pcap: lower bound on pcap, the room for a DA* batch's repair pushes.
 // allow_wg: honour opts->mode and plan the workgroup mode when it applies.
 int ddp_ga_plan(ddp_ctx *ctx, const ddp_graph *g, const ddp_astar_opts_t *o, GaGridPlan *p,
                 int64_t min_pcap = 0, bool allow_wg = false);

@@ -1,29 +1,20 @@
-// Single-query GA*.  Fresh grid-mode searches run on piles over the whole GPU
-// (grid_piles.h); the K priority queues over one persistent grid below are
-// what DA* resumes in grid mode; workgroup mode keeps all queues inside one
-// workgroup (further down).
+// Single-query GA*: planning, state and entry point.  Grid mode runs on piles over
+// the whole GPU (grid_piles.h); the other modes keep the search in one workgroup
+// (below): K lane heaps, piles (slot_search.h) or piles from both ends
+// (bidi_search.h).
 //
 // Reference loop (GA_star/GA_v2.cu:488-559): per iteration the host launches
 // extractMin, A_star_expand, keepHeapPQ, setNV (an O(N) flag scan), insertPQ,
 // copies flags and all K queue sizes back, and runs checkMIN.  Here the whole
-// loop is one kernel:
-//   * queue q is a binary heap owned by one lane (lane q % B of workgroup
-//     q / B); its first lcap entries sit in LDS, the rest spill to HBM;
-//   * each iteration every queue pops its best valid entry, the workgroup
-//     expands the popped nodes cooperatively (search_expand.h), and every
-//     improvement CASes a packed (f << 32 | parent) word -- no per-node locks;
-//   * improved nodes are appended to a push buffer with one atomic per wave
-//     (ballot + mbcnt), replacing setNV's O(N) scan; after the grid barrier
-//     queue q takes entries p with (rr + p) % K == q, the round-robin
-//     distribution of insertPQ (GA_v2.cu:241-273) made continuous across
-//     iterations so queue sizes stay balanced;
-//   * termination is decided on the device: once the target's f is <= the
-//     smallest queue top at the previous iteration's start and every f pushed
-//     during it, no open node can improve it (GA_v2.cu:277-289, 547-557).
-//     The decision reads only values frozen by the barrier, so all workgroups
-//     agree without another barrier.
-// Stale heap entries (a node improved after it was queued) are skipped when
-// popped; this replaces keepHeapPQ's in-place decrease-key repair.
+// loop is one kernel in every mode:
+//   * an iteration expands its nodes cooperatively, and every improvement goes
+//     into a packed (f << 32 | parent) word by one atomic -- no per-node locks;
+//   * improved nodes are queued by the wave that improved them, with one counter
+//     atomic per wave or workgroup, which replaces setNV's O(N) scan;
+//   * termination is decided on the device: once no open entry can lead to
+//     anything below F(t) (GA_v2.cu:277-289, 547-557).
+// Stale entries (a node improved after it was queued) are skipped when they are
+// taken; this replaces keepHeapPQ's in-place decrease-key repair.
 #include <algorithm>
 #include <chrono>
 #include <cstring>
@@ -38,7 +29,7 @@
 namespace {
 
 enum : uint32_t {
-    ERR_HEAP = GA_ERR_HEAP, ERR_PBUF = GA_ERR_PBUF, ERR_ITERS = GA_ERR_ITERS, ERR_BARRIER = GA_ERR_BARRIER,
+    ERR_HEAP = GA_ERR_HEAP, ERR_ITERS = GA_ERR_ITERS, ERR_BARRIER = GA_ERR_BARRIER,
     ERR_PATH = 16
 };
 
@@ -240,10 +231,9 @@ int ddp_ga_plan(ddp_ctx *ctx, const ddp_graph *g, const ddp_astar_opts_t *o, GaG
         }
         return DDP_OK;
     }
-    // the widest grids on wide workgroups: fewer workgroups make each
-    // device-wide barrier cheaper.  One R-MAT scale-23 search: K = 65,536 took
-    // 33 ms on 64 workgroups of 1,024 lanes and 42 ms on 256 of 256; K = 32,768
-    // took 37 ms on 128 of 256 lanes and 41 ms on 32 of 1,024.
+    // Grid mode's workgroups have 1,024 lanes whatever B is (pg_workgroups): B, given
+    // or by these steps, is what K is rounded up to and bounded by, as callers
+    // that sized K for lane heaps know it.
     if (B == 0) B = K >= 65536 ? 1024 : K >= 4096 ? 256 : 64;
     DDP_CHECK(B == 64 || B == 256 || B == 1024, ctx, DDP_ERR_ARG,
               "block must be 64, 256 or 1024 (got %d)", B);
@@ -255,6 +245,7 @@ int ddp_ga_plan(ddp_ctx *ctx, const ddp_graph *g, const ddp_astar_opts_t *o, GaG
     int64_t cap = (o && o->heap_cap) ? o->heap_cap : (2 * (int64_t)g->N + K - 1) / K + 256;
     cap = std::max<int64_t>(cap, lcap);
     DDP_CHECK(cap < (1 << 30), ctx, DDP_ERR_ARG, "heap_cap too large");
+    // room for a DA* batch's pushes (and, with E close to 2^31, a refusal of its own)
     int64_t pcap = (int64_t)K * std::max(1, g->maxdeg) + K;
     pcap = std::min<int64_t>(pcap, (int64_t)g->E + 2 * (int64_t)K + 64);
     pcap = std::max<int64_t>(pcap, std::max<int64_t>(1024, min_pcap));
@@ -265,9 +256,9 @@ int ddp_ga_plan(ddp_ctx *ctx, const ddp_graph *g, const ddp_astar_opts_t *o, GaG
     p->edges = g->E;
     p->hubcap = (uint32_t)((int64_t)g->E / kPgSeg + kPgRound + 64);
     p->delta0 = std::max<uint32_t>(1, g->meanw);
-    // K is bounded by the queues whose tops and expansion tables the device
-    // could hold at once, as callers know it (the piles themselves need no LDS
-    // per queue): workgroups of B lanes per CU by LDS and by 20 waves.
+    // The bound on K is part of the interface, not a limit of the piles (which
+    // need no LDS per queue): the lane heaps of K queues that the device could
+    // hold at once, in workgroups of B lanes, 20 waves a CU at most.
     const size_t lds = (size_t)lcap * B * 8 + 48 * (size_t)B + 392;
     const int per_cu = (int)std::min<size_t>(ctx->prop.maxSharedMemoryPerMultiProcessor / lds, 20 * 64 / B);
     DDP_CHECK((int64_t)per_cu * ctx->prop.multiProcessorCount >= nblocks, ctx, DDP_ERR_ARG,
@@ -406,7 +397,6 @@ int grid_finish(ddp_ctx *ctx, const GaGridPlan &P, const GaGridState &S, uint32_
     DDP_CHECK(!(err & ERR_ITERS), ctx, DDP_ERR_TIMEOUT, "GA*: iteration limit %d reached", P.maxit);
     DDP_CHECK(!(err & ERR_HEAP), ctx, DDP_ERR_OVERFLOW,
               "GA*: a queue exceeded heap_cap=%d entries; raise heap_cap", P.cap);
-    DDP_CHECK(!(err & ERR_PBUF), ctx, DDP_ERR_OVERFLOW, "GA*: push buffer (%d entries) overflowed", P.pcap);
     return DDP_OK;
 }
 

@@ -14,8 +14,8 @@
 // have gone stale since).  As in the slots this is a label-correcting search:
 // an entry is dropped only when it is stale or cannot lead to anything below
 // F(t), so the cost is exact for an admissible heuristic.  K sets the window:
-// a width that fed fewer than K entries doubles, one that fed more than 8K
-// halves.
+// a width that fed fewer than K entries, or few a round (kPgFeed), doubles, one
+// that fed more than 8K halves.
 //
 // Why piles and not the K lane heaps this replaced: a heap pop is a chain of
 // dependent LDS and HBM accesses (8 us an iteration on the 100,000-node random
@@ -24,8 +24,10 @@
 // workgroup with the hub), and K lanes were all the parallelism there was.
 // Measured, whole call, heaps and piles: random graph of 100,000 nodes, K = 1,024,
 // 1.5-3.1 and 0.39-0.43 ms; R-MAT scale 20, K = 16,384, 9.8-11.2 and 2.0-2.9 ms;
-// 2,048 x 2,048 maze, K = 512, 49.1 and 26.0 ms.  What is left is latency: a
-// round is seven dependent round trips and a barrier, 6 us.
+// 4,096 x 4,096 maze, K = 1,024, 26 and 18.7 ms.  What is left is latency: a round
+// is six dependent round trips (the entry; its word, row and heuristic input;
+// its edges; their ends' words and inputs; the atomics; places in the piles)
+// and a barrier, 6 us.
 //
 // RESUME (DA*): the search starts from an open set -- the first entries of far0,
 // counted on the device -- with F(t) read from the target's word, and a current

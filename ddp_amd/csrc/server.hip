@@ -647,7 +647,7 @@ __global__ void serve_grid_finish(const uint32_t *gctrl, const uint64_t *stamp, 
 {
     if (threadIdx.x != 0) return;
     const uint32_t err = gctrl[GA_RES_ERR];
-    const int32_t status = ((err & (GA_ERR_HEAP | GA_ERR_PBUF)) ? 1 : 0) | ((err & GA_ERR_ITERS) ? 2 : 0) |
+    const int32_t status = ((err & GA_ERR_HEAP) ? 1 : 0) | ((err & GA_ERR_ITERS) ? 2 : 0) |
                            ((err & GA_ERR_BARRIER) ? 8 : 0);
     __hip_atomic_store(&r->cost, (int32_t)gctrl[GA_RES_F], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __hip_atomic_store(&r->status, status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -999,8 +999,8 @@ extern "C" int ddp_server_create(ddp_ctx *ctx, const ddp_graph *g, ddp_heur_t h,
         ddp_astar_opts_t ao{};
         ao.K = grid_k;
         if ((rc = ddp_ga_plan(ctx, g, &ao, &sv->gplan))) return fail(rc);
-        // room for 8N queued entries over the K heaps (a hub-heavy graph pushes
-        // each node several times over a full search)
+        // 8N entries over the piles: a hub-heavy graph queues each node several
+        // times over a full search
         sv->gplan.cap = (int32_t)std::max<int64_t>(sv->gplan.cap, (8LL * g->N + sv->gplan.K - 1) / sv->gplan.K);
         if ((rc = ddp_ga_alloc_owned(ctx, g->N, sv->gplan, &sv->gstate))) return fail(rc);
         hipError_t ge = hipMalloc((void **)&sv->gstamp, 64);
