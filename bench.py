@@ -363,7 +363,7 @@ def run_c1(args):
     res.update({"kernel_ms": round(kms, 3), "iterations": st["iterations"], "expansions": st["expansions"],
                 "expansions_per_s": round(st["expansions"] / (kms * 1e-3), 1),
                 "edges_per_s": round(st["edges"] / (kms * 1e-3), 1),
-                "roofline": roofline(abytes, kms, "ga_grid_kernel"),
+                "roofline": roofline(abytes, kms, "ga_piles_kernel"),
                 "cpu_baseline": {"value": round(reps / el, 3), "unit": "queries/s", "cores": 1, "kind": "port",
                                  "sample": f"the same query {reps} times, oracle restatement of A_star_cpu.cpp"}})
     ctx.close()
