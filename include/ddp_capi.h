@@ -138,7 +138,10 @@ typedef struct {
  * (needs DDP_GRAPH_REVERSE), i.e. hops from v to t in g.
  * If store_as_h != 0 the result also becomes g's DDP_H_ARRAY heuristic
  * without a host round trip.  h_out may be NULL.  *levels_out (optional) gets
- * the number of BFS levels. */
+ * the number of BFS levels.  Other work may hold part of the GPU meanwhile
+ * (another context's server, say): the widest levels run on the workgroups that
+ * find room within 100 us.  The narrow ones need room for 32 workgroups of 256
+ * lanes; without it the call ends with DDP_ERR_TIMEOUT after 20 s. */
 int ddp_bfs_hops(ddp_ctx *ctx, ddp_graph *g, int32_t t, int32_t reverse,
                  int32_t scale, int32_t store_as_h, int32_t *h_out,
                  int32_t *levels_out);
@@ -167,7 +170,10 @@ typedef struct {
     int32_t block;      /* lanes per workgroup; grid mode: 64, 256 or 1024 (rounds K up to a
                            multiple; the grid's own workgroups have 1,024 lanes); 0 = auto
                            (grid mode: 64 below K = 4096, 256 below 65536, 1024 from there) */
-    int32_t heap_cap;   /* entries per queue (grid mode: K * heap_cap in all); 0 = auto */
+    int32_t heap_cap;   /* entries per queue; 0 = auto.  Grid mode: its piles take no more than
+                           the larger of K * heap_cap and 8N entries of 8 bytes, and K * heap_cap
+                           limits a search only below 2N (from there on, and so by default,
+                           piles that overflow are rebuilt from the nodes' words) */
     int32_t lds_cap;    /* heap entries per queue kept in LDS; 0 = auto */
     int32_t max_iters;  /* iteration limit; 0 = auto (bounded) */
     int32_t mode;       /* DDP_ASTAR_AUTO / _GRID / _WORKGROUP / _PILES / _BIDI */
@@ -175,8 +181,10 @@ typedef struct {
 } ddp_astar_opts_t;
 
 /* Execution modes of the single-query search.  GRID runs near/far piles over
- * the whole GPU: 64 workgroups, or one per CU on large graphs without a
- * geometric heuristic, that meet at a device-wide barrier every round.
+ * the whole GPU: 16 workgroups below 131,072 edges, one per CU on graphs of
+ * 4,194,304 edges and more without a geometric heuristic, 64 otherwise, that
+ * meet at a device-wide barrier every round.  Other work may hold part of the GPU
+ * meanwhile: the workgroups that find room within 100 us do the search.
  * WORKGROUP keeps all K <= 1024 queues in one workgroup (block = K rounded up
  * to a power of two >= 64): no device-wide barrier, but one CU's worth of
  * memory parallelism.  PILES runs the search on one workgroup of K <= 1024
@@ -203,7 +211,7 @@ typedef struct {
     int32_t iterations;     /* rounds: one pop per queue, or up to K (lanes) near entries */
     int32_t K;              /* queues used */
     int32_t block;          /* lanes per workgroup used */
-    int32_t blocks;         /* workgroups used */
+    int32_t blocks;         /* workgroups launched */
     float kernel_ms;        /* search kernel time (HIP events, ctx stream) */
     float total_ms;         /* entry point wall time */
 } ddp_astar_stats_t;
