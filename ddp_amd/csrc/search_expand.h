@@ -10,7 +10,7 @@
 // inputs and (f, parent) words), so R independent memory round trips overlap.
 //
 // Edges that beat their node's word are few (5% on R-MAT, a fifth on a road
-// map), so a wave collects them in LDS and relaxes and queues 64 at a time.
+// map), so a wave collects them in LDS and relaxes and queues 64 (128 up to 512 lanes) at a time.
 // Not for the lane-owned heaps: their pushes have to stay spread over the
 // lanes (collected, the C4 batch overflowed heaps of 2,048 entries, and with
 // the lanes taking turns it took 96-117 ms instead of 79).
